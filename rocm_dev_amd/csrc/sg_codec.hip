@@ -37,14 +37,17 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// One workgroup per row.  Thread t holds chunks t, t+T, ... of 8 bf16 each (CH of them),
-// so the row is read from memory exactly once.
-template <int CH>
-__global__ void __launch_bounds__(256) fp8_encode_rows_kernel(const uint16_t* __restrict__ X, uint8_t* __restrict__ Q,
-                                                              float* __restrict__ scales, int cols) {
-    __shared__ float wmax[4];
+// A row is held in registers, so it is read from memory exactly once: thread t of the THREADS that share a row holds
+// its chunks t, t + THREADS, ... of 8 bf16 each, CH of them.  HBM-bound at 3 bytes per element (30.5 us for 8192 x 8192 at
+// the 6.6 TB/s a stream reaches, measured 33.4); what a row shape can lose on top is idle lanes, workgroup launches and
+// the reduction of the maximum, which is why there is one build per range of row lengths (launch_fp8_encode_rows).
+//
+// One workgroup per row, the maximum through LDS.
+template <int THREADS, int CH>
+__global__ void __launch_bounds__(THREADS) fp8_encode_row_kernel(const uint16_t* __restrict__ X, uint8_t* __restrict__ Q,
+                                                                 float* __restrict__ scales, int cols) {
+    __shared__ float wmax[THREADS / 64];
     const int row = blockIdx.x;
-    const int T = blockDim.x;
     const int t = threadIdx.x;
     const int nchunks = cols >> 3;
     const u32x4* xrow = reinterpret_cast<const u32x4*>(X + (size_t)row * cols);
@@ -52,109 +55,110 @@ __global__ void __launch_bounds__(256) fp8_encode_rows_kernel(const uint16_t* __
     u32x4 raw[CH];
 #pragma unroll
     for (int c = 0; c < CH; c++) {
-        const int idx = c * T + t;
         raw[c] = u32x4{0u, 0u, 0u, 0u};
-        if (idx < nchunks) raw[c] = __builtin_nontemporal_load(xrow + idx);
+        if (c * THREADS + t < nchunks) raw[c] = __builtin_nontemporal_load(xrow + c * THREADS + t);
     }
-
     float amax = 0.0f;
 #pragma unroll
     for (int c = 0; c < CH; c++) amax = absmax8_bf16(raw[c], amax);
     amax = wave_max(amax);
-    const int nw = T >> 6;
-    if (nw > 1) {
-        if (lane_id() == 0) wmax[threadIdx.x >> 6] = amax;
+    if (THREADS > 64) {
+        if (lane_id() == 0) wmax[t >> 6] = amax;
         __syncthreads();
         amax = wmax[0];
-        for (int w = 1; w < nw; w++) amax = fmaxf(amax, wmax[w]);
+#pragma unroll
+        for (int w = 1; w < THREADS / 64; w++) amax = fmaxf(amax, wmax[w]);
     }
-
     const RowQuant rq = row_quant(amax);
     if (t == 0) scales[row] = rq.s;
-
     u32x2* qrow = reinterpret_cast<u32x2*>(Q + (size_t)row * cols);
 #pragma unroll
-    for (int c = 0; c < CH; c++) {
-        const int idx = c * T + t;
-        const u32x2 out = quantize8_bf16(raw[c], rq);
-        if (idx < nchunks) __builtin_nontemporal_store(out, qrow + idx);
-    }
+    for (int c = 0; c < CH; c++)
+        if (c * THREADS + t < nchunks) __builtin_nontemporal_store(quantize8_bf16(raw[c], rq), qrow + c * THREADS + t);
 }
 
-// Rows too long to hold in registers: two passes over the row (the second mostly from L2).
-__global__ void __launch_bounds__(256) fp8_encode_rows_long_kernel(const uint16_t* __restrict__ X, uint8_t* __restrict__ Q,
-                                                                   float* __restrict__ scales, int cols) {
-    __shared__ float wmax[4];
+// Short rows: LANES lanes of a wave (a power of two) share a row, 256 / LANES rows per workgroup, the maximum by
+// shuffles.  A workgroup per row spends a launch of its own and most of a wave's lanes on them: 16384 rows of 16 / 64 /
+// 240 / 512 columns 8.7 / 7.9 / 8.3 / 8.7 us that way, 2.7 / 3.2 / 4.8 / 6.6 this way.
+template <int LANES, int CH>
+__global__ void __launch_bounds__(256) fp8_encode_short_rows_kernel(const uint16_t* __restrict__ X, uint8_t* __restrict__ Q,
+                                                                    float* __restrict__ scales, int rows, int cols) {
+    const unsigned row = blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    const int t = (int)threadIdx.x % LANES;
+    const int nchunks = row < (unsigned)rows ? cols >> 3 : 0;      // lanes past the last row take part in the shuffles only
+    const u32x4* xrow = reinterpret_cast<const u32x4*>(X + (size_t)row * cols);
+    u32x4 raw[CH];
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        raw[c] = u32x4{0u, 0u, 0u, 0u};
+        if (c * LANES + t < nchunks) raw[c] = __builtin_nontemporal_load(xrow + c * LANES + t);
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CH; c++) amax = absmax8_bf16(raw[c], amax);
+#pragma unroll
+    for (int o = LANES / 2; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+    const RowQuant rq = row_quant(amax);
+    if (t == 0 && row < (unsigned)rows) scales[row] = rq.s;
+    u32x2* qrow = reinterpret_cast<u32x2*>(Q + (size_t)row * cols);
+#pragma unroll
+    for (int c = 0; c < CH; c++)
+        if (c * LANES + t < nchunks) __builtin_nontemporal_store(quantize8_bf16(raw[c], rq), qrow + c * LANES + t);
+}
+
+// Rows too long to hold in registers (more than 65536 columns): two passes over the row (the second mostly from L2).
+__global__ void __launch_bounds__(1024) fp8_encode_rows_long_kernel(const uint16_t* __restrict__ X, uint8_t* __restrict__ Q,
+                                                                    float* __restrict__ scales, int cols) {
+    __shared__ float wmax[16];
     const int row = blockIdx.x;
     const int t = threadIdx.x;
     const int nchunks = cols >> 3;
     const u32x4* xrow = reinterpret_cast<const u32x4*>(X + (size_t)row * cols);
     float amax = 0.0f;
-    for (int idx = t; idx < nchunks; idx += 256) {
-        const u32x4 raw = xrow[idx];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            amax = fmaxf(amax, fabsf(bf16_lo(raw[j])));
-            amax = fmaxf(amax, fabsf(bf16_hi(raw[j])));
-        }
-    }
+    for (int idx = t; idx < nchunks; idx += 1024) amax = absmax8_bf16(xrow[idx], amax);
     amax = wave_max(amax);
-    if (lane_id() == 0) wmax[threadIdx.x >> 6] = amax;
+    if (lane_id() == 0) wmax[t >> 6] = amax;
     __syncthreads();
-    amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-    const float s = (amax == 0.0f) ? 1.0f : __fdiv_rn(amax, 448.0f);
-    if (t == 0) scales[row] = s;
-    u32x2* qrow = reinterpret_cast<u32x2*>(Q + (size_t)row * cols);
-    for (int idx = t; idx < nchunks; idx += 256) {
-        const u32x4 raw = xrow[idx];
-        float q[8];
+    amax = wmax[0];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            q[2 * j] = __fdiv_rn(bf16_lo(raw[j]), s);
-            q[2 * j + 1] = __fdiv_rn(bf16_hi(raw[j]), s);
-        }
-        int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
-        w0 = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], w0, true);
-        int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], 0, false);
-        w1 = __builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], w1, true);
-        qrow[idx] = u32x2{canonical_nan_codes(w0), canonical_nan_codes(w1)};
-    }
+    for (int w = 1; w < 16; w++) amax = fmaxf(amax, wmax[w]);
+    const RowQuant rq = row_quant(amax);
+    if (t == 0) scales[row] = rq.s;
+    u32x2* qrow = reinterpret_cast<u32x2*>(Q + (size_t)row * cols);
+    for (int idx = t; idx < nchunks; idx += 1024) qrow[idx] = quantize8_bf16(xrow[idx], rq);
 }
 
-// 16 codes per thread: one 16-byte load, two 16-byte stores.  cols % 16 == 0, so a chunk
-// never straddles two rows.
+// Eight codes per thread: one 8-byte load, one 16-byte store, both contiguous over a wave, the store non-temporal.
+// (8192 x 8192: 33.3 us; with 16 codes a thread the two stores of a lane interleave at 32 bytes and the launch takes 37.8,
+// and the 64-bit division for the row, now a multiply-high, another 0.3.)  cols % 16 == 0: no chunk straddles two rows.
 __global__ void __launch_bounds__(256) fp8_decode_rows_kernel(const uint8_t* __restrict__ Q, const float* __restrict__ scales,
-                                                              uint16_t* __restrict__ Y, int cols, size_t nchunks) {
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+                                                              uint16_t* __restrict__ Y, unsigned chunks_per_row,
+                                                              unsigned inv_chunks_per_row, unsigned nchunks) {
+    const unsigned idx = blockIdx.x * 256 + threadIdx.x;
     if (idx >= nchunks) return;
-    const int chunks_per_row = cols >> 4;
-    const int row = (int)(idx / chunks_per_row);
-    const float s = scales[row];
-    const u32x4 q = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(Q) + idx);
-    u32x4 o[2];
+    const float s = scales[fast_div(idx, chunks_per_row, inv_chunks_per_row)];
+    const u32x2 q = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(Q) + idx);
+    u32x4 o;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < 2; j++) {
         const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8(q[j], false);
         const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8(q[j], true);
-        o[j >> 1][2 * (j & 1)] = cvt_bf16x2(__fmul_rn(lo.x, s), __fmul_rn(lo.y, s));
-        o[j >> 1][2 * (j & 1) + 1] = cvt_bf16x2(__fmul_rn(hi.x, s), __fmul_rn(hi.y, s));
+        o[2 * j] = cvt_bf16x2(__fmul_rn(lo.x, s), __fmul_rn(lo.y, s));
+        o[2 * j + 1] = cvt_bf16x2(__fmul_rn(hi.x, s), __fmul_rn(hi.y, s));
     }
-    // plain stores: with 32 bytes per lane the non-temporal hint costs a third of the bandwidth
-    // (measured 3.9 vs 6.0 TB/s for this 1-read : 2-write pattern)
-    u32x4* y = reinterpret_cast<u32x4*>(Y) + 2 * idx;
-    y[0] = o[0];
-    y[1] = o[1];
+    __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(Y) + idx);
 }
 
+// NBUF > 0: all buffers' codes requested before any is added; 0: any number, one after the other.
 template <int NBUF>
 __global__ void __launch_bounds__(256) fp8_reduce_rows_kernel(const uint8_t* __restrict__ Q, const float* __restrict__ scales,
                                                               uint16_t* __restrict__ Y, int nbuf_rt, size_t q_buf_stride,
-                                                              int rows, int cols, size_t nchunks) {
-    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+                                                              size_t s_buf_stride, unsigned chunks_per_row,
+                                                              unsigned inv_chunks_per_row, unsigned nchunks) {
+    const unsigned idx = blockIdx.x * 256 + threadIdx.x;
     if (idx >= nchunks) return;
     const int nbuf = NBUF > 0 ? NBUF : nbuf_rt;
-    const int chunks_per_row = cols >> 4;
-    const int row = (int)(idx / chunks_per_row);
+    const unsigned row = fast_div(idx, chunks_per_row, inv_chunks_per_row);
     float acc[16];
 #pragma unroll
     for (int e = 0; e < 16; e++) acc[e] = 0.0f;
@@ -177,14 +181,14 @@ __global__ void __launch_bounds__(256) fp8_reduce_rows_kernel(const uint8_t* __r
 #pragma unroll
         for (int b = 0; b < NBUF; b++) {
             q[b] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(Q + (size_t)b * q_buf_stride) + idx);
-            s[b] = scales[(size_t)b * rows + row];
+            s[b] = scales[(size_t)b * s_buf_stride + row];
         }
 #pragma unroll
         for (int b = 0; b < NBUF; b++) accumulate(q[b], s[b]);
     } else {
         for (int b = 0; b < nbuf; b++) {
             const u32x4 q = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(Q + (size_t)b * q_buf_stride) + idx);
-            accumulate(q, scales[(size_t)b * rows + row]);
+            accumulate(q, scales[(size_t)b * s_buf_stride + row]);
         }
     }
 
@@ -192,8 +196,8 @@ __global__ void __launch_bounds__(256) fp8_reduce_rows_kernel(const uint8_t* __r
 #pragma unroll
     for (int j = 0; j < 8; j++) o[j >> 2][j & 3] = cvt_bf16x2(acc[2 * j], acc[2 * j + 1]);
     // plain stores: with 32 bytes per lane the non-temporal hint costs a third of the bandwidth
-    // (measured 3.9 vs 6.0 TB/s for this 1-read : 2-write pattern)
-    u32x4* y = reinterpret_cast<u32x4*>(Y) + 2 * idx;
+    // (measured 3.9 vs 6.0 TB/s for a 1-read : 2-write pattern)
+    u32x4* y = reinterpret_cast<u32x4*>(Y) + 2 * (size_t)idx;
     y[0] = o[0];
     y[1] = o[1];
 }
@@ -205,25 +209,56 @@ int launch_fp8_encode_rows(const void* X, uint8_t* Q, float* scales, int rows, i
     if (!aligned16(X) || !aligned16(Q)) return SG_BAD_ALIGNMENT;
     const int nchunks = cols >> 3;
     const uint16_t* x = reinterpret_cast<const uint16_t*>(X);
-    int threads = 256;
-    if (nchunks <= 64) threads = 64;
-    else if (nchunks <= 128) threads = 128;
-    const int ch = (nchunks + threads - 1) / threads;
-    if (ch <= 1) fp8_encode_rows_kernel<1><<<rows, threads, 0, stream>>>(x, Q, scales, cols);
-    else if (ch <= 2) fp8_encode_rows_kernel<2><<<rows, threads, 0, stream>>>(x, Q, scales, cols);
-    else if (ch <= 4) fp8_encode_rows_kernel<4><<<rows, threads, 0, stream>>>(x, Q, scales, cols);
-    else if (ch <= 8) fp8_encode_rows_kernel<8><<<rows, threads, 0, stream>>>(x, Q, scales, cols);
-    else fp8_encode_rows_long_kernel<<<rows, 256, 0, stream>>>(x, Q, scales, cols);
+#define SG_SHORT(LANES, CH) \
+    fp8_encode_short_rows_kernel<LANES, CH><<<((unsigned)rows + 256 / LANES - 1) / (256 / LANES), 256, 0, stream>>>(x, Q, scales, rows, cols)
+#define SG_ROW(THREADS, CH) fp8_encode_row_kernel<THREADS, CH><<<rows, THREADS, 0, stream>>>(x, Q, scales, cols)
+    // The smallest group of threads that holds the row in two chunks each (from 32 columns on), lanes of a shared wave up
+    // to 512 columns and a workgroup beyond; with many rows fewer threads of four chunks from 8192 columns on.  us, cold,
+    // against 64 / 128 / 256 threads a row as many as needed: 16384 x 1024 16.4 -> 10.0, 16384 x 2048 27.9 -> 18.0,
+    // 8192 x 4096 19.1 -> 18.7, 1024 x 8192 6.7 -> 6.4, 16 x 14336 4.3 -> 3.6, 2048 x 16384 19.8 -> 18.9; above 16384
+    // columns against two passes over the row: 512 x 32768 22.7 -> 10.4, 64 x 65536 29.4 -> 7.8.
+    if (nchunks <= 2) SG_SHORT(2, 1);
+    else if (nchunks <= 4) SG_SHORT(4, 1);
+    else if (nchunks <= 8) SG_SHORT(8, 1);
+    else if (nchunks <= 16) SG_SHORT(16, 1);
+    else if (nchunks <= 32) SG_SHORT(16, 2);
+    else if (nchunks <= 64) SG_SHORT(32, 2);
+    else if (nchunks <= 128) SG_ROW(64, 2);
+    else if (nchunks <= 256) SG_ROW(128, 2);
+    else if (nchunks <= 512) SG_ROW(256, 2);
+    else if (nchunks <= 1024 && rows <= 2048) SG_ROW(512, 2);
+    else if (nchunks <= 1024) SG_ROW(256, 4);
+    else if (nchunks <= 2048 && rows <= 256) SG_ROW(1024, 2);
+    else if (nchunks <= 2048) SG_ROW(512, 4);
+    else if (nchunks <= 4096) SG_ROW(1024, 4);
+    else if (nchunks <= 8192) SG_ROW(1024, 8);
+    else fp8_encode_rows_long_kernel<<<rows, 1024, 0, stream>>>(x, Q, scales, cols);
+#undef SG_SHORT
+#undef SG_ROW
     return hipGetLastError() == hipSuccess ? SG_SUCCESS : SG_LAUNCH_FAILED;
+}
+
+// The decode and reduce kernels count chunks in 32 bits: a larger matrix goes in slabs of whole rows, at most 2^30 chunks
+// each.  launch(first row, rows) enqueues one slab.
+template <class Launch>
+static int in_slabs(int rows, unsigned chunks_per_row, Launch&& launch) {
+    const size_t slab = 0x40000000u / chunks_per_row;   // (cols is an int: at least four rows)
+    for (size_t r0 = 0; r0 < (size_t)rows; r0 += slab) {
+        launch(r0, (size_t)rows - r0 < slab ? (size_t)rows - r0 : slab);
+        if (hipGetLastError() != hipSuccess) return SG_LAUNCH_FAILED;
+    }
+    return SG_SUCCESS;
 }
 
 int launch_fp8_decode_rows(const uint8_t* Q, const float* scales, void* Y, int rows, int cols, hipStream_t stream) {
     if (!Q || !scales || !Y || rows <= 0 || cols <= 0 || (cols & 15)) return SG_BAD_ARGUMENT;
     if (!aligned16(Q) || !aligned16(Y)) return SG_BAD_ALIGNMENT;
-    const size_t nchunks = (size_t)rows * (cols >> 4);
-    const unsigned grid = (unsigned)((nchunks + 255) / 256);
-    fp8_decode_rows_kernel<<<grid, 256, 0, stream>>>(Q, scales, reinterpret_cast<uint16_t*>(Y), cols, nchunks);
-    return hipGetLastError() == hipSuccess ? SG_SUCCESS : SG_LAUNCH_FAILED;
+    const unsigned per_row = (unsigned)cols >> 3, inv = div_reciprocal(per_row);
+    return in_slabs(rows, per_row, [&](size_t r0, size_t nrows) {
+        const unsigned nchunks = (unsigned)nrows * per_row;
+        fp8_decode_rows_kernel<<<(nchunks + 255) / 256, 256, 0, stream>>>(
+            Q + r0 * (size_t)cols, scales + r0, reinterpret_cast<uint16_t*>(Y) + r0 * (size_t)cols, per_row, inv, nchunks);
+    });
 }
 
 int launch_fp8_reduce_rows(const uint8_t* Q, const float* scales, void* Y, int nbuf, size_t q_buf_stride, int rows,
@@ -231,18 +266,27 @@ int launch_fp8_reduce_rows(const uint8_t* Q, const float* scales, void* Y, int n
     if (!Q || !scales || !Y || nbuf <= 0 || rows <= 0 || cols <= 0 || (cols & 15)) return SG_BAD_ARGUMENT;
     if (!aligned16(Q) || !aligned16(Y) || (q_buf_stride & 15)) return SG_BAD_ALIGNMENT;
     if (nbuf > 1 && q_buf_stride < (size_t)rows * cols) return SG_BAD_ARGUMENT;
-    const size_t nchunks = (size_t)rows * (cols >> 4);
-    const unsigned grid = (unsigned)((nchunks + 255) / 256);
-    uint16_t* y = reinterpret_cast<uint16_t*>(Y);
-    if (nbuf == 8)
-        fp8_reduce_rows_kernel<8><<<grid, 256, 0, stream>>>(Q, scales, y, nbuf, q_buf_stride, rows, cols, nchunks);
-    else if (nbuf == 4)
-        fp8_reduce_rows_kernel<4><<<grid, 256, 0, stream>>>(Q, scales, y, nbuf, q_buf_stride, rows, cols, nchunks);
-    else if (nbuf == 2)
-        fp8_reduce_rows_kernel<2><<<grid, 256, 0, stream>>>(Q, scales, y, nbuf, q_buf_stride, rows, cols, nchunks);
-    else
-        fp8_reduce_rows_kernel<0><<<grid, 256, 0, stream>>>(Q, scales, y, nbuf, q_buf_stride, rows, cols, nchunks);
-    return hipGetLastError() == hipSuccess ? SG_SUCCESS : SG_LAUNCH_FAILED;
+    const unsigned per_row = (unsigned)cols >> 4, inv = div_reciprocal(per_row);
+    return in_slabs(rows, per_row, [&](size_t r0, size_t nrows) {
+        const unsigned nchunks = (unsigned)nrows * per_row;
+        const unsigned grid = (nchunks + 255) / 256;
+        const uint8_t* q = Q + r0 * (size_t)cols;
+        uint16_t* y = reinterpret_cast<uint16_t*>(Y) + r0 * (size_t)cols;
+#define SG_REDUCE(NBUF) \
+    fp8_reduce_rows_kernel<NBUF><<<grid, 256, 0, stream>>>(q, scales + r0, y, nbuf, q_buf_stride, (size_t)rows, per_row, inv, nchunks)
+        switch (nbuf) {
+            case 1: SG_REDUCE(1); break;
+            case 2: SG_REDUCE(2); break;
+            case 3: SG_REDUCE(3); break;
+            case 4: SG_REDUCE(4); break;
+            case 5: SG_REDUCE(5); break;
+            case 6: SG_REDUCE(6); break;
+            case 7: SG_REDUCE(7); break;
+            case 8: SG_REDUCE(8); break;
+            default: SG_REDUCE(0); break;
+        }
+#undef SG_REDUCE
+    });
 }
 
 }  // namespace sg

@@ -181,6 +181,42 @@ def test_tiled_sum_reduce_lds_queue_short_batches(sg, oracle, b):
         assert np.array_equal(D.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 16), (129, 16), (65, 32), (33, 48), (31, 64), (17, 80), (16, 128), (9, 144), (15, 256), (7, 272),
+                                       (9, 512), (3, 528), (2, 1024), (2, 1040), (2, 2048), (2, 2064), (3, 4096), (2, 4112), (2049, 4112),
+                                       (2, 8192), (257, 8208), (2, 8208), (2, 16400), (2, 32768), (2, 32784), (2, 65536), (2, 65552)])
+def test_codec_row_length_ranges(sg, oracle, rows, cols):
+    """Every build of the encoder at the shortest and longest rows it takes (lanes of a shared wave, one workgroup per row,
+    two passes), with a row count that leaves the last workgroup partly filled, and the decoder and the one-buffer reduce on
+    the result; bit for bit, and nothing beyond the outputs is written."""
+    X = oracle.normal_bf16_outliers((rows, cols), seed=cols, stream_id=3, frac=0.01, mag=50.0)
+    X[-1, -1] = 0x4416                                       # 600: the maximum in the last chunk of the last row
+    Xd = dev(X)
+    Q = torch.full((rows + 1, cols), 0xEE, dtype=torch.uint8, device="cuda")
+    S = torch.full((rows + 1,), -1.0, dtype=torch.float32, device="cuda")
+    assert sg.fp8_encode_rows(Xd, Q[:rows], S[:rows]) == 0
+    q_ref, s_ref = oracle.fp8_encode_rows(X)
+    assert np.array_equal(Q[:rows].cpu().numpy(), q_ref) and torch.all(Q[rows] == 0xEE)
+    assert np.array_equal(S[:rows].cpu().numpy(), s_ref) and S[rows].item() == -1.0
+    Y = torch.full((rows + 1, cols), 7.0, dtype=torch.bfloat16, device="cuda")
+    want = oracle.fp8_decode_rows(q_ref, s_ref)
+    assert sg.fp8_decode_rows(Q[:rows], S[:rows], Y[:rows]) == 0
+    assert np.array_equal(bits(Y[:rows]), want) and torch.all(Y[rows] == 7.0)
+    Y[:rows] = 0
+    assert sg.fp8_reduce_rows(Q[None, :rows], S[None, :rows], Y[:rows]) == 0
+    assert np.array_equal(bits(Y[:rows]), oracle.fp8_reduce_rows(q_ref[None], s_ref[None])) and torch.all(Y[rows] == 7.0)
+
+
+@pytest.mark.parametrize("nbuf", [6, 7, 8, 9])
+def test_reduce_more_counts(sg, oracle, nbuf):
+    """The builds for six to eight buffers and the loop for more."""
+    rows, cols = 19, 272
+    pairs = [oracle.fp8_encode_rows(oracle.normal_bf16_outliers((rows, cols), seed=20 + i, stream_id=3)) for i in range(nbuf)]
+    q_ref, s_ref = np.stack([p[0] for p in pairs]), np.stack([p[1] for p in pairs])
+    Y = torch.empty((rows, cols), dtype=torch.bfloat16, device="cuda")
+    assert sg.fp8_reduce_rows(dev(q_ref), dev(s_ref), Y) == 0
+    assert np.array_equal(bits(Y), oracle.fp8_reduce_rows(q_ref, s_ref))
+
+
 def test_encode_special_values_bit_exact(sg, oracle):
     """Infinities, NaNs, denormals and signed zeros: same codes and scales as the oracle (whose values for these rows
     are pinned in closed form by tests/test_oracle_gemm.py), and the decoder turns them back bit for bit."""
