@@ -16,7 +16,7 @@ import enum
 
 import torch
 
-from ._lib import lib
+from ._lib import host, lib
 
 
 class SgReturnCode(enum.IntEnum):
@@ -64,6 +64,9 @@ def _dev(t, *dtypes):
 
 _FP8 = (torch.uint8, torch.float8_e4m3fn)
 
+# The entry points that programs call per layer first offer their operands to the extension module (`host`), which
+# launches plain ones in a few hundred nanoseconds and returns None for everything else - other devices, layouts the
+# kernels would misread, tensor subclasses.  What follows the offer is the complete rule, and the error message.
 
 # The C ABI takes raw pointers with the shapes it is told: everything it will assume about a tensor is checked here,
 # before the call - a transposed or sliced operand would otherwise be read with the wrong strides, and a weight matrix
@@ -134,6 +137,9 @@ def skinny_gemm(A, B, D, scale_tensor, split_k, A_producers, B_producers, consum
 
 def skinny_gemm_fastpath(A, B, D, scale_tensor, check=False):
     """Library-chosen configuration; B is [n, k] (row stride taken from the tensor)."""
+    rc = host.skinny_gemm_fastpath(A, B, D, scale_tensor)
+    if rc is not None:
+        return _done(rc, check)
     m, n, k, b_stride = _gemm_operands(A, B, D, scale_tensor)
     with torch.cuda.device(A.device):
         rc = lib.sg_skinny_gemm_auto(_dev(A, *_FP8), _dev(B, *_FP8), _dev(D, torch.bfloat16),
@@ -158,6 +164,9 @@ def tuning_as_dict(t):
 
 def skinny_gemm_rowcol(A, B, D, scale_tensor=None, row_scales=None, col_scales=None, check=False):
     """D = bf16(((A @ B^T) * scale) * row_scales[:, None] * col_scales[None, :]); any factor may be None."""
+    rc = host.skinny_gemm_rowcol(A, B, D, scale_tensor, row_scales, col_scales)
+    if rc is not None:
+        return _done(rc, check)
     m, n, k, b_stride = _gemm_operands(A, B, D, scale_tensor, extra=(row_scales, col_scales))
     _vector(row_scales, m, "row_scales")
     _vector(col_scales, n, "col_scales")
@@ -175,6 +184,10 @@ def skinny_gemm_bf16act(X, B, D, scale_tensor=None, col_scales=None, row_scales_
     D = bf16(((q(X) @ B^T) * scale) * row_scale[:, None] * col_scales[None, :]); row_scales_out, if given, receives the
     row scales.  One launch where the fused kernel pays (skinny_gemm_bf16act_choice), two inside the library otherwise;
     with `tuning` (an SgTuning; engine 0 = the library's record for the shape) always the fused kernel."""
+    if tuning is None:
+        rc = host.skinny_gemm_bf16act(X, B, D, scale_tensor, col_scales, row_scales_out)
+        if rc is not None:
+            return _done(rc, check)
     m, n, k, b_stride = _gemm_operands(X, B, D, scale_tensor, extra=(col_scales, row_scales_out))
     _vector(col_scales, n, "col_scales")
     _vector(row_scales_out, m, "row_scales_out")
@@ -359,6 +372,10 @@ class HFRK_skinny_gemm:
 
 def sparse24_gemm(A, B_vals, B_meta, D, scale_tensor, tuning=None, check=False):
     """2:4 sparse weights: B_vals [n, k/2] kept codes, B_meta [n, k/8] position nibbles (include/sgemm.h)."""
+    if tuning is None:
+        rc = host.sparse24_gemm(A, B_vals, B_meta, D, scale_tensor)
+        if rc is not None:
+            return _done(rc, check)
     if A.dim() != 2 or A.shape[1] % 8:
         raise ValueError("A must be [m, k] with k a multiple of 8, got %s" % (tuple(A.shape),))
     m, n, k, _ = _gemm_operands(A, B_vals, D, scale_tensor, weight_cols=A.shape[1] // 2, extra=(B_meta,))
@@ -379,6 +396,9 @@ def sparse24_gemm(A, B_vals, B_meta, D, scale_tensor, tuning=None, check=False):
 def sparse24_compress(B, B_vals, B_meta, check=False):
     """Prune dense E4M3 weights B [n, k] to 2:4 (two largest magnitudes per group of four) and compress them
     into B_vals [n, k/2] and B_meta [n, k/8] (format of include/sgemm.h)."""
+    rc = host.sparse24_compress(B, B_vals, B_meta)
+    if rc is not None:
+        return _done(rc, check)
     if B.dim() != 2 or B.shape[1] % 8:
         raise ValueError("B must be [n, k] with k a multiple of 8, got %s" % (tuple(B.shape),))
     n, k = B.shape
@@ -409,6 +429,10 @@ def async_gemm(A, B, D, check=False):
 def tiled_sum_reduce(A, B, D, check=False, lds_queue=False):
     """D[m,n] = sum_b (A[b,m,n] + B[b,m,n]) in fp32, batch order.  lds_queue=True runs the variant that stages the
     batches through a queue in LDS (tiled_sum_reduce_async/src.cu:179-200); the result bits are the same."""
+    if not lds_queue:
+        rc = host.tiled_sum_reduce(A, B, D)
+        if rc is not None:
+            return _done(rc, check)
     if A.dim() != 3 or B.shape != A.shape or tuple(D.shape) != tuple(A.shape[1:]):
         raise ValueError("A and B must be [b, m, n] and D [m, n], got %s, %s, %s" % (tuple(A.shape), tuple(B.shape), tuple(D.shape)))
     for t, name in ((A, "A"), (B, "B"), (D, "D")):
@@ -433,6 +457,9 @@ def _codec_operands(X, Q, scales, nbuf=None):
 
 
 def fp8_encode_rows(X, Q, scales, check=False):
+    rc = host.fp8_encode_rows(X, Q, scales)
+    if rc is not None:
+        return _done(rc, check)
     _codec_operands(X, Q, scales)
     rows, cols = X.shape
     with torch.cuda.device(X.device):
@@ -442,6 +469,9 @@ def fp8_encode_rows(X, Q, scales, check=False):
 
 
 def fp8_decode_rows(Q, scales, Y, check=False):
+    rc = host.fp8_decode_rows(Q, scales, Y)
+    if rc is not None:
+        return _done(rc, check)
     _codec_operands(Y, Q, scales)
     rows, cols = Q.shape
     with torch.cuda.device(Q.device):
@@ -452,6 +482,9 @@ def fp8_decode_rows(Q, scales, Y, check=False):
 
 def fp8_reduce_rows(Q, scales, Y, check=False):
     """Q [nbuf, rows, cols], scales [nbuf, rows] -> Y [rows, cols] bfloat16."""
+    rc = host.fp8_reduce_rows(Q, scales, Y)
+    if rc is not None:
+        return _done(rc, check)
     if Q.dim() != 3:
         raise ValueError("Q must be [nbuf, rows, cols], got %s" % (tuple(Q.shape),))
     _codec_operands(Y, Q, scales, nbuf=Q.shape[0])
