@@ -27,8 +27,10 @@ __device__ __forceinline__ uint32_t bf16_bits(float x) {
     uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
     return ((u & 0x7fffffffu) > 0x7f800000u) ? ((u >> 16) | 0x40u) : r;
 }
+// Two at once by v_cvt_pk_bf16_f32: bf16_bits' result for each of the 2^32 inputs, NaNs included (compared on the device).
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-    return bf16_bits(lo) | (bf16_bits(hi) << 16);
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
