@@ -14,13 +14,21 @@ extern "C" {
 #endif
 
 /* Profiling aid, no counterpart in the reference.  While a buffer is set, every launch of the LDS-ring GEMM
- * kernels (per-tile and persistent), of the mid-batch GEMM kernel and of the 2:4 kernels takes the next grid * 8 words of it and each workgroup leaves eight 64-bit
+ * kernels (per-tile and persistent), of the mid-batch and wide-tile GEMM kernels and of the 2:4 kernels takes the next grid * 8 words of it and each workgroup leaves eight 64-bit
  * words there when it is done: [0] kernel entry, [1] prologue DMAs issued, [2] first stage landed, [3] last stage
  * consumed, [4] outputs stored and acknowledged - 10 ns ticks of the device's constant 100 MHz clock -
  * [5], [6] shader clock at entry and end, [7] XCC_ID << 32 | HW_ID.  Launches that no longer fit leave nothing.
  * A launch recorded into a HIP graph keeps its slice on every replay.  Process-wide; set it from one thread while
  * no other thread launches.  sg_debug_stamps(NULL, 0) switches the stamps off again. */
 int sg_debug_stamps(unsigned long long* device_buffer, size_t n_words);
+
+/* The GEMM of sg_skinny_gemm_rowcol on the wide-tile kernel with a given tile, for tests and timings of single tiles: the
+ * library chooses between them by itself above 128 rows.  The tile is 32 * row_tiles weight rows (row_tiles 4..8) by
+ * 32 * m_blocks activation rows (8, or 4 with row_tiles 4 and 8); split_k > 1 sums its partials in a second launch.
+ * scale, row_scales and col_scales may be NULL; k a multiple of 16 beyond 128. */
+int sg_debug_wide_gemm(const uint8_t* A, const uint8_t* B, void* D_bf16, const float* scale, const float* row_scales,
+                       const float* col_scales, int m, int n, int k, int b_stride, int row_tiles, int m_blocks, int split_k,
+                       void* stream);
 
 /* Profiling aid, no counterpart in the reference: reads the n x k weight matrix B (row stride b_stride, k % 1024 == 0)
  * the way the persistent LDS-ring GEMM streams it - one workgroup per CU walking row tiles, eight waves sharing K,

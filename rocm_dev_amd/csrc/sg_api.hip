@@ -243,6 +243,7 @@ struct Config {
     int nt;       // weights loaded with the non-temporal hint
     int persist;  // LDS engine: 0 = one workgroup per tile; n > 0 = n persistent workgroups per CU walking the tiles
     const Workspace* fixed_ws = nullptr;   // split-K partials and counters to use instead of the stream's own workspace
+    bool wide = false;   // mid-batch engine: the wide-tile kernel (only the library itself asks for it: wide_config)
     int wavetile; // LDS engine, bits 0-1: 1 = every wave owns whole tiles, activations resident in LDS (persist = workgroups per CU);
                   //             2 = persistent K-split workgroups with the activations resident in LDS
                   //             3 = ... resident in the waves' registers (k = 256 * waves * {1, 2, 4});  bit 2: epilogue wave
@@ -463,8 +464,30 @@ static int launch_ring(const RingConfig& c, StreamArgs a, hipStream_t stream) {
 // partial last block, which exist for the tiles and rings pick_mid chooses.
 static bool mid_partial_block_k(int k) { return k % 128 != 0 && k % 16 == 0 && k > 128; }
 
+// The wide-tile kernel: four waves, two along n x two along m, c.rg x c.mt fragments each, a K split's sum always in a
+// second launch.  Rows are addressed by 32-bit offsets inside a tile of at most 256 rows.
+constexpr int kWidePitch = 1 << 23;
+static int launch_wide_engine(const Config& c, StreamArgs a, hipStream_t stream) {
+    if (c.waves != 4 || c.rg < 4 || c.rg > 8 || (c.mt != 4 && c.mt != 8) || a.b_stride > kWidePitch || a.k > kWidePitch) return SG_INVALID_CONFIG;
+    const int bn = 32 * c.rg, bm = 32 * c.mt;
+    a.waves = c.waves;
+    a.split_k = c.split_k;
+    a.n_tiles = (a.n + bn - 1) / bn;
+    a.m_tiles = (a.m + bm - 1) / bm;
+    if (c.split_k < 1 || c.split_k > a.k / 128) return SG_INVALID_CONFIG;
+    const size_t tiles = (size_t)a.n_tiles * a.m_tiles;
+    if (tiles * c.split_k > 0x7fffffffu) return SG_BAD_ARGUMENT;
+    if (int rc = attach_workspace(c, a, tiles, (size_t)c.waves * c.rg * c.mt * 1024, stream)) return rc;
+    set_reciprocals(a);
+    a.defer_reduce = c.split_k > 1 ? 1 : 0;
+    a.stamps = take_stamps((unsigned)(tiles * c.split_k));
+    if (int rc = launch_wide(c.rg, c.mt, a, (unsigned)(tiles * c.split_k), stream)) return rc;
+    return a.defer_reduce ? launch_mid_reduce(c.rg, c.mt, 2, a, stream) : SG_SUCCESS;
+}
+
 static int launch_mid_engine(const Config& c, StreamArgs a, hipStream_t stream) {
     if (a.k % 128 != 0 && !mid_partial_block_k(a.k)) return SG_K_NOT_DIVISIBLE_BY_WARPTILE_K;
+    if (c.wide) return launch_wide_engine(c, a, stream);
     if ((c.rg != 2 && c.rg != 4) || (c.mt != 2 && c.mt != 4 && c.mt != 8) || c.depth < 2) return SG_INVALID_CONFIG;
     if (c.waves != 4 && c.waves != 8 && c.waves != 14) return SG_INVALID_CONFIG;
     const int wn = c.waves / 2;                   // waves = wn (along n) x 2 (along m)
@@ -759,7 +782,7 @@ static void workspace_need(const Config& c, int m, int n, size_t* partial_bytes,
     if (c.split_k <= 1) return;
     size_t tiles, per_tile;
     if (c.engine == ENGINE_MID) {
-        const int wn = c.waves / 2;
+        const int wn = c.waves / 2;            // (wide tiles are 2 x 2 waves as well)
         const int bn = 16 * c.rg * (wn > 0 ? wn : 1), bm = 32 * c.mt;
         tiles = (size_t)((n + bn - 1) / bn) * ((m + bm - 1) / bm);
         per_tile = (size_t)c.waves * c.rg * c.mt * 1024;
@@ -1182,6 +1205,62 @@ static Config heuristic_config(int m, int n, int k, int cu_count) {
     return pick_config(m, n, k, cu_count);
 }
 
+// More than 128 activation rows and enough work: the wide-tile kernel (sg_wide_kernel.h) in place of heuristic_config's
+// mid-batch record, on the tile and K split that this model puts first.  Microseconds with every CU busy: a launch costs
+// 2.1, a round of workgroups its tile's fixed part (first loads, epilogue) plus one of the tile's stages per 128 bytes of
+// K, a partly filled last round at least 0.81 of that, a K that 128 does not divide 1.4 times (rows off their 128-byte
+// lines), a K split 1.6 and 0.21 per MB of partials, and nothing is faster than its weights at 6 TB/s.  Fitted to 2000
+// timings of these tiles on 243 random shapes (129..2048 rows, K of 512..32768, odd ones among them): 5.5 % off (rms),
+// and the tile it puts first is 0.2 % behind the best of them (geometric mean).  Against the mid-batch record: ahead by
+// 1.1-1.6 times on most shapes where the model says 24 us or more (718 x 15360 x 13568 169.8 -> 123.8 us, 1024 x 57344 x
+// 8192 500 -> 375, 640 x 21120 x 23552 402 -> 248, 449 x 54816 x 512 54.2 -> 35.5), one of 120 behind by more than 3 % (320 x
+// 35680 x 1408 33.8 -> 35.3).  Below 24 us, where a tile's fixed part rules, and on launches that fill less than 9/16 of
+// the CUs (320 x 1408 x 17536 26.0 against 31.4) the mid-batch tiles are ahead.
+// Whose workspace it is does not change the result, so a K split of wide tiles is taken only where its partials fit what
+// sg_workspace_query asks for the mid-batch record; a tile without that split must then be within 10 % of the first.
+struct WideTile { int rg, mt; double stage_us, tile_us; };
+static const WideTile kWideTiles[] = {{4, 8, 0.829, 6.45}, {5, 8, 0.933, 7.48}, {6, 8, 1.064, 8.96}, {7, 8, 1.149, 9.83},
+                                      {8, 8, 1.249, 11.03}, {8, 4, 0.949, 6.48}, {4, 4, 0.620, 3.93}};
+static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, int cu_count, const Workspace* fixed_ws, Config* out) {
+    if (m <= 128 || mid.engine != ENGINE_MID || b_stride > kWidePitch || k > kWidePitch) return false;
+    size_t partial_limit, counters;
+    workspace_need(mid, m, n, &partial_limit, &counters);
+    if (fixed_ws && fixed_ws->partial_bytes < partial_limit) partial_limit = fixed_ws->partial_bytes;
+    const int blocks = (k + 127) / 128;
+    double first = 0, best = 0;       // of all tiles and splits, of those whose partials fit
+    long best_wgs = 0;
+    Config c{};
+    for (const WideTile& t : kWideTiles) {
+        const int bn = 32 * t.rg, bm = 32 * t.mt;
+        const long n_tiles = (n + bn - 1) / bn, tiles = n_tiles * ((m + bm - 1) / bm);
+        for (int sk = 1; sk <= 4; sk++) {
+            const long wgs = tiles * sk;
+            const double partials = (double)wgs * bn * bm * 4;
+            if (sk > 1 && (blocks / sk < 12 || wgs > cu_count)) continue;
+            const long full = wgs / cu_count, rest = wgs % cu_count;
+            const double rounds = full + (rest ? 0.81 + 0.19 * rest / cu_count : 0.0);
+            double us = 2.1 + rounds * blocks / sk * t.stage_us * (k % 128 ? 1.4 : 1.0) + (full + (rest ? 1 : 0)) * t.tile_us;
+            if (sk > 1) us += 1.6 + 0.214e-6 * partials;
+            const double weights = (double)n_tiles * bn * k / 6.0e6 + 6.1;
+            if (us < weights) us = weights;
+            if (first == 0 || us < first) first = us;
+            if (sk > 1 && (partials > (double)partial_limit || (fixed_ws && (size_t)tiles > fixed_ws->n_counters))) continue;
+            if (best == 0 || us < best) {
+                best = us;
+                best_wgs = wgs;
+                c.rg = t.rg; c.mt = t.mt; c.split_k = sk;
+            }
+        }
+    }
+    if (best < 24.0 || best > 1.1 * first || best_wgs * 16 < (long)cu_count * 9) return false;
+    c.engine = ENGINE_MID;
+    c.waves = 4;
+    c.wide = true;
+    c.nt = 1;
+    *out = c;
+    return true;
+}
+
 // ---- per-shape tuning table ---------------------------------------------------------------
 // What a tuning driver measured to be the best record for a shape; consulted before the
 // heuristics by the launchers that choose their own configuration.  Process-wide, any thread.
@@ -1245,7 +1324,12 @@ static int launch_chosen(const StreamArgs& a, int cu_count, hipStream_t stream, 
             if (!rejected_before_launch(rc)) return rc;
         }
     }
-    Config c = heuristic_config(a.m, a.n, a.k, cu_count);
+    Config c = heuristic_config(a.m, a.n, a.k, cu_count), wide;
+    if (wide_config(c, a.m, a.n, a.k, a.b_stride, cu_count, fixed_ws, &wide)) {
+        wide.fixed_ws = fixed_ws;
+        const int rc = launch_config(wide, a, stream);
+        if (!rejected_before_launch(rc)) return rc;
+    }
     c.fixed_ws = fixed_ws;
     int rc = launch_config(c, a, stream);
     if (rejected_before_launch(rc) && c.split_k > 1) {
@@ -1417,6 +1501,25 @@ int sg_debug_stamps(unsigned long long* device_buffer, size_t n_words) {
     return SG_SUCCESS;
 }
 
+int sg_debug_wide_gemm(const uint8_t* A, const uint8_t* B, void* D, const float* scale, const float* row_scales,
+                       const float* col_scales, int m, int n, int k, int b_stride, int row_tiles, int m_blocks, int split_k,
+                       void* stream) {
+    if (n % 2 != 0) return SG_N_NOT_EVEN;
+    if (k % 16 != 0 || k <= 128) return SG_K_NOT_DIVISIBLE_BY_WARPTILE_K;
+    if (int rc = check_pointers(A, B, D, m, n, k, b_stride)) return rc;
+    DeviceInfo* dev;
+    if (int rc = get_device_info(&dev)) return rc;
+    Config c{};
+    c.engine = ENGINE_MID;
+    c.wide = true;
+    c.waves = 4; c.rg = row_tiles; c.mt = m_blocks; c.split_k = split_k;
+    StreamArgs a{};
+    a.A = A; a.B = B; a.D = D; a.scale = scale; a.row_scale = row_scales; a.col_scale = col_scales;
+    a.m = m; a.n = n; a.k = k; a.b_stride = b_stride;
+    a.out_f32 = 0;
+    return launch_config(c, a, static_cast<hipStream_t>(stream));
+}
+
 int sg_debug_read_stream(const uint8_t* B, int n, int k, int b_stride, int segment_bytes, void* stream) {
     if (!B || n <= 0 || k <= 0 || k % 1024 != 0 || b_stride < k || (b_stride & 15) || (reinterpret_cast<uintptr_t>(B) & 15u))
         return SG_BAD_ARGUMENT;
@@ -1526,7 +1629,11 @@ int sg_skinny_gemm_tuned(const uint8_t* A, const uint8_t* B, void* D, const floa
     DeviceInfo* dev;
     if (int rc = get_device_info(&dev)) return rc;
     Config c = config_from_tuning(*t);
-    if (c.engine == ENGINE_AUTO) c = heuristic_config(m, n, k, dev->cu_count);
+    if (c.engine == ENGINE_AUTO) {
+        c = heuristic_config(m, n, k, dev->cu_count);
+        Config wide;
+        if (wide_config(c, m, n, k, b_stride, dev->cu_count, nullptr, &wide)) c = wide;
+    }
     if (c.engine != ENGINE_MID && c.mt != 1 && c.mt != 2) return SG_INVALID_CONFIG;
     StreamArgs a{};
     a.A = A; a.B = B; a.D = D; a.scale = scale_tensor;
@@ -1550,6 +1657,8 @@ int sg_skinny_gemm_tuned_noalloc(const uint8_t* A, const uint8_t* B, void* D, co
     Config c = config_from_tuning(*t);
     if (c.engine == ENGINE_AUTO) {
         c = heuristic_config(m, n, k, dev->cu_count);
+        Config wide;
+        if (wide_config(c, m, n, k, b_stride, dev->cu_count, &w, &wide)) c = wide;
         // the library's own choice is made to fit the array: a K split whose partials or counters do not, is not taken
         size_t partial_bytes, counters;
         workspace_need(c, m, n, &partial_bytes, &counters);

@@ -45,6 +45,8 @@ int SG_RING_LAUNCHER(2)(int bl, int xu, int nt, const RingArgs& ra, unsigned gri
 int launch_xreg(int mt, int rg, int pt, int depth, const StreamArgs& a, unsigned grid, unsigned threads, size_t lds,
                 hipStream_t stream);
 int launch_mid(int rgw, int mh, int depth, int dx, int wn, const StreamArgs& a, unsigned grid, size_t lds, hipStream_t stream);
+// wide tiles on four waves, rgw x mh fragments each (sg_wide_kernel.h)
+int launch_wide(int rgw, int mh, const StreamArgs& a, unsigned grid, hipStream_t stream);
 // second launch of a mid-batch GEMM with StreamArgs::defer_reduce: sums the split-K partials of every output fragment
 int launch_mid_reduce(int rgw, int mh, int wn, const StreamArgs& a, hipStream_t stream);
 

@@ -1,6 +1,7 @@
 // Instantiates the mid-batch kernel for every compiled (RGW, MH, DEPTH) and exposes the
 // launcher the dispatcher in sg_api.hip calls.
 #include "sg_mid_kernel.h"
+#include "sg_mid_reduce_kernel.h"
 #include "sg_host.h"
 
 namespace sg {
@@ -52,7 +53,7 @@ static int launch_mid_tail(int rgw, int mh, int depth, int dx, int wn, const Str
 }
 
 int launch_mid_reduce(int rgw, int mh, int wn, const StreamArgs& a, hipStream_t stream) {
-    const int frags_wg = 2 * wn * rgw * mh;                    // fragments of a tile; a workgroup of four waves takes 4 * kReduceFrags
+    const int frags_wg = 2 * wn * rgw * mh;                   // fragments of a tile; a workgroup of four waves takes 4 * kReduceFrags
     if ((rgw * mh) % kReduceFrags != 0) return SG_INVALID_CONFIG;
     const size_t grid = (size_t)a.n_tiles * a.m_tiles * ((frags_wg + 4 * kReduceFrags - 1) / (4 * kReduceFrags));
     if (grid == 0 || grid > 0x7fffffffu) return SG_BAD_ARGUMENT;

@@ -378,51 +378,4 @@ __global__ void __launch_bounds__(WN * 128) mid_gemm_kernel(const StreamArgs a) 
     stamps.end(a);
 }
 
-
-// Second launch of a mid-batch GEMM whose split-K sum was deferred: every wave adds the split_k partials of
-// kReduceFrags 16 x 16 fragments of the output in split order - what the last workgroup to arrive does in the single
-// launch, so the result bits are the same - and applies scale, row and column factors and the rounding.  A wave's
-// work is a chain of round trips (partials, scale, store), so it takes several fragments at once and requests all
-// their partials of a split before it adds any: with one fragment per wave the launch took 7-12 us for 8-33 MB of
-// partials that the GEMM had just left in the caches.  The tile geometry comes as run-time values: rgw x mh
-// fragments per wave of the GEMM, wn x 2 waves per tile.
-constexpr int kReduceFrags = 4;
-__global__ void __launch_bounds__(256) mid_reduce_kernel(const StreamArgs a, int rgw, int mh, int wn) {
-    const int fr = rgw * mh, frags_wg = 2 * wn * fr;      // fr is a multiple of kReduceFrags (rgw, mh are 2, 4 or 8)
-    const int lane = lane_id();
-    // a workgroup takes 4 * kReduceFrags consecutive fragments of one tile; the workgroups of a weight tile sit on the
-    // XCD that computed it (the grid is n_tiles * m_tiles * chunks workgroups, chunks per tile)
-    const int chunks = (frags_wg + 4 * kReduceFrags - 1) / (4 * kReduceFrags);   // (the last one may have idle waves)
-    int pos;
-    const int tile_n = xcd_weight_tile((int)blockIdx.x, (int)gridDim.x, a.m_tiles * chunks, a.n_tiles, pos);
-    const int tile_m = pos / chunks, chunk = pos - tile_m * chunks;
-    if (tile_n >= a.n_tiles || tile_m >= a.m_tiles) return;
-    const unsigned tile_id = (unsigned)(tile_m * a.n_tiles + tile_n);
-    const unsigned rem = (unsigned)((chunk * 4 + wave_id()) * kReduceFrags);     // (wave of the tile, fragment of the wave)
-    if (rem >= (unsigned)frags_wg) return;
-    const float scale = a.scale ? a.scale[0] : 1.0f;
-    const int wave = (int)rem / fr, f0 = (int)rem - wave * fr;
-    const int wq = wave % wn, wm = wave / wn;
-    const f32x4* p = reinterpret_cast<const f32x4*>(a.ws + ((size_t)tile_id * a.split_k) * ((size_t)frags_wg * 256) +
-                                                    (size_t)wave * (fr * 256) + (size_t)f0 * 256) + lane;
-    const size_t split_stride = (size_t)frags_wg * 64;
-    f32x4 v[kReduceFrags];
-#pragma unroll
-    for (int j = 0; j < kReduceFrags; j++) v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int sp = 0; sp < a.split_k; sp++) {
-        f32x4 t[kReduceFrags];
-#pragma unroll
-        for (int j = 0; j < kReduceFrags; j++) t[j] = p[(size_t)sp * split_stride + j * 64];
-#pragma unroll
-        for (int j = 0; j < kReduceFrags; j++) v[j] += t[j];
-    }
-    const int r = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int j = 0; j < kReduceFrags; j++) {
-        const int f = f0 + j, rg = f / mh, mb = f - rg * mh;
-        store_fragment(a, v[j], scale, tile_m * (32 * mh) + (wm * mh + mb) * 16 + r, tile_n * (16 * rgw * wn) + (wq * rgw + rg) * 16 + 4 * g);
-    }
-}
-
 }  // namespace sg
