@@ -9,8 +9,8 @@
 // channel and bank, different rows - and what decides the rate is how much of a DRAM row a
 // stream takes per visit: 32 KB per workgroup and stream (CH = 8) with one batch in flight
 // reaches 6.4-7.0 TB/s on 8-16 batches of 16-32 MB, 4 KB with four batches in flight 5.3-5.6.
-// Small problems keep CH = 1, which gives them enough workgroups.  Any m, n: the tail is
-// handled element-wise.
+// Small problems keep CH = 1, which gives them enough workgroups.  Any m, n: only the last m*n % 4
+// elements are handled one by one.
 //
 // tiled_sum_reduce_async/src.cu:13-177 stages the same sum through an LDS queue: producer waves copy
 // batch slices of A and B into QSIZE slots, consumer waves wait on flag bytes, add and free the slots.
@@ -36,33 +36,56 @@ __device__ __forceinline__ void tiled_sum_reduce_elementwise(const float* A, con
     }
 }
 
-template <int CH>
-__global__ void __launch_bounds__(256) tiled_sum_reduce_kernel(const float* __restrict__ A, const float* __restrict__ B,
-                                                               float* __restrict__ D, int b, size_t mn) {
-    if ((mn & 3) == 0 && (size_t)(blockIdx.x + 1) * (1024 * CH) <= mn) {
-        const size_t base = (size_t)blockIdx.x * (1024 * CH) + threadIdx.x * 4;
-        f32x4 acc[CH];
+// A piece is loaded as four floats at an address that is a multiple of four bytes only: batch ib of an m*n that four does
+// not divide starts 4, 8 or 12 bytes off, and the memory pipeline takes such 16-byte loads as they are.  One float per
+// lane, step and batch - a chain of 4 * CH * b round trips - is what those sizes, and the last, partial workgroup of every
+// size, took before.  8 x 1023 x 8191 163 -> 92 us, 2 x 2051 x 2051 36.6 -> 17.6, 8 x 1024 x 8190 (a ragged end) 114 -> 89.
+using f32x4_at4 = f32x4 __attribute__((aligned(4)));
+
+// The sums of a lane's CH pieces; PARTIAL: the pieces that end beyond mn are read from [mn - 4, mn) and not stored.
+template <int CH, bool PARTIAL>
+__device__ __forceinline__ void tiled_sum_reduce_pieces(const float* A, const float* B, float* D, int b, size_t mn, size_t base) {
+    auto place = [&](int c) __attribute__((always_inline)) {
+        const size_t i = base + c * 1024;
+        return !PARTIAL || i + 4 <= mn ? i : mn - 4;
+    };
+    f32x4 acc[CH];
 #pragma unroll
-        for (int c = 0; c < CH; c++) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int ib = 0; ib < b; ib++) {
-            f32x4 va[CH], vb[CH];
+    for (int c = 0; c < CH; c++) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ib = 0; ib < b; ib++) {
+        f32x4 va[CH], vb[CH];
 #pragma unroll
-            for (int c = 0; c < CH; c++) {
-                va[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(A + (size_t)ib * mn + base + c * 1024));
-                vb[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(B + (size_t)ib * mn + base + c * 1024));
-            }
-#pragma unroll
-            for (int c = 0; c < CH; c++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[c][e] = __fadd_rn(acc[c][e], __fadd_rn(va[c][e], vb[c][e]));
+        for (int c = 0; c < CH; c++) {
+            va[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_at4*>(A + (size_t)ib * mn + place(c)));
+            vb[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_at4*>(B + (size_t)ib * mn + place(c)));
         }
 #pragma unroll
-        for (int c = 0; c < CH; c++) *reinterpret_cast<f32x4*>(D + base + c * 1024) = acc[c];
-    } else {
-        // the last, partial workgroup, or m*n not a multiple of four (batches then start at unaligned addresses):
-        // one float per lane and step, neighbouring lanes on neighbouring floats
-        tiled_sum_reduce_elementwise(A, B, D, b, mn, (size_t)blockIdx.x * (1024 * CH) + threadIdx.x, 4 * CH, 256);
+        for (int c = 0; c < CH; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[c][e] = __fadd_rn(acc[c][e], __fadd_rn(va[c][e], vb[c][e]));
     }
+#pragma unroll
+    for (int c = 0; c < CH; c++)
+        if (!PARTIAL || base + c * 1024 + 4 <= mn) *reinterpret_cast<f32x4*>(D + base + c * 1024) = acc[c];
+}
+
+// `whole` workgroups of CH pieces a lane, then one-piece workgroups for what is left: a ragged end costs no workgroup
+// 8 pieces of mostly nothing.  Six waves per SIMD: with registers for all 16 loads of a batch the compiler issues them at
+// once and the launch is slower for it (8 x 1024 x 8192 93.0 us on 128 registers, 88.2 on 79).
+template <int CH>
+__global__ void __launch_bounds__(256, 6) tiled_sum_reduce_kernel(const float* __restrict__ A, const float* __restrict__ B,
+                                                                  float* __restrict__ D, int b, size_t mn, unsigned whole) {
+    if (blockIdx.x < whole) {
+        tiled_sum_reduce_pieces<CH, false>(A, B, D, b, mn, (size_t)blockIdx.x * (1024 * CH) + threadIdx.x * 4);
+        return;
+    }
+    if (mn >= 4) {
+        const size_t base = (size_t)whole * (1024 * CH) + (size_t)(blockIdx.x - whole) * 1024 + threadIdx.x * 4;
+        tiled_sum_reduce_pieces<1, true>(A, B, D, b, mn, base);
+    }
+    // the last mn % 4 floats
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x < (mn & 3))
+        tiled_sum_reduce_elementwise(A, B, D, b, mn, (mn & ~(size_t)3) + threadIdx.x, 1, 0);
 }
 
 // LDS-queue variant.  WAVES waves per workgroup, each owning P pieces of 1 KB (256 floats), contiguous, of every
@@ -137,11 +160,10 @@ int launch_tiled_sum_reduce(const float* A, const float* B, float* D, int b, int
     const size_t mn = (size_t)m * n;
     // 32 KB per workgroup and stream once that still leaves two workgroups for every CU
     const int ch = mn >= ((size_t)4 << 20) ? 8 : 1;
-    const size_t per_wg = (size_t)1024 * ch;
-    const size_t grid = (mn + per_wg - 1) / per_wg;
+    const size_t whole = mn / (1024 * ch), grid = whole + (mn - whole * 1024 * ch + 1023) / 1024;
     if (grid > 0x7fffffffu) return SG_BAD_ARGUMENT;
-    if (ch == 8) tiled_sum_reduce_kernel<8><<<(unsigned)grid, 256, 0, stream>>>(A, B, D, b, mn);
-    else tiled_sum_reduce_kernel<1><<<(unsigned)grid, 256, 0, stream>>>(A, B, D, b, mn);
+    if (ch == 8) tiled_sum_reduce_kernel<8><<<(unsigned)grid, 256, 0, stream>>>(A, B, D, b, mn, (unsigned)whole);
+    else tiled_sum_reduce_kernel<1><<<(unsigned)grid, 256, 0, stream>>>(A, B, D, b, mn, (unsigned)whole);
     return hipGetLastError() == hipSuccess ? SG_SUCCESS : SG_LAUNCH_FAILED;
 }
 

@@ -165,6 +165,22 @@ def test_tiled_sum_reduce(sg, oracle, b, m, n, lds_queue):
     assert np.array_equal(D.cpu().numpy(), oracle.tiled_sum_reduce(A, B))
 
 
+# element counts below, at and just above a lane's four floats and a workgroup's 1024 and 8192, with every remainder by four
+@pytest.mark.parametrize("m,n", [(1, 1), (1, 3), (1, 4), (1, 5), (1, 1023), (5, 205), (1, 1026), (2, 2 ** 21 + 1), (1, 2 ** 22 + 8191),
+                                 (3, 1398103)])
+def test_tiled_sum_reduce_remainders(sg, oracle, m, n):
+    b = 3
+    A = oracle.uniform_f32((b, m, n), 0, 7, -0.5, 0.5)
+    B = oracle.uniform_f32((b, m, n), 0, 8, -0.5, 0.5)
+    # guard floats around the output
+    room = torch.full((m * n + 8,), 7.0, dtype=torch.float32, device="cuda")
+    D = room[4:m * n + 4].view(m, n)
+    assert sg.tiled_sum_reduce(dev(A), dev(B), D) == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(D.cpu().numpy(), oracle.tiled_sum_reduce(A, B))
+    assert bool((room[:4] == 7.0).all()) and bool((room[m * n + 4:] == 7.0).all())
+
+
 @pytest.mark.parametrize("b", [0, 1, 2, 3, 4, 5, 7])
 def test_tiled_sum_reduce_lds_queue_short_batches(sg, oracle, b):
     """Fewer batches than queue slots, exactly as many, and a few more: the drain must count what was really issued.
