@@ -55,11 +55,23 @@ __device__ __forceinline__ void wait_vmcnt_if(int on) {
 // The matrix instruction as text, accumulators in the accumulation registers: up to 256 of them beside 200 of
 // everything else, which the builtin (free to take either file) turns into 300 moves a stage.  Volatile, so it stays where
 // it is written among the memory instructions.  The two idle states in front of it are what a vector instruction that
-// wrote an operand would need; whoever reads accumulators waits for the last instruction first (mfma_drain).
+// wrote an operand would need.
+//
+// The compiler does not know how long the result takes and may read, copy or spill an accumulator right behind the text.
+// So the instruction that ends a stage is followed, in its own text, by the 32 idle states the longest one needs, where
+// `left` (wave-uniform) is not positive: behind the last stage every accumulator is complete before anything else can be
+// issued.  (Inside the loop nothing but the next stage's instruction touches one: tests/test_wide_codegen.py.)
 __device__ __forceinline__ void mfma_acc(f32x4& c, const i32x8& a, const i32x8& b) {
     asm volatile("s_nop 1\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
 }
-__device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
+__device__ __forceinline__ void mfma_acc_drain(f32x4& c, const i32x8& a, const i32x8& b, int left) {
+    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0\n\ts_cmp_gt_i32 %3, 0\n\ts_cbranch_scc1 .Lwide%=\n\t"
+                 "s_nop 15\n\ts_nop 15\n.Lwide%=:"
+                 : "+a"(c) : "v"(a), "v"(b), "s"(left) : "memory", "scc");
+}
+// Holds the copy of an accumulator to vector registers back to where the epilogue uses it.  On the largest tile the compiler
+// otherwise copies all 256 at the epilogue's top and spills what does not fit (21 registers; the smaller tiles fit).
+__device__ __forceinline__ void keep_in_accumulator(f32x4& c) { asm volatile("" : "+a"(c)); }
 
 // RGW x MH fragments per wave on WN x 2 waves; DW, DX: ring slots of the weights and of the activations (2 <= DX <= DW)
 template <int RGW, int MH, int WN, int DW, int DX, bool TAIL>
@@ -241,7 +253,8 @@ __global__ void __launch_bounds__(WN * 128) wide_gemm_kernel(const StreamArgs a)
                         issue_w(op, koff_w, prev_w, fill_w);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                mfma_acc(acc[rg][mb], w[(u * RGW + rg) % WR], x[u & 1][mb]);
+                if (rg == RGW - 1 && mb == MH - 1) mfma_acc_drain(acc[rg][mb], w[(u * RGW + rg) % WR], x[u & 1][mb], n_blk - 1 - s);
+                else mfma_acc(acc[rg][mb], w[(u * RGW + rg) % WR], x[u & 1][mb]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -254,7 +267,6 @@ __global__ void __launch_bounds__(WN * 128) wide_gemm_kernel(const StreamArgs a)
         stage(s + 1, std::integral_constant<int, 1>{});
     }
     if (s < n_blk) stage(s, std::integral_constant<int, 0>{});
-    mfma_drain();
     stamps.mark(3);
 
     // ---- epilogue --------------------------------------------------------------------------------
@@ -286,6 +298,7 @@ __global__ void __launch_bounds__(WN * 128) wide_gemm_kernel(const StreamArgs a)
         const f32x4 cs = col_scale_ahead(a, n_wave + rg * 16 + 4 * g);
 #pragma unroll
         for (int mb = 0; mb < MH; mb++) {
+            if (RGW * MH == 64) keep_in_accumulator(acc[rg][mb]);
             f32x4 v = acc[rg][mb];
             // scale, then the row factor, then the column factors: three separately rounded fp32 products
             v *= scale;
