@@ -51,6 +51,25 @@ def test_every_tile_at_its_edges(oracle, m, n, k, pad):
             assert bool((room[:8] == 7.0).all()) and bool((room[m + 8:] == 7.0).all()), (rg, mb, sk)
 
 
+# every remainder of n by the 8 outputs of a 16-byte store, on a D that is aligned to 16 bytes and to 8 only, and a tile
+# whose last columns are all beyond n
+@pytest.mark.parametrize("n", [260, 262, 264, 266, 390])
+@pytest.mark.parametrize("off", [0, 4])
+def test_rows_off_their_16_byte_pieces(oracle, n, off):
+    m, k = 131, 256
+    a8, b8, scale = oracle.make_gemm_operands(m, n, k, seed=n)
+    ref = rowcol_reference(oracle, a8, b8, scale, None, None, model=True)
+    A, B, S = dev(a8), dev(b8), scale_tensor(scale)
+    for rg, mb in TILES:
+        room = torch.full((m * n + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
+        D = room[8 + off:8 + off + m * n].view(m, n)
+        assert D.data_ptr() % 16 == 2 * off
+        assert _wide(A, B, D, S, None, None, rg, mb, 1) == 0
+        torch.cuda.synchronize()
+        assert oracle.max_rel_err_bf16(bits(D), ref) <= GEMM_TOL, (rg, mb)
+        assert bool((room[:8 + off] == 7.0).all()) and bool((room[8 + off + m * n:] == 7.0).all()), (rg, mb)
+
+
 # shapes the library itself runs on wide tiles: unsplit on a full round, K split, partial last block with padded rows
 @pytest.mark.parametrize("m,n,k,pad", [(300, 16384, 2048, 0), (257, 1536, 16384, 0), (1030, 4098, 3088, 16)])
 def test_the_librarys_choice(oracle, m, n, k, pad):
