@@ -411,7 +411,8 @@ def main():
                     "mhz": np.median((t[j, :, 6].astype(np.int64) - t[j, :, 5].astype(np.int64)) / np.maximum(end[j] - ent[j], tick))})
             med = {key: float(np.median([r[key] for r in rows])) for key in rows[0]}
             t_choice, _ = sg.skinny_gemm_choice(args.m, n, k)
-            what = "2:4, the library's choice" if args.sparse else sg.api.tuning_as_dict(t_choice)
+            what = ("2:4, the library's choice" if args.sparse else sg.api.skinny_gemm_wide_choice(args.m, n, k) or
+                    sg.api.tuning_as_dict(t_choice))
             print("%-18s %5d x %5d  grid %4d  event-pair period %.2f | period %.2f = gap %.2f + span %.2f | entry spread %.2f | "
                   "workgroup (median): prologue issue %.2f, first stage landed %.2f (max %.2f), streaming %.2f, reduce+store %.2f, "
                   "total %.2f (max %.2f) | last end - median end %.2f | shader clock %.0f MHz | %s"
@@ -656,8 +657,10 @@ def main():
                 if lib.sg_tuning_set(m, n, k, ctypes.byref(forced)) != 0:
                     sys.exit("bench.py: --record is not a valid tuning record")
             t, _ = sg.skinny_gemm_choice(m, n, k)
-            print("%s: %s" % (spec, {f: getattr(t, f) for f in ("engine", "split_k", "waves", "row_tiles", "m_blocks", "depth", "k_chunks",
-                                                                 "persistent_wgs_per_cu", "wave_tiles")}), file=sys.stderr)
+            wide = sg.api.skinny_gemm_wide_choice(m, n, k)
+            print("%s: %s" % (spec, "wide tile %d x %d, K split %d" % (32 * wide[0], 32 * wide[1], wide[2]) if wide else
+                              {f: getattr(t, f) for f in ("engine", "split_k", "waves", "row_tiles", "m_blocks", "depth", "k_chunks",
+                                                          "persistent_wgs_per_cu", "wave_tiles")}), file=sys.stderr)
             for i in range(3):
                 rc = lib.sg_skinny_gemm_auto(a8.data_ptr(), wb[i % copies].data_ptr(), d.data_ptr(), one.data_ptr(), m, n, k, k, None)
                 if rc != 0:
@@ -902,7 +905,8 @@ def main():
 
     def choice(m, n, k):
         t, from_table = sg.skinny_gemm_choice(m, n, k)
-        d = sg.api.tuning_as_dict(t)
+        wide = sg.api.skinny_gemm_wide_choice(m, n, k)
+        d = dict(zip(("wide_row_tiles", "wide_m_blocks", "split_k"), wide)) if wide else sg.api.tuning_as_dict(t)
         d["from_table"] = bool(from_table)
         return d
 

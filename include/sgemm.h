@@ -233,8 +233,9 @@ int sg_skinny_gemm_pick(int m, int n, int k, int out[8]);
 
 /* The complete record sg_skinny_gemm_auto would launch for the shape: the tuning table's entry when
  * there is one (*from_table = 1), the built-in heuristics' otherwise (0).  from_table may be NULL.
- * Above 128 rows the heuristics may run the wide-tile kernel instead, which no record describes: the record is then
- * the mid-batch launch that it replaces, and engine = 0 replays what sg_skinny_gemm_auto runs. */
+ * Above 128 rows the library may run the wide-tile kernel in place of the heuristics' record, and no record describes
+ * that kernel: sg_debug_wide_choice (sgemm_debug.h) says whether it does and on which tile, engine = 0 replays it, and the
+ * record is the mid-batch launch that it replaces (stored in the table it is what runs from then on). */
 int sg_skinny_gemm_choice(int m, int n, int k, SgTuning* out, int* from_table);
 
 /* Per-shape tuning table - the run-time form of what the reference's grid search produces: there the

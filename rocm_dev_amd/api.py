@@ -301,12 +301,23 @@ def skinny_gemm_pick(m, n, k):
 
 def skinny_gemm_choice(m, n, k):
     """(record, from_table): the complete SgTuning the fastpath would launch for the shape, and whether it comes
-    from the tuning table rather than the built-in heuristics."""
+    from the tuning table rather than the built-in heuristics.  Above 128 rows a wide tile, which no record describes, may
+    run in the place of the heuristics' record: skinny_gemm_wide_choice."""
     t, from_table = SgTuning(), C.c_int(0)
     rc = lib.sg_skinny_gemm_choice(m, n, k, C.byref(t), C.byref(from_table))
     if rc != 0:
         raise SgError(rc)
     return t, bool(from_table.value)
+
+
+def skinny_gemm_wide_choice(m, n, k, b_stride=None):
+    """(row_tiles, m_blocks, split_k) of the wide tile the fastpath launches for the shape, or None where it launches the
+    record that skinny_gemm_choice reports."""
+    out = (C.c_int * 3)()
+    rc = lib.sg_debug_wide_choice(m, n, k, k if b_stride is None else b_stride, C.byref(out))
+    if rc != 0:
+        raise SgError(rc)
+    return tuple(out) if out[0] else None
 
 
 def tuning_set(m, n, k, tuning):

@@ -180,6 +180,15 @@ def same_launch(a, b):
     return norm(a) == norm(b)
 
 
+def builtin_record(m, n, k):
+    """The record the library launches for the shape by itself; None where it runs a wide tile, which no record describes."""
+    from .api import skinny_gemm_choice, skinny_gemm_wide_choice
+    if skinny_gemm_wide_choice(m, n, k):
+        return None
+    own, _ = skinny_gemm_choice(m, n, k)
+    return {f: getattr(own, f) for f in FIELDS}
+
+
 def format_table(entries):
     """entries: iterable of ((m, n, k), record dict) -> text of a tuning file."""
     lines = ["sgemm-tuning 1", "# m n k " + " ".join(FIELDS)]
@@ -352,16 +361,15 @@ def main(argv=None):
         for us, r in kept[:args.top]:
             print("   %.2f us  %s" % (us, " ".join("%s=%d" % (f, r[f]) for f in FIELDS)), flush=True)
         # a winner that is the library's own choice under another spelling is timing noise, not a finding
-        from .api import skinny_gemm_choice
-        own, _ = skinny_gemm_choice(m, n, k)
-        own = {f: getattr(own, f) for f in FIELDS}
-        if kept and kept[0][0] < base_us * (1.0 - args.min_gain) and (args.min_gain < 0 or not same_launch(kept[0][1], own)):
+        own = builtin_record(m, n, k)
+        is_own = bool(kept) and own is not None and same_launch(kept[0][1], own)
+        if kept and kept[0][0] < base_us * (1.0 - args.min_gain) and (args.min_gain < 0 or not is_own):
             entries[(m, n, k)] = kept[0][1]
         else:
             entries.pop((m, n, k), None)
         report.append({"m": m, "n": n, "k": k, "builtin_us": round(base_us, 3), "candidates": tried,
                        "best_us": round(kept[0][0], 3) if kept else None, "best": kept[0][1] if kept else None,
-                       "best_is_builtin": bool(kept) and same_launch(kept[0][1], own), "in_table": (m, n, k) in entries})
+                       "best_is_builtin": is_own, "in_table": (m, n, k) in entries})
     with open(args.out, "w") as f:
         f.write(format_table(entries.items()))
     if args.report:

@@ -1520,6 +1520,21 @@ int sg_debug_wide_gemm(const uint8_t* A, const uint8_t* B, void* D, const float*
     return launch_config(c, a, static_cast<hipStream_t>(stream));
 }
 
+int sg_debug_wide_choice(int m, int n, int k, int b_stride, int out[3]) {
+    if (!out || m <= 0 || n <= 0 || k <= 0 || b_stride < k) return SG_BAD_ARGUMENT;
+    out[0] = out[1] = out[2] = 0;
+    SgTuning t;
+    if (table_lookup(m, n, k, &t) && t.engine != ENGINE_AUTO) return SG_SUCCESS;
+    DeviceInfo* dev;
+    int cu = 256;
+    if (get_device_info(&dev) == SG_SUCCESS) cu = dev->cu_count;
+    Config wide;
+    if (wide_config(heuristic_config(m, n, k, cu), m, n, k, b_stride, cu, nullptr, &wide)) {
+        out[0] = wide.rg; out[1] = wide.mt; out[2] = wide.split_k;
+    }
+    return SG_SUCCESS;
+}
+
 int sg_debug_read_stream(const uint8_t* B, int n, int k, int b_stride, int segment_bytes, void* stream) {
     if (!B || n <= 0 || k <= 0 || k % 1024 != 0 || b_stride < k || (b_stride & 15) || (reinterpret_cast<uintptr_t>(B) & 15u))
         return SG_BAD_ARGUMENT;

@@ -314,3 +314,30 @@ def test_the_shipped_table_is_loaded_once_unless_the_environment_says_otherwise(
             env["SGEMM_TUNING_TABLE"] = value
         out = subprocess.run([sys.executable, "-c", code], cwd=root, env=env, capture_output=True, text=True, check=True)
         assert [int(v) for v in out.stdout.split()] == want, (value, out.stdout, out.stderr)
+
+
+def test_the_tuner_keeps_the_record_a_wide_tile_replaced(table, tmp_path, monkeypatch):
+    """Above 128 rows the library may run a wide tile, which no record describes, in place of the record it reports.  A search
+    that finds that record ahead of what ran has found something; where the record itself ran, it is timing noise."""
+    sg = table
+    for shape, wide in (((1024, 57344, 8192), True), ((320, 4096, 4096), False)):
+        assert (api.skinny_gemm_wide_choice(*shape) is not None) == wide
+        choice, _ = sg.skinny_gemm_choice(*shape)
+        rec = autotune_fields(choice)
+        monkeypatch.setattr(autotune, "tune_shape", lambda *a, **kw: ([(90.0, rec)], 100.0, 7))
+        out = tmp_path / "t.txt"
+        assert autotune.main(["--shapes", "%dx%dx%d" % shape, "--out", str(out), "--report", str(tmp_path / "r.json")]) == 0
+        assert autotune.parse_table(out.read_text()) == ({shape: rec} if wide else {})
+        sg.tuning_load(out)
+        assert api.skinny_gemm_wide_choice(*shape) is None              # stored, the record is what runs
+
+
+def test_wide_choice_of_shapes_and_refusals():
+    assert api.skinny_gemm_wide_choice(128, 57344, 8192) is None        # 128 rows: the mid-batch kernel
+    assert api.skinny_gemm_wide_choice(1024, 57344, 8192, 8192 + 128) is not None
+    assert api.skinny_gemm_wide_choice(1024, 512, 8192, (1 << 23) + 16) is None     # rows too far apart for its offsets
+    for bad in ((0, 512, 512), (512, 0, 512), (512, 512, 0)):
+        with pytest.raises(api.SgError):
+            api.skinny_gemm_wide_choice(*bad)
+    with pytest.raises(api.SgError):
+        api.skinny_gemm_wide_choice(512, 512, 512, 496)
