@@ -1209,18 +1209,45 @@ static Config heuristic_config(int m, int n, int k, int cu_count) {
 // mid-batch record, on the tile and K split that this model puts first.  Microseconds with every CU busy: a launch costs
 // 2.1, a round of workgroups its tile's fixed part (first loads, epilogue) plus one of the tile's stages per 128 bytes of
 // K, a partly filled last round at least 0.81 of that, a K that 128 does not divide 1.4 times (rows off their 128-byte
-// lines), a K split 1.6 and 0.21 per MB of partials, and nothing is faster than its weights at 6 TB/s.  Fitted to 2000
-// timings of these tiles on 243 random shapes (129..2048 rows, K of 512..32768, odd ones among them): 5.5 % off (rms),
-// and the tile it puts first is 0.2 % behind the best of them (geometric mean).  Against the mid-batch record: ahead by
-// 1.1-1.6 times on most shapes where the model says 24 us or more (718 x 15360 x 13568 169.8 -> 123.8 us, 1024 x 57344 x
-// 8192 500 -> 375, 640 x 21120 x 23552 402 -> 248, 449 x 54816 x 512 54.2 -> 35.5), one of 120 behind by more than 3 % (320 x
-// 35680 x 1408 33.8 -> 35.3).  Below 24 us, where a tile's fixed part rules, and on launches that fill less than 9/16 of
-// the CUs (320 x 1408 x 17536 26.0 against 31.4) the mid-batch tiles are ahead.
+// lines), a K split 1.6 and 0.21 per MB of partials, and nothing is faster than its weights at 6 TB/s.  Fitted to timings of
+// these tiles on 243 random shapes (129..2048 rows, K of 512..32768, odd ones among them).  It ranks the tiles: on 1069
+// other shapes the times were 1.1 times what it says (geometric mean; 0.83 to 1.6, the highest with rows off their lines
+// at a K that 128 divides).  Below 24 us, where a tile's fixed part rules, and on launches that fill less than 9/16 of
+// the CUs (320 x 1408 x 17536 26.0 against 31.4) the mid-batch tiles are ahead, and where mid_stays_ahead says so;
+// elsewhere the wide ones, by up to 1.6 times (718 x 15360 x 13568 169.8 -> 123.8 us, 1024 x 57344 x 8192 466 -> 361,
+// 640 x 21120 x 23552 402 -> 248, 449 x 54816 x 512 54.2 -> 35.5).
 // Whose workspace it is does not change the result, so a K split of wide tiles is taken only where its partials fit what
 // sg_workspace_query asks for the mid-batch record; a tile without that split must then be within 10 % of the first.
 struct WideTile { int rg, mt; double stage_us, tile_us; };
 static const WideTile kWideTiles[] = {{4, 8, 0.829, 6.45}, {5, 8, 0.933, 7.48}, {6, 8, 1.064, 8.96}, {7, 8, 1.149, 9.83},
                                       {8, 8, 1.249, 11.03}, {8, 4, 0.949, 6.48}, {4, 4, 0.620, 3.93}};
+// Mid-batch launches that the model does not know of and that a wide tile loses to.  Of 1960 shapes timed
+// on both (129..2048 rows, 900 random, the others drawn from where the rules lie) 955 go to a wide tile, 1.18 times faster
+// (geometric mean), 34 of them behind by more than 3 % and 6 by more than 10 % (151 x 16708 x 24192 by 17 %); without
+// these rules 113 of 1069 were, up to 1.34 times.
+static bool mid_stays_ahead(const Config& mid, const Config& wide, double wide_us, int m, int n, int k, int b_stride, int cu_count) {
+    // A K split five to eight ways, where a wide tile goes to four at most and mid_model_us (which knows whole K blocks only)
+    // puts the mid-batch launch 5 % ahead of four ways or 9 % ahead of three: 208 x 2304 x 20864 29.6 us against 37.9,
+    // 525 x 1024 x 28032 40.6 against 49.9, 856 x 1536 x 27776 61.4 against 67.9.
+    if (k % 128 == 0 && mid.split_k > 4 && wide.split_k >= 3)
+        return mid_model_us(m, n, k, 8 * mid.rg * mid.waves, 32 * mid.mt, mid.split_k, cu_count) < (wide.split_k == 4 ? 0.95 : 0.91) * wide_us;
+    // The fourteen-wave tiles - except where four does not divide n, which costs the mid-batch epilogue more than any tile.
+    if (mid.waves != 14 || n % 4 != 0) return false;
+    const bool whole_lines = k % 128 == 0 && b_stride % 128 == 0;
+    if (mid.mt == 4) {
+        // 224 x 128 tiles against wide ones of the same 128 rows: level to 17 % ahead on 26 shapes (266 x 17856 x 4432 54.1 us
+        // against 63.3, 384 x 18432 x 3072 level) ...
+        if (wide.rg == 8 && wide.mt == 4) return true;
+        // ... and wherever they fill every round, on rows of whole lines: 1024 x 7168 x 4096 37.2 us against 39.9, 512 x 14336 x
+        // 7168 60.9 against 64.9 (rows off their lines, 1024 x 7168 x 10240: 118 against 97).
+        const long wgs = (long)((n + 223) / 224) * ((m + 127) / 128);
+        return whole_lines && wgs % cu_count == 0;
+    }
+    // 224 x 256 tiles on rows off their 128-byte lines with a short K and few rows, where loads and stores are all there is:
+    // level to 13 % ahead on 23 shapes (315 x 53428 x 640, rows 656 apart, 35.2 us against 39.7).
+    return mid.mt == 8 && !whole_lines && m < 400 && k <= 2000;
+}
+
 static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, int cu_count, const Workspace* fixed_ws, Config* out) {
     if (m <= 128 || mid.engine != ENGINE_MID || b_stride > kWidePitch || k > kWidePitch) return false;
     size_t partial_limit, counters;
@@ -1253,6 +1280,7 @@ static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, in
         }
     }
     if (best < 24.0 || best > 1.1 * first || best_wgs * 16 < (long)cu_count * 9) return false;
+    if (mid_stays_ahead(mid, c, best, m, n, k, b_stride, cu_count)) return false;
     c.engine = ENGINE_MID;
     c.waves = 4;
     c.wide = true;
