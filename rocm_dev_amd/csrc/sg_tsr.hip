@@ -9,8 +9,8 @@
 // channel and bank, different rows - and what decides the rate is how much of a DRAM row a
 // stream takes per visit: 32 KB per workgroup and stream (CH = 8) with one batch in flight
 // reaches 6.4-7.0 TB/s on 8-16 batches of 16-32 MB, 4 KB with four batches in flight 5.3-5.6.
-// Small problems keep CH = 1, which gives them enough workgroups.  Any m, n: only the last m*n % 4
-// elements are handled one by one.
+// Small problems keep CH = 1, which gives them enough workgroups.  Any m, n: the piece that crosses m*n is summed
+// four floats back and stored in part.
 //
 // tiled_sum_reduce_async/src.cu:13-177 stages the same sum through an LDS queue: producer waves copy
 // batch slices of A and B into QSIZE slots, consumer waves wait on flag bytes, add and free the slots.
@@ -42,13 +42,9 @@ __device__ __forceinline__ void tiled_sum_reduce_elementwise(const float* A, con
 // size, took before.  8 x 1023 x 8191 163 -> 92 us, 2 x 2051 x 2051 36.6 -> 17.6, 8 x 1024 x 8190 (a ragged end) 114 -> 89.
 using f32x4_at4 = f32x4 __attribute__((aligned(4)));
 
-// The sums of a lane's CH pieces; PARTIAL: the pieces that end beyond mn are read from [mn - 4, mn) and not stored.
-template <int CH, bool PARTIAL>
+// The sums of a lane's CH pieces, all inside [0, mn).
+template <int CH>
 __device__ __forceinline__ void tiled_sum_reduce_pieces(const float* A, const float* B, float* D, int b, size_t mn, size_t base) {
-    auto place = [&](int c) __attribute__((always_inline)) {
-        const size_t i = base + c * 1024;
-        return !PARTIAL || i + 4 <= mn ? i : mn - 4;
-    };
     f32x4 acc[CH];
 #pragma unroll
     for (int c = 0; c < CH; c++) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -56,8 +52,8 @@ __device__ __forceinline__ void tiled_sum_reduce_pieces(const float* A, const fl
         f32x4 va[CH], vb[CH];
 #pragma unroll
         for (int c = 0; c < CH; c++) {
-            va[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_at4*>(A + (size_t)ib * mn + place(c)));
-            vb[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_at4*>(B + (size_t)ib * mn + place(c)));
+            va[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_at4*>(A + (size_t)ib * mn + base + c * 1024));
+            vb[c] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_at4*>(B + (size_t)ib * mn + base + c * 1024));
         }
 #pragma unroll
         for (int c = 0; c < CH; c++)
@@ -65,27 +61,52 @@ __device__ __forceinline__ void tiled_sum_reduce_pieces(const float* A, const fl
             for (int e = 0; e < 4; e++) acc[c][e] = __fadd_rn(acc[c][e], __fadd_rn(va[c][e], vb[c][e]));
     }
 #pragma unroll
-    for (int c = 0; c < CH; c++)
-        if (!PARTIAL || base + c * 1024 + 4 <= mn) *reinterpret_cast<f32x4*>(D + base + c * 1024) = acc[c];
+    for (int c = 0; c < CH; c++) *reinterpret_cast<f32x4*>(D + base + c * 1024) = acc[c];
+}
+
+// One piece a lane at the ragged end (mn >= 4).  The piece that crosses mn is read from [mn - 4, mn), and its floats from
+// `base` on are stored.  A small launch is a chain of round trips, so four batches are asked for at once (15 x 1 x 617
+// 6.2 us with floats one by one, 3.1 this way); with eight the kernel takes 76 registers, two waves per SIMD fewer, and
+// 14 x 1416 x 1220 goes from 34 to 40 us.
+__device__ __forceinline__ void tiled_sum_reduce_end(const float* A, const float* B, float* D, int b, size_t mn, size_t base) {
+    if (base >= mn) return;
+    const size_t at = base + 4 <= mn ? base : mn - 4;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int ib = 0; ib < b; ib += 4) {
+        f32x4 va[4], vb[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (ib + j < b) {
+                va[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_at4*>(A + (size_t)(ib + j) * mn + at));
+                vb[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_at4*>(B + (size_t)(ib + j) * mn + at));
+            }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (ib + j < b)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[e] = __fadd_rn(acc[e], __fadd_rn(va[j][e], vb[j][e]));
+    }
+    if (at == base) {
+        *reinterpret_cast<f32x4*>(D + base) = acc;
+    } else {
+#pragma unroll
+        for (int e = 1; e < 4; e++)
+            if (at + e >= base) D[at + e] = acc[e];
+    }
 }
 
 // `whole` workgroups of CH pieces a lane, then one-piece workgroups for what is left: a ragged end costs no workgroup
 // 8 pieces of mostly nothing.  Six waves per SIMD: with registers for all 16 loads of a batch the compiler issues them at
-// once and the launch is slower for it (8 x 1024 x 8192 93.0 us on 128 registers, 88.2 on 79).
+// once and the launch is slower for it (8 x 1024 x 8192 93.0 us on 128 registers, 88.2 on 79).  Eight waves with one piece.
 template <int CH>
-__global__ void __launch_bounds__(256, 6) tiled_sum_reduce_kernel(const float* __restrict__ A, const float* __restrict__ B,
+__global__ void __launch_bounds__(256, CH == 1 ? 8 : 6) tiled_sum_reduce_kernel(const float* __restrict__ A, const float* __restrict__ B,
                                                                   float* __restrict__ D, int b, size_t mn, unsigned whole) {
-    if (blockIdx.x < whole) {
-        tiled_sum_reduce_pieces<CH, false>(A, B, D, b, mn, (size_t)blockIdx.x * (1024 * CH) + threadIdx.x * 4);
-        return;
-    }
-    if (mn >= 4) {
-        const size_t base = (size_t)whole * (1024 * CH) + (size_t)(blockIdx.x - whole) * 1024 + threadIdx.x * 4;
-        tiled_sum_reduce_pieces<1, true>(A, B, D, b, mn, base);
-    }
-    // the last mn % 4 floats
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x < (mn & 3))
-        tiled_sum_reduce_elementwise(A, B, D, b, mn, (mn & ~(size_t)3) + threadIdx.x, 1, 0);
+    if (blockIdx.x < whole)
+        tiled_sum_reduce_pieces<CH>(A, B, D, b, mn, (size_t)blockIdx.x * (1024 * CH) + threadIdx.x * 4);
+    else if (mn > 256)
+        tiled_sum_reduce_end(A, B, D, b, mn, (size_t)whole * (1024 * CH) + (size_t)(blockIdx.x - whole) * 1024 + threadIdx.x * 4);
+    else   // a float a lane is all there is: the shorter code is ahead (9 x 1 x 5 2.13 us, 2.58 by pieces; 2 x 1 x 82 2.07, 2.16)
+        tiled_sum_reduce_elementwise(A, B, D, b, mn, threadIdx.x, 1, 0);
 }
 
 // LDS-queue variant.  WAVES waves per workgroup, each owning P pieces of 1 KB (256 floats), contiguous, of every

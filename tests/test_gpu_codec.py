@@ -169,7 +169,17 @@ def test_tiled_sum_reduce(sg, oracle, b, m, n, lds_queue):
 @pytest.mark.parametrize("m,n", [(1, 1), (1, 3), (1, 4), (1, 5), (1, 1023), (5, 205), (1, 1026), (2, 2 ** 21 + 1), (1, 2 ** 22 + 8191),
                                  (3, 1398103)])
 def test_tiled_sum_reduce_remainders(sg, oracle, m, n):
-    b = 3
+    _ragged_sum(sg, oracle, 3, m, n)
+
+
+# the ragged end on both sides of 256 floats, every remainder by four, batch counts around its groups of four
+@pytest.mark.parametrize("b", [1, 3, 4, 5, 8, 15])     # (no batch at all is refused: empty tensors have no address)
+@pytest.mark.parametrize("mn", [255, 256, 257, 258, 259, 260, 1027])
+def test_tiled_sum_reduce_ragged_end(sg, oracle, b, mn):
+    _ragged_sum(sg, oracle, b, 1, mn)
+
+
+def _ragged_sum(sg, oracle, b, m, n):
     A = oracle.uniform_f32((b, m, n), 0, 7, -0.5, 0.5)
     B = oracle.uniform_f32((b, m, n), 0, 8, -0.5, 0.5)
     # guard floats around the output
