@@ -39,9 +39,44 @@ __device__ __forceinline__ float wave_max(float v) {
 
 // A row is held in registers, so it is read from memory exactly once: thread t of the THREADS that share a row holds
 // its chunks t, t + THREADS, ... of 8 bf16 each, CH of them.  HBM-bound at 3 bytes per element (30.5 us for 8192 x 8192 at
-// the 6.6 TB/s a stream reaches, measured 33.4); what a row shape can lose on top is idle lanes, workgroup launches and
+// the 6.6 TB/s a stream reaches, measured 34.4); what a row shape can lose on top is idle lanes, workgroup launches and
 // the reduction of the maximum, which is why there is one build per range of row lengths (launch_fp8_encode_rows).
 //
+// All chunks are asked for before any is looked at.  A thread beyond the row's end takes its last chunk again, which changes
+// no maximum, and stores nothing: a load that only some lanes issue, into registers that are zero in the others, made the
+// compiler wait for the second load before it issued the third (2048 x 4112 8.3 us, 7.2 this way).
+template <int STEP, int CH>
+__device__ __forceinline__ float load_chunks(u32x4 (&raw)[CH], const u32x4* xrow, int t, int nchunks) {
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        // a 32-bit offset from the row: one register of address a load where the row is the workgroup's
+        const unsigned at = (unsigned)(c * STEP + t < nchunks ? c * STEP + t : nchunks - 1) * 16;
+        raw[c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(reinterpret_cast<const uint8_t*>(xrow) + at));
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CH; c++) amax = absmax8_bf16(raw[c], amax);
+    return amax;
+}
+template <int STEP, int CH>
+__device__ __forceinline__ void store_chunks(const u32x4 (&raw)[CH], RowQuant rq, u32x2* qrow, int t, int nchunks) {
+    auto store = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const u32x2 q = quantize8_bf16(raw[c], rq);
+            if (c * STEP + t < nchunks) __builtin_nontemporal_store(q, qrow + c * STEP + t);
+        }
+    };
+    // one branch over all chunks
+    if (rq.fast) {
+        rq.fast = true;
+        store();
+    } else {
+        rq.fast = false;
+        store();
+    }
+}
+
 // One workgroup per row, the maximum through LDS.
 template <int THREADS, int CH>
 __global__ void __launch_bounds__(THREADS) fp8_encode_row_kernel(const uint16_t* __restrict__ X, uint8_t* __restrict__ Q,
@@ -50,18 +85,8 @@ __global__ void __launch_bounds__(THREADS) fp8_encode_row_kernel(const uint16_t*
     const int row = blockIdx.x;
     const int t = threadIdx.x;
     const int nchunks = cols >> 3;
-    const u32x4* xrow = reinterpret_cast<const u32x4*>(X + (size_t)row * cols);
-
     u32x4 raw[CH];
-#pragma unroll
-    for (int c = 0; c < CH; c++) {
-        raw[c] = u32x4{0u, 0u, 0u, 0u};
-        if (c * THREADS + t < nchunks) raw[c] = __builtin_nontemporal_load(xrow + c * THREADS + t);
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int c = 0; c < CH; c++) amax = absmax8_bf16(raw[c], amax);
-    amax = wave_max(amax);
+    float amax = wave_max(load_chunks<THREADS>(raw, reinterpret_cast<const u32x4*>(X + (size_t)row * cols), t, nchunks));
     if (THREADS > 64) {
         if (lane_id() == 0) wmax[t >> 6] = amax;
         __syncthreads();
@@ -69,41 +94,30 @@ __global__ void __launch_bounds__(THREADS) fp8_encode_row_kernel(const uint16_t*
 #pragma unroll
         for (int w = 1; w < THREADS / 64; w++) amax = fmaxf(amax, wmax[w]);
     }
-    const RowQuant rq = row_quant(amax);
+    RowQuant rq = row_quant(amax);
+    rq.fast = __builtin_amdgcn_readfirstlane(rq.fast);      // the row is the workgroup's
     if (t == 0) scales[row] = rq.s;
-    u32x2* qrow = reinterpret_cast<u32x2*>(Q + (size_t)row * cols);
-#pragma unroll
-    for (int c = 0; c < CH; c++)
-        if (c * THREADS + t < nchunks) __builtin_nontemporal_store(quantize8_bf16(raw[c], rq), qrow + c * THREADS + t);
+    store_chunks<THREADS>(raw, rq, reinterpret_cast<u32x2*>(Q + (size_t)row * cols), t, nchunks);
 }
 
 // Short rows: LANES lanes of a wave (a power of two) share a row, 256 / LANES rows per workgroup, the maximum by
 // shuffles.  A workgroup per row spends a launch of its own and most of a wave's lanes on them: 16384 rows of 16 / 64 /
-// 240 / 512 columns 8.7 / 7.9 / 8.3 / 8.7 us that way, 2.7 / 3.2 / 4.8 / 6.6 this way.
+// 240 / 512 columns 8.7 / 7.8 / 8.3 / 8.1 us that way, 2.5 / 2.9 / 4.5 / 6.7 this way.
 template <int LANES, int CH>
 __global__ void __launch_bounds__(256) fp8_encode_short_rows_kernel(const uint16_t* __restrict__ X, uint8_t* __restrict__ Q,
                                                                     float* __restrict__ scales, int rows, int cols) {
-    const unsigned row = blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    const unsigned mine = blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    const unsigned row = mine < (unsigned)rows ? mine : (unsigned)rows - 1;      // lanes past the last row store nothing
     const int t = (int)threadIdx.x % LANES;
-    const int nchunks = row < (unsigned)rows ? cols >> 3 : 0;      // lanes past the last row take part in the shuffles only
-    const u32x4* xrow = reinterpret_cast<const u32x4*>(X + (size_t)row * cols);
+    const int nchunks = cols >> 3;
     u32x4 raw[CH];
-#pragma unroll
-    for (int c = 0; c < CH; c++) {
-        raw[c] = u32x4{0u, 0u, 0u, 0u};
-        if (c * LANES + t < nchunks) raw[c] = __builtin_nontemporal_load(xrow + c * LANES + t);
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int c = 0; c < CH; c++) amax = absmax8_bf16(raw[c], amax);
+    float amax = load_chunks<LANES>(raw, reinterpret_cast<const u32x4*>(X + (size_t)row * cols), t, nchunks);
 #pragma unroll
     for (int o = LANES / 2; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
     const RowQuant rq = row_quant(amax);
-    if (t == 0 && row < (unsigned)rows) scales[row] = rq.s;
-    u32x2* qrow = reinterpret_cast<u32x2*>(Q + (size_t)row * cols);
-#pragma unroll
-    for (int c = 0; c < CH; c++)
-        if (c * LANES + t < nchunks) __builtin_nontemporal_store(quantize8_bf16(raw[c], rq), qrow + c * LANES + t);
+    if (mine >= (unsigned)rows) return;
+    if (t == 0) scales[row] = rq.s;
+    store_chunks<LANES>(raw, rq, reinterpret_cast<u32x2*>(Q + (size_t)row * cols), t, nchunks);
 }
 
 // Rows too long to hold in registers (more than 65536 columns): two passes over the row (the second mostly from L2).
@@ -213,10 +227,12 @@ int launch_fp8_encode_rows(const void* X, uint8_t* Q, float* scales, int rows, i
     fp8_encode_short_rows_kernel<LANES, CH><<<((unsigned)rows + 256 / LANES - 1) / (256 / LANES), 256, 0, stream>>>(x, Q, scales, rows, cols)
 #define SG_ROW(THREADS, CH) fp8_encode_row_kernel<THREADS, CH><<<rows, THREADS, 0, stream>>>(x, Q, scales, cols)
     // The smallest group of threads that holds the row in two chunks each (from 32 columns on), lanes of a shared wave up
-    // to 512 columns and a workgroup beyond; with many rows fewer threads of four chunks from 8192 columns on.  us, cold,
-    // against 64 / 128 / 256 threads a row as many as needed: 16384 x 1024 16.4 -> 10.0, 16384 x 2048 27.9 -> 18.0,
-    // 8192 x 4096 19.1 -> 18.7, 1024 x 8192 6.7 -> 6.4, 16 x 14336 4.3 -> 3.6, 2048 x 16384 19.8 -> 18.9; above 16384
-    // columns against two passes over the row: 512 x 32768 22.7 -> 10.4, 64 x 65536 29.4 -> 7.8.
+    // to 512 columns and a workgroup beyond; from 4112 columns on, with more than 1024 rows (and 256 beyond 8192 columns),
+    // half as many threads of four chunks (2048 x 4112 7.8 us in two chunks, 7.2 in four; 1024 x 4112 the other way round).
+    // us, cold, against 64 / 128 / 256 threads a row as many as needed: 16384 x 1024 15.0 -> 11.1, 16384 x 2048 28.5 -> 19.7,
+    // 8192 x 4096 19.8 -> 19.1, 1024 x 8192 6.5 -> 6.3, 16 x 14336 4.2 -> 3.2, 2048 x 16384 20.9 -> 19.6, but 1500 x 6144
+    // 6.9 -> 7.3 and 1200 x 8192 7.3 -> 7.6; above 16384 columns against two passes over the row: 512 x 32768 23.3 -> 11.4,
+    // 64 x 65536 29.3 -> 7.6.
     if (nchunks <= 2) SG_SHORT(2, 1);
     else if (nchunks <= 4) SG_SHORT(4, 1);
     else if (nchunks <= 8) SG_SHORT(8, 1);
@@ -226,7 +242,7 @@ int launch_fp8_encode_rows(const void* X, uint8_t* Q, float* scales, int rows, i
     else if (nchunks <= 128) SG_ROW(64, 2);
     else if (nchunks <= 256) SG_ROW(128, 2);
     else if (nchunks <= 512) SG_ROW(256, 2);
-    else if (nchunks <= 1024 && rows <= 2048) SG_ROW(512, 2);
+    else if (nchunks <= 1024 && rows <= 1024) SG_ROW(512, 2);
     else if (nchunks <= 1024) SG_ROW(256, 4);
     else if (nchunks <= 2048 && rows <= 256) SG_ROW(1024, 2);
     else if (nchunks <= 2048) SG_ROW(512, 4);
