@@ -6,7 +6,7 @@ same library without ctypes.  There is no fallback: if either has not been built
 import ctypes as C
 import os
 
-import torch  # noqa: F401  (the extension module links against its libraries)
+import torch  # (the extension module links against its libraries)
 
 from .build import HOST_PATH, LIB_PATH
 
@@ -20,6 +20,8 @@ lib = C.CDLL(LIB_PATH)
 
 from . import _torch_host as host  # noqa: E402
 
+if host.torch_version != torch.__version__:    # it reads torch's own structures
+    raise ImportError("%s was built against torch %s, this is %s: build it again" % (HOST_PATH, host.torch_version, torch.__version__))
 host.bind(lib._handle)
 
 _vp, _i, _sz = C.c_void_p, C.c_int, C.c_size_t

@@ -335,4 +335,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_host", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_host(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__torch_host(void) {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", SG_TORCH_VERSION) != 0) {   // what it was built against (_lib.py)
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}
