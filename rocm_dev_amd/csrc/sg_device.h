@@ -27,7 +27,8 @@ __device__ __forceinline__ uint32_t bf16_bits(float x) {
     uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
     return ((u & 0x7fffffffu) > 0x7f800000u) ? ((u >> 16) | 0x40u) : r;
 }
-// Two at once by v_cvt_pk_bf16_f32: bf16_bits' result for each of the 2^32 inputs, NaNs included (compared on the device).
+// Two at once by v_cvt_pk_bf16_f32: the same result, NaNs included (tests/test_gpu_gemm.py, every upper half of a float over
+// the lower halves around the rounding boundary).
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));

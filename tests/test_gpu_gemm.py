@@ -912,3 +912,22 @@ def test_two_activation_tiles_on_the_skinny_ring(sg, oracle, m, n, k, tile_rows)
     # (against the model of the matrix instruction's summation: with these factors the sequential host sum itself lies
     # 0.0104 from it in one of the 524,288 outputs of 128 x 4096 x 4096, whichever kernel runs)
     assert oracle.max_rel_err_bf16(bits(D), rowcol_reference(oracle, a8, b8, scale, rs, cs, model=True)) <= GEMM_TOL
+
+
+@pytest.mark.parametrize("low", [0x0000, 0x0001, 0x7FFF, 0x8000, 0x8001, 0xFFFF])
+def test_rounding_to_bf16_of_every_upper_half(sg, oracle, low):
+    """The epilogues round pairs by one instruction: round to nearest even, NaN to a quiet NaN of the same sign and payload.
+    The sum is exactly 1 and the column factors are every upper half of a float - all signs, exponents, infinities, NaNs and
+    denormals - over the lower halves at and around the rounding boundary; a lower half acts only by how it compares to it."""
+    n, k = 65536, 256
+    u = (np.arange(n, dtype=np.uint32) << 16) | np.uint32(low)
+    one = np.zeros((1, k), dtype=np.uint8)
+    one[0, 7] = 0x38                                        # 1.0
+    cols = torch.from_numpy(u.view(np.float32)).cuda()
+    W = dev(np.repeat(one, n, 0))
+    D = torch.zeros((1, n), dtype=torch.bfloat16, device="cuda")
+    assert sg.skinny_gemm_rowcol(dev(one), W, D, None, None, cols) == 0
+    torch.cuda.synchronize()
+    nan = (u & 0x7FFFFFFF) > 0x7F800000
+    want = np.where(nan, (u >> 16) | 0x40, (u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    assert np.array_equal(bits(D)[0], want)

@@ -333,6 +333,9 @@ def test_the_tuner_keeps_the_record_a_wide_tile_replaced(table, tmp_path, monkey
 
 
 def test_wide_choice_of_shapes_and_refusals():
+    # below 24 us of work, below 9/16 of the CUs, and with no K split to take because the mid-batch record has none
+    for shape in ((300, 16384, 2048), (320, 1408, 17536), (1024, 8192, 28672)):
+        assert api.skinny_gemm_wide_choice(*shape) is None
     assert api.skinny_gemm_wide_choice(128, 57344, 8192) is None        # 128 rows: the mid-batch kernel
     assert api.skinny_gemm_wide_choice(1024, 57344, 8192, 8192 + 128) is not None
     assert api.skinny_gemm_wide_choice(1024, 512, 8192, (1 << 23) + 16) is None     # rows too far apart for its offsets
