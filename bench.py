@@ -110,6 +110,9 @@ def main():
                     help="only run the ingest probe (sg_debug_cu_ingest): what a CU takes in through direct-to-LDS loads from "
                          "beyond its XCD's L2 (cold), from inside it (hot), and from both at once out of the same or out of "
                          "different waves, with 16 and with 256 workgroups; prints a table, no JSON line")
+    ap.add_argument("--wide-against-mid", type=int, metavar="COUNT",
+                    help="only time COUNT seeded random shapes (129..2048 rows) that the library runs on a wide tile against the "
+                         "mid-batch record the tile replaces, in alternating rounds on cold weights; prints a table, no JSON line")
     ap.add_argument("--sparse", action="store_true",
                     help="with --stamps --launch-shapes: the 2:4 GEMM (sg_sparse24_gemm on weights pruned and compressed here) "
                          "instead of the dense one")
@@ -329,6 +332,37 @@ def main():
                                        rec[0], rec[1], rec[2], rec[3], rec[4], op_m, ops, None)
                 torch.cuda.synchronize()
             del wb
+        return
+
+    if args.wide_against_mid:
+        import math
+        import random
+        from rocm_dev_amd import autotune
+        rng = random.Random(0)
+        sg.tuning_clear()
+        ratios = []
+        print("| M x N x K | wide tile (split) | us | mid-batch record: tile (split) | us | ratio |\n|---|---|---|---|---|---|")
+        while len(ratios) < args.wide_against_mid:
+            m, n, k = (int(lo * (hi / lo) ** rng.random()) for lo, hi in ((129, 2049), (256, 60000), (256, 28672)))
+            step = 128 if rng.random() < 0.5 else 16          # every other one with whole K blocks and whole groups of columns
+            n, k = n // (64 if step == 128 else 2) * (64 if step == 128 else 2), k // step * step
+            if k <= 128 or n < 256 or n * k > 400 << 20 or 2 * m * n * k > 4e11 or not sg.api.skinny_gemm_wide_choice(m, n, k):
+                continue
+            rg, mb, split = sg.api.skinny_gemm_wide_choice(m, n, k)
+            mid, _ = sg.skinny_gemm_choice(m, n, k)
+            bench = autotune.Bench(m, n, k)
+            us = [[], []]
+            for _ in range(4):
+                for side, t in enumerate((sg.SgTuning(0, 1, 1, 1, 1, 2, 4, 1, 0, 0), mid)):
+                    us[side].append(bench.time(lib, t, launches=8, repeats=2))
+            wide_us, mid_us = (sorted(v)[1] for v in us)
+            ratios.append(wide_us / mid_us)
+            print("| %d x %d x %d | %d x %d (%d) | %.2f | %d x %d (%d) | %.2f | %.3f |"
+                  % (m, n, k, 32 * rg, 32 * mb, split, wide_us, 8 * mid.row_tiles * mid.waves, 32 * mid.m_blocks, mid.split_k, mid_us,
+                     ratios[-1]), flush=True)
+            del bench
+        print("geometric mean %.3f; %d of %d behind by more than 3 %%, the worst by %.0f %%"
+              % (math.exp(sum(map(math.log, ratios)) / len(ratios)), sum(r > 1.03 for r in ratios), len(ratios), 100 * (max(ratios) - 1)))
         return
 
     if args.stamps:
