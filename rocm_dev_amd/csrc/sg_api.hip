@@ -1213,9 +1213,9 @@ static Config heuristic_config(int m, int n, int k, int cu_count) {
 // these tiles on 243 random shapes (129..2048 rows, K of 512..32768, odd ones among them).  It ranks the tiles: on 1069
 // other shapes the times were 1.1 times what it says (geometric mean; 0.83 to 1.6, the highest with rows off their lines
 // at a K that 128 divides).  Below 24 us, where a tile's fixed part rules, and on launches that fill less than 9/16 of
-// the CUs (320 x 1408 x 17536 26.0 against 31.4) the mid-batch tiles are ahead, and where mid_stays_ahead says so;
-// elsewhere the wide ones, by up to 1.6 times (718 x 15360 x 13568 169.8 -> 123.8 us, 1024 x 57344 x 8192 466 -> 361,
-// 640 x 21120 x 23552 402 -> 248, 449 x 54816 x 512 54.2 -> 35.5).
+// the CUs (320 x 1408 x 17536 25.9 against 31.4) the mid-batch tiles are ahead, and where mid_stays_ahead says so;
+// elsewhere the wide ones (718 x 15360 x 13568 169 -> 124 us, 1024 x 57344 x 8192 469 -> 366,
+// 640 x 21120 x 23552 367 -> 261, 1024 x 10240 x 8192 106 -> 73).
 // Whose workspace it is does not change the result, so a K split of wide tiles is taken only where its partials fit what
 // sg_workspace_query asks for the mid-batch record; a tile without that split must then be within 10 % of the first.
 struct WideTile { int rg, mt; double stage_us, tile_us; };

@@ -9,15 +9,16 @@
 //
 // With one wave per SIMD whatever that wave waits for is idle time of its matrix core, so nothing is read in front of
 // its use and no burst of memory instructions stands between two MFMAs:
-//   * the wave's activation fragments of a stage are held in registers, two sets; the weight fragments stream
-//     through a ring of four, read three groups (of MH MFMAs) ahead of their use;
-//   * the barrier between two stages stands three groups before the end of a stage, where the last LDS read of the
-//     stage has been issued; behind it the three remaining groups read the next stage's first operands;
+//   * the wave's activation fragments of a stage are held in registers, two sets; the weight fragments stream through a
+//     ring of WR, read AHEAD groups (of MH MFMAs) ahead of their use: WR is RGW, 4 on the 8 x 8 tile, whose registers that
+//     leaves, and AHEAD one less, five at most;
+//   * the barrier between two stages stands AHEAD groups before the end of a stage, where the last LDS read of the stage
+//     has been issued; behind it the remaining groups read the next stage's first operands;
 //   * LDS reads and refills are dealt out one by one to the MFMAs they are issued in front of.
-// 1024 x 57344 x 8192 on 224 x 256 tiles, four full rounds: 2290 clocks a stage (1792 of MFMA; 1940 with the refill left
-// out, a direct-to-LDS instruction costs its wave 15) at 1.88 GHz, the clock that power leaves (2.39 on zeros), 500 -> 375
-// us; 1024 x 10240 x 8192 on 160 x 256 tiles 96 -> 74.  Tried and not kept: eight waves (410), loads masked by EXEC
-// instead of skipped by a branch (100 clocks a stage more).
+// 1024 x 57344 x 8192 on 224 x 256 tiles, four full rounds: 2310 clocks a stage, 1792 of them MFMA, at 1.92 GHz, the clock
+// that power leaves (profiles/wide_tile_gemm_time_stamps_and_counters.md; the mid-batch kernel 3230), 469 -> 366 us;
+// 1024 x 10240 x 8192 on 160 x 256 tiles 106 -> 73.  Tried and not kept: eight waves (410 us on the first), loads masked by
+// EXEC instead of skipped by a branch (100 clocks a stage more).
 //
 // All workgroups of one XCD walk K in step (the start of the walk depends on the XCD only), so that one XCD's L2
 // serves an activation line to all of them while it is there; the mid-batch kernel's rotation by weight tile spreads
