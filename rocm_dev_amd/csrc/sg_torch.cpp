@@ -120,9 +120,13 @@ struct Gemm {
 template <class Launch>
 PyObject* enqueue(Launch&& launch) {
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = launch();
-    Py_END_ALLOW_THREADS
+    {
+        struct Unlocked {      // (not the macros: an exception out of the launch must find the lock held again)
+            PyThreadState* state = PyEval_SaveThread();
+            ~Unlocked() { PyEval_RestoreThread(state); }
+        } unlocked;
+        rc = launch();
+    }
     return PyLong_FromLong(rc);
 }
 
