@@ -145,10 +145,10 @@ __global__ void __launch_bounds__(1024) fp8_encode_rows_long_kernel(const uint16
 // Eight codes per thread: one 8-byte load, one 16-byte store, both contiguous over a wave, the store non-temporal.
 // (8192 x 8192: 33.3 us; with 16 codes a thread the two stores of a lane interleave at 32 bytes and the launch takes 37.8,
 // and the 64-bit division for the row, now a multiply-high, another 0.3.)  cols % 16 == 0: no chunk straddles two rows.
-__global__ void __launch_bounds__(512) fp8_decode_rows_kernel(const uint8_t* __restrict__ Q, const float* __restrict__ scales,
+__global__ void __launch_bounds__(256) fp8_decode_rows_kernel(const uint8_t* __restrict__ Q, const float* __restrict__ scales,
                                                               uint16_t* __restrict__ Y, unsigned chunks_per_row,
                                                               unsigned inv_chunks_per_row, unsigned nchunks) {
-    const unsigned idx = blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned idx = blockIdx.x * 256 + threadIdx.x;
     if (idx >= nchunks) return;
     const float s = scales[fast_div(idx, chunks_per_row, inv_chunks_per_row)];
     const u32x2 q = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(Q) + idx);
@@ -272,9 +272,7 @@ int launch_fp8_decode_rows(const uint8_t* Q, const float* scales, void* Y, int r
     const unsigned per_row = (unsigned)cols >> 3, inv = div_reciprocal(per_row);
     return in_slabs(rows, per_row, [&](size_t r0, size_t nrows) {
         const unsigned nchunks = (unsigned)nrows * per_row;
-        // (small matrices in workgroups of 512: five workgroups take 0.13 us longer than three, 128 x 64 2.00 us, 1.82 this way)
-        const unsigned threads = nchunks <= 4096 ? 512 : 256;
-        fp8_decode_rows_kernel<<<(nchunks + threads - 1) / threads, threads, 0, stream>>>(
+        fp8_decode_rows_kernel<<<(nchunks + 255) / 256, 256, 0, stream>>>(
             Q + r0 * (size_t)cols, scales + r0, reinterpret_cast<uint16_t*>(Y) + r0 * (size_t)cols, per_row, inv, nchunks);
     });
 }
