@@ -316,21 +316,25 @@ __global__ void __launch_bounds__(WN * 128) wide_gemm_kernel(const StreamArgs a)
     // (With eight 2-byte stores a piece where 8 does not divide n: 1159 x 22756 x 880 78.0 us, now 44.7; 778 x 22364 x 2048
     // 80.1, now 51.8; the mid-batch kernel takes 48.6 and 63.0.)
     using u32x4_at4 = u32x4 __attribute__((aligned(4)));
+    auto store_rows = [&](auto ragged) __attribute__((always_inline)) {
 #pragma unroll 4
-    for (int i = lane; i < ROWS * PIECES; i += 64) {
-        const int row = i / PIECES, c = i - row * PIECES;
-        const int m_idx = m_wave + row, n_idx = n_wave + 8 * c;
-        if (m_idx >= a.m || n_idx >= a.n) continue;
-        uint16_t* const to = d + (size_t)m_idx * a.n + n_idx;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(mine + row * PITCH + 16 * c);
-        if (n_idx + 8 <= a.n) {
-            *reinterpret_cast<u32x4_at4*>(to) = v;
-        } else {
+        for (int i = lane; i < ROWS * PIECES; i += 64) {
+            const int row = i / PIECES, c = i - row * PIECES;
+            const int m_idx = m_wave + row, n_idx = n_wave + 8 * c;
+            if (m_idx >= a.m || n_idx >= a.n) continue;
+            uint16_t* const to = d + (size_t)m_idx * a.n + n_idx;
+            const u32x4 v = *reinterpret_cast<const u32x4*>(mine + row * PITCH + 16 * c);
+            if (!decltype(ragged)::value || n_idx + 8 <= a.n) {
+                *reinterpret_cast<u32x4_at4*>(to) = v;
+            } else {
 #pragma unroll
-            for (int e = 0; e < 3; e++)
-                if (n_idx + 2 * e < a.n) reinterpret_cast<uint32_t*>(to)[e] = v[e];
+                for (int e = 0; e < 3; e++)
+                    if (n_idx + 2 * e < a.n) reinterpret_cast<uint32_t*>(to)[e] = v[e];
+            }
         }
-    }
+    };
+    if ((a.n & 7) == 0) store_rows(std::false_type{});   // no piece crosses n
+    else store_rows(std::true_type{});
     stamps.end(a);
 }
 
