@@ -30,9 +30,10 @@ int sg_debug_wide_gemm(const uint8_t* A, const uint8_t* B, void* D_bf16, const f
                        const float* col_scales, int m, int n, int k, int b_stride, int row_tiles, int m_blocks, int split_k,
                        void* stream);
 
-/* Which wide tile sg_skinny_gemm_auto launches for the shape and row stride: out = {row_tiles, m_blocks, split_k} as
- * sg_debug_wide_gemm takes them, or three zeros where it launches the record that sg_skinny_gemm_choice reports. */
-int sg_debug_wide_choice(int m, int n, int k, int b_stride, int out[3]);
+/* Which wide tile sg_skinny_gemm_auto - with factors: sg_skinny_gemm_rowcol with row or column factors - launches for the
+ * shape and row stride: out = {row_tiles, m_blocks, split_k} as sg_debug_wide_gemm takes them, or three zeros where it
+ * launches the record that sg_skinny_gemm_choice reports. */
+int sg_debug_wide_choice(int m, int n, int k, int b_stride, int factors, int out[3]);
 
 /* Profiling aid, no counterpart in the reference: reads the n x k weight matrix B (row stride b_stride, k % 1024 == 0)
  * the way the persistent LDS-ring GEMM streams it - one workgroup per CU walking row tiles, eight waves sharing K,

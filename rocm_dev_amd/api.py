@@ -310,11 +310,11 @@ def skinny_gemm_choice(m, n, k):
     return t, bool(from_table.value)
 
 
-def skinny_gemm_wide_choice(m, n, k, b_stride=None):
-    """(row_tiles, m_blocks, split_k) of the wide tile the fastpath launches for the shape, or None where it launches the
-    record that skinny_gemm_choice reports."""
+def skinny_gemm_wide_choice(m, n, k, b_stride=None, factors=False):
+    """(row_tiles, m_blocks, split_k) of the wide tile the fastpath (with factors: skinny_gemm_rowcol with row or column
+    factors) launches for the shape, or None where it launches the record that skinny_gemm_choice reports."""
     out = (C.c_int * 3)()
-    rc = lib.sg_debug_wide_choice(m, n, k, k if b_stride is None else b_stride, C.byref(out))
+    rc = lib.sg_debug_wide_choice(m, n, k, k if b_stride is None else b_stride, 1 if factors else 0, C.byref(out))
     if rc != 0:
         raise SgError(rc)
     return tuple(out) if out[0] else None

@@ -1225,14 +1225,16 @@ static const WideTile kWideTiles[] = {{4, 8, 0.829, 6.45}, {5, 8, 0.933, 7.48}, 
 // on both (129..2048 rows, 900 random, the others drawn from where the rules lie) 955 go to a wide tile, 1.18 times faster
 // (geometric mean), 34 of them behind by more than 3 % and 6 by more than 10 % (151 x 16708 x 24192 by 17 %); without
 // these rules 113 of 1069 were, up to 1.34 times.
-static bool mid_stays_ahead(const Config& mid, const Config& wide, double wide_us, int m, int n, int k, int b_stride, int cu_count) {
+static bool mid_stays_ahead(const Config& mid, const Config& wide, double wide_us, int m, int n, int k, int b_stride, bool factors, int cu_count) {
     // A K split five to eight ways, where a wide tile goes to four at most and mid_model_us (which knows whole K blocks only)
     // puts the mid-batch launch 5 % ahead of four ways or 9 % ahead of three: 208 x 2304 x 20864 29.6 us against 37.9,
     // 525 x 1024 x 28032 40.6 against 49.9, 856 x 1536 x 27776 61.4 against 67.9.
     if (k % 128 == 0 && mid.split_k > 4 && wide.split_k >= 3)
         return mid_model_us(m, n, k, 8 * mid.rg * mid.waves, 32 * mid.mt, mid.split_k, cu_count) < (wide.split_k == 4 ? 0.95 : 0.91) * wide_us;
-    // The fourteen-wave tiles - except where four does not divide n, which costs the mid-batch epilogue more than any tile.
-    if (mid.waves != 14 || n % 4 != 0) return false;
+    // The fourteen-wave tiles - except where four does not divide n or where there are row or column factors: either costs the
+    // mid-batch epilogue more than any tile (363 x 23320 x 1088 with factors 34.8 us against 24.9; of the 52 shapes timed that
+    // the rules below would name, three were ahead with factors, the 52 1.11 times slower in the geometric mean).
+    if (mid.waves != 14 || n % 4 != 0 || factors) return false;
     const bool whole_lines = k % 128 == 0 && b_stride % 128 == 0;
     if (mid.mt == 4) {
         // 224 x 128 tiles against wide ones of the same 128 rows: level to 17 % ahead on 26 shapes (266 x 17856 x 4432 54.1 us
@@ -1248,7 +1250,7 @@ static bool mid_stays_ahead(const Config& mid, const Config& wide, double wide_u
     return mid.mt == 8 && !whole_lines && m < 400 && k <= 2000;
 }
 
-static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, int cu_count, const Workspace* fixed_ws, Config* out) {
+static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, bool factors, int cu_count, const Workspace* fixed_ws, Config* out) {
     if (m <= 128 || mid.engine != ENGINE_MID || b_stride > kWidePitch || k > kWidePitch) return false;
     size_t partial_limit, counters;
     workspace_need(mid, m, n, &partial_limit, &counters);
@@ -1280,7 +1282,7 @@ static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, in
         }
     }
     if (best < 24.0 || best > 1.1 * first || best_wgs * 16 < (long)cu_count * 9) return false;
-    if (mid_stays_ahead(mid, c, best, m, n, k, b_stride, cu_count)) return false;
+    if (mid_stays_ahead(mid, c, best, m, n, k, b_stride, factors, cu_count)) return false;
     c.engine = ENGINE_MID;
     c.waves = 4;
     c.wide = true;
@@ -1353,7 +1355,7 @@ static int launch_chosen(const StreamArgs& a, int cu_count, hipStream_t stream, 
         }
     }
     Config c = heuristic_config(a.m, a.n, a.k, cu_count), wide;
-    if (wide_config(c, a.m, a.n, a.k, a.b_stride, cu_count, fixed_ws, &wide)) {
+    if (wide_config(c, a.m, a.n, a.k, a.b_stride, a.row_scale || a.col_scale, cu_count, fixed_ws, &wide)) {
         wide.fixed_ws = fixed_ws;
         const int rc = launch_config(wide, a, stream);
         if (!rejected_before_launch(rc)) return rc;
@@ -1548,7 +1550,7 @@ int sg_debug_wide_gemm(const uint8_t* A, const uint8_t* B, void* D, const float*
     return launch_config(c, a, static_cast<hipStream_t>(stream));
 }
 
-int sg_debug_wide_choice(int m, int n, int k, int b_stride, int out[3]) {
+int sg_debug_wide_choice(int m, int n, int k, int b_stride, int factors, int out[3]) {
     if (!out || m <= 0 || n <= 0 || k <= 0 || b_stride < k) return SG_BAD_ARGUMENT;
     out[0] = out[1] = out[2] = 0;
     SgTuning t;
@@ -1557,7 +1559,7 @@ int sg_debug_wide_choice(int m, int n, int k, int b_stride, int out[3]) {
     int cu = 256;
     if (get_device_info(&dev) == SG_SUCCESS) cu = dev->cu_count;
     Config wide;
-    if (wide_config(heuristic_config(m, n, k, cu), m, n, k, b_stride, cu, nullptr, &wide)) {
+    if (wide_config(heuristic_config(m, n, k, cu), m, n, k, b_stride, factors != 0, cu, nullptr, &wide)) {
         out[0] = wide.rg; out[1] = wide.mt; out[2] = wide.split_k;
     }
     return SG_SUCCESS;
@@ -1675,7 +1677,7 @@ int sg_skinny_gemm_tuned(const uint8_t* A, const uint8_t* B, void* D, const floa
     if (c.engine == ENGINE_AUTO) {
         c = heuristic_config(m, n, k, dev->cu_count);
         Config wide;
-        if (wide_config(c, m, n, k, b_stride, dev->cu_count, nullptr, &wide)) c = wide;
+        if (wide_config(c, m, n, k, b_stride, false, dev->cu_count, nullptr, &wide)) c = wide;
     }
     if (c.engine != ENGINE_MID && c.mt != 1 && c.mt != 2) return SG_INVALID_CONFIG;
     StreamArgs a{};
@@ -1701,7 +1703,7 @@ int sg_skinny_gemm_tuned_noalloc(const uint8_t* A, const uint8_t* B, void* D, co
     if (c.engine == ENGINE_AUTO) {
         c = heuristic_config(m, n, k, dev->cu_count);
         Config wide;
-        if (wide_config(c, m, n, k, b_stride, dev->cu_count, &w, &wide)) c = wide;
+        if (wide_config(c, m, n, k, b_stride, false, dev->cu_count, &w, &wide)) c = wide;
         // the library's own choice is made to fit the array: a K split whose partials or counters do not, is not taken
         size_t partial_bytes, counters;
         workspace_need(c, m, n, &partial_bytes, &counters);

@@ -358,3 +358,6 @@ def test_mid_batch_launches_that_stay_ahead_of_the_wide_tile():
             (1024, 57344, 8192, 8192): True, (1024, 28672, 4096, 4096): True}
     for (m, n, k, stride), wide in want.items():
         assert (api.skinny_gemm_wide_choice(m, n, k, stride) is not None) == wide, (m, n, k, stride)
+        # with row or column factors, which the fourteen-wave tiles pay most for, only the K splits stay
+        split = api.skinny_gemm_choice(m, n, k)[0].split_k > 4
+        assert (api.skinny_gemm_wide_choice(m, n, k, stride, factors=True) is not None) == (wide or not split), (m, n, k, stride)
