@@ -1240,10 +1240,13 @@ static bool mid_stays_ahead(const Config& mid, const Config& wide, double wide_u
         // 224 x 128 tiles against wide ones of the same 128 rows: level to 17 % ahead on 26 shapes (266 x 17856 x 4432 54.1 us
         // against 63.3, 384 x 18432 x 3072 level) ...
         if (wide.rg == 8 && wide.mt == 4) return true;
-        // ... and wherever they fill every round, on rows of whole lines: 1024 x 7168 x 4096 37.2 us against 39.9, 512 x 14336 x
-        // 7168 60.9 against 64.9 (rows off their lines, 1024 x 7168 x 10240: 118 against 97).
-        const long wgs = (long)((n + 223) / 224) * ((m + 127) / 128);
-        return whole_lines && wgs % cu_count == 0;
+        // ... and where more than two of them, all but full, stand over m and they fill every round, on rows of whole lines:
+        // 1024 x 7168 x 4096 37.2 us against 39.9, 512 x 14336 x 7168 60.9 against 64.9, 1..7 % on 27 of 36 shapes, within 2 % on
+        // the others.  (Part of a tile empty, 412 x 14208 x 4096: 39.6 against 33.9; two tiles: level; rows off their lines,
+        // 1024 x 7168 x 10240: 118 against 97.)
+        const int m_tiles = (m + 127) / 128;
+        const long wgs = (long)((n + 223) / 224) * m_tiles;
+        return whole_lines && m_tiles > 2 && m * 16L > m_tiles * 128L * 15 && wgs % cu_count == 0;
     }
     // 224 x 256 tiles on rows off their 128-byte lines with a short K and few rows, where loads and stores are all there is:
     // level to 13 % ahead on 23 shapes (315 x 53428 x 640, rows 656 apart, 35.2 us against 39.7).

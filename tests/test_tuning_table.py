@@ -352,7 +352,8 @@ def test_mid_batch_launches_that_stay_ahead_of_the_wide_tile():
     224 x 128, a short K with rows off their lines.  (m, n, k, row stride) -> a wide tile?"""
     want = {(208, 2304, 20864, 20864): False, (525, 1024, 28032, 28032): False, (856, 1536, 27776, 27776): False,
             (720, 3904, 17920, 18048): True, (1202, 1792, 12800, 12800): True,
-            (1024, 7168, 4096, 4096): False, (512, 14336, 7168, 7168): False, (1024, 7168, 10240, 10256): True, (1024, 6144, 8192, 8192): True,
+            (1024, 7168, 4096, 4096): False, (512, 14336, 7168, 7168): False, (1024, 7168, 10240, 10256): True,
+            (412, 14208, 4096, 4096): True, (250, 28608, 4096, 4096): True, (1024, 6144, 8192, 8192): True,
             (266, 17856, 4432, 4432): False, (289, 37688, 9936, 10064): False, (309, 36386, 688, 688): True,
             (315, 53428, 640, 656): False, (297, 46296, 576, 704): False, (645, 37240, 256, 272): True,
             (1024, 57344, 8192, 8192): True, (1024, 28672, 4096, 4096): True}
