@@ -1221,21 +1221,31 @@ static Config heuristic_config(int m, int n, int k, int cu_count) {
 struct WideTile { int rg, mt; double stage_us, tile_us; };
 static const WideTile kWideTiles[] = {{4, 8, 0.829, 6.45}, {5, 8, 0.933, 7.48}, {6, 8, 1.064, 8.96}, {7, 8, 1.149, 9.83},
                                       {8, 8, 1.249, 11.03}, {8, 4, 0.949, 6.48}, {4, 4, 0.620, 3.93}};
-// Mid-batch launches that the model does not know of and that a wide tile loses to.  Of 1960 shapes timed
-// on both (129..2048 rows, 900 random, the others drawn from where the rules lie) 955 go to a wide tile, 1.18 times faster
-// (geometric mean), 34 of them behind by more than 3 % and 6 by more than 10 % (151 x 16708 x 24192 by 17 %); without
-// these rules 113 of 1069 were, up to 1.34 times.
+// Mid-batch launches that the model does not know of and that a wide tile loses to.  Of 3220 shapes timed
+// on both (129..2048 rows, 900 random, the others drawn from where the rules lie) 1468 go to a wide tile, 1.15 times faster
+// (geometric mean), 60 of them behind by more than 3 % and 10 by more than 10 % (266 x 6296 x 3088 by 18 %); without these
+// rules 170 of 1635 were, up to 1.34 times (profiles/wide_tile_against_mid_batch.md, which has them with factors too).
 static bool mid_stays_ahead(const Config& mid, const Config& wide, double wide_us, int m, int n, int k, int b_stride, bool factors, int cu_count) {
     // A K split five to eight ways, where a wide tile goes to four at most and mid_model_us (which knows whole K blocks only)
     // puts the mid-batch launch 5 % ahead of four ways or 9 % ahead of three: 208 x 2304 x 20864 29.6 us against 37.9,
     // 525 x 1024 x 28032 40.6 against 49.9, 856 x 1536 x 27776 61.4 against 67.9.
     if (k % 128 == 0 && mid.split_k > 4 && wide.split_k >= 3)
         return mid_model_us(m, n, k, 8 * mid.rg * mid.waves, 32 * mid.mt, mid.split_k, cu_count) < (wide.split_k == 4 ? 0.95 : 0.91) * wide_us;
+    const bool whole_lines = k % 128 == 0 && b_stride % 128 == 0;
+    // A round of 64-row tiles, unsplit, on rows of whole lines, where m lies just beyond a multiple of the wide tile's height
+    // and its fewer workgroups multiply padding: 295 x 6368 x 5248 250 workgroups against 150, 27.8 us against 33.4; 428 x 4508
+    // x 4608 25.2 against 29.7.  Level to 20 % ahead on 13 shapes, with factors on 7 of 8 (rows off their lines: from 18 %
+    // ahead to 20 % behind).
+    if (mid.split_k == 1 && mid.mt == 2 && n % 4 == 0 && whole_lines) {
+        const int bn = 8 * mid.rg * mid.waves;
+        const long wgs = (long)((n + bn - 1) / bn) * ((m + 63) / 64);
+        const long wide_wgs = (long)((n + 32 * wide.rg - 1) / (32 * wide.rg)) * ((m + 32 * wide.mt - 1) / (32 * wide.mt)) * wide.split_k;
+        if (wgs <= cu_count && wgs * 5 > wide_wgs * 6) return true;
+    }
     // The fourteen-wave tiles - except where four does not divide n or where there are row or column factors: either costs the
     // mid-batch epilogue more than any tile (363 x 23320 x 1088 with factors 34.8 us against 24.9; of the 52 shapes timed that
     // the rules below would name, three were ahead with factors, the 52 1.11 times slower in the geometric mean).
     if (mid.waves != 14 || n % 4 != 0 || factors) return false;
-    const bool whole_lines = k % 128 == 0 && b_stride % 128 == 0;
     if (mid.mt == 4) {
         // 224 x 128 tiles against wide ones of the same 128 rows: level to 17 % ahead on 26 shapes (266 x 17856 x 4432 54.1 us
         // against 63.3, 384 x 18432 x 3072 level) ...

@@ -349,16 +349,17 @@ def test_wide_choice_of_shapes_and_refusals():
 def test_mid_batch_launches_that_stay_ahead_of_the_wide_tile():
     """Shapes on which the wide tile was timed behind the mid-batch launch it would have replaced, with one beside each kind
     on which it is ahead: K splits of five ways and more, 224 x 128 tiles that fill every round, 256 x 128 wide tiles against
-    224 x 128, a short K with rows off their lines.  (m, n, k, row stride) -> a wide tile?"""
+    224 x 128, a short K with rows off their lines, a round of 64-row tiles just beyond 128 or 256 rows.  (m, n, k, row stride) -> a wide tile?"""
     want = {(208, 2304, 20864, 20864): False, (525, 1024, 28032, 28032): False, (856, 1536, 27776, 27776): False,
             (720, 3904, 17920, 18048): True, (1202, 1792, 12800, 12800): True,
             (1024, 7168, 4096, 4096): False, (512, 14336, 7168, 7168): False, (1024, 7168, 10240, 10256): True,
             (412, 14208, 4096, 4096): True, (250, 28608, 4096, 4096): True, (1024, 6144, 8192, 8192): True,
             (266, 17856, 4432, 4432): False, (289, 37688, 9936, 10064): False, (309, 36386, 688, 688): True,
             (315, 53428, 640, 656): False, (297, 46296, 576, 704): False, (645, 37240, 256, 272): True,
+            (295, 6368, 5248, 5248): False, (131, 9348, 4992, 4992): False, (384, 6368, 5248, 5248): True,
             (1024, 57344, 8192, 8192): True, (1024, 28672, 4096, 4096): True}
     for (m, n, k, stride), wide in want.items():
         assert (api.skinny_gemm_wide_choice(m, n, k, stride) is not None) == wide, (m, n, k, stride)
-        # with row or column factors, which the fourteen-wave tiles pay most for, only the K splits stay
-        split = api.skinny_gemm_choice(m, n, k)[0].split_k > 4
-        assert (api.skinny_gemm_wide_choice(m, n, k, stride, factors=True) is not None) == (wide or not split), (m, n, k, stride)
+        # with row or column factors, which the fourteen-wave tiles pay most for, the other kinds stay
+        fourteen = api.skinny_gemm_choice(m, n, k)[0].waves == 14
+        assert (api.skinny_gemm_wide_choice(m, n, k, stride, factors=True) is not None) == (wide or fourteen), (m, n, k, stride)
