@@ -359,10 +359,13 @@ static int launch_lds(const Config& c, StreamArgs a, hipStream_t stream) {
         if (threads > 1024) return SG_TOO_MANY_WARPS;
         size_t lds_x = (size_t)c.waves * c.depth * c.rg * 4096 + 2u * c.waves * c.rg * c.mt * 1024;
         if (lds_x > 159 * 1024) return SG_INVALID_CONFIG;
+        const size_t factor_bytes = workgroup_factor_bytes(a, tiles, grid, 16 * c.rg, lds_x, 160 * 1024);
         // room for one more 4 KB staging block per wave (the kernel has no static LDS: all 160 KB may be asked for):
         // the activation fragments then reach the registers without the first weight stages being waited for
-        a.x_extra = (c.mt == 2 && pt == 2 && lds_x + (size_t)c.waves * 4096 <= 160 * 1024) ? 1 : 0;
+        a.x_extra = (c.mt == 2 && pt == 2 && lds_x + factor_bytes + (size_t)c.waves * 4096 <= 160 * 1024) ? 1 : 0;
         if (a.x_extra) lds_x += (size_t)c.waves * 4096;
+        a.factor_off = factor_bytes ? (int)lds_x : 0;
+        lds_x += factor_bytes;
         a.stamps = take_stamps(grid);
         return launch_xreg(c.mt, c.rg, pt, c.depth, a, grid, threads, lds_x, stream);
     } else if (c.persist > 0) {
@@ -378,6 +381,11 @@ static int launch_lds(const Config& c, StreamArgs a, hipStream_t stream) {
         DeviceInfo* dev;
         if (int rc = get_device_info(&dev)) return rc;
         grid = level_persistent_grid(grid, (size_t)dev->cu_count * c.persist);
+        if (a.m_tiles == 1) {
+            const size_t factor_bytes = workgroup_factor_bytes(a, tiles, grid, 16 * c.rg, lds, 159 * 1024);
+            a.factor_off = factor_bytes ? (int)lds : 0;
+            lds += factor_bytes;
+        }
     }
     if (lds > 159 * 1024) return SG_INVALID_CONFIG;  // 160 KB per CU, minus the kernel's static LDS
     if (a.A16) {   // only the resident-activation kernel quantises bf16 activations itself

@@ -33,6 +33,7 @@ struct StreamArgs {
     int split_k, waves;
     int n_tiles, m_tiles;
     int out_f32;
+    int factor_off;         // register-resident kernel: where in the launch's LDS the row and column factors are staged, or 0
     unsigned inv_n_tiles, inv_split_k, inv_waves;  // div_reciprocal() of n_tiles, split_k, waves (set_reciprocals)
     unsigned long long* stamps;  // profiling aid, normally nullptr: kStampWords time stamps per workgroup (sg_debug_stamps)
     int x_extra;            // register-resident kernel: 1 = the launch's LDS has one more 4 KB staging block per wave behind the reduction scratch
@@ -105,43 +106,48 @@ __device__ __forceinline__ int blocks_of_wave(const StreamArgs& a, int n_blk, in
     return wave < n_blk ? (int)fast_div((unsigned)(n_blk - wave + a.waves - 1), (unsigned)a.waves, a.inv_waves) : 0;
 }
 
-// Writes one finished 16(n) x 16(m) fragment: lane owns m = m_base + l%16, n = n_base + 4*(l/16)..+3.
-// `lds_row_scale`, when given, is a per-row factor table in LDS (the scales of activations quantised in the kernel)
-// that takes the place of a.row_scale.
-// `col_factors`, when given, holds a.col_scale[n_idx .. n_idx + 3] fetched ahead of time (col_scale_ahead).
+// The scale as a scalar load: the pointer's memory does not change during a launch, and a vector load would put a wait for
+// every outstanding DMA (the compiler does not see those) in front of its first use.
+__device__ __forceinline__ float scalar_scale(const StreamArgs& a) {
+    return a.scale ? *(const __attribute__((address_space(4))) float*)a.scale : 1.0f;
+}
+// 64 lanes x 4 bytes from global memory to LDS [lds_base + 4*lane]; lds_base is wave-uniform
+__device__ __forceinline__ void dma_256b(const void* gptr, unsigned lds_base) {
+    lds_base = __builtin_amdgcn_readfirstlane(lds_base);
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(gptr), "s"(lds_base) : "memory", "m0");
+}
+// What a lane multiplies its part of a fragment with, 1.0f where there is no such factor: a.col_scale[n_idx .. n_idx + 3]
+// and a.row_scale[m_idx].  Column factors are floats, so 4-byte aligned; one load where all four exist.  Indices past the
+// edge give a value that is never stored.
+typedef float f32x4_at4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned int u32x2_at4 __attribute__((ext_vector_type(2), aligned(4)));
 __device__ __forceinline__ f32x4 col_scale_ahead(const StreamArgs& a, int n_idx) {
     f32x4 c = {1.0f, 1.0f, 1.0f, 1.0f};
     if (a.col_scale) {
+        if (n_idx + 3 < a.n) {
+            c = *reinterpret_cast<const f32x4_at4*>(a.col_scale + n_idx);
+        } else {
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-            if (n_idx + e < a.n) c[e] = a.col_scale[n_idx + e];
+            for (int e = 0; e < 3; e++)
+                if (n_idx + e < a.n) c[e] = a.col_scale[n_idx + e];
+        }
     }
     return c;
 }
+__device__ __forceinline__ float row_scale_ahead(const StreamArgs& a, int m_idx) {
+    return a.row_scale ? a.row_scale[m_idx < a.m ? m_idx : a.m - 1] : 1.0f;
+}
+
+// Writes one finished and scaled 16(n) x 16(m) fragment: lane owns m = m_base + l%16, n = n_base + 4*(l/16)..+3.
 // Columns from `n_limit` on belong to another tile (24-row tiles computed with two 16-row fragments) and are not written.
-__device__ __forceinline__ void store_fragment(const StreamArgs& a, f32x4 v, float scale, int m_idx, int n_idx,
-                                               const float* lds_row_scale = nullptr, const f32x4* col_factors = nullptr,
-                                               int n_limit = 0x7fffffff) {
-    // Pin the fragment before the lane-divergent exit below.  An MFMA needs every lane of the wave
-    // (it reads all lanes' operand registers), but the compiler is free to sink the loads and the
-    // MFMA that produce `v` into the region where only lanes with m_idx < m are active - it did so
-    // with the 16x16x128 instruction - and the operand rows supplied by the masked lanes are then garbage.
-    asm volatile("" : "+v"(v));
+// One store where all four columns exist: 4-byte alignment is all that it needs, which an even n gives a bf16 row.
+__device__ __forceinline__ void store_scaled(const StreamArgs& a, f32x4 v, int m_idx, int n_idx, int n_limit = 0x7fffffff) {
     if (m_idx >= a.m || n_idx >= n_limit) return;
-    // scale, then the row factor, then the column factors: three separately rounded fp32 products
-    v *= scale;
-    if (lds_row_scale) v *= lds_row_scale[m_idx];
-    else if (a.row_scale) v *= a.row_scale[m_idx];
-    if (a.col_scale) {
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            if (n_idx + e < a.n) v[e] *= col_factors ? (*col_factors)[e] : a.col_scale[n_idx + e];
-    }
     const size_t off = (size_t)m_idx * a.n + n_idx;
     if (a.out_f32) {
         float* d = reinterpret_cast<float*>(a.D) + off;
-        if (n_idx + 3 < a.n && (a.n & 3) == 0) {
-            *reinterpret_cast<f32x4*>(d) = v;
+        if (n_idx + 3 < a.n) {
+            *reinterpret_cast<f32x4_at4*>(d) = v;
         } else {
 #pragma unroll
             for (int e = 0; e < 4; e++)
@@ -149,9 +155,9 @@ __device__ __forceinline__ void store_fragment(const StreamArgs& a, f32x4 v, flo
         }
     } else {
         uint16_t* d = reinterpret_cast<uint16_t*>(a.D) + off;
-        if (n_idx + 3 < a.n && (a.n & 3) == 0) {
+        if (n_idx + 3 < a.n && (a.n & 1) == 0) {
             u32x2 p = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-            *reinterpret_cast<u32x2*>(d) = p;
+            *reinterpret_cast<u32x2_at4*>(d) = p;
         } else {
 #pragma unroll
             for (int e = 0; e < 4; e++)
@@ -160,23 +166,114 @@ __device__ __forceinline__ void store_fragment(const StreamArgs& a, f32x4 v, flo
     }
 }
 
+// Scales a finished fragment and writes it: scale, then the row factor, then the column factors, three separately rounded
+// fp32 products.  The factors either come along, requested ahead by a wave that has nothing else under way, or are loaded
+// here - inside the branches, so that a launch without them waits for nothing.
+// Either way `v` is pinned before the first lane-divergent branch.  An MFMA needs every lane of the wave (it reads all
+// lanes' operand registers), but the compiler is free to sink the loads and the MFMA that produce `v` into the region where
+// only lanes with m_idx < m are active - it did so with the 16x16x128 instruction - and the operand rows supplied by the
+// masked lanes are then garbage.
+__device__ __forceinline__ void store_fragment(const StreamArgs& a, f32x4 v, float scale, int m_idx, int n_idx, float row, const f32x4& col) {
+    asm volatile("" : "+v"(v));
+    v *= scale;
+    v *= row;
+    v *= col;
+    store_scaled(a, v, m_idx, n_idx);
+}
+__device__ __forceinline__ void store_fragment(const StreamArgs& a, f32x4 v, float scale, int m_idx, int n_idx) {
+    asm volatile("" : "+v"(v));
+    v *= scale;
+    if (a.row_scale) v *= row_scale_ahead(a, m_idx);
+    if (a.col_scale) v *= col_scale_ahead(a, n_idx);
+    store_scaled(a, v, m_idx, n_idx);
+}
+
+// The row and column factors of one tile (up to 32 activation rows, 64 weight rows), in LDS by way of the same direct
+// loads as the operands: the first ones of wave 0's queue, so that they have landed long before the epilogue, where a
+// load would be a round trip with nothing else under way (and was four of them, one branch per column:
+// with factors 8 x 4096 x 4096 5.35 -> 5.07 us, 8 x 6144 x 4096 6.88 -> 6.62, 32 x 6144 x 4096 8.77 -> 7.99; without 4.95, 6.53
+// and 7.9).
+constexpr int kStagedFactors = 64 + 64;   // columns, rows; floats
+struct StagedFactors {
+    const float* lds;
+    // called by one wave; complete once its vmcnt says so, visible to the others behind a barrier
+    __device__ __forceinline__ void fetch(const StreamArgs& a, int m0, int n0, int lane) const {
+        const unsigned to = (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)lds;
+        if (a.col_scale) dma_256b(a.col_scale + (n0 + lane < a.n ? n0 + lane : a.n - 1), to);
+        if (a.row_scale) dma_256b(a.row_scale + (m0 + lane < a.m ? m0 + lane : a.m - 1), to + 256);
+    }
+    __device__ __forceinline__ void apply(const StreamArgs& a, f32x4& v, int rg, int mt, int r, int g) const {
+        if (a.row_scale) v *= lds[64 + mt * 16 + r];
+        if (a.col_scale) v *= *reinterpret_cast<const f32x4*>(lds + rg * 16 + 4 * g);
+    }
+};
+
+// The same for a persistent workgroup, whose tiles are consecutive: 64 row factors (up to 32 used), then the column factors
+// of all its tiles.  Its waves store between their stages, and a load that such a wave waits for drains its ring, a load
+// that any streaming wave issues makes every later vmcnt(n) wait for one DMA more; the epilogue wave, where there is one,
+// would pay a round trip per tile (8 x 28672 x 4096 with factors 21.8 -> 19.8 us, 12 x 57344 x 8192 78.5 -> 74.3,
+// 32 x 28672 x 4096 26.3 -> 22.8; without 19.8, 73.9 and 21.9).  Where the launch's LDS has no
+// room (lds is null) store_fragment loads them.
+struct WorkgroupFactors {
+    const float* lds;
+    // by the streaming waves `wave` of `waves`, in front of everything else in their queues
+    __device__ __forceinline__ void fetch(const StreamArgs& a, int first, int count, int wave, int waves, int lane) const {
+        if (!lds) return;
+        const unsigned to = (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)lds;
+        if (a.row_scale && wave == 0) dma_256b(a.row_scale + (lane < a.m ? lane : a.m - 1), to);
+        if (a.col_scale)
+            for (int c = wave * 64; c < count; c += waves * 64)
+                dma_256b(a.col_scale + (first + c + lane < a.n ? first + c + lane : a.n - 1), to + 256 + (unsigned)c * 4);
+    }
+    // Scales and writes a finished fragment (v pinned as in store_fragment): m, n_idx its place, i that of n_idx among the
+    // workgroup's columns; xscale: row factors in LDS that take the place of a.row_scale, or nullptr.  Every load stands in
+    // a branch with its use, so that none makes the others wait for what is outstanding in the wave's queue.
+    __device__ __forceinline__ void store(const StreamArgs& a, f32x4 v, float scale, const float* xscale, int m, int n_idx, int i) const {
+        asm volatile("" : "+v"(v));
+        v *= scale;
+        if (xscale) v *= xscale[m];
+        else if (a.row_scale) {
+            if (lds) v *= lds[m];
+            else v *= row_scale_ahead(a, m);
+        }
+        if (a.col_scale) {
+            if (lds) v *= *reinterpret_cast<const f32x4*>(lds + 64 + i);
+            else v *= col_scale_ahead(a, n_idx);
+        }
+        store_scaled(a, v, m, n_idx);
+    }
+};
+// ... and the LDS it takes on top of `used` of at most `limit` bytes (0: no factors, or no room)
+inline size_t workgroup_factor_bytes(const StreamArgs& a, size_t tiles, size_t grid, int tile_rows, size_t used, size_t limit) {
+    if (!a.row_scale && !a.col_scale) return 0;
+    const size_t bytes = 256 + (((tiles + grid - 1) / grid * tile_rows + 63) / 64) * 256;
+    return used + bytes <= limit ? bytes : 0;
+}
+
 template <int RG, int MT>
 __device__ __forceinline__ void finish_tile(const StreamArgs& a, f32x4 (&acc)[RG][MT], f32x4* red, unsigned* arrival_lds,
-                                            int tile_m, int tile_n, int split, int m0, int n0, int n_limit = 0x7fffffff) {
+                                            float scale, const StagedFactors& factors, int tile_m, int tile_n, int split, int m0, int n0,
+                                            int n_limit = 0x7fffffff) {
     constexpr int FRAGS = RG * MT;
     const int lane = lane_id();
     const int wave = wave_id();
     const int waves = a.waves;
     const int r = lane & 15, g = lane >> 4;
     unsigned& arrival = *arrival_lds;
-    const float scale = a.scale ? a.scale[0] : 1.0f;
     const int tile_id = tile_m * a.n_tiles + tile_n;
     float* ws_tile = a.ws + ((size_t)tile_id * a.split_k) * (FRAGS * 256);
 
-    auto finish = [&](int f, f32x4 v) __attribute__((always_inline)) {
+    // scale, then the row factor, then the column factors: three separately rounded fp32 products (v pinned as above)
+    auto finish_output = [&](int f, f32x4 v) __attribute__((always_inline)) {
         const int rg = f / MT, mt = f % MT;
+        asm volatile("" : "+v"(v));
+        v *= scale;
+        factors.apply(a, v, rg, mt, r, g);
+        store_scaled(a, v, m0 + mt * 16 + r, n0 + rg * 16 + 4 * g, n_limit);
+    };
+    auto finish = [&](int f, f32x4 v) __attribute__((always_inline)) {
         if (a.split_k == 1) {
-            store_fragment(a, v, scale, m0 + mt * 16 + r, n0 + rg * 16 + 4 * g, nullptr, nullptr, n_limit);
+            finish_output(f, v);
         } else {
             // agent-scope stores go through to memory, past this XCD's L2, so that a workgroup on
             // another XCD can read them without any cache-wide write-back or invalidate
@@ -223,8 +320,7 @@ __device__ __forceinline__ void finish_tile(const StreamArgs& a, f32x4 (&acc)[RG
 #pragma unroll
             for (int e = 0; e < 4; e++) v[e] += __hip_atomic_load(q + e * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        const int rg = f / MT, mt = f % MT;
-        store_fragment(a, v, scale, m0 + mt * 16 + r, n0 + rg * 16 + 4 * g, nullptr, nullptr, n_limit);
+        finish_output(f, v);
     }
     if (threadIdx.x == 0)  // ready for the next launch
         __hip_atomic_store(&a.counters[tile_id], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -190,6 +190,7 @@ template <int MT, int RG, int XU, int DEPTH, bool NT, bool HALF2 = false, bool T
 __global__ void __launch_bounds__(lds_launch_bound(MT, RG)) lds_gemm_kernel(const StreamArgs a) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t ring[];  // [wave][DEPTH][stage]
     __shared__ unsigned arrival;
+    __shared__ __attribute__((aligned(16))) float factor_lds[kStagedFactors];
 
     static_assert(!HALF2 || RG == 2, "24-row tiles are two fragments");
     constexpr int W_INSTR = HALF2 ? 6 : RG * 4;    // weight DMA instructions per stage (4 rows each)
@@ -284,10 +285,14 @@ __global__ void __launch_bounds__(lds_launch_bound(MT, RG)) lds_gemm_kernel(cons
         else mma_block_256<MT, RG>(slot, slot + W_INSTR * 1024, acc);
     };
 
+    const StagedFactors factors{factor_lds};
+    if (wave == 0) factors.fetch(a, m0, n0, lane);
+    const float scale = scalar_scale(a);
     if (mine >= DEPTH) {
 #pragma unroll
         for (int d = 0; d < DEPTH; d++) issue(d);
         stamps.mark(1);
+        asm volatile("" ::"s"(scale));   // (here, not where the outputs are ready)
         int i = 0;
         for (; i + DEPTH < mine; i++) {
             wait_vmcnt<(DEPTH - 1) * PER_STAGE>();   // stage i has landed; DEPTH-1 stages still in flight
@@ -305,6 +310,7 @@ __global__ void __launch_bounds__(lds_launch_bound(MT, RG)) lds_gemm_kernel(cons
     } else {
         for (int i = 0; i < mine; i++) issue(i);
         stamps.mark(1);
+        asm volatile("" ::"s"(scale));
         wait_vmcnt<0>();
         stamps.mark(2);
         if constexpr (TAIL) {
@@ -319,7 +325,7 @@ __global__ void __launch_bounds__(lds_launch_bound(MT, RG)) lds_gemm_kernel(cons
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     stamps.mark(3);
     __syncthreads();
-    finish_tile<RG, MT>(a, acc, reinterpret_cast<f32x4*>(ring), &arrival, tile_m, tile_n, split, m0, n0, n0 + TILE_ROWS);
+    finish_tile<RG, MT>(a, acc, reinterpret_cast<f32x4*>(ring), &arrival, scale, factors, tile_m, tile_n, split, m0, n0, n0 + TILE_ROWS);
     stamps.end(a);
 }
 
@@ -493,7 +499,6 @@ lds_gemm_persistent_kernel(const StreamArgs a) {
     // bf16 activations quantised here (resident kernel only): the row scales live behind the reduction scratch
     constexpr bool quant = QUANT;
     float* xscale = reinterpret_cast<float*>(red + (size_t)2 * FRAGS * waves * 64);
-    const float* row_factors = quant ? xscale : nullptr;
 
     // Tiles are walked n fastest.  Both the issuing and the finishing side keep their tile's (n, m) coordinates as
     // counters that are stepped when a tile ends: dividing by run-time values per stage (tile index, tile
@@ -563,7 +568,13 @@ lds_gemm_persistent_kernel(const StreamArgs a) {
         mma_block_256<MT, RG>(slot, xs, acc);
     };
 
-    const float scale = a.scale ? a.scale[0] : 1.0f;
+    const float scale = scalar_scale(a);
+    const WorkgroupFactors factors{a.factor_off ? reinterpret_cast<const float*>(ring + a.factor_off) : nullptr};
+    if (wave == 0) factors.fetch(a, run.first * (16 * RG), my_tiles * (16 * RG), 0, 1, lane);
+    auto store = [&](const f32x4& v, int f, int j, int m0, int n0) __attribute__((always_inline)) {
+        const int m = m0 + (f % MT) * 16 + r, n = (f / MT) * 16 + 4 * g;
+        factors.store(a, v, scale, quant ? xscale : nullptr, m, n0 + n, j * (16 * RG) + n);
+    };
     int red_turn = 0;
     // Reduce the waves' partial tiles of the j-th tile in wave order, scale, round, store.
     auto tile_done = [&](int j) __attribute__((always_inline)) {
@@ -574,20 +585,13 @@ lds_gemm_persistent_kernel(const StreamArgs a) {
         }
         if (waves == 1 && !epilogue_wave) {
 #pragma unroll
-            for (int f = 0; f < FRAGS; f++)
-                store_fragment(a, acc[f / MT][f % MT], scale, m0 + (f % MT) * 16 + r, n0 + (f / MT) * 16 + 4 * g, row_factors);
+            for (int f = 0; f < FRAGS; f++) store(acc[f / MT][f % MT], f, j, m0, n0);
         } else {
             f32x4* buf = red + (size_t)(j & 1) * (FRAGS * waves * 64);
             if (wave < waves) {
 #pragma unroll
                 for (int f = 0; f < FRAGS; f++) buf[(f * waves + wave) * 64 + lane] = acc[f / MT][f % MT];
             }
-            // per-column factors of this tile, requested before the barrier: fetched when needed, their memory
-            // latency (a different line per tile) would be paid once per tile by the wave that stores
-            f32x4 colf[RG];
-#pragma unroll
-            for (int rg = 0; rg < RG; rg++) colf[rg] = col_scale_ahead(a, n0 + rg * 16 + 4 * g);
-            __syncthreads();
             // without an epilogue wave the reducing wave rotates with the tile, so that the cost is
             // spread over the waves
             int first = wave - red_turn, step = waves;        // red_turn = j % waves, kept as a counter
@@ -597,14 +601,11 @@ lds_gemm_persistent_kernel(const StreamArgs a) {
                 first = wave == waves ? 0 : FRAGS;
                 step = 1;
             }
+            __syncthreads();
             for (int f = first; f < FRAGS; f += step) {
                 f32x4 v = buf[(f * waves) * 64 + lane];
                 for (int w = 1; w < waves; w++) v += buf[(f * waves + w) * 64 + lane];
-                f32x4 cf = colf[0];    // colf[f / MT] without indexing registers by a run-time value
-#pragma unroll
-                for (int rg = 1; rg < RG; rg++)
-                    if (f / MT == rg) cf = colf[rg];
-                store_fragment(a, v, scale, m0 + (f % MT) * 16 + r, n0 + (f / MT) * 16 + 4 * g, row_factors, &cf);
+                store(v, f, j, m0, n0);
             }
         }
 #pragma unroll
@@ -790,7 +791,7 @@ __global__ void __launch_bounds__(lds_persistent_launch_bound(MT, RG)) lds_gemm_
         else mma_block_256<MT, RG>(slot, ring + (size_t)kb * (XU * 1024) + rd_off, acc);
     };
 
-    const float scale = a.scale ? a.scale[0] : 1.0f;
+    const float scale = scalar_scale(a);
     int tile_j = 0;
     auto after_consume = [&]() __attribute__((always_inline)) {
         if (++kb_cur == blocks) {   // the tile is complete: scale, round, store, start the next one

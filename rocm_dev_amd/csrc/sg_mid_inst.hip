@@ -57,7 +57,8 @@ int launch_mid_reduce(int rgw, int mh, int wn, const StreamArgs& a, hipStream_t 
     if ((rgw * mh) % kReduceFrags != 0) return SG_INVALID_CONFIG;
     const size_t grid = (size_t)a.n_tiles * a.m_tiles * ((frags_wg + 4 * kReduceFrags - 1) / (4 * kReduceFrags));
     if (grid == 0 || grid > 0x7fffffffu) return SG_BAD_ARGUMENT;
-    mid_reduce_kernel<<<dim3((unsigned)grid), dim3(256), 0, stream>>>(a, rgw, mh, wn);
+    if (a.row_scale || a.col_scale) mid_reduce_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, stream>>>(a, rgw, mh, wn);
+    else mid_reduce_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, stream>>>(a, rgw, mh, wn);
     return report_hip("mid_reduce_kernel launch", hipGetLastError()) == hipSuccess ? SG_SUCCESS : SG_LAUNCH_FAILED;
 }
 

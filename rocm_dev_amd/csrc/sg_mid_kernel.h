@@ -315,13 +315,33 @@ __global__ void __launch_bounds__(WN * 128) mid_gemm_kernel(const StreamArgs a) 
     stamps.mark(3);
 
     // ---- epilogue --------------------------------------------------------------------------------
-    const float scale = a.scale ? a.scale[0] : 1.0f;
+    // the factors of all the wave's fragments at once: one round trip instead of one per fragment and column
+    const float scale = scalar_scale(a);
     auto store_all = [&](auto&& get) __attribute__((always_inline)) {
+        const int m_wave = m0 + wm * MH * 16 + r, n_wave = n0 + wn * RGW * 16 + 4 * g;
+        if (a.row_scale || a.col_scale) {
+            f32x4 colf[RGW];
+            float rowf[MH];
 #pragma unroll
-        for (int rg = 0; rg < RGW; rg++)
+            for (int rg = 0; rg < RGW; rg++) colf[rg] = col_scale_ahead(a, n_wave + rg * 16);
 #pragma unroll
-            for (int mb = 0; mb < MH; mb++)
-                store_fragment(a, get(rg, mb), scale, m0 + (wm * MH + mb) * 16 + r, n0 + (wn * RGW + rg) * 16 + 4 * g);
+            for (int mb = 0; mb < MH; mb++) rowf[mb] = row_scale_ahead(a, m_wave + mb * 16);
+#pragma unroll
+            for (int rg = 0; rg < RGW; rg++)
+#pragma unroll
+                for (int mb = 0; mb < MH; mb++)
+                    store_fragment(a, get(rg, mb), scale, m_wave + mb * 16, n_wave + rg * 16, rowf[mb], colf[rg]);
+        } else {
+#pragma unroll
+            for (int rg = 0; rg < RGW; rg++)
+#pragma unroll
+                for (int mb = 0; mb < MH; mb++) {
+                    f32x4 v = get(rg, mb);
+                    asm volatile("" : "+v"(v));   // (as in store_fragment)
+                    v *= scale;
+                    store_scaled(a, v, m_wave + mb * 16, n_wave + rg * 16);
+                }
+        }
     };
     if (a.split_k == 1) {
         store_all([&](int rg, int mb) { return acc[rg][mb]; });

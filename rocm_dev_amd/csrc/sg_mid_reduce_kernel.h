@@ -12,7 +12,10 @@ namespace sg {
 // their partials of a split before it adds any: with one fragment per wave the launch took 7-12 us for 8-33 MB of
 // partials that the GEMM had just left in the caches.  The tile geometry comes as run-time values: rgw x mh
 // fragments per wave of the GEMM, wn x 2 waves per tile.
+// FACTORS: there are row or column factors (requested ahead of the partials, in 34 registers that the other build does not
+// hold: five workgroups a SIMD instead of eight).
 constexpr int kReduceFrags = 4;
+template <bool FACTORS>
 __global__ void __launch_bounds__(256) mid_reduce_kernel(const StreamArgs a, int rgw, int mh, int wn) {
     const int fr = rgw * mh, frags_wg = 2 * wn * fr;   // fr is a multiple of kReduceFrags (launch_mid_reduce)
     const int lane = lane_id();
@@ -26,9 +29,26 @@ __global__ void __launch_bounds__(256) mid_reduce_kernel(const StreamArgs a, int
     const unsigned tile_id = (unsigned)(tile_m * a.n_tiles + tile_n);
     const unsigned rem = (unsigned)((chunk * 4 + wave_id()) * kReduceFrags);     // (wave of the tile, fragment of the wave)
     if (rem >= (unsigned)frags_wg) return;
-    const float scale = a.scale ? a.scale[0] : 1.0f;
     const int wave = (int)rem / fr, f0 = (int)rem - wave * fr;
     const int wq = wave % wn, wm = wave / wn;
+    const int r = lane & 15, g = lane >> 4;
+    const float scale = scalar_scale(a);
+    auto place = [&](int j, int& m_idx, int& n_idx) __attribute__((always_inline)) {
+        const int f = f0 + j, rg = f / mh, mb = f - rg * mh;
+        m_idx = tile_m * (32 * mh) + (wm * mh + mb) * 16 + r;
+        n_idx = tile_n * (16 * rgw * wn) + (wq * rgw + rg) * 16 + 4 * g;
+    };
+    f32x4 col[kReduceFrags];
+    float row[kReduceFrags];
+    if constexpr (FACTORS) {
+#pragma unroll
+        for (int j = 0; j < kReduceFrags; j++) {
+            int m_idx, n_idx;
+            place(j, m_idx, n_idx);
+            col[j] = col_scale_ahead(a, n_idx);
+            row[j] = row_scale_ahead(a, m_idx);
+        }
+    }
     const f32x4* p = reinterpret_cast<const f32x4*>(a.ws + ((size_t)tile_id * a.split_k) * ((size_t)frags_wg * 256) +
                                                     (size_t)wave * (fr * 256) + (size_t)f0 * 256) + lane;
     const size_t split_stride = (size_t)frags_wg * 64;
@@ -43,11 +63,16 @@ __global__ void __launch_bounds__(256) mid_reduce_kernel(const StreamArgs a, int
 #pragma unroll
         for (int j = 0; j < kReduceFrags; j++) v[j] += t[j];
     }
-    const int r = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int j = 0; j < kReduceFrags; j++) {
-        const int f = f0 + j, rg = f / mh, mb = f - rg * mh;
-        store_fragment(a, v[j], scale, tile_m * (32 * mh) + (wm * mh + mb) * 16 + r, tile_n * (16 * rgw * wn) + (wq * rgw + rg) * 16 + 4 * g);
+        int m_idx, n_idx;
+        place(j, m_idx, n_idx);
+        if constexpr (FACTORS) {
+            store_fragment(a, v[j], scale, m_idx, n_idx, row[j], col[j]);
+        } else {
+            v[j] *= scale;
+            store_scaled(a, v[j], m_idx, n_idx);
+        }
     }
 }
 

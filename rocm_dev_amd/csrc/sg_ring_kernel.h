@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(1024) ring_gemm_kernel(const RingArgs ra) {
     // ---------------------------------- consumers ----------------------------------------------
     const int c = wave - PA - PB;
     const int rd_off = 1024 * (r >> 2) + 64 * (r & 3) + 16 * ((g16 - (r >> 2)) & 3);
-    const float scale = a.scale ? a.scale[0] : 1.0f;
+    const float scale = scalar_scale(a);
 
     f32x4 acc[BL][MT];
 #pragma unroll

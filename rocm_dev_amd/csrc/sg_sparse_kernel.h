@@ -218,6 +218,7 @@ __global__ void __launch_bounds__(sparse_launch_bound(MT, RG)) sparse24_gemm_ker
         }
     };
 
+    const float scale = scalar_scale(a);
     if constexpr (PAIRS) {
         if (mine > 0) {   // the first pair's metadata ahead of everything
             issue_meta(0, 0);
@@ -228,6 +229,7 @@ __global__ void __launch_bounds__(sparse_launch_bound(MT, RG)) sparse24_gemm_ker
 #pragma unroll
         for (int d = 0; d < DEPTH; d++) issue(d);
         stamps.mark(1);
+        asm volatile("" ::"s"(scale));   // (here, not where the outputs are ready)
         int i = 0;
         for (; i + DEPTH < mine; i++) {
             wait_vmcnt<(DEPTH - 1) * PER_STAGE>();
@@ -242,6 +244,7 @@ __global__ void __launch_bounds__(sparse_launch_bound(MT, RG)) sparse24_gemm_ker
     } else {
         for (int i = 0; i < mine; i++) issue(i);
         stamps.mark(1);
+        asm volatile("" ::"s"(scale));   // (here, not where the outputs are ready)
         wait_vmcnt<0>();
         stamps.mark(2);
         for (int i = 0; i < mine; i++) consume(i);
@@ -250,7 +253,7 @@ __global__ void __launch_bounds__(sparse_launch_bound(MT, RG)) sparse24_gemm_ker
 
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __syncthreads();
-    finish_tile<RG, MT>(a, acc, reinterpret_cast<f32x4*>(ring), &arrival, tile_m, tile_n, split, m0, n0);
+    finish_tile<RG, MT>(a, acc, reinterpret_cast<f32x4*>(ring), &arrival, scale, StagedFactors{nullptr}, tile_m, tile_n, split, m0, n0);
     stamps.end(a);
 }
 
@@ -404,7 +407,7 @@ __global__ void __launch_bounds__(RG == 4 ? 512 : 1024) sparse24_gemm_wavetile_k
         }
     };
 
-    const float scale = a.scale ? a.scale[0] : 1.0f;
+    const float scale = scalar_scale(a);
     int tile_j = 0;
     auto after_consume = [&]() __attribute__((always_inline)) {
         if (++kb_cur == blocks) {   // the tile is complete: scale, round, store, start the next one

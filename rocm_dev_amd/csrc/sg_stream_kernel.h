@@ -85,6 +85,7 @@ __global__ void __launch_bounds__(stream_launch_bound(MT, RG, KU, DEPTH))
 stream_gemm_kernel(const StreamArgs a) {
     extern __shared__ f32x4 red[];  // [frag][wave][64]
     __shared__ unsigned arrival;
+    __shared__ __attribute__((aligned(16))) float factor_lds[kStagedFactors];
 
     constexpr int FRAGS = RG * MT;
     constexpr int STAGE_K = KU * 64;
@@ -180,7 +181,13 @@ stream_gemm_kernel(const StreamArgs a) {
         mma_stage<MT, RG, KU>(st[0], acc);
     }
 
-    finish_tile<RG, MT>(a, acc, red, &arrival, tile_m, tile_n, split, m0, n0);
+    const StagedFactors factors{factor_lds};
+    if (a.row_scale || a.col_scale) {
+        if (wave == 0) factors.fetch(a, m0, n0, lane);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    finish_tile<RG, MT>(a, acc, red, &arrival, scalar_scale(a), factors, tile_m, tile_n, split, m0, n0);
 }
 
 }  // namespace sg

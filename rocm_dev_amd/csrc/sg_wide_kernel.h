@@ -286,14 +286,14 @@ __global__ void __launch_bounds__(WN * 128) wide_gemm_kernel(const StreamArgs a)
     // The wave turns its tile around in LDS and stores whole runs of 32 * RGW bytes a row (a fragment as it is ends in
     // 32-byte runs: 9.5 us for the stores of a 256 x 256 tile, 7.5 this way).  No barrier: nobody reads the ring any more, and no load
     // is under way (behind the last stages' barriers).
-    const float scale = a.scale ? a.scale[0] : 1.0f;
+    const float scale = scalar_scale(a);
     constexpr int PITCH = 32 * RGW + 16;                    // bytes; + 16 spreads the rows over the banks
     constexpr int ROWS = 16 * MH;
     uint8_t* const mine = ring + (size_t)wave * (ROWS * PITCH);
     const int m_wave = m0 + wm * ROWS, n_wave = n0 + wn * RGW * 16;
     float rs[MH];
 #pragma unroll
-    for (int mb = 0; mb < MH; mb++) rs[mb] = a.row_scale ? a.row_scale[m_wave + mb * 16 + r < a.m ? m_wave + mb * 16 + r : a.m - 1] : 1.0f;
+    for (int mb = 0; mb < MH; mb++) rs[mb] = row_scale_ahead(a, m_wave + mb * 16 + r);
 #pragma unroll
     for (int rg = 0; rg < RGW; rg++) {
         const f32x4 cs = col_scale_ahead(a, n_wave + rg * 16 + 4 * g);

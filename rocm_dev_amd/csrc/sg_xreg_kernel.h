@@ -112,13 +112,17 @@ __global__ void __launch_bounds__(xreg_launch_bound(MT, RG, PT)) lds_gemm_xreg_k
             }
     };
 
-    const float scale = a.scale ? a.scale[0] : 1.0f;
+    const float scale = scalar_scale(a);
+    const WorkgroupFactors factors{a.factor_off ? reinterpret_cast<const float*>(ring + a.factor_off) : nullptr};
+    auto store = [&](const f32x4& v, int f, int j) __attribute__((always_inline)) {
+        const int m = (f % MT) * 16 + r, n = (f / MT) * 16 + 4 * g;
+        factors.store(a, v, scale, nullptr, m, (run.first + j) * (16 * RG) + n, j * (16 * RG) + n);
+    };
     // Reduce the waves' partial tiles of the j-th tile in wave order, scale, round, store.
     auto tile_done = [&](int j) __attribute__((always_inline)) {
-        const int n0 = (run.first + j) * (16 * RG);
         if (waves == 1 && !epilogue_wave) {
 #pragma unroll
-            for (int f = 0; f < FRAGS; f++) store_fragment(a, acc[f / MT][f % MT], scale, (f % MT) * 16 + r, n0 + (f / MT) * 16 + 4 * g);
+            for (int f = 0; f < FRAGS; f++) store(acc[f / MT][f % MT], f, j);
         } else {
             f32x4* buf = red + (size_t)(j & 1) * (FRAGS * waves * 64);
             if (streaming) {
@@ -135,7 +139,7 @@ __global__ void __launch_bounds__(xreg_launch_bound(MT, RG, PT)) lds_gemm_xreg_k
             for (int f = first; f < FRAGS; f += step) {
                 f32x4 v = buf[(f * waves) * 64 + lane];
                 for (int w = 1; w < waves; w++) v += buf[(f * waves + w) * 64 + lane];
-                store_fragment(a, v, scale, (f % MT) * 16 + r, n0 + (f / MT) * 16 + 4 * g);
+                store(v, f, j);
             }
         }
 #pragma unroll
@@ -144,6 +148,7 @@ __global__ void __launch_bounds__(xreg_launch_bound(MT, RG, PT)) lds_gemm_xreg_k
             for (int mt = 0; mt < MT; mt++) acc[rg][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
 
+    if (streaming) factors.fetch(a, run.first * (16 * RG), my_tiles * (16 * RG), wave, waves, lane);
     if (!streaming) {   // epilogue wave: takes part in every barrier, reduces and stores
         __syncthreads();   // the reduction scratch is free (it staged activations, see below)
         for (int j = 0; j < my_tiles; j++) tile_done(j);
