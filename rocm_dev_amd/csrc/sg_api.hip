@@ -244,6 +244,7 @@ struct Config {
     int persist;  // LDS engine: 0 = one workgroup per tile; n > 0 = n persistent workgroups per CU walking the tiles
     const Workspace* fixed_ws = nullptr;   // split-K partials and counters to use instead of the stream's own workspace
     bool wide = false;   // mid-batch engine: the wide-tile kernel (only the library itself asks for it: wide_config)
+    bool line = false;   // mid-batch engine: the kernel for rows off their 128-byte lines (likewise: line_config)
     int wavetile; // LDS engine, bits 0-1: 1 = every wave owns whole tiles, activations resident in LDS (persist = workgroups per CU);
                   //             2 = persistent K-split workgroups with the activations resident in LDS
                   //             3 = ... resident in the waves' registers (k = 256 * waves * {1, 2, 4});  bit 2: epilogue wave
@@ -493,9 +494,29 @@ static int launch_wide_engine(const Config& c, StreamArgs a, hipStream_t stream)
     return a.defer_reduce ? launch_mid_reduce(c.rg, c.mt, 2, a, stream) : SG_SUCCESS;
 }
 
+// The kernel for rows off their lines: c.waves / 2 waves along n x two along m, a K split's sum always in a second launch.
+static int launch_line_engine(const Config& c, StreamArgs a, hipStream_t stream) {
+    if ((c.waves != 4 && c.waves != 8) || c.rg < 1 || c.mt < 2 || a.b_stride > kWidePitch || a.k > kWidePitch) return SG_INVALID_CONFIG;
+    const int wn = c.waves / 2, bn = 16 * c.rg * wn, bm = 32 * c.mt;
+    a.waves = c.waves;
+    a.split_k = c.split_k;
+    a.n_tiles = (a.n + bn - 1) / bn;
+    a.m_tiles = (a.m + bm - 1) / bm;
+    if (c.split_k < 1 || c.split_k > a.k / 128) return SG_INVALID_CONFIG;
+    const size_t tiles = (size_t)a.n_tiles * a.m_tiles;
+    if (tiles * c.split_k > 0x7fffffffu) return SG_BAD_ARGUMENT;
+    if (int rc = attach_workspace(c, a, tiles, (size_t)c.waves * c.rg * c.mt * 1024, stream)) return rc;
+    set_reciprocals(a);
+    a.defer_reduce = c.split_k > 1 ? 1 : 0;
+    a.stamps = take_stamps((unsigned)(tiles * c.split_k));
+    if (int rc = launch_line(c.rg, c.mt, wn, a, (unsigned)(tiles * c.split_k), stream)) return rc;
+    return a.defer_reduce ? launch_mid_reduce(c.rg, c.mt, wn, a, stream) : SG_SUCCESS;
+}
+
 static int launch_mid_engine(const Config& c, StreamArgs a, hipStream_t stream) {
     if (a.k % 128 != 0 && !mid_partial_block_k(a.k)) return SG_K_NOT_DIVISIBLE_BY_WARPTILE_K;
     if (c.wide) return launch_wide_engine(c, a, stream);
+    if (c.line) return launch_line_engine(c, a, stream);
     if ((c.rg != 2 && c.rg != 4) || (c.mt != 2 && c.mt != 4 && c.mt != 8) || c.depth < 2) return SG_INVALID_CONFIG;
     if (c.waves != 4 && c.waves != 8 && c.waves != 14) return SG_INVALID_CONFIG;
     const int wn = c.waves / 2;                   // waves = wn (along n) x 2 (along m)
@@ -1271,7 +1292,8 @@ static bool mid_stays_ahead(const Config& mid, const Config& wide, double wide_u
     return mid.mt == 8 && !whole_lines && m < 400 && k <= 2000;
 }
 
-static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, bool factors, int cu_count, const Workspace* fixed_ws, Config* out) {
+static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, bool factors, int cu_count, const Workspace* fixed_ws, Config* out,
+                        double* us_out = nullptr) {
     if (m <= 128 || mid.engine != ENGINE_MID || b_stride > kWidePitch || k > kWidePitch) return false;
     size_t partial_limit, counters;
     workspace_need(mid, m, n, &partial_limit, &counters);
@@ -1309,7 +1331,126 @@ static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, bo
     c.wide = true;
     c.nt = 1;
     *out = c;
+    if (us_out) *us_out = best;
     return true;
+}
+
+// More than 32 rows, weights or activations off their 128-byte lines (a row stride or a k that 128 does not divide): the
+// kernel that follows the lines (sg_line_kernel.h) in place of heuristic_config's record or the wide tile, where the model
+// of its own time is 5 % ahead of the model of theirs.  Microseconds with every CU busy, all fitted to timings of 302 random
+// shapes of that kind (33..700 rows, 512..32768 weight rows, K of 512..20000), every tile and K split of this kernel and
+// the launch it would replace: a launch costs c0, a round of workgroups its tile's stage per 128 bytes of K (and one more,
+// for the line behind the last), a partly filled last round at least 0.85 of that, a K split 2.2 and 0.21 per MB of
+// partials.  What it picks is 1.007 times the best tile and split (geometric mean), and the choice between the kernels 0.838
+// of the times before it (a perfect one: 0.835), two shapes behind by more than 3 % (up to 7 %): 468 x 566 x 9200 37.0 -> 16.4 us,
+// 47 x 28666 x 10320 83.9 -> 52.9, 128 x 8192 x 8208 36.7 -> 24.9, 96 x 4828 x 11984 43.5 -> 23.1.  The others stay ahead
+// on small weight matrices with K below about 4000 (the ring over several activation tiles: 49 x 4092 x 1680 5.2 against 10.3)
+// and where many rows fill rounds of wide tiles (207 x 27442 x 6800 62.9 against 83.4).
+// Beyond 768 rows it was not timed and is not taken.  The K split's partials: a workspace of the library's own, or one of
+// the size that sg_workspace_query asks for, has room for them where 128 does not divide k; where only the stride is off
+// the lines, which the query does not know, they have to fit what the record needs.  Either way the result does not depend
+// on whose workspace it is, as long as it has the size asked for.
+struct LineTile { int waves, rg, mt; double stage_us; };
+static const LineTile kLineTiles[] = {{4, 2, 2, 0.388}, {8, 2, 2, 0.513}, {8, 2, 4, 0.737}, {8, 2, 6, 1.016}, {8, 3, 4, 0.919}};
+constexpr int kLineMaxM = 768, kLineMaxSplit = 12;
+
+// rounds of `wgs` workgroups on the device, a partly filled last one counting at least `part`
+static double rounds_of(long wgs, int cu_count, double part) {
+    const long rest = wgs % cu_count;
+    return (double)(wgs / cu_count) + (rest ? part + (1.0 - part) * (double)rest / cu_count : 0.0);
+}
+
+// the launch that the record stands for, on rows off their lines
+static double off_line_us(const Config& c, int m, int n, int k, int cu_count) {
+    const int wn = c.engine == ENGINE_MID ? c.waves / 2 : 1;
+    const int bn = c.engine == ENGINE_MID ? 16 * c.rg * wn : 16 * c.rg, bm = (c.engine == ENGINE_MID ? 32 : 16) * c.mt;
+    const long wgs = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm) * c.split_k;
+    if (c.engine == ENGINE_LDS) {     // the skinny ring over several activation tiles (two_pass_config)
+        const double fill = (double)wgs / cu_count, stages = (double)((k + 255) / 256) / c.split_k;
+        return 3.04 + stages * (0.111 + c.rg * (0.088 + 0.048 * fill)) * (fill > 1.0 ? 1.71 : 1.0) + (c.split_k > 1 ? 1.36 : 0.0);
+    }
+    const double stages = (double)((k + 127) / 128) / c.split_k;
+    double us = 2.46 + 1.68 * (double)((wgs + cu_count - 1) / cu_count) +
+                rounds_of(wgs, cu_count, 0.8) * stages * (0.097 + 0.435 * bn / 128 + 0.088 * bm / 128 + 0.414 * bn * bm / 16384);
+    if (c.split_k > 1) us += 4.0 + 0.8e-6 * (double)wgs * bn * bm;
+    return us;
+}
+
+static bool line_config(const Config& record, const Config* wide, double wide_us, int m, int n, int k, int b_stride, int cu_count,
+                        const Workspace* fixed_ws, Config* out) {
+    if (m <= 32 || m > kLineMaxM || k <= 128 || (k % 128 == 0 && b_stride % 128 == 0)) return false;
+    if ((record.engine != ENGINE_MID && record.engine != ENGINE_LDS) || b_stride > kWidePitch || k > kWidePitch) return false;
+    if (m > 128 && k <= 1024) return false;     // stores of D, not loads: 1.09 times slower on 14 shapes (412 x 25130 x 768 32.0 us, 18.9)
+    size_t partial_limit = kMaxPartialBytes, counters;
+    if (k % 128 == 0) workspace_need(record, m, n, &partial_limit, &counters);
+    if (fixed_ws && fixed_ws->partial_bytes < partial_limit) partial_limit = fixed_ws->partial_bytes;
+    const int blocks = (k + 127) / 128;
+    double best = 0;
+    Config c{};
+    for (const LineTile& t : kLineTiles) {
+        const int bn = 8 * t.waves * t.rg, bm = 32 * t.mt;
+        if (bm >= 2 * m && t.mt > 2) continue;
+        const long n_tiles = (n + bn - 1) / bn, tiles = n_tiles * ((m + bm - 1) / bm);
+        if (fixed_ws && (size_t)tiles > fixed_ws->n_counters && partial_limit > 0) continue;
+        for (int sk = 1; sk <= kLineMaxSplit; sk++) {
+            const long wgs = tiles * sk;
+            const double partials = (double)wgs * bn * bm * 4;
+            if (sk > 1 && (blocks / sk < 5 || wgs > 2L * cu_count || partials > (double)partial_limit)) break;
+            const double stages = (double)((blocks + sk - 1) / sk + 1);
+            double us = 3.07 + rounds_of(wgs, cu_count, 0.85) * stages * t.stage_us + 2.27 * (double)((wgs + cu_count - 1) / cu_count);
+            if (sk > 1) us += 2.18 + 0.209e-6 * partials;
+            const double weights = (double)n_tiles * bn * k / 5.69e6 + 4.29;
+            if (us < weights) us = weights;
+            if (best == 0 || us < best) {
+                best = us;
+                c.waves = t.waves; c.rg = t.rg; c.mt = t.mt; c.split_k = sk;
+            }
+        }
+    }
+    double other;
+    if (wide) {     // wide_config's model of a K that 128 does not divide, refitted; it knows nothing of strides
+        const double fixed = 2.1;
+        other = 0.925 * (fixed + (wide_us - fixed) * (k % 128 ? 1.04 : 1.35));
+    } else {
+        other = off_line_us(record, m, n, k, cu_count);
+    }
+    if (best == 0 || best > 0.95 * other) return false;
+    c.engine = ENGINE_MID;
+    c.line = true;
+    c.nt = 1;
+    *out = c;
+    return true;
+}
+
+// What stands in for heuristic_config's record, if anything does: a wide tile or the kernel for rows off their lines.
+static bool stand_in_config(const Config& record, int m, int n, int k, int b_stride, bool factors, int cu_count, const Workspace* fixed_ws,
+                            Config* out) {
+    double wide_us = 0;
+    const bool wide = wide_config(record, m, n, k, b_stride, factors, cu_count, fixed_ws, out, &wide_us);
+    Config line;
+    if (!line_config(record, wide ? out : nullptr, wide_us, m, n, k, b_stride, cu_count, fixed_ws, &line)) return wide;
+    *out = line;
+    return true;
+}
+
+// The record that sg_skinny_gemm_choice reports: heuristic_config's - or, where that has no K split and the kernel for rows
+// off their lines takes one in its place, the mid-batch record of that split on the tile nearest to that kernel's, so that a
+// record without a K split still says that no workspace is needed.  (Launches that cannot have the split, on a caller's
+// smaller workspace for instance, run heuristic_config's.)
+static Config reported_config(int m, int n, int k, int cu_count) {
+    const Config base = heuristic_config(m, n, k, cu_count);
+    Config c;
+    if (k % 128 == 0 || base.split_k > 1 || !stand_in_config(base, m, n, k, k, false, cu_count, nullptr, &c) || !c.line || c.split_k == 1) return base;
+    Config r{};
+    r.engine = ENGINE_MID;
+    r.waves = c.waves;
+    r.rg = c.rg == 3 ? 4 : c.rg;
+    r.mt = c.mt == 6 ? 8 : c.mt;
+    r.split_k = c.split_k;
+    r.depth = r.rg == 4 || r.mt == 8 ? 3 : 4;
+    r.nt = 1;
+    r.wavetile = 1;
+    return r;
 }
 
 // ---- per-shape tuning table ---------------------------------------------------------------
@@ -1375,10 +1516,10 @@ static int launch_chosen(const StreamArgs& a, int cu_count, hipStream_t stream, 
             if (!rejected_before_launch(rc)) return rc;
         }
     }
-    Config c = heuristic_config(a.m, a.n, a.k, cu_count), wide;
-    if (wide_config(c, a.m, a.n, a.k, a.b_stride, a.row_scale || a.col_scale, cu_count, fixed_ws, &wide)) {
-        wide.fixed_ws = fixed_ws;
-        const int rc = launch_config(wide, a, stream);
+    Config c = heuristic_config(a.m, a.n, a.k, cu_count), instead;
+    if (stand_in_config(c, a.m, a.n, a.k, a.b_stride, a.row_scale || a.col_scale, cu_count, fixed_ws, &instead)) {
+        instead.fixed_ws = fixed_ws;
+        const int rc = launch_config(instead, a, stream);
         if (!rejected_before_launch(rc)) return rc;
     }
     c.fixed_ws = fixed_ws;
@@ -1493,21 +1634,33 @@ int sg_release_workspaces(void) {
 constexpr size_t kCallerCounters = 16384;
 constexpr size_t kCallerCounterBytes = kCallerCounters * sizeof(unsigned);
 
-int sg_workspace_query(int m, int n, int k, size_t* bytes) {
-    if (!bytes || m <= 0 || n <= 0 || k <= 0) return SG_BAD_ARGUMENT;
+// *least: what sg_skinny_gemm_auto_ws refuses to go below, the records' own partials; *bytes: with those of what stands in
+// for the record, where that is known from the shape - a caller that has less gets the record.
+static void workspace_sizes(int m, int n, int k, size_t* least, size_t* bytes) {
     DeviceInfo* dev;
     int cu = 256;
     if (get_device_info(&dev) == SG_SUCCESS) cu = dev->cu_count;
     SgTuning t;
-    Config c = (table_lookup(m, n, k, &t) && t.engine != ENGINE_AUTO) ? config_from_tuning(t) : heuristic_config(m, n, k, cu);
-    size_t partial, counters;
-    workspace_need(c, m, n, &partial, &counters);
-    // (should the table's record be refused at launch, the heuristics' record runs: it must fit as well)
+    const bool from_table = table_lookup(m, n, k, &t) && t.engine != ENGINE_AUTO;
     const Config h = heuristic_config(m, n, k, cu);
-    size_t partial_h, counters_h;
-    workspace_need(h, m, n, &partial_h, &counters_h);
-    if (partial_h > partial) partial = partial_h;
+    size_t partial, counters, other;
+    workspace_need(from_table ? config_from_tuning(t) : h, m, n, &partial, &counters);
+    // (should the table's record be refused at launch, the heuristics' record runs: it must fit as well)
+    workspace_need(h, m, n, &other, &counters);
+    partial = std::max(partial, other);
+    *least = partial ? kCallerCounterBytes + partial : 0;
+    Config c;
+    if (stand_in_config(h, m, n, k, k, false, cu, nullptr, &c)) {
+        workspace_need(c, m, n, &other, &counters);
+        partial = std::max(partial, other);
+    }
     *bytes = partial ? kCallerCounterBytes + partial : 0;
+}
+
+int sg_workspace_query(int m, int n, int k, size_t* bytes) {
+    if (!bytes || m <= 0 || n <= 0 || k <= 0) return SG_BAD_ARGUMENT;
+    size_t least;
+    workspace_sizes(m, n, k, &least, bytes);
     return SG_SUCCESS;
 }
 
@@ -1525,12 +1678,12 @@ int sg_skinny_gemm_auto_ws(const uint8_t* A, const uint8_t* B, void* D, const fl
     if (workspace && (reinterpret_cast<uintptr_t>(workspace) & 255u)) return SG_BAD_ALIGNMENT;
     DeviceInfo* dev;
     if (int rc = get_device_info(&dev)) return rc;
-    size_t need = 0;
-    if (int rc = sg_workspace_query(m, n, k, &need)) return rc;
-    if (need > 0 && (!workspace || workspace_bytes < need)) return SG_WORKSPACE_TOO_SMALL;
+    size_t least = 0, need = 0;
+    workspace_sizes(m, n, k, &least, &need);
+    if (least > 0 && (!workspace || workspace_bytes < least)) return SG_WORKSPACE_TOO_SMALL;
     // a launch without a K split gets a workspace nothing fits into: whatever would want one is refused, never allocated
     Workspace w;
-    if (need > 0) {
+    if (need > 0 && workspace && workspace_bytes > kCallerCounterBytes) {
         w.counters = static_cast<unsigned*>(workspace);
         w.n_counters = kCallerCounters;
         w.partials = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + kCallerCounterBytes);
@@ -1571,6 +1724,25 @@ int sg_debug_wide_gemm(const uint8_t* A, const uint8_t* B, void* D, const float*
     return launch_config(c, a, static_cast<hipStream_t>(stream));
 }
 
+int sg_debug_line_gemm(const uint8_t* A, const uint8_t* B, void* D, const float* scale, const float* row_scales,
+                       const float* col_scales, int m, int n, int k, int b_stride, int waves, int row_tiles, int m_blocks, int split_k,
+                       void* stream) {
+    if (n % 2 != 0) return SG_N_NOT_EVEN;
+    if (k % 16 != 0 || k <= 128) return SG_K_NOT_DIVISIBLE_BY_WARPTILE_K;
+    if (int rc = check_pointers(A, B, D, m, n, k, b_stride)) return rc;
+    DeviceInfo* dev;
+    if (int rc = get_device_info(&dev)) return rc;
+    Config c{};
+    c.engine = ENGINE_MID;
+    c.line = true;
+    c.waves = waves; c.rg = row_tiles; c.mt = m_blocks; c.split_k = split_k;
+    StreamArgs a{};
+    a.A = A; a.B = B; a.D = D; a.scale = scale; a.row_scale = row_scales; a.col_scale = col_scales;
+    a.m = m; a.n = n; a.k = k; a.b_stride = b_stride;
+    a.out_f32 = 0;
+    return launch_config(c, a, static_cast<hipStream_t>(stream));
+}
+
 int sg_debug_wide_choice(int m, int n, int k, int b_stride, int factors, int out[3]) {
     if (!out || m <= 0 || n <= 0 || k <= 0 || b_stride < k) return SG_BAD_ARGUMENT;
     out[0] = out[1] = out[2] = 0;
@@ -1579,9 +1751,24 @@ int sg_debug_wide_choice(int m, int n, int k, int b_stride, int factors, int out
     DeviceInfo* dev;
     int cu = 256;
     if (get_device_info(&dev) == SG_SUCCESS) cu = dev->cu_count;
-    Config wide;
-    if (wide_config(heuristic_config(m, n, k, cu), m, n, k, b_stride, factors != 0, cu, nullptr, &wide)) {
-        out[0] = wide.rg; out[1] = wide.mt; out[2] = wide.split_k;
+    Config c;
+    if (stand_in_config(heuristic_config(m, n, k, cu), m, n, k, b_stride, factors != 0, cu, nullptr, &c) && c.wide) {
+        out[0] = c.rg; out[1] = c.mt; out[2] = c.split_k;
+    }
+    return SG_SUCCESS;
+}
+
+int sg_debug_line_choice(int m, int n, int k, int b_stride, int factors, int out[4]) {
+    if (!out || m <= 0 || n <= 0 || k <= 0 || b_stride < k) return SG_BAD_ARGUMENT;
+    out[0] = out[1] = out[2] = out[3] = 0;
+    SgTuning t;
+    if (table_lookup(m, n, k, &t) && t.engine != ENGINE_AUTO) return SG_SUCCESS;
+    DeviceInfo* dev;
+    int cu = 256;
+    if (get_device_info(&dev) == SG_SUCCESS) cu = dev->cu_count;
+    Config c;
+    if (stand_in_config(heuristic_config(m, n, k, cu), m, n, k, b_stride, factors != 0, cu, nullptr, &c) && c.line) {
+        out[0] = c.waves; out[1] = c.rg; out[2] = c.mt; out[3] = c.split_k;
     }
     return SG_SUCCESS;
 }
@@ -1723,8 +1910,8 @@ int sg_skinny_gemm_tuned_noalloc(const uint8_t* A, const uint8_t* B, void* D, co
     Config c = config_from_tuning(*t);
     if (c.engine == ENGINE_AUTO) {
         c = heuristic_config(m, n, k, dev->cu_count);
-        Config wide;
-        if (wide_config(c, m, n, k, b_stride, false, dev->cu_count, &w, &wide)) c = wide;
+        Config instead;
+        if (stand_in_config(c, m, n, k, b_stride, false, dev->cu_count, &w, &instead)) c = instead;
         // the library's own choice is made to fit the array: a K split whose partials or counters do not, is not taken
         size_t partial_bytes, counters;
         workspace_need(c, m, n, &partial_bytes, &counters);
@@ -1769,7 +1956,7 @@ int sg_skinny_gemm_choice(int m, int n, int k, SgTuning* out, int* from_table) {
     DeviceInfo* dev;
     int cu = 256;
     if (get_device_info(&dev) == SG_SUCCESS) cu = dev->cu_count;
-    const Config c = heuristic_config(m, n, k, cu);
+    const Config c = reported_config(m, n, k, cu);
     out->engine = c.engine; out->split_k = c.split_k; out->waves = c.waves; out->row_tiles = c.rg; out->m_blocks = c.mt;
     out->depth = c.depth; out->k_chunks = c.ku; out->non_temporal = c.nt; out->persistent_wgs_per_cu = c.persist;
     out->wave_tiles = c.wavetile;

@@ -47,6 +47,8 @@ int launch_xreg(int mt, int rg, int pt, int depth, const StreamArgs& a, unsigned
 int launch_mid(int rgw, int mh, int depth, int dx, int wn, const StreamArgs& a, unsigned grid, size_t lds, hipStream_t stream);
 // wide tiles on four waves, rgw x mh fragments each (sg_wide_kernel.h)
 int launch_wide(int rgw, int mh, const StreamArgs& a, unsigned grid, hipStream_t stream);
+// mid-batch tiles on rows off their 128-byte lines (sg_line_kernel.h)
+int launch_line(int rgw, int mh, int wn, const StreamArgs& a, unsigned grid, hipStream_t stream);
 // second launch of a mid-batch GEMM with StreamArgs::defer_reduce: sums the split-K partials of every output fragment
 int launch_mid_reduce(int rgw, int mh, int wn, const StreamArgs& a, hipStream_t stream);
 

@@ -285,12 +285,15 @@ __global__ void __launch_bounds__(lds_launch_bound(MT, RG)) lds_gemm_kernel(cons
         else mma_block_256<MT, RG>(slot, slot + W_INSTR * 1024, acc);
     };
 
+    // the factors behind the first stage, which then does not wait for their arguments; older than every other stage
     const StagedFactors factors{factor_lds};
-    if (wave == 0) factors.fetch(a, m0, n0, lane);
     const float scale = scalar_scale(a);
     if (mine >= DEPTH) {
 #pragma unroll
-        for (int d = 0; d < DEPTH; d++) issue(d);
+        for (int d = 0; d < DEPTH; d++) {
+            issue(d);
+            if (d == 0 && wave == 0) factors.fetch(a, m0, n0, lane);
+        }
         stamps.mark(1);
         asm volatile("" ::"s"(scale));   // (here, not where the outputs are ready)
         int i = 0;
@@ -309,6 +312,7 @@ __global__ void __launch_bounds__(lds_launch_bound(MT, RG)) lds_gemm_kernel(cons
         else drain_ring<0, DEPTH, PER_STAGE>(consume, i);
     } else {
         for (int i = 0; i < mine; i++) issue(i);
+        if (wave == 0) factors.fetch(a, m0, n0, lane);
         stamps.mark(1);
         asm volatile("" ::"s"(scale));
         wait_vmcnt<0>();

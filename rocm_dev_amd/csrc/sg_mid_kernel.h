@@ -54,6 +54,46 @@ constexpr int mid_activation_waves(int instr, int waves) {
     return best;
 }
 
+// Scales and stores a wave's RGW x MH fragments, get(rg, mb) each; m_wave, n_wave: the lane's place in the first.  The factors
+// of all fragments are requested at once: one round trip instead of one per fragment and column.
+template <int RGW, int MH, class Get>
+__device__ __forceinline__ void store_wave_tile(const StreamArgs& a, Get&& get, int m_wave, int n_wave) {
+    const float scale = scalar_scale(a);
+    if (a.row_scale || a.col_scale) {
+        f32x4 col[RGW];
+        float row[MH];
+#pragma unroll
+        for (int rg = 0; rg < RGW; rg++) col[rg] = col_scale_ahead(a, n_wave + rg * 16);
+#pragma unroll
+        for (int mb = 0; mb < MH; mb++) row[mb] = row_scale_ahead(a, m_wave + mb * 16);
+#pragma unroll
+        for (int rg = 0; rg < RGW; rg++)
+#pragma unroll
+            for (int mb = 0; mb < MH; mb++)
+                store_fragment(a, get(rg, mb), scale, m_wave + mb * 16, n_wave + rg * 16, row[mb], col[rg]);
+    } else {
+#pragma unroll
+        for (int rg = 0; rg < RGW; rg++)
+#pragma unroll
+            for (int mb = 0; mb < MH; mb++) {
+                f32x4 v = get(rg, mb);
+                asm volatile("" : "+v"(v));   // (as in store_fragment)
+                v *= scale;
+                store_scaled(a, v, m_wave + mb * 16, n_wave + rg * 16);
+            }
+    }
+}
+// Stores a wave's partials of a K split for mid_reduce_kernel: [tile][split][wave][fragment][lane], 16 bytes a lane.
+template <int RGW, int MH, int WAVES>
+__device__ __forceinline__ void store_wave_partials(const StreamArgs& a, const f32x4 (&acc)[RGW][MH], int tile_id, int split, int wave, int lane) {
+    f32x4* mine = reinterpret_cast<f32x4*>(a.ws + ((size_t)tile_id * a.split_k + split) * (WAVES * RGW * MH * 256) +
+                                           (size_t)wave * (RGW * MH * 256)) + lane;
+#pragma unroll
+    for (int rg = 0; rg < RGW; rg++)
+#pragma unroll
+        for (int mb = 0; mb < MH; mb++) mine[(rg * MH + mb) * 64] = acc[rg][mb];
+}
+
 // TAIL: k is not a multiple of 128 (but of 16, and beyond 128).  The last 128-byte K block of both operands is loaded
 //      from k - 128 - a window that ends with the row, nothing past it is read - and the activation fragments of that
 //      stage are zero in the 16-byte pieces the block before has already multiplied: lane (r, g) holds pieces g and
@@ -315,36 +355,9 @@ __global__ void __launch_bounds__(WN * 128) mid_gemm_kernel(const StreamArgs a) 
     stamps.mark(3);
 
     // ---- epilogue --------------------------------------------------------------------------------
-    // the factors of all the wave's fragments at once: one round trip instead of one per fragment and column
-    const float scale = scalar_scale(a);
-    auto store_all = [&](auto&& get) __attribute__((always_inline)) {
-        const int m_wave = m0 + wm * MH * 16 + r, n_wave = n0 + wn * RGW * 16 + 4 * g;
-        if (a.row_scale || a.col_scale) {
-            f32x4 colf[RGW];
-            float rowf[MH];
-#pragma unroll
-            for (int rg = 0; rg < RGW; rg++) colf[rg] = col_scale_ahead(a, n_wave + rg * 16);
-#pragma unroll
-            for (int mb = 0; mb < MH; mb++) rowf[mb] = row_scale_ahead(a, m_wave + mb * 16);
-#pragma unroll
-            for (int rg = 0; rg < RGW; rg++)
-#pragma unroll
-                for (int mb = 0; mb < MH; mb++)
-                    store_fragment(a, get(rg, mb), scale, m_wave + mb * 16, n_wave + rg * 16, rowf[mb], colf[rg]);
-        } else {
-#pragma unroll
-            for (int rg = 0; rg < RGW; rg++)
-#pragma unroll
-                for (int mb = 0; mb < MH; mb++) {
-                    f32x4 v = get(rg, mb);
-                    asm volatile("" : "+v"(v));   // (as in store_fragment)
-                    v *= scale;
-                    store_scaled(a, v, m_wave + mb * 16, n_wave + rg * 16);
-                }
-        }
-    };
+    const int m_wave = m0 + wm * MH * 16 + r, n_wave = n0 + wn * RGW * 16 + 4 * g;
     if (a.split_k == 1) {
-        store_all([&](int rg, int mb) { return acc[rg][mb]; });
+        store_wave_tile<RGW, MH>(a, [&](int rg, int mb) { return acc[rg][mb]; }, m_wave, n_wave);
         stamps.end(a);
         return;
     }
@@ -354,12 +367,7 @@ __global__ void __launch_bounds__(WN * 128) mid_gemm_kernel(const StreamArgs a) 
     const int tile_id = tile_m * a.n_tiles + tile_n;
     float* ws_tile = a.ws + ((size_t)tile_id * a.split_k) * (FRAGS_WG * 256);
     if (a.defer_reduce) {
-        // partials only: [tile][split][wave][fragment][lane] as one 16-byte store per lane and fragment
-        f32x4* mine = reinterpret_cast<f32x4*>(ws_tile + (size_t)split * (FRAGS_WG * 256) + (size_t)wave * (RGW * MH * 256)) + lane;
-#pragma unroll
-        for (int rg = 0; rg < RGW; rg++)
-#pragma unroll
-            for (int mb = 0; mb < MH; mb++) mine[(rg * MH + mb) * 64] = acc[rg][mb];
+        store_wave_partials<RGW, MH, WAVES>(a, acc, tile_id, split, wave, lane);
         stamps.end(a);
         return;
     }
@@ -384,7 +392,7 @@ __global__ void __launch_bounds__(WN * 128) mid_gemm_kernel(const StreamArgs a) 
         stamps.end(a);
         return;
     }
-    store_all([&](int rg, int mb) {
+    store_wave_tile<RGW, MH>(a, [&](int rg, int mb) {
         const float* p = ws_tile + (size_t)wave * (RGW * MH * 256) + (rg * MH + mb) * 256 + lane;
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         for (int sp = 0; sp < a.split_k; sp++) {
@@ -393,7 +401,7 @@ __global__ void __launch_bounds__(WN * 128) mid_gemm_kernel(const StreamArgs a) 
             for (int e = 0; e < 4; e++) v[e] += __hip_atomic_load(q + e * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return v;
-    });
+    }, m_wave, n_wave);
     if (threadIdx.x == 0) __hip_atomic_store(&a.counters[tile_id], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     stamps.end(a);
 }

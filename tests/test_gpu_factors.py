@@ -10,6 +10,13 @@ from gpu_util import bits, scale_tensor
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture(scope="module")
+def sg():
+    import rocm_dev_amd
+    return rocm_dev_amd
+
+
 # m, n, k, pad: n = 2 mod 4 (the last fragment ends inside a lane's four columns) except where a kernel wants whole tiles
 SHAPES = [
     (1, 2, 512, 0), (8, 4098, 4096, 0), (13, 6146, 4112, 16), (30, 4098, 14336, 0), (32, 1026, 8192, 0),   # per-tile ring, K splits

@@ -1,0 +1,151 @@
+"""The mid-batch kernel for rows off their 128-byte lines (sg_line_kernel.h): every compiled tile at the sizes where its edges
+can go wrong, every place a row can start on its line, and the library's own choice of it."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import GEMM_TOL, bits, dev, rowcol_reference, scale_tensor
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def sg():
+    import rocm_dev_amd
+    rocm_dev_amd.tuning_clear()
+    yield rocm_dev_amd
+    rocm_dev_amd.tuning_clear()
+
+
+TILES = [(4, 2, 2), (8, 2, 2), (8, 2, 4), (8, 2, 6), (8, 3, 4)]     # waves, row tiles, activation blocks
+
+
+def _line(A, B, D, S, rs, cs, tile, sk):
+    from rocm_dev_amd._lib import lib
+    m, k = A.shape
+    return lib.sg_debug_line_gemm(A.data_ptr(), B.data_ptr(), D.data_ptr(), S.data_ptr(), rs.data_ptr() if rs is not None else None,
+                                  cs.data_ptr() if cs is not None else None, m, B.shape[0], k, B.stride(0), *tile, sk,
+                                  torch.cuda.current_stream().cuda_stream)
+
+
+def _in_nans(codes, stride, offset):
+    """`codes` with rows `stride` apart, `offset` bytes into a buffer whose every other byte is a NaN code: a result that
+    took anything but the rows themselves is NaN."""
+    rows, k = codes.shape
+    buf = torch.full((256 + offset + rows * stride + 256,), 0x7f, dtype=torch.uint8, device="cuda")
+    view = buf[256 + offset:256 + offset + rows * stride].view(rows, stride)[:, :k]
+    view.copy_(dev(codes))
+    return view
+
+
+# one block and a piece, the last block of one piece and of seven, one tile's rows and one more, a single weight row pair;
+# 192 rows of either operand; whole blocks on a stride that is off the lines
+SHAPES = [(33, 2, 144, 0), (65, 130, 272, 0), (128, 128, 1040, 16), (129, 190, 656, 48), (193, 194, 2032, 0), (64, 258, 384, 16),
+          (100, 322, 1936, 112), (40, 66, 1280, 32)]
+
+
+@pytest.mark.parametrize("m,n,k,pad", SHAPES)
+def test_every_tile_at_its_edges(oracle, m, n, k, pad):
+    a8, b8, scale = oracle.make_gemm_operands(m, n, k, seed=m + n)
+    # (the oracle's model of the instruction's own sum at every k, as for the wide tiles)
+    ref = rowcol_reference(oracle, a8, b8, scale, None, None, model=True)
+    rs = np.random.default_rng(1).uniform(0.5, 2.0, size=m).astype(np.float32)
+    cs = np.random.default_rng(2).uniform(0.5, 2.0, size=n).astype(np.float32)
+    ref_rc = rowcol_reference(oracle, a8, b8, scale, rs, cs, model=True)
+    A, B, S, R, C = _in_nans(a8, k, 16), _in_nans(b8, k + pad, 48), scale_tensor(scale), dev(rs), dev(cs)
+    for tile in TILES:
+        for sk in (1, 2, 3, 5):
+            if sk > k // 128:
+                continue
+            G = torch.full((m + 8, n), 9.0, dtype=torch.bfloat16, device="cuda")   # guard rows around the output
+            D = G[4:4 + m]
+            for r, c, want in ((None, None, ref), (R, C, ref_rc)):
+                D.fill_(float("nan"))
+                assert _line(A, B, D, S, r, c, tile, sk) == 0, (tile, sk)
+                torch.cuda.synchronize()
+                assert (G[:4] == 9).all() and (G[4 + m:] == 9).all(), (tile, sk)
+                err = oracle.max_rel_err_bf16(bits(D), want)
+                assert err <= GEMM_TOL, (tile, sk, err)
+
+
+@pytest.mark.parametrize("pitch", range(16, 129, 16))
+def test_every_place_on_the_line(oracle, pitch):
+    """Weight rows `pitch` bytes further on their line each (eight pitches), both operands starting at each of its eight
+    pieces, on a k of whole blocks and on one that ends within a block; several weight tiles, so that the walk of K starts
+    at other blocks than the first."""
+    m, n = 40, 20 * 64 + 2
+    for k in (640, 640 + 48):
+        a8, b8, scale = oracle.make_gemm_operands(m, n, k, seed=pitch)
+        ref = rowcol_reference(oracle, a8, b8, scale, None, None, model=True)
+        S = scale_tensor(scale)
+        stride = 768 + pitch
+        for offset in range(0, 128, 16):
+            A, B = _in_nans(a8, k, offset), _in_nans(b8, stride, 112 - offset)
+            for tile, sk in (((4, 2, 2), 1), ((8, 2, 2), 2)):
+                D = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+                assert _line(A, B, D, S, None, None, tile, sk) == 0
+                err = oracle.max_rel_err_bf16(bits(D), ref)
+                assert err <= GEMM_TOL, (k, offset, tile, err)
+
+
+def test_nan_codes_poison_their_row_and_column_only(oracle):
+    """A NaN in the pieces of the last block, which pieces behind the end of a row repeat."""
+    m, n, k = 70, 200, 1040
+    a8, b8, scale = oracle.make_gemm_operands(m, n, k, seed=3)
+    a8[7, k - 1] = 0x7f
+    b8[150, k - 16] = 0x7f
+    A, B, S = dev(a8), dev(b8), scale_tensor(scale)
+    want = np.zeros((m, n), bool)
+    want[7] = True
+    want[:, 150] = True
+    for tile in TILES:
+        for sk in (1, 3):
+            D = torch.zeros((m, n), dtype=torch.bfloat16, device="cuda")
+            assert _line(A, B, D, S, None, None, tile, sk) == 0
+            assert np.array_equal(torch.isnan(D).cpu().numpy(), want), (tile, sk)
+
+
+# unsplit and split, a record of either engine and a wide tile in its place; the last one off its lines by the stride only
+@pytest.mark.parametrize("m,n,k,pad", [(47, 28666, 2064, 0), (100, 2374, 5440, 16), (96, 4828, 11984, 0), (300, 2300, 9200, 0),
+                                       (264, 10178, 9952, 112), (100, 4096, 8192, 16)])
+def test_the_choice_and_whose_workspace(sg, m, n, k, pad):
+    """The library's own launch is the tile that the choice names, bit for bit, eagerly, in a replayed graph and on a
+    workspace of the caller's of the size the query asks for; with what the record alone needs the call still runs."""
+    import ctypes as C
+    from rocm_dev_amd import api
+    from rocm_dev_amd._lib import lib
+    out = (C.c_int * 4)()
+    assert lib.sg_debug_line_choice(m, n, k, k + pad, 0, C.byref(out)) == 0
+    waves, rg, mb, sk = out
+    assert waves, "not a shape of this kernel"
+    assert api.skinny_gemm_wide_choice(m, n, k, k + pad) is None
+    g = torch.Generator().manual_seed(m)
+    W = torch.zeros((n, k + pad), dtype=torch.uint8)
+    W[:, :k] = torch.randn((n, k), generator=g).to(torch.float8_e4m3fn).view(torch.uint8)
+    A, W = torch.randn((m, k), generator=g).to(torch.float8_e4m3fn).view(torch.uint8).cuda(), W.cuda()[:, :k]
+    S = scale_tensor(0.5)
+    want, D = (torch.empty((m, n), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    assert _line(A, W, want, S, None, None, (waves, rg, mb), sk) == 0
+    assert sg.skinny_gemm_fastpath(A, W, D, S) == 0
+    assert torch.equal(D, want)
+    need = sg.workspace_query(m, n, k)
+    ws = torch.empty(max(need, 1 << 17), dtype=torch.uint8, device="cuda")
+    sg.workspace_init(ws)
+    D.zero_()
+    assert sg.skinny_gemm_auto_ws(A, W, D, S, ws) == 0
+    assert torch.equal(D, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        sg.skinny_gemm_auto_ws(A, W, D, S, ws, check=True)
+    for _ in range(3):
+        D.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(D, want)
+    if sk > 1 and k % 128:
+        record, _ = sg.skinny_gemm_choice(m, n, k)
+        if record.split_k == 1:     # the record needs no workspace: without one the call runs on something unsplit
+            D.zero_()
+            assert sg.skinny_gemm_auto_ws(A, W, D, S, None) == 0
+            err = (D.float() - want.float()).norm() / want.float().norm()
+            assert float(err) < 7e-3     # one bf16 rounding each, 1.6e-3 measured: four times that

@@ -1,0 +1,65 @@
+"""Which launches the kernel for rows off their 128-byte lines takes (no GPU: the choice is the library's host code)."""
+import ctypes as C
+import random
+
+import pytest
+
+TILES = {(4, 2, 2), (8, 2, 2), (8, 2, 4), (8, 2, 6), (8, 3, 4)}
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from rocm_dev_amd._lib import lib
+    return lib
+
+
+def _choice(lib, m, n, k, stride):
+    out = (C.c_int * 4)()
+    assert lib.sg_debug_line_choice(m, n, k, stride, 0, C.byref(out)) == 0
+    return tuple(out)
+
+
+def test_only_rows_off_their_lines_and_only_compiled_tiles(lib):
+    import rocm_dev_amd as sg
+    r = random.Random(7)
+    taken = 0
+    for _ in range(4000):
+        m, n = r.randint(1, 900), 2 * r.randint(1, 20000)
+        k, pad = 16 * r.randint(1, 1500), 16 * r.randint(0, 9)
+        waves, rg, mb, sk = _choice(lib, m, n, k, k + pad)
+        if not waves:
+            continue
+        taken += 1
+        assert 32 < m <= 768 and k > 128 and (k % 128 or (k + pad) % 128)
+        assert (waves, rg, mb) in TILES and 1 <= sk <= k // 128
+        bn, bm = 8 * waves * rg, 32 * mb
+        if sk > 1 and k % 128:      # room for the partials in a workspace of the size that the query asks for
+            partials = -(-n // bn) * -(-m // bm) * sk * bn * bm * 4
+            assert sg.workspace_query(m, n, k) >= 65536 + partials
+    assert taken > 500
+
+
+def test_shapes_timed_on_both_sides_of_the_rule(lib):
+    # line kernel / what it replaces, us: 16.4 / 37.0, 52.9 / 83.9, 24.9 / 36.7, 23.1 / 43.5, 65.9 / 75.8 (a wide tile)
+    for m, n, k, pad in [(468, 566, 9200, 0), (47, 28666, 10320, 0), (128, 8192, 8208, 0), (96, 4828, 11984, 0), (599, 7284, 9728, 16)]:
+        assert _choice(lib, m, n, k, k + pad)[0], (m, n, k)
+    # 10.3 / 5.2, 11.4 / 8.4, 83.4 / 62.9, 91.6 / 75.0, 32.0 / 18.9
+    for m, n, k, pad in [(49, 4092, 1680, 112), (120, 1422, 4000, 112), (207, 27442, 6800, 112), (440, 22664, 6208, 0), (412, 25130, 768, 112)]:
+        assert not _choice(lib, m, n, k, k + pad)[0], (m, n, k)
+    for m, n, k in [(128, 8192, 8192), (64, 57344, 8320), (300, 2300, 9216)]:     # whole lines
+        assert not _choice(lib, m, n, k, k)[0], (m, n, k)
+
+
+def test_the_reported_record_is_launchable_and_split_where_a_workspace_is_asked_for(lib):
+    import launch_rules
+    import rocm_dev_amd as sg
+    from rocm_dev_amd import api
+    r = random.Random(8)
+    for _ in range(2000):
+        m, n, k = r.randint(33, 768), 2 * r.randint(100, 16000), 16 * r.randint(20, 1200)
+        record, from_table = sg.skinny_gemm_choice(m, n, k)
+        assert not from_table
+        d = api.tuning_as_dict(record)
+        if record.engine == 4:
+            assert launch_rules.expect_mid(m, n, k, d) == launch_rules.OK, (m, n, k, d)
+        assert (record.split_k > 1) == (sg.workspace_query(m, n, k) > 0), (m, n, k, d)
