@@ -985,7 +985,10 @@ static Config pick_config(int m, int n, int k, int cu_count) {
                 const int pt = blocks / w;   // compiled for 1, 2 and 4 blocks per wave
                 if (blocks % w != 0 || pt * c.mt > 4 || pt == 3) continue;
                 c.waves = w;
-                c.depth = blocks / w == 1 ? (w <= 2 ? 4 : 2) : 3;
+                // (eight waves at 17..32 rows on two slots: 32 x 28672 x 4096 22.05 -> 21.7 us, 32 x 14336 x 4096 13.3 -> 13.1 - with
+                // factors, which then find LDS beside the third staging area, 22.9 -> 22.1 and 14.3 -> 13.8; on six and
+                // seven waves, and up to 16 rows, level or behind: 12 x 14336 x 8192 24.4 -> 24.9)
+                c.depth = blocks / w == 1 ? (w <= 2 ? 4 : 2) : (c.mt == 2 && w == 8 ? 2 : 3);
                 c.wavetile = 3;
                 return c;
             }
