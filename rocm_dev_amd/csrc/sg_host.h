@@ -55,6 +55,7 @@ int launch_mid_reduce(int rgw, int mh, int wn, const StreamArgs& a, hipStream_t 
 struct SparseArgs;
 int launch_sparse(int mt, int rg, int xu2, int depth, bool pairs, const SparseArgs& sa, unsigned grid, unsigned threads,
                   size_t lds, hipStream_t stream);
+int launch_sparse_xreg(int pt, const SparseArgs& sa, unsigned grid, hipStream_t stream);
 int launch_sparse_wavetile(int rg, int xu2, int depth, bool pairs, const SparseArgs& sa, unsigned grid, unsigned threads,
                            size_t lds, hipStream_t stream);
 

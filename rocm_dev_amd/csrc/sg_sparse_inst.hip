@@ -41,6 +41,23 @@ int launch_sparse(int mt, int rg, int xu2, int depth, bool pairs, const SparseAr
     return SG_INVALID_CONFIG;
 }
 
+// register-resident activations (17..32 rows): k = 512 * pt * waves, as many ring slots as 160 KB allow
+int launch_sparse_xreg(int pt, const SparseArgs& sa, unsigned grid, hipStream_t stream) {
+    const int waves = sa.g.waves;
+    if (waves < 2 || waves > 8 || sa.g.k != 512 * pt * waves || sa.g.m > 32) return SG_INVALID_CONFIG;
+    auto go = [&](auto kernel, int depth, LdsGranted& granted) {
+        const size_t lds = (size_t)waves * sparse_xreg_wave_bytes(depth);
+        if (int rc = request_dynamic_lds(reinterpret_cast<const void*>(kernel), lds, granted)) return rc;
+        kernel<<<dim3(grid), dim3((unsigned)waves * 64), lds, stream>>>(sa);
+        return report_hip("sparse24_gemm_xreg_kernel launch", hipGetLastError()) == hipSuccess ? (int)SG_SUCCESS : (int)SG_LAUNCH_FAILED;
+    };
+    static LdsGranted granted[4];
+    const bool three = waves * sparse_xreg_wave_bytes(3) <= 160 * 1024;
+    if (pt == 1) return three ? go(sparse24_gemm_xreg_kernel<1, 3>, 3, granted[0]) : go(sparse24_gemm_xreg_kernel<1, 2>, 2, granted[1]);
+    if (pt == 2) return three ? go(sparse24_gemm_xreg_kernel<2, 3>, 3, granted[2]) : go(sparse24_gemm_xreg_kernel<2, 2>, 2, granted[3]);
+    return SG_INVALID_CONFIG;
+}
+
 template <int RG, int XU2, int DEPTH, bool TAIL, bool PAIRS>
 static int launch_wavetile(const SparseArgs& sa, unsigned grid, unsigned threads, size_t lds, hipStream_t stream) {
     if (threads > (RG == 4 ? 512u : 1024u)) return SG_INVALID_CONFIG;

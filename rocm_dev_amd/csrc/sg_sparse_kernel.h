@@ -465,5 +465,136 @@ __global__ void __launch_bounds__(RG == 4 ? 512 : 1024) sparse24_gemm_wavetile_k
     stamps.end(a);
 }
 
+// ---------------------------------------------------------------------------------------------
+// Persistent variant with the activations in registers, for 17..32 rows and more than two tiles per CU.  There a workgroup
+// per tile streams 32 rows of activations beside 16 or 32 rows of weights, more L2 hits than misses, and a CU's L1 serves
+// them in turn: 32 x 14336 x 4096 takes 459 KB of activations and 143 KB of weights into every CU.  Here wave w of a
+// workgroup works on K stages w, w + waves, ... (PT of them) of every tile the workgroup walks, and keeps the activation
+// fragments of those stages (64 registers each): they cross the L1 once a CU, 128 KB, and the ring carries weights only.
+// As in sg_xreg_kernel.h the fragments reach the registers through LDS, the waves' partial tiles meet in LDS and the wave
+// that sums them rotates with the tile.  us, before -> now: 32 x 28672 x 4096 (24 rows) 19.5 -> 16.5, 32 x 28672 x 7168
+// 35.8 -> 25.7, 32 x 16384 x 8192 23.8 -> 19.2, 32 x 28672 x 2048 13.4 -> 10.3, 30 x 20480 x 3072 15.7 -> 11.3,
+// 32 x 14336 x 4096 11.3 -> 10.8.  The activations go first, all of a stage at once; with the first weight stages in front of
+// their second half, which leaves nothing in flight while it is read, 10.8 is 11.0, 16.5 is 17.2 and 11.3 is 12.0.
+constexpr int sparse_xreg_wave_bytes(int DEPTH) { return DEPTH * 5120 + 8192; }
+
+// k = 512 * PT * waves
+template <int PT, int DEPTH>
+__global__ void __launch_bounds__(512) sparse24_gemm_xreg_kernel(const SparseArgs sa) {
+    // [wave][DEPTH][5 KB] | [wave][8 KB of staging], the latter then the partial tiles [2][FRAGS][wave][64]
+    extern __shared__ __attribute__((aligned(1024))) uint8_t ring[];
+    const StreamArgs& a = sa.g;
+    Stamps stamps;
+    stamps.begin();
+    constexpr int MT = 2, FRAGS = MT, PER_STAGE = 5, STAGE_BYTES = 5120;
+    static_assert(DEPTH >= 2, "the second half of a stage's activations is staged in two ring slots");
+
+    const int lane = lane_id();
+    const int wave = wave_id();
+    const int waves = a.waves;
+    const int r = lane & 15, g = lane >> 4;
+    const TileRun run = persistent_tile_run(a.n_tiles);
+    const int my_tiles = run.count, total = PT * my_tiles;
+    const size_t v_stride = (size_t)(a.k >> 1), t_stride = (size_t)(a.k >> 3);
+
+    const int v_row = lane >> 4, v_pp = lane & 15;     // values / activations: 4 rows x 16 pieces an instruction
+    const int t_row = lane >> 2, t_pp = lane & 3;      // metadata: 16 rows x 4 pieces
+    const uint8_t* const my_ring = ring + (size_t)wave * (DEPTH * STAGE_BYTES);
+    const unsigned my_ring_lds = lds_addr(my_ring);
+    uint8_t* const areas = ring + (size_t)waves * (DEPTH * STAGE_BYTES);
+    const uint8_t* const my_area = areas + (size_t)wave * 8192;
+    f32x4* const red = reinterpret_cast<f32x4*>(areas);
+
+    auto issue = [&](int i) __attribute__((always_inline)) {   // stage i = tile i / PT, K stage wave + (i % PT) * waves
+        const int j = i / PT, kb = wave + (i % PT) * waves;
+        const int n0 = (run.first + j) * 16, last = a.n - 1 - n0;   // rows past the edge re-read the last row, never stored
+        const unsigned slot = my_ring_lds + (unsigned)(i % DEPTH) * STAGE_BYTES;
+        const uint8_t* v_base = a.B + (size_t)n0 * v_stride + ((size_t)kb << 8);
+        const uint8_t* t_base = sa.meta + (size_t)n0 * t_stride + ((size_t)kb << 6);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int row16 = 4 * u + v_row, row = row16 < last ? row16 : last;
+            dma_1kb_stream_at(v_base, (unsigned)row * (unsigned)v_stride + ((v_pp ^ row16) << 4), slot + u * 1024);
+        }
+        const int row = t_row < last ? t_row : last;
+        dma_1kb_stream_at(t_base, (unsigned)row * (unsigned)t_stride + ((t_pp ^ (t_row >> 2)) << 4), slot + 4096);
+    };
+
+    // ---- activations: rows 0..15 of a stage through the wave's staging area, rows 16..31 through its first two slots ------
+    i32x4 x[PT][MT][8];
+    const int x_rd = ((r >> 2) * 2 + (g >> 1)) * 1024 + (r & 3) * 256;
+    const float scale = scalar_scale(a);
+#pragma unroll
+    for (int t = 0; t < PT; t++) {
+        const size_t k0 = (size_t)(wave + t * waves) << 9;
+#pragma unroll
+        for (int i2 = 0; i2 < 16; i2++) {
+            const int row_l = 4 * (i2 >> 1) + v_row;
+            const int row = row_l < a.m ? row_l : a.m - 1;
+            dma_1kb(a.A + (size_t)row * a.k + k0 + (i2 & 1) * 256 + ((v_pp ^ (row_l & 15)) << 4),
+                    (i2 < 8 ? lds_addr(my_area) : my_ring_lds) + (i2 & 7) * 1024);
+        }
+        wait_vmcnt<0>();
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int p = 0; p < 8; p++)
+                x[t][mt][p] = *reinterpret_cast<const i32x4*>((mt ? my_ring : my_area) + x_rd + (((8 * (g & 1) + p) ^ r) << 4));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // in registers before the areas are written again
+    }
+    asm volatile("" ::"s"(scale));
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++)
+        if (d < total) issue(d);
+    stamps.mark(1);
+    __syncthreads();   // every wave has its fragments: the staging areas may take partial tiles
+
+    const int v_rd = (r >> 2) * 1024 + (r & 3) * 256;
+    const int t_rd = 4096 + r * 64 + ((g ^ (r >> 2)) << 4);
+    int turn = 0;
+    for (int j = 0; j < my_tiles; j++) {
+        f32x4 acc[MT] = {};
+#pragma unroll
+        for (int t = 0; t < PT; t++) {
+            const int i = j * PT + t, behind = total - 1 - i;
+            if (behind >= DEPTH - 1) wait_vmcnt<(DEPTH - 1) * PER_STAGE>();
+            else wait_vmcnt_upto(behind * PER_STAGE);
+            if (i == 0) stamps.mark(2);
+            const uint8_t* slot = my_ring + (size_t)(i % DEPTH) * STAGE_BYTES;
+            const i32x4 idx = *reinterpret_cast<const i32x4*>(slot + t_rd);
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                const i32x4 v = *reinterpret_cast<const i32x4*>(slot + v_rd + (((4 * g + p) ^ r) << 4));
+                const i32x2 v_lo = {v.x, v.y}, v_hi = {v.z, v.w};
+                const int id_lo = idx[p] & 0xffff, id_hi = (unsigned)idx[p] >> 16;
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) {
+                    acc[mt] = __builtin_amdgcn_smfmac_f32_16x16x64_fp8_fp8(v_lo, x[t][mt][2 * p], acc[mt], id_lo, 0, 0);
+                    acc[mt] = __builtin_amdgcn_smfmac_f32_16x16x64_fp8_fp8(v_hi, x[t][mt][2 * p + 1], acc[mt], id_hi, 0, 0);
+                }
+            }
+            // the slot is refilled only after its reads have returned
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            if (i + DEPTH < total) issue(i + DEPTH);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (j == my_tiles - 1) stamps.mark(3);
+        // sum the waves' partial tiles in wave order; double-buffered by tile parity: one barrier a tile
+        f32x4* buf = red + (size_t)(j & 1) * (FRAGS * waves * 64);
+#pragma unroll
+        for (int f = 0; f < FRAGS; f++) buf[(f * waves + wave) * 64 + lane] = acc[f];
+        __syncthreads();
+        int first = wave - turn;
+        first = first < 0 ? first + waves : first;
+        turn = turn + 1 == waves ? 0 : turn + 1;
+        for (int f = first; f < FRAGS; f += waves) {
+            f32x4 v = buf[(f * waves) * 64 + lane];
+            for (int w = 1; w < waves; w++) v += buf[(f * waves + w) * 64 + lane];
+            store_fragment(a, v, scale, f * 16 + r, (run.first + j) * 16 + 4 * g);
+        }
+    }
+    stamps.end(a);
+}
 
 }  // namespace sg
