@@ -80,7 +80,9 @@ int    sg_release_workspaces(void);
  * sg_skinny_gemm_auto_ws does the same - its split-K partials and arrival counters live in `workspace` and nowhere
  * else, nothing is allocated, and a launch that would need more than it is given returns SG_WORKSPACE_TOO_SMALL.
  *   sg_workspace_query  *bytes = what sg_skinny_gemm_auto_ws needs for the shape with the tuning table as it is now
- *                       (0 when the launch it would choose has no K split; then workspace may be NULL)
+ *                       (0 when the launch it would choose has no K split; then workspace may be NULL) to run what
+ *                       sg_skinny_gemm_auto runs, bit for bit; where the kernel for rows off their 128-byte lines would
+ *                       split K, less - or NULL - is accepted too and runs what fits
  *   sg_workspace_init   zeroes the counter region (the first 64 KB) of a workspace with a kernel in stream order:
  *                       once per buffer, before its first use; every launch that completes leaves it zero again
  * workspace: device memory, 256-byte aligned, [16384 arrival counters][fp32 partials]; one buffer serves launches of
@@ -233,6 +235,9 @@ int sg_skinny_gemm_pick(int m, int n, int k, int out[8]);
 
 /* The complete record sg_skinny_gemm_auto would launch for the shape: the tuning table's entry when
  * there is one (*from_table = 1), the built-in heuristics' otherwise (0).  from_table may be NULL.
+ * From 33 rows on, where k or b_stride is no multiple of 128, the library may run the kernel for rows off their lines in
+ * place of the heuristics' record (sg_debug_line_choice, sgemm_debug.h); where that splits K and the record does not, the
+ * mid-batch record of the same split is reported.
  * Above 128 rows the library may run the wide-tile kernel in place of the heuristics' record, and no record describes
  * that kernel: sg_debug_wide_choice (sgemm_debug.h) says whether it does and on which tile, engine = 0 replays it, and the
  * record is the mid-batch launch that it replaces (stored in the table it is what runs from then on). */

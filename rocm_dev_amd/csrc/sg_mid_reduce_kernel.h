@@ -13,7 +13,7 @@ namespace sg {
 // partials that the GEMM had just left in the caches.  The tile geometry comes as run-time values: rgw x mh
 // fragments per wave of the GEMM, wn x 2 waves per tile.
 // FACTORS: there are row or column factors (requested ahead of the partials, in 34 registers that the other build does not
-// hold: five workgroups a SIMD instead of eight).
+// hold: five waves a SIMD instead of eight).
 constexpr int kReduceFrags = 4;
 template <bool FACTORS>
 __global__ void __launch_bounds__(256) mid_reduce_kernel(const StreamArgs a, int rgw, int mh, int wn) {
