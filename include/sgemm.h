@@ -52,8 +52,10 @@ typedef enum SgReturnCode {
 const char* sg_strerror(int code);
 
 /* Library-owned split-K workspaces (fp32 partial fragments + one arrival counter per output tile), one per
- * device and stream: launches on one stream run in order and share a workspace, launches on different
- * streams may overlap and never share one.  A workspace is created, or grown, by the first launch on its
+ * device and stream: calls on one stream run in order and share a workspace, calls on different
+ * streams may overlap and never share one.  Host threads may call on one stream at the same time: a call whose
+ * launches hand each other memory (a GEMM and the sum of its K split's partials, the row encoder and the GEMM on
+ * its codes) enqueues them with no other such call of the library's in between.  A workspace is created, or grown, by the first launch on its
  * stream that needs it (split_k > 1, also when the library chooses the split itself); at most 512 MB of
  * partials per launch, beyond that SG_WORKSPACE_TOO_SMALL.  An outgrown buffer is kept until it is released
  * (below).  A launch recorded into a HIP graph keeps the workspace of the stream it was captured on: run no

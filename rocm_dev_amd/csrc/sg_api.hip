@@ -181,6 +181,29 @@ int get_workspace(hipStream_t stream, size_t partial_bytes, size_t n_counters, W
     return SG_SUCCESS;
 }
 
+// ---- calls of more than one launch ---------------------------------------------------------------
+// A call whose K split is summed by a second launch, or whose activations an encoder launch quantises first, hands memory of
+// its stream's (or of the caller's, or the fixed array below) from one launch to the next.  Stream order keeps calls apart
+// only as whole calls: with two host threads on one stream another call's launch on the same memory could come in between,
+// and the sum would be of that call's partials.  So every launch that uses such memory is enqueued inside its stream's turn,
+// which a call holds from its first launch to its last.  A mutex per stream modulo kTurns: nothing to allocate or to
+// give back with a stream; streams that share one wait for each other's enqueuing, never for the device.  (Uncontended it
+// costs such a call about 20 ns of host time; a call without a K split takes none.)
+constexpr int kTurns = 64;
+static std::recursive_mutex g_turn[kTurns];    // (recursive: the encoder's call holds it around the GEMM's)
+class StreamTurn {
+    std::unique_lock<std::recursive_mutex> lock_;
+public:
+    StreamTurn(bool needed, hipStream_t stream) {
+        if (!needed) return;
+        int dev = 0;
+        (void)current_device(&dev);
+        const unsigned long long key = (unsigned long long)reinterpret_cast<uintptr_t>(stream) + (unsigned long long)dev;
+        lock_ = std::unique_lock<std::recursive_mutex>(g_turn[(key * 0x9E3779B97F4A7C15ull) >> 58]);
+    }
+};
+static_assert(kTurns == 64, "the top six bits of the product");
+
 // ---- scratch for the entry point that allocates nothing -------------------------------------------
 // Split-K partials and arrival counters of sg_skinny_gemm_tuned_noalloc live in this array instead of a
 // workspace from hipMalloc.  Every device the library runs on holds its own copy at its own address; in host
@@ -412,6 +435,7 @@ struct RingConfig {
 };
 
 static int launch_ring(const RingConfig& c, StreamArgs a, hipStream_t stream) {
+    const StreamTurn turn(c.split_k > 1, stream);
     if (a.k % 256 != 0) return SG_K_NOT_DIVISIBLE_BY_WARPTILE_K;
     if (c.a_producers < 1 || c.b_producers < 1 || c.consumers < 1 || c.qsize < 1) return SG_INVALID_CONFIG;
     if (c.a_producers + c.b_producers + c.consumers > 16) return SG_TOO_MANY_WARPS;
@@ -712,6 +736,7 @@ static bool sparse_k_ok(int k) { return k >= 512 && k % 128 == 0; }
 
 // 2:4 sparse engine: c.rg row tiles per wave, c.waves waves splitting K, c.depth ring slots.
 static int launch_sparse_engine(const Config& c, StreamArgs a, const uint8_t* meta, hipStream_t stream) {
+    const StreamTurn turn(c.split_k > 1, stream);
     if (!sparse_k_ok(a.k)) return SG_K_NOT_DIVISIBLE_BY_WARPTILE_K;
     const int blocks = (a.k + 511) / 512;   // 512-k stages, the last one partly used when 512 does not divide k
     size_t tiles;
@@ -847,6 +872,7 @@ static void workspace_need(const Config& c, int m, int n, size_t* partial_bytes,
 }
 
 static int launch_config(const Config& c, const StreamArgs& a, hipStream_t stream) {
+    const StreamTurn turn(c.split_k > 1, stream);
     if (c.engine == ENGINE_DIRECT) return launch_stream(c, a, stream);
     if (c.engine == ENGINE_LDS) return launch_lds(c, a, stream);
     if (c.engine == ENGINE_MID) return launch_mid_engine(c, a, stream);
@@ -2051,6 +2077,7 @@ int sg_skinny_gemm_bf16act(const void* X_bf16, const uint8_t* B, void* D, const 
         a.row_scale_out = nullptr;
     }
     // two launches: the row encoder into the stream's scratch, then the GEMM with its scales in the epilogue
+    const StreamTurn turn(true, st);
     uint8_t* scratch = nullptr;
     const size_t q_bytes = ((size_t)m * k + 255) & ~(size_t)255;
     if (int rc = get_act_scratch(st, q_bytes + (size_t)m * sizeof(float), &scratch)) return rc;

@@ -149,3 +149,40 @@ def test_the_choice_and_whose_workspace(sg, m, n, k, pad):
             assert sg.skinny_gemm_auto_ws(A, W, D, S, None) == 0
             err = (D.float() - want.float()).norm() / want.float().norm()
             assert float(err) < 7e-3     # one bf16 rounding each, 1.6e-3 measured: four times that
+
+
+def test_split_launches_of_threads_on_one_stream_and_on_two(sg):
+    """K splits of this kernel, of the mid-batch kernel and the encoder's two launches, from threads that share a stream (and
+    with it a workspace) and threads on a stream of their own: the bits of each call by itself."""
+    import threading
+    g = torch.Generator().manual_seed(1)
+    jobs = []
+    for m, n, k in [(100, 2374, 5456), (190, 940, 7600), (64, 8192, 8192)]:
+        W = torch.randn((n, k), generator=g).to(torch.float8_e4m3fn).view(torch.uint8).cuda()
+        A = torch.randn((m, k), generator=g)
+        jobs.append((sg.skinny_gemm_fastpath, A.to(torch.float8_e4m3fn).view(torch.uint8).cuda(), W, scale_tensor(0.5)))
+        jobs.append((sg.skinny_gemm_bf16act, A.bfloat16().cuda(), W, scale_tensor(0.25)))
+    want = []
+    for entry, A, W, S in jobs:
+        want.append(torch.empty((A.shape[0], W.shape[0]), dtype=torch.bfloat16, device="cuda"))
+        assert entry(A, W, want[-1], S) == 0
+    torch.cuda.synchronize()
+    shared, codes, outs = torch.cuda.Stream(), [], []
+
+    def work(i, stream):
+        with torch.cuda.stream(stream):
+            for r in range(12):
+                entry, A, W, S = jobs[(i + r) % len(jobs)]
+                D = torch.empty_like(want[(i + r) % len(jobs)])
+                codes.append(entry(A, W, D, S))
+                outs.append((D, want[(i + r) % len(jobs)]))
+
+    threads = [threading.Thread(target=work, args=(i, shared if i < 4 else torch.cuda.Stream())) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert codes == [0] * 72
+    for D, w in outs:
+        assert torch.equal(D.view(torch.int16), w.view(torch.int16))
