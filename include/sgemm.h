@@ -154,7 +154,8 @@ int sg_skinny_gemm_rowcol(const uint8_t* A, const uint8_t* B, void* D_bf16, cons
  * whose tunables are compile-time #defines rewritten by its grid-search script
  * (grid.py:106-116); this is the run-time equivalent a tuning driver sweeps. */
 typedef struct SgTuning {
-    int engine;        /* 0 library's choice, 1 direct (global -> VGPR -> MFMA), 2 LDS ring (global -> LDS DMA -> MFMA),
+    int engine;        /* 0 library's choice (what sg_skinny_gemm_auto runs without a table entry, also where no record
+                          describes it), 1 direct (global -> VGPR -> MFMA), 2 LDS ring (global -> LDS DMA -> MFMA),
                           4 mid-batch (32 < m: weights streamed once, both operands staged in LDS for 2x2 or 4x2 waves;
                           k a multiple of 128, or - for the tile and ring combinations the library itself chooses - any
                           multiple of 16 beyond 128, the last 128-byte stage then loaded from k - 128) */

@@ -1935,8 +1935,8 @@ int sg_skinny_gemm_tuned(const uint8_t* A, const uint8_t* B, void* D, const floa
     Config c = config_from_tuning(*t);
     if (c.engine == ENGINE_AUTO) {
         c = heuristic_config(m, n, k, dev->cu_count);
-        Config wide;
-        if (wide_config(c, m, n, k, b_stride, false, dev->cu_count, nullptr, &wide)) c = wide;
+        Config instead;
+        if (stand_in_config(c, m, n, k, b_stride, false, dev->cu_count, nullptr, &instead)) c = instead;
     }
     if (c.engine != ENGINE_MID && c.mt != 1 && c.mt != 2) return SG_INVALID_CONFIG;
     StreamArgs a{};

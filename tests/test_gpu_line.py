@@ -128,6 +128,9 @@ def test_the_choice_and_whose_workspace(sg, m, n, k, pad):
     assert _line(A, W, want, S, None, None, (waves, rg, mb), sk) == 0
     assert sg.skinny_gemm_fastpath(A, W, D, S) == 0
     assert torch.equal(D, want)
+    D.zero_()
+    assert sg.skinny_gemm_tuned(A, W, D, S, engine=0) == 0
+    assert torch.equal(D, want)
     need = sg.workspace_query(m, n, k)
     ws = torch.empty(max(need, 1 << 17), dtype=torch.uint8, device="cuda")
     sg.workspace_init(ws)
