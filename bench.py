@@ -42,6 +42,16 @@ def gemm_bytes(m, n, k):
     return k * (m + n) + 2 * m * n
 
 
+def unrecorded_launch(sg, m, n, k):
+    """What the library launches for the shape where no tuning record describes it, or None."""
+    wide, line = sg.api.skinny_gemm_wide_choice(m, n, k), sg.api.skinny_gemm_line_choice(m, n, k)
+    if wide:
+        return "wide tile %d x %d, K split %d" % (32 * wide[0], 32 * wide[1], wide[2])
+    if line:
+        return "rows off their lines, tile %d x %d, K split %d" % (8 * line[0] * line[1], 32 * line[2], line[3])
+    return None
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -445,7 +455,7 @@ def main():
                     "mhz": np.median((t[j, :, 6].astype(np.int64) - t[j, :, 5].astype(np.int64)) / np.maximum(end[j] - ent[j], tick))})
             med = {key: float(np.median([r[key] for r in rows])) for key in rows[0]}
             t_choice, _ = sg.skinny_gemm_choice(args.m, n, k)
-            what = ("2:4, the library's choice" if args.sparse else sg.api.skinny_gemm_wide_choice(args.m, n, k) or
+            what = ("2:4, the library's choice" if args.sparse else unrecorded_launch(sg, args.m, n, k) or
                     sg.api.tuning_as_dict(t_choice))
             print("%-18s %5d x %5d  grid %4d  event-pair period %.2f | period %.2f = gap %.2f + span %.2f | entry spread %.2f | "
                   "workgroup (median): prologue issue %.2f, first stage landed %.2f (max %.2f), streaming %.2f, reduce+store %.2f, "
@@ -691,8 +701,7 @@ def main():
                 if lib.sg_tuning_set(m, n, k, ctypes.byref(forced)) != 0:
                     sys.exit("bench.py: --record is not a valid tuning record")
             t, _ = sg.skinny_gemm_choice(m, n, k)
-            wide = sg.api.skinny_gemm_wide_choice(m, n, k)
-            print("%s: %s" % (spec, "wide tile %d x %d, K split %d" % (32 * wide[0], 32 * wide[1], wide[2]) if wide else
+            print("%s: %s" % (spec, unrecorded_launch(sg, m, n, k) or
                               {f: getattr(t, f) for f in ("engine", "split_k", "waves", "row_tiles", "m_blocks", "depth", "k_chunks",
                                                           "persistent_wgs_per_cu", "wave_tiles")}), file=sys.stderr)
             for i in range(3):
@@ -939,8 +948,9 @@ def main():
 
     def choice(m, n, k):
         t, from_table = sg.skinny_gemm_choice(m, n, k)
-        wide = sg.api.skinny_gemm_wide_choice(m, n, k)
-        d = dict(zip(("wide_row_tiles", "wide_m_blocks", "split_k"), wide)) if wide else sg.api.tuning_as_dict(t)
+        wide, line = sg.api.skinny_gemm_wide_choice(m, n, k), sg.api.skinny_gemm_line_choice(m, n, k)
+        d = (dict(zip(("wide_row_tiles", "wide_m_blocks", "split_k"), wide)) if wide else
+             dict(zip(("line_waves", "line_row_tiles", "line_m_blocks", "split_k"), line)) if line else sg.api.tuning_as_dict(t))
         d["from_table"] = bool(from_table)
         return d
 

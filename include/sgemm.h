@@ -233,17 +233,18 @@ int sg_skinny_gemm_bf16act_choice(int m, int n, int k, SgTuning* out, int* fused
  * The eight cannot say everything a launch here depends on (persistent workgroups, resident activations,
  * the epilogue wave, the mid-batch tiles): passed back through sg_skinny_gemm they select a kernel of the
  * same ring geometry, not necessarily the one sg_skinny_gemm_auto runs.  sg_skinny_gemm_choice below
- * returns the complete record, and sg_skinny_gemm_tuned replays exactly that. */
+ * returns the complete record, and sg_skinny_gemm_tuned replays exactly that - but for the two kernels that no
+ * record describes, which engine = 0 replays. */
 int sg_skinny_gemm_pick(int m, int n, int k, int out[8]);
 
 /* The complete record sg_skinny_gemm_auto would launch for the shape: the tuning table's entry when
  * there is one (*from_table = 1), the built-in heuristics' otherwise (0).  from_table may be NULL.
- * From 33 rows on, where k or b_stride is no multiple of 128, the library may run the kernel for rows off their lines in
- * place of the heuristics' record (sg_debug_line_choice, sgemm_debug.h); where that splits K and the record does not, the
- * mid-batch record of the same split is reported.
- * Above 128 rows the library may run the wide-tile kernel in place of the heuristics' record, and no record describes
- * that kernel: sg_debug_wide_choice (sgemm_debug.h) says whether it does and on which tile, engine = 0 replays it, and the
- * record is the mid-batch launch that it replaces (stored in the table it is what runs from then on). */
+ * Two kernels that no record describes may run in place of the heuristics' record; engine = 0 replays them, sgemm_debug.h
+ * says whether they do and on which tile, and the record, stored in the table, is what runs from then on:
+ *   rows off their 128-byte lines (sg_debug_line_choice; 33 to 768 rows, k or b_stride no multiple of 128).  The record is
+ *     the launch that it replaces - or, where it splits K and that launch does not, a mid-batch record of the same split on
+ *     the tile nearest to its own, so that split_k says of either whether a workspace is needed (k = b_stride)
+ *   wide tiles (sg_debug_wide_choice; above 128 rows).  The record is the mid-batch launch that it replaces. */
 int sg_skinny_gemm_choice(int m, int n, int k, SgTuning* out, int* from_table);
 
 /* Per-shape tuning table - the run-time form of what the reference's grid search produces: there the

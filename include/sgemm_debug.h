@@ -14,7 +14,8 @@ extern "C" {
 #endif
 
 /* Profiling aid, no counterpart in the reference.  While a buffer is set, every launch of the LDS-ring GEMM
- * kernels (per-tile and persistent), of the mid-batch (whole lines or not) and wide-tile GEMM kernels and of the 2:4 kernels takes the next grid * 8 words of it and each workgroup leaves eight 64-bit
+ * kernels (per-tile and persistent), of the mid-batch (whole lines or not) and wide-tile GEMM kernels and of the 2:4
+ * kernels takes the next grid * 8 words of it and each workgroup leaves eight 64-bit
  * words there when it is done: [0] kernel entry, [1] prologue DMAs issued, [2] first stage landed, [3] last stage
  * consumed, [4] outputs stored and acknowledged - 10 ns ticks of the device's constant 100 MHz clock -
  * [5], [6] shader clock at entry and end, [7] XCC_ID << 32 | HW_ID.  Launches that no longer fit leave nothing.
@@ -30,21 +31,22 @@ int sg_debug_wide_gemm(const uint8_t* A, const uint8_t* B, void* D_bf16, const f
                        const float* col_scales, int m, int n, int k, int b_stride, int row_tiles, int m_blocks, int split_k,
                        void* stream);
 
-/* ... and which tile of that kernel sg_skinny_gemm_auto launches for the shape and row stride: out = {waves, row_tiles,
- * m_blocks, split_k}, or four zeros where it launches something else. */
-int sg_debug_line_choice(int m, int n, int k, int b_stride, int factors, int out[4]);
-
 /* Which wide tile sg_skinny_gemm_auto - with factors: sg_skinny_gemm_rowcol with row or column factors - launches for the
  * shape and row stride: out = {row_tiles, m_blocks, split_k} as sg_debug_wide_gemm takes them, or three zeros where it
- * launches the record that sg_skinny_gemm_choice reports. */
+ * launches something else. */
 int sg_debug_wide_choice(int m, int n, int k, int b_stride, int factors, int out[3]);
 
-/* The same on the kernel for rows that start off their 128-byte lines: the tile is 8 * waves * row_tiles weight rows by
- * 32 * m_blocks activation rows, (waves, row_tiles, m_blocks) one of (4, 2, 2), (8, 2, 2), (8, 2, 4), (8, 2, 6) and
- * (8, 3, 4); a K split sums its partials in a second launch.  Any k and stride the library takes, also on whole lines. */
+/* The GEMM of sg_debug_wide_gemm on the kernel for rows that start off their 128-byte lines: the tile is
+ * 8 * waves * row_tiles weight rows by 32 * m_blocks activation rows, (waves, row_tiles, m_blocks) one of (4, 2, 2),
+ * (8, 2, 2), (8, 2, 4), (8, 2, 6) and (8, 3, 4); a K split sums its partials in a second launch.  Any k and stride the
+ * library takes, also on whole lines. */
 int sg_debug_line_gemm(const uint8_t* A, const uint8_t* B, void* D_bf16, const float* scale, const float* row_scales,
                        const float* col_scales, int m, int n, int k, int b_stride, int waves, int row_tiles, int m_blocks,
                        int split_k, void* stream);
+
+/* ... and which tile of that kernel sg_skinny_gemm_auto - with factors: sg_skinny_gemm_rowcol - launches for the shape and
+ * row stride: out = {waves, row_tiles, m_blocks, split_k}, or four zeros where it launches something else. */
+int sg_debug_line_choice(int m, int n, int k, int b_stride, int factors, int out[4]);
 
 /* Profiling aid, no counterpart in the reference: reads the n x k weight matrix B (row stride b_stride, k % 1024 == 0)
  * the way the persistent LDS-ring GEMM streams it - one workgroup per CU walking row tiles, eight waves sharing K,

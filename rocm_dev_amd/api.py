@@ -301,8 +301,9 @@ def skinny_gemm_pick(m, n, k):
 
 def skinny_gemm_choice(m, n, k):
     """(record, from_table): the complete SgTuning the fastpath would launch for the shape, and whether it comes
-    from the tuning table rather than the built-in heuristics.  Above 128 rows a wide tile, which no record describes, may
-    run in the place of the heuristics' record: skinny_gemm_wide_choice."""
+    from the tuning table rather than the built-in heuristics.  Two kernels that no record describes may run in the place of
+    the heuristics' record: the one for rows off their 128-byte lines (skinny_gemm_line_choice) and, above 128 rows, a wide
+    tile (skinny_gemm_wide_choice)."""
     t, from_table = SgTuning(), C.c_int(0)
     rc = lib.sg_skinny_gemm_choice(m, n, k, C.byref(t), C.byref(from_table))
     if rc != 0:
@@ -312,9 +313,20 @@ def skinny_gemm_choice(m, n, k):
 
 def skinny_gemm_wide_choice(m, n, k, b_stride=None, factors=False):
     """(row_tiles, m_blocks, split_k) of the wide tile the fastpath (with factors: skinny_gemm_rowcol with row or column
-    factors) launches for the shape, or None where it launches the record that skinny_gemm_choice reports."""
+    factors) launches for the shape, or None where it launches something else."""
     out = (C.c_int * 3)()
     rc = lib.sg_debug_wide_choice(m, n, k, k if b_stride is None else b_stride, 1 if factors else 0, C.byref(out))
+    if rc != 0:
+        raise SgError(rc)
+    return tuple(out) if out[0] else None
+
+
+def skinny_gemm_line_choice(m, n, k, b_stride=None, factors=False):
+    """(waves, row_tiles, m_blocks, split_k) of the kernel for rows off their 128-byte lines where the fastpath (with factors:
+    skinny_gemm_rowcol with row or column factors) launches it for the shape, or None where it launches something else.  Its
+    tile is 8 * waves * row_tiles weight rows by 32 * m_blocks activation rows."""
+    out = (C.c_int * 4)()
+    rc = lib.sg_debug_line_choice(m, n, k, k if b_stride is None else b_stride, 1 if factors else 0, C.byref(out))
     if rc != 0:
         raise SgError(rc)
     return tuple(out) if out[0] else None

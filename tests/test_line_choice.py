@@ -63,3 +63,26 @@ def test_the_reported_record_is_launchable_and_split_where_a_workspace_is_asked_
         if record.engine == 4:
             assert launch_rules.expect_mid(m, n, k, d) == launch_rules.OK, (m, n, k, d)
         assert (record.split_k > 1) == (sg.workspace_query(m, n, k) > 0), (m, n, k, d)
+
+
+def test_the_tuner_keeps_a_record_that_beats_this_kernel(tmp_path, monkeypatch):
+    """No record describes the kernel, so a search that finds the reported record ahead of what ran has found something;
+    where the record itself ran (the row above it on whole lines), it is timing noise."""
+    import rocm_dev_amd as sg
+    from rocm_dev_amd import api, autotune
+    for shape, line in (((337, 6582, 1392), True), ((96, 4828, 11984), True), ((96, 4828, 11904), False)):
+        assert (api.skinny_gemm_line_choice(*shape) is not None) == line
+        assert (autotune.builtin_record(*shape) is None) == line
+        rec = api.tuning_as_dict(sg.skinny_gemm_choice(*shape)[0])
+        monkeypatch.setattr(autotune, "tune_shape", lambda *a, **kw: ([(90.0, rec)], 100.0, 7))
+        out = tmp_path / "t.txt"
+        try:
+            assert autotune.main(["--shapes", "%dx%dx%d" % shape, "--out", str(out)]) == 0
+            assert autotune.parse_table(out.read_text()) == ({shape: rec} if line else {})
+            sg.tuning_load(out)
+            assert api.skinny_gemm_line_choice(*shape) is None       # stored, the record is what runs
+        finally:
+            sg.tuning_clear()
+    for bad in ((0, 512, 512), (512, 0, 512), (512, 512, 0)):
+        with pytest.raises(api.SgError):
+            api.skinny_gemm_line_choice(*bad)
