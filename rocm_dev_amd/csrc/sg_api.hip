@@ -1434,6 +1434,7 @@ static bool line_config(const Config& record, const Config* wide, double wide_us
     if (m > 128 && k <= 1024) return false;     // stores of D, not loads: 1.09 times slower on 14 shapes (412 x 25130 x 768 32.0 us, 18.9)
     size_t partial_limit = kMaxPartialBytes, counters;
     if (k % 128 == 0) workspace_need(record, m, n, &partial_limit, &counters);
+    // (no look at its counters: a split, which comes with at most two workgroups per CU, has fewer tiles than any workspace)
     if (fixed_ws && fixed_ws->partial_bytes < partial_limit) partial_limit = fixed_ws->partial_bytes;
     const int blocks = (k + 127) / 128;
     double best = 0;
@@ -1442,7 +1443,6 @@ static bool line_config(const Config& record, const Config* wide, double wide_us
         const int bn = 8 * t.waves * t.rg, bm = 32 * t.mt;
         if (bm >= 2 * m && t.mt > 2) continue;
         const long n_tiles = (n + bn - 1) / bn, tiles = n_tiles * ((m + bm - 1) / bm);
-        if (fixed_ws && (size_t)tiles > fixed_ws->n_counters && partial_limit > 0) continue;
         for (int sk = 1; sk <= kLineMaxSplit; sk++) {
             const long wgs = tiles * sk;
             const double partials = (double)wgs * bn * bm * 4;

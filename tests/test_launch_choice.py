@@ -45,3 +45,28 @@ def test_engine_0_of_the_tuned_entry_point_is_the_librarys_choice(fake):
     differ, kernels = launch_recorder.scenario(fake, "test_launch_choice", "engine_0_and_auto", 3000)
     assert not differ, (len(differ), differ[:3])
     assert all(kernels.get(name, 0) > 20 for name in ("line_gemm_kernel", "mid_gemm_kernel", "wide_gemm_kernel", "lds_gemm_kernel")), kernels
+
+
+def noalloc_and_auto(rec, count):
+    """The same of sg_skinny_gemm_tuned_noalloc with engine 0, on shapes whose partials fit its array; large weight matrices too"""
+    own_choice, differ, seen, r = (C.c_int * 10)(), [], 0, random.Random(3)
+    need = C.c_size_t()
+    shapes = list(_shapes(count, 2))
+    shapes += [(r.randint(33, 768), 2 * r.randint(15000, 400000), k, stride) for _, _, k, stride in _shapes(count, 4)]
+    for m, n, k, stride in shapes:
+        assert rec.call("sg_workspace_query", m, n, k, C.byref(need)) == 0
+        if need.value > 65536 + (8 << 20):
+            continue
+        seen += 1
+        rc, auto = rec.of("sg_skinny_gemm_auto", rec.A, rec.B, rec.D, rec.S, m, n, k, stride, None)
+        rc2, own = rec.of("sg_skinny_gemm_tuned_noalloc", rec.A, rec.B, rec.D, rec.S, m, n, k, stride, own_choice, None)
+        assert rc == rc2 == 0, (m, n, k, stride, rc, rc2)
+        if _gemms(auto) != _gemms(own):
+            differ.append([(m, n, k, stride), _gemms(auto), _gemms(own)])
+    return differ, seen
+
+
+def test_the_fixed_array_changes_no_launch_that_fits_it(fake):
+    differ, seen = launch_recorder.scenario(fake, "test_launch_choice", "noalloc_and_auto", 3000)
+    assert not differ, (len(differ), differ[:3])
+    assert seen > 3000
