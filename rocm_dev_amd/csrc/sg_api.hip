@@ -1553,6 +1553,16 @@ static bool rejected_before_launch(int rc) {
            rc == SG_WORKSPACE_TOO_SMALL;
 }
 
+// Launches what stands in for heuristic_config's record, if anything does.  False with nothing enqueued: nothing does, or it
+// was refused, or there is no device memory for the partials of its K split - the record may need none.
+static bool launch_stand_in(const Config& record, const StreamArgs& a, int cu_count, hipStream_t stream, const Workspace* fixed_ws, int* rc) {
+    Config c;
+    if (!stand_in_config(record, a.m, a.n, a.k, a.b_stride, a.row_scale || a.col_scale, cu_count, fixed_ws, &c)) return false;
+    c.fixed_ws = fixed_ws;
+    *rc = launch_config(c, a, stream);
+    return !rejected_before_launch(*rc) && !(c.split_k > 1 && *rc == SG_NO_DEVICE);
+}
+
 // The table's record for the shape if it has a usable one, the heuristics' otherwise.  Should a launch
 // function refuse the heuristics' own record before anything is enqueued (split-K partials beyond the
 // workspace limit, a combination nothing is compiled for), the same record without the K split and then
@@ -1567,14 +1577,11 @@ static int launch_chosen(const StreamArgs& a, int cu_count, hipStream_t stream, 
             if (!rejected_before_launch(rc)) return rc;
         }
     }
-    Config c = heuristic_config(a.m, a.n, a.k, cu_count), instead;
-    if (stand_in_config(c, a.m, a.n, a.k, a.b_stride, a.row_scale || a.col_scale, cu_count, fixed_ws, &instead)) {
-        instead.fixed_ws = fixed_ws;
-        const int rc = launch_config(instead, a, stream);
-        if (!rejected_before_launch(rc)) return rc;
-    }
+    Config c = heuristic_config(a.m, a.n, a.k, cu_count);
+    int rc;
+    if (launch_stand_in(c, a, cu_count, stream, fixed_ws, &rc)) return rc;
     c.fixed_ws = fixed_ws;
-    int rc = launch_config(c, a, stream);
+    rc = launch_config(c, a, stream);
     if (rejected_before_launch(rc) && c.split_k > 1) {
         c.split_k = 1;
         rc = launch_config(c, a, stream);
@@ -1932,17 +1939,17 @@ int sg_skinny_gemm_tuned(const uint8_t* A, const uint8_t* B, void* D, const floa
     if (!scale_tensor) return SG_BAD_ARGUMENT;
     DeviceInfo* dev;
     if (int rc = get_device_info(&dev)) return rc;
-    Config c = config_from_tuning(*t);
-    if (c.engine == ENGINE_AUTO) {
-        c = heuristic_config(m, n, k, dev->cu_count);
-        Config instead;
-        if (stand_in_config(c, m, n, k, b_stride, false, dev->cu_count, nullptr, &instead)) c = instead;
-    }
-    if (c.engine != ENGINE_MID && c.mt != 1 && c.mt != 2) return SG_INVALID_CONFIG;
     StreamArgs a{};
     a.A = A; a.B = B; a.D = D; a.scale = scale_tensor;
     a.m = m; a.n = n; a.k = k; a.b_stride = b_stride;
     a.out_f32 = 0;
+    Config c = config_from_tuning(*t);
+    if (c.engine == ENGINE_AUTO) {
+        c = heuristic_config(m, n, k, dev->cu_count);
+        int rc;
+        if (launch_stand_in(c, a, dev->cu_count, static_cast<hipStream_t>(stream), nullptr, &rc)) return rc;
+    }
+    if (c.engine != ENGINE_MID && c.mt != 1 && c.mt != 2) return SG_INVALID_CONFIG;
     return launch_config(c, a, static_cast<hipStream_t>(stream));
 }
 

@@ -70,3 +70,22 @@ def test_the_fixed_array_changes_no_launch_that_fits_it(fake):
     differ, seen = launch_recorder.scenario(fake, "test_launch_choice", "noalloc_and_auto", 3000)
     assert not differ, (len(differ), differ[:3])
     assert seen > 3000
+
+
+def without_room_for_partials(rec):
+    """Launches where the device has no memory left for a workspace, of both entry points that would allocate one"""
+    own_choice, out = (C.c_int * 10)(), []
+    rec.fake.rec_largest_allocation(1 << 20)
+    for m, n, k in UNSPLIT_RECORDS:
+        out.append(rec.of("sg_skinny_gemm_auto", rec.A, rec.B, rec.D, rec.S, m, n, k, k, None))
+        out.append(rec.of("sg_skinny_gemm_tuned", rec.A, rec.B, rec.D, rec.S, m, n, k, k, own_choice, None))
+    return out
+
+
+# shapes whose heuristic record has no K split where the kernel for rows off their lines takes one
+UNSPLIT_RECORDS = [(100, 2374, 5456), (190, 940, 7600), (468, 566, 9200)]
+
+
+def test_a_split_that_stands_in_for_an_unsplit_launch_is_left_where_no_workspace_can_be_had(fake):
+    for rc, launches in launch_recorder.scenario(fake, "test_launch_choice", "without_room_for_partials"):
+        assert rc == 0 and len(launches) == 1 and "line_gemm" not in launches[0][0], (rc, launches)
