@@ -1397,13 +1397,17 @@ static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, bo
 // 47 x 28666 x 10320 83.9 -> 52.9, 128 x 8192 x 8208 36.7 -> 24.9, 96 x 4828 x 11984 43.5 -> 23.1.  The others stay ahead
 // on small weight matrices with K below about 4000 (the ring over several activation tiles: 49 x 4092 x 1680 5.2 against 10.3)
 // and where many rows fill rounds of wide tiles (207 x 27442 x 6800 62.9 against 83.4).
-// Beyond 768 rows it was not timed and is not taken.  The K split's partials: a workspace of the library's own, or one of
+// What lies outside the fit was timed against the launch replaced (234 shapes that this rule takes): below 512 weight rows 0.71
+// of the time before in the geometric mean (five of 68 behind by 10 to 21 %, eleven and twelve K splits against a ring that
+// takes 9-12 us), 32770..131072 rows 0.80 (three of 104 behind by 10 to 15 %), K of 20000..65536 0.69 (none behind),
+// 701..768 rows 0.81 (none).  Beyond 768 rows, 131072 weight rows or a K of 65536 it was not timed and is not taken.
+// The K split's partials: a workspace of the library's own, or one of
 // the size that sg_workspace_query asks for, has room for them where 128 does not divide k; where only the stride is off
 // the lines, which the query does not know, they have to fit what the record needs.  Either way the result does not depend
 // on whose workspace it is, as long as it has the size asked for.
 struct LineTile { int waves, rg, mt; double stage_us; };
 static const LineTile kLineTiles[] = {{4, 2, 2, 0.388}, {8, 2, 2, 0.513}, {8, 2, 4, 0.737}, {8, 2, 6, 1.016}, {8, 3, 4, 0.919}};
-constexpr int kLineMaxM = 768, kLineMaxSplit = 12;
+constexpr int kLineMaxM = 768, kLineMaxN = 131072, kLineMaxK = 65536, kLineMaxSplit = 12;
 
 // rounds of `wgs` workgroups on the device, a partly filled last one counting at least `part`
 static double rounds_of(long wgs, int cu_count, double part) {
@@ -1429,8 +1433,8 @@ static double off_line_us(const Config& c, int m, int n, int k, int cu_count) {
 
 static bool line_config(const Config& record, const Config* wide, double wide_us, int m, int n, int k, int b_stride, int cu_count,
                         const Workspace* fixed_ws, Config* out) {
-    if (m <= 32 || m > kLineMaxM || k <= 128 || (k % 128 == 0 && b_stride % 128 == 0)) return false;
-    if ((record.engine != ENGINE_MID && record.engine != ENGINE_LDS) || b_stride > kWidePitch || k > kWidePitch) return false;
+    if (m <= 32 || m > kLineMaxM || n > kLineMaxN || k <= 128 || k > kLineMaxK || (k % 128 == 0 && b_stride % 128 == 0)) return false;
+    if ((record.engine != ENGINE_MID && record.engine != ENGINE_LDS) || b_stride > kWidePitch) return false;
     if (m > 128 && k <= 1024) return false;     // stores of D, not loads: 1.09 times slower on 14 shapes (412 x 25130 x 768 32.0 us, 18.9)
     size_t partial_limit = kMaxPartialBytes, counters;
     if (k % 128 == 0) workspace_need(record, m, n, &partial_limit, &counters);

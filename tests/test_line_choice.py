@@ -50,6 +50,13 @@ def test_shapes_timed_on_both_sides_of_the_rule(lib):
         assert not _choice(lib, m, n, k, k)[0], (m, n, k)
 
 
+def test_nothing_beyond_the_timed_ranges(lib):
+    for m, n, k, pad in [(768, 3234, 10864, 0), (66, 131072, 2064, 0), (123, 206, 65520, 16), (96, 34, 14288, 0)]:
+        assert _choice(lib, m, n, k, k + pad)[0], (m, n, k)
+    for m, n, k, pad in [(769, 3234, 10864, 0), (66, 131074, 2064, 0), (64, 600002, 2064, 16), (123, 206, 65552, 16), (300, 900, 300016, 0)]:
+        assert not _choice(lib, m, n, k, k + pad)[0], (m, n, k)
+
+
 def test_the_reported_record_is_launchable_and_split_where_a_workspace_is_asked_for(lib):
     import launch_rules
     import rocm_dev_amd as sg
