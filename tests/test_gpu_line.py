@@ -39,9 +39,23 @@ def _in_nans(codes, stride, offset):
 
 
 # one block and a piece, the last block of one piece and of seven, one tile's rows and one more, a single weight row pair;
-# 192 rows of either operand; whole blocks on a stride that is off the lines
+# 192 rows of either operand; whole blocks on a stride that is off the lines; eighteen weight tiles of 192 rows, so that of
+# every tile some workgroups start K at another block than the first and wrap, past the end of every ring
 SHAPES = [(33, 2, 144, 0), (65, 130, 272, 0), (128, 128, 1040, 16), (129, 190, 656, 48), (193, 194, 2032, 0), (64, 258, 384, 16),
-          (100, 322, 1936, 112), (40, 66, 1280, 32)]
+          (100, 322, 1936, 112), (40, 66, 1280, 32), (200, 3300, 1040, 0), (130, 3300, 2064, 32), (66, 3300, 1536, 80)]
+
+
+def _rotations(n, k, tile, sk):
+    """The blocks other than its split's first that some workgroup starts K at (tile_n / 8 * 5 modulo the split's blocks)"""
+    blocks = -(-k // 128)
+    sizes = {blocks * (s + 1) // sk - blocks * s // sk for s in range(sk)}
+    return {(t // 8 * 5) % b for t in range(-(-n // (8 * tile[0] * tile[1]))) for b in sizes} - {0}
+
+
+def test_the_shapes_start_k_at_other_blocks_on_every_tile():
+    for tile in TILES:
+        for sk in (1, 2, 3):
+            assert any(_rotations(n, k, tile, sk) for _, n, k, _ in SHAPES if sk <= k // 128), (tile, sk)
 
 
 @pytest.mark.parametrize("m,n,k,pad", SHAPES)
@@ -74,11 +88,12 @@ def test_every_place_on_the_line(oracle, pitch):
     pieces, on a k of whole blocks and on one that ends within a block; several weight tiles, so that the walk of K starts
     at other blocks than the first."""
     m, n = 40, 20 * 64 + 2
-    for k in (640, 640 + 48):
+    for k in (768, 768 + 48):
+        assert _rotations(n, k, (4, 2, 2), 1) and _rotations(n, k, (8, 2, 2), 2)
         a8, b8, scale = oracle.make_gemm_operands(m, n, k, seed=pitch)
         ref = rowcol_reference(oracle, a8, b8, scale, None, None, model=True)
         S = scale_tensor(scale)
-        stride = 768 + pitch
+        stride = 1024 + pitch
         for offset in range(0, 128, 16):
             A, B = _in_nans(a8, k, offset), _in_nans(b8, stride, 112 - offset)
             for tile, sk in (((4, 2, 2), 1), ((8, 2, 2), 2)):
@@ -109,8 +124,8 @@ def test_nan_codes_poison_their_row_and_column_only(oracle):
 @pytest.mark.parametrize("m,n,k,pad", [(47, 28666, 2064, 0), (100, 2374, 5440, 16), (96, 4828, 11984, 0), (300, 2300, 9200, 0),
                                        (264, 10178, 9952, 112), (100, 4096, 8192, 16)])
 def test_the_choice_and_whose_workspace(sg, m, n, k, pad):
-    """The library's own launch is the tile that the choice names, bit for bit, eagerly, in a replayed graph and on a
-    workspace of the caller's of the size the query asks for; with what the record alone needs the call still runs."""
+    """The library's own launch is the tile that the choice names, bit for bit, eagerly, by engine 0, in a replayed graph and
+    on a workspace of the caller's of the size the query asks for."""
     import ctypes as C
     from rocm_dev_amd import api
     from rocm_dev_amd._lib import lib
@@ -145,13 +160,32 @@ def test_the_choice_and_whose_workspace(sg, m, n, k, pad):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(D, want)
-    if sk > 1 and k % 128:
-        record, _ = sg.skinny_gemm_choice(m, n, k)
-        if record.split_k == 1:     # the record needs no workspace: without one the call runs on something unsplit
-            D.zero_()
-            assert sg.skinny_gemm_auto_ws(A, W, D, S, None) == 0
-            err = (D.float() - want.float()).norm() / want.float().norm()
-            assert float(err) < 7e-3     # one bf16 rounding each, 1.6e-3 measured: four times that
+
+
+# the record has no K split where this kernel takes one: the mid-batch engine, the ring over several activation tiles
+@pytest.mark.parametrize("m,n,k", [(100, 2374, 5456), (190, 940, 7600), (468, 566, 9200)])
+def test_less_workspace_than_the_query_asks_for(sg, oracle, m, n, k):
+    """A caller whose workspace has no room for this kernel's partials, or who has none, gets a launch that fits, within the
+    tolerance of the oracle, and nothing behind the workspace is written."""
+    from rocm_dev_amd import api
+    sk = api.skinny_gemm_line_choice(m, n, k)[3]
+    need = sg.workspace_query(m, n, k)
+    assert sk > 1 and need > 65536
+    a8, b8, scale = oracle.make_gemm_operands(m, n, k, seed=n)
+    ref = rowcol_reference(oracle, a8, b8, scale, None, None, model=True)
+    A, B, S = dev(a8), dev(b8), scale_tensor(scale)
+    room = torch.full((need + 4096,), 0xA5, dtype=torch.uint8, device="cuda")
+    partials = need - 65536
+    for size in (None, 65536, 65536 + partials // sk, need - 1, need):
+        ws = None if size is None else room[:size]
+        room.fill_(0xA5)
+        if ws is not None:
+            sg.workspace_init(ws)
+        D = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert sg.skinny_gemm_auto_ws(A, B, D, S, ws) == 0, size
+        torch.cuda.synchronize()
+        assert oracle.max_rel_err_bf16(bits(D), ref) <= GEMM_TOL, size
+        assert bool((room[size or 0:] == 0xA5).all()), size
 
 
 def test_split_launches_of_threads_on_one_stream_and_on_two(sg):
