@@ -822,7 +822,8 @@ def test_k_with_part_of_a_block_at_its_end(sg, oracle, m, n, k):
     """k beyond 256 that is not a multiple of it (the intermediate sizes 29568, 1408 and 10944 of some models, their
     tensor-parallel shards 3696 and 7392): the library's own choice is the per-tile LDS ring, K splits and 24-row tiles
     included, or above 32 rows the mid-batch engine, with the last block loaded from k - 256 (k - 128) and its new bytes
-    used; against the oracle, and through the row/column-scaled entry point."""
+    used - or the kernel for rows off their lines, which stands in for both on some of these shapes (the mid-batch engine's own
+    builds: the next test); against the oracle, and through the row/column-scaled entry point."""
     t, from_table = sg.skinny_gemm_choice(m, n, k)
     assert not from_table and (t.engine == 4 if m > 256 else t.engine in (2, 4) if m > 32 else t.engine == 2)
     assert t.engine == 4 or t.persistent_wgs_per_cu == 0 or t.wave_tiles == 1
@@ -851,6 +852,40 @@ def test_k_with_part_of_a_block_at_its_end(sg, oracle, m, n, k):
     torch.cuda.synchronize()
     want = np.stack([oracle.e4m3_decode(b8[:, cols[i % len(cols)]]) for i in range(m)])
     assert np.array_equal(oracle.bf16_to_f32(bits(D1)), want.astype(np.float32))
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 4096, 7392), (256, 8192, 1424), (200, 14336, 2064), (64, 28672, 1168), (300, 1024, 3696),
+                                   (320, 4096, 4112), (40, 10240, 10944)])
+def test_mid_batch_builds_with_part_of_a_block_at_the_end_of_k(sg, oracle, m, n, k):
+    """The mid-batch engine's builds with a partial last 128-byte block on shapes that the kernel for rows off their lines takes
+    from them: the record reported, and two and three K splits of it summed by a second launch and by the last workgroup, stored
+    in the table - then they are what runs, with and without factors; against the oracle."""
+    assert sg.api.skinny_gemm_line_choice(m, n, k), "not a shape of the other kernel: this test would repeat the one above"
+    record = sg.api.tuning_as_dict(sg.skinny_gemm_choice(m, n, k)[0])
+    assert record["engine"] == 4
+    a8, b8, scale = oracle.make_gemm_operands(m, n, k, seed=5)
+    rs = np.random.default_rng(k).uniform(0.5, 2.0, size=m).astype(np.float32)
+    cs = np.random.default_rng(n).uniform(0.5, 2.0, size=n).astype(np.float32)
+    ref, ref_rc = (rowcol_reference(oracle, a8, b8, scale, r, c, model=True) for r, c in ((None, None), (rs, cs)))
+    A, B, S, R, C = dev(a8), dev(b8), scale_tensor(scale), dev(rs), dev(cs)
+    try:
+        for split_k, wave_tiles in ((1, 0), (2, 1), (2, 0), (3, 1), (3, 0)):
+            if split_k > k // 128:
+                continue
+            sg.tuning_set(m, n, k, sg.SgTuning(**dict(record, split_k=split_k, wave_tiles=wave_tiles)))
+            assert sg.api.skinny_gemm_line_choice(m, n, k) is None
+            alone = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+            rc = sg.skinny_gemm_tuned(A, B, alone, S, **dict(record, split_k=split_k, wave_tiles=wave_tiles))
+            assert rc == 0, (split_k, wave_tiles, sg.strerror(rc))     # (the table would pass over a record that is refused)
+            for r, c, want in ((None, None, ref), (R, C, ref_rc)):
+                D = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+                assert sg.skinny_gemm_rowcol(A, B, D, S, r, c) == 0
+                torch.cuda.synchronize()
+                assert oracle.max_rel_err_bf16(bits(D), want) <= GEMM_TOL, (split_k, wave_tiles, r is not None)
+                if r is None:
+                    assert torch.equal(D.view(torch.int16), alone.view(torch.int16))
+    finally:
+        sg.tuning_clear()
 
 
 # (m, n, k) -> (waves, wave_tiles) the library chooses for many-tile shapes away from k = 4096: one wave per K
