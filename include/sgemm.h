@@ -84,7 +84,8 @@ int    sg_release_workspaces(void);
  *   sg_workspace_query  *bytes = what sg_skinny_gemm_auto_ws needs for the shape with the tuning table as it is now
  *                       (0 when the launch it would choose has no K split; then workspace may be NULL) to run what
  *                       sg_skinny_gemm_auto runs, bit for bit; where the kernel for rows off their 128-byte lines would
- *                       split K, less - or NULL - is accepted too and runs what fits
+ *                       split K, less is accepted too, down to what the launch that it replaces needs (NULL, if
+ *                       that has no K split), and runs what fits
  *   sg_workspace_init   zeroes the counter region (the first 64 KB) of a workspace with a kernel in stream order:
  *                       once per buffer, before its first use; every launch that completes leaves it zero again
  * workspace: device memory, 256-byte aligned, [16384 arrival counters][fp32 partials]; one buffer serves launches of
@@ -213,8 +214,8 @@ int sg_skinny_gemm_tuned_noalloc(const uint8_t* A, const uint8_t* B, void* D_bf1
  * The fused kernel applies where one activation tile covers m (m <= 32), k % 256 == 0 and the codes fit LDS beside
  * the weight rings of four waves: every workgroup quantises its own copy of the activations while its first weight
  * stages are in flight.  That repeats the quantisation in every workgroup, so the library uses it only where it
- * measured faster than the two launches - m <= 8 and at least three 16-row tiles per CU (8 x 28672 x 4096: 26.9
- * against 29.0 us) - and otherwise runs the two launches itself, with the codes in a per-stream scratch buffer it
+ * measured faster than the two launches - m <= 8 and at least three 16-row tiles per CU (8 x 28672 x 4096: 22.5
+ * against 22.8 us, 4 rows 21.0 against 23.8) - and otherwise runs the two launches itself, with the codes in a per-stream scratch buffer it
  * keeps.  sg_skinny_gemm_bf16act_choice says which (*fused) and with which record.  sg_skinny_gemm_bf16act_tuned
  * always runs the fused kernel: with the given record (LDS ring, persistent_wgs_per_cu >= 1, wave_tiles 2 or 6,
  * row_tiles 1, depth 2; at most 8 streaming waves), or - engine 0 - the library's own for the shape;

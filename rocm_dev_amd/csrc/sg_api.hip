@@ -1160,8 +1160,9 @@ static bool fused_config(int m, int k, Config* out) {
 
 // ... and where it pays.  Every workgroup repeats the quantisation of all m x k activations (about 2.4 us of vector
 // work per workgroup at m = 8, k = 4096), which is only hidden where the workgroup goes on to stream several tiles:
-// 8 x 28672 x 4096 takes 26.9 us fused against 29.0 us for the two launches, 8 x 4096 x 4096 8.5 against 8.4,
-// 8 x 6144 x 4096 10.8 against 9.9, and at 16 rows or with a share too long for registers the two launches win.
+// 8 x 28672 x 4096 takes 22.5 us fused against 22.8 us for the two launches (4 rows 21.0 against 23.8), 8 x 4096 x 4096 8.1
+// against 7.4, 8 x 6144 x 4096 9.6 against 9.1, and at 16 rows (16 x 28672 x 4096 25.2 against 23.6) or with a share too long
+// for registers (8 x 4096 x 14336 29.3 against 14.4) the two launches win.
 static bool pick_bf16act(int m, int n, int k, int cu_count, Config* out) {
     Config c;
     if (!fused_config(m, k, &c)) return false;
@@ -1390,11 +1391,11 @@ static bool wide_config(const Config& mid, int m, int n, int k, int b_stride, bo
 // kernel that follows the lines (sg_line_kernel.h) in place of heuristic_config's record or the wide tile, where the model
 // of its own time is 5 % ahead of the model of theirs.  Microseconds with every CU busy, all fitted to timings of 302 random
 // shapes of that kind (33..700 rows, 512..32768 weight rows, K of 512..20000), every tile and K split of this kernel and
-// the launch it would replace: a launch costs c0, a round of workgroups its tile's stage per 128 bytes of K (and one more,
-// for the line behind the last), a partly filled last round at least 0.85 of that, a K split 2.2 and 0.21 per MB of
-// partials.  What it picks is 1.007 times the best tile and split (geometric mean), and the choice between the kernels 0.838
-// of the times before it (a perfect one: 0.835), two shapes behind by more than 3 % (up to 7 %): 468 x 566 x 9200 37.0 -> 16.4 us,
-// 47 x 28666 x 10320 83.9 -> 52.9, 128 x 8192 x 8208 36.7 -> 24.9, 96 x 4828 x 11984 43.5 -> 23.1.  The others stay ahead
+// the launch it would replace: a launch costs 3.1, a round of workgroups 2.3 and its tile's stage per 128 bytes of K (and one
+// more, for the line behind the last), a partly filled last round at least 0.85 of its stages, a K split 2.2 and 0.21 per MB of
+// partials.  What the model puts first is 1.003 times the best tile and split (geometric mean).  The rule takes 186 of the 302
+// shapes, 0.76 of the times before; all 302 together 0.842 (a perfect choice: 0.833), two behind by more than 3 % (5 and 6 %):
+// 468 x 566 x 9200 37.0 -> 16.4 us, 47 x 28666 x 10320 83.9 -> 52.9, 128 x 8192 x 8208 36.7 -> 24.9, 96 x 4828 x 11984 43.5 -> 23.1.  The others stay ahead
 // on small weight matrices with K below about 4000 (the ring over several activation tiles: 49 x 4092 x 1680 5.2 against 10.3)
 // and where many rows fill rounds of wide tiles (207 x 27442 x 6800 62.9 against 83.4).
 // What lies outside the fit was timed against the launch replaced (234 shapes that this rule takes): below 512 weight rows 0.71

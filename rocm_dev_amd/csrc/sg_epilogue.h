@@ -33,7 +33,7 @@ struct StreamArgs {
     int split_k, waves;
     int n_tiles, m_tiles;
     int out_f32;
-    int factor_off;         // register-resident kernel: where in the launch's LDS the row and column factors are staged, or 0
+    int factor_off;         // persistent and register-resident kernels: where in the launch's LDS the row and column factors are staged, or 0
     unsigned inv_n_tiles, inv_split_k, inv_waves;  // div_reciprocal() of n_tiles, split_k, waves (set_reciprocals)
     unsigned long long* stamps;  // profiling aid, normally nullptr: kStampWords time stamps per workgroup (sg_debug_stamps)
     int x_extra;            // register-resident kernel: 1 = the launch's LDS has one more 4 KB staging block per wave behind the reduction scratch

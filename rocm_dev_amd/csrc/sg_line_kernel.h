@@ -18,7 +18,8 @@
 // row's last block holds as well.
 //
 // Waves, K splits (summed by mid_reduce_kernel) and the rotated start of K are the mid-batch kernel's; both operands have the
-// same ring, as deep as 160 KB allow, because two lines are in use at once.  What it comes to (us, before -> now, cold weights):
+// same ring, as deep as 160 KB allow, because two lines are in use at once (the 64 x 64 tile's nine slots, 144 KB, measured ahead
+// of the ten that fit: 60 x 12192 x 2064 12.4 us against 12.8, 266 x 1308 x 5760 16.2 against 16.6, level at best).  What it comes to (us, before -> now, cold weights):
 // 128 x 8192 x 8208 36.7 -> 24.9, where rows on their lines (K = 8320) take 24.2; 47 x 28666 x 10320 83.9 -> 52.9,
 // 96 x 4828 x 11984 43.5 -> 23.1, 352 x 9388 x 17200 143 -> 101, 100 x 2374 x 5440 on a stride of 5456 15.6 -> 13.1.  Which
 // shapes and tiles: line_config (sg_api.hip).

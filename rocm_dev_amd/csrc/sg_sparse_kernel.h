@@ -472,7 +472,7 @@ __global__ void __launch_bounds__(RG == 4 ? 512 : 1024) sparse24_gemm_wavetile_k
 // workgroup works on K stages w, w + waves, ... (PT of them) of every tile the workgroup walks, and keeps the activation
 // fragments of those stages (64 registers each): they cross the L1 once a CU, 128 KB, and the ring carries weights only.
 // As in sg_xreg_kernel.h the fragments reach the registers through LDS, the waves' partial tiles meet in LDS and the wave
-// that sums them rotates with the tile.  us, before -> now: 32 x 28672 x 4096 (24 rows) 19.5 -> 16.5, 32 x 28672 x 7168
+// that sums them rotates with the tile.  us, before -> now: 24 x 28672 x 4096 19.5 -> 16.5, 32 x 28672 x 7168
 // 35.8 -> 25.7, 32 x 16384 x 8192 23.8 -> 19.2, 32 x 28672 x 2048 13.4 -> 10.3, 30 x 20480 x 3072 15.7 -> 11.3,
 // 32 x 14336 x 4096 11.3 -> 10.8.  The activations go first, all of a stage at once; with the first weight stages in front of
 // their second half, which leaves nothing in flight while it is read, 10.8 is 11.0, 16.5 is 17.2 and 11.3 is 12.0.
