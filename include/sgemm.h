@@ -55,7 +55,8 @@ const char* sg_strerror(int code);
  * device and stream: calls on one stream run in order and share a workspace, calls on different
  * streams may overlap and never share one.  Host threads may call on one stream at the same time: a call whose
  * launches hand each other memory (a GEMM and the sum of its K split's partials, the row encoder and the GEMM on
- * its codes) enqueues them with no other such call of the library's in between.  A workspace is created, or grown, by the first launch on its
+ * its codes) enqueues them with no other such call of the library's in between.  (hipStreamPerThread is one handle
+ * for a stream of every thread's own: pass it from one thread only.)  A workspace is created, or grown, by the first launch on its
  * stream that needs it (split_k > 1, also when the library chooses the split itself); at most 512 MB of
  * partials per launch, beyond that SG_WORKSPACE_TOO_SMALL.  An outgrown buffer is kept until it is released
  * (below).  A launch recorded into a HIP graph keeps the workspace of the stream it was captured on: run no
@@ -72,7 +73,7 @@ size_t sg_workspace_bytes(void);
  * sg_skinny_gemm_bf16act): sg_release_stream waits for `stream` and frees what the library holds for it on the
  * current device - call it before destroying a stream, whose handle the runtime may hand out again -;
  * sg_release_workspaces waits for the device and frees everything, after which sg_workspace_bytes() is 0.  Later
- * launches allocate afresh.  A HIP graph that recorded a launch keeps pointing at the workspace of its capture
+ * launches allocate afresh.  No other thread may be inside a call on what is released.  A HIP graph that recorded a launch keeps pointing at the workspace of its capture
  * stream: release only after such graphs are destroyed. */
 int    sg_release_stream(void* stream);
 int    sg_release_workspaces(void);
