@@ -1,4 +1,4 @@
-"""Row and column factors in every epilogue, and outputs whose rows are off their 8-byte pieces.
+"""Row and column factors in every epilogue but the wide tile's (test_gpu_wide.py), and outputs whose rows are off their 8-byte pieces.
 
 Factors that are powers of two commute with every rounding on the way (no output here is subnormal), so the product with
 factors must be, bit for bit, the product without them times the factors."""
@@ -20,13 +20,15 @@ def sg():
 # m, n, k, pad: n = 2 mod 4 (the last fragment ends inside a lane's four columns) except where a kernel wants whole tiles
 SHAPES = [
     (1, 2, 512, 0), (8, 4098, 4096, 0), (13, 6146, 4112, 16), (30, 4098, 14336, 0), (32, 1026, 8192, 0),   # per-tile ring, K splits
+    (17, 14338, 2816, 0), (32, 14338, 5120, 0),                                                            # ... on 64-row tiles
     (8, 28674, 4096, 0), (16, 9218, 4096, 0), (5, 12290, 3072, 128),                                       # persistent, activations in LDS
-    (32, 28674, 4096, 0), (17, 14338, 2816, 0), (16, 14338, 8192, 0), (32, 40962, 1792, 0),                # persistent, in registers
-    (12, 14338, 9472, 0), (32, 14338, 5120, 0),                                                            # neither fits
-    (8, 16386, 512, 0), (32, 28674, 1040, 0),                                                              # whole tiles per wave
-    (9, 302, 208, 0), (40, 130, 144, 16),                                                                  # register streaming
-    (100, 2374, 5440, 16), (64, 6146, 4096, 0), (40, 1026, 28672, 0),                                      # several activation tiles
-    (100, 10946, 3696, 16), (100, 3698, 10944, 16), (128, 8194, 8192, 0), (33, 57346, 640, 0),             # mid-batch, with and without a K split
+    (32, 28674, 4096, 0), (16, 14338, 8192, 0),                                                            # persistent, in registers
+    (12, 14338, 9472, 0),                                                                                  # persistent, in the ring
+    (8, 16386, 512, 0), (32, 28674, 1040, 0), (32, 40962, 1792, 0),                                        # whole tiles per wave
+    (9, 302, 208, 0),                                                                                      # register streaming
+    (64, 6146, 4096, 0), (40, 1026, 28672, 0),                                                             # several activation tiles
+    (40, 130, 144, 16), (128, 8194, 8192, 0), (33, 57346, 640, 0),                                         # mid-batch, with and without a K split
+    (100, 2374, 5440, 16), (100, 10946, 3696, 16), (100, 3698, 10944, 16),                                 # rows off their lines, the same
 ]
 
 
