@@ -49,6 +49,10 @@ def unrecorded_launch(sg, m, n, k):
         return "wide tile %d x %d, K split %d" % (32 * wide[0], 32 * wide[1], wide[2])
     if line:
         return "rows off their lines, tile %d x %d, K split %d" % (8 * line[0] * line[1], 32 * line[2], line[3])
+    skinny = sg.api.skinny_gemm_skinny_line_choice(m, n, k)
+    if skinny:
+        return "rows off their lines, %d waves, %d rows, %d slots, K split %d%s" % (
+            skinny[0], 16 * skinny[1], skinny[2], skinny[3], ", activations resident" if skinny[4] else "")
     return None
 
 

@@ -48,6 +48,19 @@ int sg_debug_line_gemm(const uint8_t* A, const uint8_t* B, void* D_bf16, const f
  * row stride: out = {waves, row_tiles, m_blocks, split_k}, or four zeros where it launches something else. */
 int sg_debug_line_choice(int m, int n, int k, int b_stride, int factors, int out[4]);
 
+/* The GEMM of sg_skinny_gemm_rowcol at up to 32 rows on one of the skinny kernels for rows that start off their 128-byte
+ * lines, k beyond 256.  resident = 0: a workgroup of `waves` waves per tile of 16 * row_tiles weight rows, K shared among them
+ * and among split_k workgroups, `depth` ring slots a wave: (row_tiles, depth) = (1, 4), (2, 3) and (2, 4), (4, 3) - from 9 rows on;
+ * above 16 rows (1, 4), (2, 4) and (4, 3).  resident = 1: one workgroup per CU with all activations in LDS, whose waves own
+ * whole 16-row tiles (row_tiles and split_k 1, depth 3 or 4). */
+int sg_debug_skinny_line_gemm(const uint8_t* A, const uint8_t* B, void* D_bf16, const float* scale, const float* row_scales,
+                              const float* col_scales, int m, int n, int k, int b_stride, int resident, int waves, int row_tiles,
+                              int depth, int split_k, void* stream);
+
+/* ... and what sg_skinny_gemm_auto launches of them for the shape and row stride: out = {waves, row_tiles, depth, split_k,
+ * resident}, or five zeros where it launches something else. */
+int sg_debug_skinny_line_choice(int m, int n, int k, int b_stride, int out[5]);
+
 /* Profiling aid, no counterpart in the reference: reads the n x k weight matrix B (row stride b_stride, k % 1024 == 0)
  * the way the persistent LDS-ring GEMM streams it - one workgroup per CU walking row tiles, eight waves sharing K,
  * direct-to-LDS loads with the streaming hint, two 4 KB slots per wave - and does nothing with it.  Its duration is the

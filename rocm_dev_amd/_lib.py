@@ -39,6 +39,8 @@ SIGNATURES = {
     "sg_debug_stamps": (_i, [_vp, _sz]),
     "sg_debug_wide_gemm": (_i, [_vp] * 6 + [_i] * 7 + [_vp]),
     "sg_debug_line_gemm": (_i, [_vp] * 6 + [_i] * 8 + [_vp]),
+    "sg_debug_skinny_line_gemm": (_i, [_vp] * 6 + [_i] * 9 + [_vp]),
+    "sg_debug_skinny_line_choice": (_i, [_i, _i, _i, _i, C.POINTER(_i * 5)]),
     "sg_debug_line_choice": (_i, [_i, _i, _i, _i, _i, C.POINTER(_i * 4)]),
     "sg_debug_wide_choice": (_i, [_i, _i, _i, _i, _i, C.POINTER(_i * 3)]),
     "sg_debug_read_stream": (_i, [_vp, _i, _i, _i, _i, _vp]),

@@ -301,9 +301,9 @@ def skinny_gemm_pick(m, n, k):
 
 def skinny_gemm_choice(m, n, k):
     """(record, from_table): the complete SgTuning the fastpath would launch for the shape, and whether it comes
-    from the tuning table rather than the built-in heuristics.  Two kernels that no record describes may run in the place of
-    the heuristics' record: the one for rows off their 128-byte lines (skinny_gemm_line_choice) and, above 128 rows, a wide
-    tile (skinny_gemm_wide_choice)."""
+    from the tuning table rather than the built-in heuristics.  Kernels that no record describes may run in the place of the
+    heuristics' record: those for rows off their 128-byte lines (skinny_gemm_line_choice; up to 32 rows
+    skinny_gemm_skinny_line_choice) and, above 128 rows, a wide tile (skinny_gemm_wide_choice)."""
     t, from_table = SgTuning(), C.c_int(0)
     rc = lib.sg_skinny_gemm_choice(m, n, k, C.byref(t), C.byref(from_table))
     if rc != 0:
@@ -327,6 +327,16 @@ def skinny_gemm_line_choice(m, n, k, b_stride=None, factors=False):
     tile is 8 * waves * row_tiles weight rows by 32 * m_blocks activation rows."""
     out = (C.c_int * 4)()
     rc = lib.sg_debug_line_choice(m, n, k, k if b_stride is None else b_stride, 1 if factors else 0, C.byref(out))
+    if rc != 0:
+        raise SgError(rc)
+    return tuple(out) if out[0] else None
+
+
+def skinny_gemm_skinny_line_choice(m, n, k, b_stride=None):
+    """(waves, row_tiles, depth, split_k, resident) of the skinny kernel for rows off their 128-byte lines where the fastpath
+    launches it for the shape (up to 32 rows), or None where it launches something else."""
+    out = (C.c_int * 5)()
+    rc = lib.sg_debug_skinny_line_choice(m, n, k, k if b_stride is None else b_stride, C.byref(out))
     if rc != 0:
         raise SgError(rc)
     return tuple(out) if out[0] else None

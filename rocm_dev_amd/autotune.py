@@ -182,9 +182,9 @@ def same_launch(a, b):
 
 def builtin_record(m, n, k):
     """The record the library launches for the shape by itself; None where it runs a kernel that no record describes, a wide
-    tile or the one for rows off their 128-byte lines."""
-    from .api import skinny_gemm_choice, skinny_gemm_line_choice, skinny_gemm_wide_choice
-    if skinny_gemm_wide_choice(m, n, k) or skinny_gemm_line_choice(m, n, k):
+    tile or one for rows off their 128-byte lines."""
+    from .api import skinny_gemm_choice, skinny_gemm_line_choice, skinny_gemm_skinny_line_choice, skinny_gemm_wide_choice
+    if skinny_gemm_wide_choice(m, n, k) or skinny_gemm_line_choice(m, n, k) or skinny_gemm_skinny_line_choice(m, n, k):
         return None
     own, _ = skinny_gemm_choice(m, n, k)
     return {f: getattr(own, f) for f in FIELDS}

@@ -339,7 +339,36 @@ static unsigned level_persistent_grid(unsigned tiles, size_t most) {
 // multiples of 256 only).
 static bool lds_half_block_k(int k) { return k % 256 != 0 && k % 16 == 0 && k > 256; }
 
+// activation DMA instructions of a stage: 4 rows each, rounded up to a compiled count
+static int activation_instructions(int mt, int m) { return mt == 2 ? 8 : (m <= 4 ? 1 : (m <= 8 ? 2 : 4)); }
+
+// The skinny kernels for rows off their lines: a workgroup of c.waves waves per 16 * c.rg row tile and K split, or one per CU
+// with the activations resident in LDS, whose waves own whole 16-row tiles.
+constexpr size_t kSkinnyLineLds = 159 * 1024;     // 160 KB per CU, minus the kernel's static LDS
+static size_t skinny_line_lds(const Config& c, int m, int k) {
+    const size_t xu = (size_t)activation_instructions(c.mt, m);
+    // + 4 KB: lanes of activation rows that are not loaded read past the last slot
+    return c.wavetile == 1 ? (size_t)((k + 255) / 256) * xu * 1024 + (size_t)c.waves * c.depth * 4096 + 4096
+                           : (size_t)c.waves * c.depth * (c.rg * 4 + xu) * 1024 + 4096;
+}
+static int launch_skinny_line_engine(const Config& c, StreamArgs a, hipStream_t stream) {
+    if (c.mt != (a.m <= 16 ? 1 : 2) || a.m > 32 || a.k <= 256) return SG_INVALID_CONFIG;
+    size_t tiles;
+    if (int rc = prepare(c, a, 256, &tiles, stream)) return rc;
+    const int xu = activation_instructions(c.mt, a.m);
+    const bool resident = c.wavetile == 1;
+    if (resident && c.split_k != 1) return SG_INVALID_CONFIG;
+    const size_t lds = skinny_line_lds(c, a.m, a.k);
+    if (lds > kSkinnyLineLds) return SG_INVALID_CONFIG;
+    DeviceInfo* dev;
+    if (int rc = get_device_info(&dev)) return rc;
+    const unsigned grid = resident ? (unsigned)std::min(tiles, (size_t)dev->cu_count) : (unsigned)(tiles * c.split_k);
+    a.stamps = take_stamps(grid);
+    return launch_skinny_line(c.mt, c.rg, xu, c.depth, resident, a, grid, (unsigned)c.waves * 64, lds, stream);
+}
+
 static int launch_lds(const Config& c, StreamArgs a, hipStream_t stream) {
+    if (c.line) return launch_skinny_line_engine(c, a, stream);
     if (a.k % 256 != 0 && !(lds_half_block_k(a.k) && !a.A16 && ((c.persist == 0 && (c.wavetile & 7) == 0) || c.wavetile == 1)))
         return SG_K_NOT_DIVISIBLE_BY_WARPTILE_K;
     // wave_tiles bit 3: 24-row tiles (two fragments, the second half used), one workgroup per tile
@@ -1478,9 +1507,100 @@ static bool line_config(const Config& record, const Config* wide, double wide_us
     return true;
 }
 
-// What stands in for heuristic_config's record, if anything does: a wide tile or the kernel for rows off their lines.
+// Up to 32 activation rows and weight rows off their lines (a row stride that 128 does not divide): the skinny kernels of
+// sg_skinny_line_kernel.h in place of heuristic_config's record.  Which of them was read off timings of all their builds
+// (waves, ring slots, row tiles, K splits) against that record on 510 random shapes, n of 128..65536, K of 272..32768, 236 of
+// which the rule takes: 0.88 of the time before in the geometric mean (the best build of each shape: 0.87), and seven behind by
+// more than 2 %, at most 6 %.  32 x 32768 x 4112 35.7 -> 26.7 us, 1 x 16384 x 4112 15.5 -> 13.8, 13 x 20660 x 9664 57.5 -> 35.6,
+// 5 x 39438 x 4016 35.6 -> 28.1, 28 x 13116 x 6960 25.0 -> 20.7, 5 x 2434 x 21584 18.0 -> 13.5, 1 x 8522 x 2832 7.3 -> 6.8.
+// What it leaves alone - weights of a megabyte or two, two K blocks, few tiles with a K below about 7000 at up to 16 rows - is
+// bound by the launch, or runs as fast there on its deeper rings.  Beyond those ranges it was not timed and is not taken.
+// The K splits of a stride that sg_workspace_query does not know (128 divides k) are not taken either, so that the result does
+// not depend on whose workspace it is.
+constexpr int kSkinnyLineMaxN = 65536, kSkinnyLineMaxK = 32768;
+
+static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, Config* out) {
+    if (m > 32 || k <= 256 || k > kSkinnyLineMaxK || n < 128 || n > kSkinnyLineMaxN || b_stride % 128 == 0) return false;
+    const int tiles = (n + 15) / 16, blocks = (k + 255) / 256, cu = cu_count;
+    const bool split_ok = k % 128 != 0;
+    Config c{};
+    c.engine = ENGINE_LDS;
+    c.line = true;
+    c.nt = 1;
+    c.ku = 4;
+    c.mt = m <= 16 ? 1 : 2;
+    auto tile = [&](int waves, int row_tiles, int depth, int split) {
+        c.wavetile = 0; c.persist = 0; c.waves = waves; c.rg = row_tiles; c.depth = depth; c.split_k = split;
+    };
+    auto resident = [&](int waves, int depth) {      // ... where everything fits the LDS
+        c.wavetile = 1; c.persist = 1; c.waves = waves; c.rg = 1; c.depth = depth; c.split_k = 1;
+        return skinny_line_lds(c, m, k) <= kSkinnyLineLds;
+    };
+    if (c.mt == 1) {
+        if (tiles * 2 <= cu) {                       // few tiles: only long K, on K splits
+            if (!split_ok || blocks < (tiles * 5 <= cu ? 100 : 60) || (tiles * 5 > cu && tiles * 3 <= cu)) return false;
+            tile(4, 1, 4, tiles * 5 <= cu ? 4 : 2);
+        } else if (tiles <= cu) {
+            if (blocks < 28) return false;
+            tile(4, 1, 4, 1);
+        } else if (tiles <= 2 * cu) {                // 32-row tiles; a long K on four waves, whose K offsets spread over the
+            if (blocks < (m > 8 || (m > 4 && tiles * 2 > 3 * cu) ? 16 : 28)) return false;   // memory channels (pitch 16448: 34.8 -> 24.7 us)
+            if (blocks >= 60) tile(4, 2, 3, 1);
+            else tile(2, 2, 4, 1);
+        } else if (blocks < 3) {
+            return false;
+        } else if (tiles <= 4 * cu) {
+            if (resident(4, 4)) {}
+            else if (m > 8 && tiles > 3 * cu) tile(2, 4, 3, 1);
+            else if (tiles <= 3 * cu) tile(1, 1, 4, 1);
+            else tile(1, 2, 4, 1);
+        } else if (tiles <= 6 * cu) {                // (eight waves all find a tile)
+            if ((blocks <= 10 && resident(8, 4)) || resident(8, 3)) {}
+            else tile(1, 2, 3, 1);
+        } else {
+            if (blocks <= 6 && (resident(8, 4) || resident(8, 3))) {}
+            else if (tiles > 12 * cu && resident(8, 3)) {}
+            else if (resident(4, 4)) {}
+            else if (m > 8) tile(1, 4, 3, 1);
+            else tile(1, 2, 4, 1);
+        }
+    } else {                                         // the activations weigh as much: taller tiles share them
+        if (tiles <= cu) {
+            if (blocks < (tiles * 4 <= cu ? 20 : 9)) return false;
+            if (tiles * 2 <= cu && blocks >= 20) {
+                if (!split_ok) return false;
+                tile(2, 1, 4, tiles * 4 <= cu ? 4 : 2);
+            } else if (tiles * 20 > 17 * cu && blocks >= 48) {
+                if (!split_ok) return false;
+                tile(2, 2, 4, 2);
+            } else {
+                if (blocks > 96 || (!split_ok && blocks < 48)) return false;
+                tile(2, 1, 4, 1);
+            }
+        } else if (tiles <= 2 * cu) {
+            if (blocks < 12) return false;
+            tile(2, 2, 4, 1);
+        } else if (blocks < 3) {
+            return false;
+        } else if (tiles <= 4 * cu) {
+            if (resident(4, 4)) {}
+            else if (blocks < 20 && tiles <= 3 * cu) tile(1, 2, 4, 1);
+            else tile(2, 4, 3, 1);
+        } else {
+            if (blocks <= 7 && resident(8, 3)) {}
+            else if (resident(4, 4)) {}
+            else tile(1, 4, 3, 1);
+        }
+    }
+    if (skinny_line_lds(c, m, k) > kSkinnyLineLds) return false;
+    *out = c;
+    return true;
+}
+
+// What stands in for heuristic_config's record, if anything does: a wide tile or a kernel for rows off their lines.
 static bool stand_in_config(const Config& record, int m, int n, int k, int b_stride, bool factors, int cu_count, const Workspace* fixed_ws,
                             Config* out) {
+    if (m <= 32) return skinny_line_config(m, n, k, b_stride, cu_count, out);
     double wide_us = 0;
     const bool wide = wide_config(record, m, n, k, b_stride, factors, cu_count, fixed_ws, out, &wide_us);
     Config line;
@@ -1489,14 +1609,18 @@ static bool stand_in_config(const Config& record, int m, int n, int k, int b_str
     return true;
 }
 
-// The record that sg_skinny_gemm_choice reports: heuristic_config's - or, where that has no K split and the kernel for rows
-// off their lines takes one in its place, the mid-batch record of that split on the tile nearest to that kernel's, so that a
-// record without a K split still says that no workspace is needed.  (Launches that cannot have the split, on a caller's
+// The record that sg_skinny_gemm_choice reports: heuristic_config's - or, where that has no K split and a kernel for rows
+// off their lines takes one in its place, the record of that split on the tile nearest to that kernel's (mid-batch or, up to
+// 32 rows, the LDS ring's), so that a record without a K split still says that no workspace is needed.  (Launches that cannot have the split, on a caller's
 // smaller workspace for instance, run heuristic_config's.)
 static Config reported_config(int m, int n, int k, int cu_count) {
     const Config base = heuristic_config(m, n, k, cu_count);
     Config c;
     if (k % 128 == 0 || base.split_k > 1 || !stand_in_config(base, m, n, k, k, false, cu_count, nullptr, &c) || !c.line || c.split_k == 1) return base;
+    if (m <= 32) {
+        c.line = false;
+        return c;
+    }
     Config r{};
     r.engine = ENGINE_MID;
     r.waves = c.waves;
@@ -1806,6 +1930,26 @@ int sg_debug_line_gemm(const uint8_t* A, const uint8_t* B, void* D, const float*
     return launch_config(c, a, static_cast<hipStream_t>(stream));
 }
 
+int sg_debug_skinny_line_gemm(const uint8_t* A, const uint8_t* B, void* D, const float* scale, const float* row_scales,
+                              const float* col_scales, int m, int n, int k, int b_stride, int resident, int waves, int row_tiles, int depth,
+                              int split_k, void* stream) {
+    if (n % 2 != 0) return SG_N_NOT_EVEN;
+    if (k % 16 != 0 || k <= 256) return SG_K_NOT_DIVISIBLE_BY_WARPTILE_K;
+    if (int rc = check_pointers(A, B, D, m, n, k, b_stride)) return rc;
+    DeviceInfo* dev;
+    if (int rc = get_device_info(&dev)) return rc;
+    Config c{};
+    c.engine = ENGINE_LDS;
+    c.line = true;
+    c.mt = m <= 16 ? 1 : 2;
+    c.waves = waves; c.rg = row_tiles; c.depth = depth; c.split_k = split_k; c.wavetile = resident ? 1 : 0;
+    StreamArgs a{};
+    a.A = A; a.B = B; a.D = D; a.scale = scale; a.row_scale = row_scales; a.col_scale = col_scales;
+    a.m = m; a.n = n; a.k = k; a.b_stride = b_stride;
+    a.out_f32 = 0;
+    return launch_config(c, a, static_cast<hipStream_t>(stream));
+}
+
 int sg_debug_wide_choice(int m, int n, int k, int b_stride, int factors, int out[3]) {
     if (!out || m <= 0 || n <= 0 || k <= 0 || b_stride < k) return SG_BAD_ARGUMENT;
     out[0] = out[1] = out[2] = 0;
@@ -1830,8 +1974,23 @@ int sg_debug_line_choice(int m, int n, int k, int b_stride, int factors, int out
     int cu = 256;
     if (get_device_info(&dev) == SG_SUCCESS) cu = dev->cu_count;
     Config c;
-    if (stand_in_config(heuristic_config(m, n, k, cu), m, n, k, b_stride, factors != 0, cu, nullptr, &c) && c.line) {
+    if (stand_in_config(heuristic_config(m, n, k, cu), m, n, k, b_stride, factors != 0, cu, nullptr, &c) && c.line && m > 32) {
         out[0] = c.waves; out[1] = c.rg; out[2] = c.mt; out[3] = c.split_k;
+    }
+    return SG_SUCCESS;
+}
+
+int sg_debug_skinny_line_choice(int m, int n, int k, int b_stride, int out[5]) {
+    if (!out || m <= 0 || n <= 0 || k <= 0 || b_stride < k) return SG_BAD_ARGUMENT;
+    for (int i = 0; i < 5; i++) out[i] = 0;
+    SgTuning t;
+    if (table_lookup(m, n, k, &t) && t.engine != ENGINE_AUTO) return SG_SUCCESS;
+    DeviceInfo* dev;
+    int cu = 256;
+    if (get_device_info(&dev) == SG_SUCCESS) cu = dev->cu_count;
+    Config c;
+    if (skinny_line_config(m, n, k, b_stride, cu, &c)) {
+        out[0] = c.waves; out[1] = c.rg; out[2] = c.depth; out[3] = c.split_k; out[4] = c.wavetile;
     }
     return SG_SUCCESS;
 }
@@ -2079,8 +2238,10 @@ int sg_skinny_gemm_bf16act(const void* X_bf16, const uint8_t* B, void* D, const 
     a.col_scale = col_scales;
     a.m = m; a.n = n; a.k = k; a.b_stride = b_stride;
     a.out_f32 = 0;
-    Config c;
-    if (pick_bf16act(m, n, k, dev->cu_count, &c)) {
+    // (a GEMM on rows off their lines adds up K in another order than the fused kernel: there the two launches run, as
+    // sg_fp8_encode_rows and sg_skinny_gemm_rowcol would)
+    Config c, line;
+    if (pick_bf16act(m, n, k, dev->cu_count, &c) && !skinny_line_config(m, n, k, b_stride, dev->cu_count, &line)) {
         a.A16 = static_cast<const uint16_t*>(X_bf16);
         a.row_scale_out = row_scales_out;
         const int rc = launch_config(c, a, st);

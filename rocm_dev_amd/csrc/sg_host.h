@@ -49,6 +49,9 @@ int launch_mid(int rgw, int mh, int depth, int dx, int wn, const StreamArgs& a, 
 int launch_wide(int rgw, int mh, const StreamArgs& a, unsigned grid, hipStream_t stream);
 // mid-batch tiles on rows off their 128-byte lines (sg_line_kernel.h)
 int launch_line(int rgw, int mh, int wn, const StreamArgs& a, unsigned grid, hipStream_t stream);
+// up to 32 activation rows on rows off their lines (sg_skinny_line_kernel.h)
+int launch_skinny_line(int mt, int rg, int xu, int depth, bool resident, const StreamArgs& a, unsigned grid, unsigned threads, size_t lds,
+                       hipStream_t stream);
 // second launch of a mid-batch GEMM with StreamArgs::defer_reduce: sums the split-K partials of every output fragment
 int launch_mid_reduce(int rgw, int mh, int wn, const StreamArgs& a, hipStream_t stream);
 
