@@ -294,8 +294,9 @@ int sg_async_gemm_bf16(const uint8_t* A, const uint8_t* B, void* D_bf16, int m, 
  * k must be a multiple of 128 and at least 512 (a k that 512 does not divide costs one partly used stage), n even;
  * all pointers 16-byte aligned.  The weights are the
  * sparse operand of gfx950's v_smfmac_f32_16x16x64_fp8_fp8; HBM traffic is 0.625 bytes per
- * dense weight.  The _tuned form takes row_tiles, waves, depth, split_k and m_blocks from
- * the record (engine 0 = library's choice); wave_tiles = 1 with persistent_wgs_per_cu >= 1
+ * dense weight.  Few weight rows with a long k take a K split in the stream's workspace (above), except under capture:
+ * a recorded launch uses no workspace, so its sums may be added up in another order than an eager call's.  The _tuned
+ * form takes row_tiles, waves, depth, split_k and m_blocks from the record (engine 0 = library's choice); wave_tiles = 1 with persistent_wgs_per_cu >= 1
  * selects the kernel that keeps the activation matrix resident in LDS and gives every wave
  * whole 16*row_tiles-row tiles (m <= 16, split_k = 1, row_tiles 1 or 2).  Where k is a multiple of 1024 (and
  * split_k <= k / 1024) the metadata is fetched by whole 128-byte lines, two K stages per row and request, as long as

@@ -821,7 +821,48 @@ static int launch_sparse_engine(const Config& c, StreamArgs a, const uint8_t* me
     return launch_sparse(c.mt, c.rg, xu2, c.depth, pairs, sa, (unsigned)(tiles * c.split_k), (unsigned)c.waves * 64, lds, stream);
 }
 
-static Config pick_sparse(int m, int n, int k, int cu_count) {
+// Row tiles, waves, ring slots and K splits of sparse24_gemm_kernel for up to 32 rows, as read off timings of 1, 2 and 4 of the
+// first two, 2..4 slots and up to eight splits on 139 random shapes (1..32 rows, n of 64..32768, k of 512..28672; every side
+// timed in turn, cold weights): 0.885 of the time of what ran before in the geometric mean, the best of them 0.878, none behind
+// by more than 3 %; on 169 further shapes whose launch it changes 0.83.  Few tiles and a long K: splits until the CUs have one each (14 x 198 x 24576 12.0 -> 7.2 us,
+// 25 x 930 x 24576 17.7 -> 9.4, 19 x 1378 x 27776 20.5 -> 13.9); a K too short for one wave's ring on two of them (9 x 328 x 6144
+// 5.74 -> 4.67, 2 x 2308 x 7168 6.09 -> 4.84); 17..32 rows on one to two tiles per CU on 32-row tiles, which share the
+// activations (23 x 7542 x 10240 18.8 -> 15.2), or, up to four stages, on one wave (24 x 4464 x 1024 6.41 -> 3.83); beyond two
+// tiles per CU 16-row tiles where all workgroups are resident in as few rounds (17 x 10622 x 1792 7.74 -> 6.73).  No more slots
+// than a wave has stages.  `split` false: as many K splits as there can be without a workspace, none.
+static void pick_sparse_tile(Config& c, int m, int tiles16, int blocks, int cu, bool split) {
+    const int xu2 = c.mt == 2 ? 16 : 2 * activation_instructions(1, m);
+    int most = 1;
+    c.rg = 1;
+    if (tiles16 <= cu) {
+        if (c.mt == 2) {
+            if (blocks >= 10) most = std::min((blocks + 2) / 4, blocks >= 24 ? 6 : 4);
+            c.waves = blocks >= 4 && blocks != 5 ? 2 : 1;      // (five stages on one wave of four slots)
+        } else {
+            if (blocks >= 20 && (m > 4 || tiles16 * 3 <= cu)) most = std::min(blocks / (m > 4 ? 8 : 12), 4);
+            c.waves = blocks >= 8 ? 2 : 1;
+        }
+    } else if (c.mt == 2 && tiles16 <= 2 * cu) {
+        c.rg = c.waves = blocks <= 4 ? 1 : 2;
+    } else if (c.mt == 2) {
+        // three workgroups of 16-row tiles on a CU, or two of 32-row tiles
+        c.rg = (tiles16 + 3 * cu - 1) / (3 * cu) <= (tiles16 + 4 * cu - 1) / (4 * cu) ? 1 : 2;
+        c.waves = c.rg == 2 && blocks >= 16 ? 2 : 1;
+    } else {
+        if (m > 8 ? tiles16 > 4 * cu : tiles16 >= 4 * cu && (m > 4 || blocks > 2 || tiles16 > 6 * cu)) c.rg = 2;
+        c.waves = 1;
+    }
+    c.split_k = split ? std::max(1, std::min(cu / tiles16, most)) : 1;
+    c.depth = 4;
+    if (c.mt == 2) c.depth = c.split_k > 1 || c.rg == 2 || tiles16 > 2 * cu ? 2 : (blocks == 5 && tiles16 <= cu ? 4 : 3);
+    else if (tiles16 > 2 * cu) c.depth = c.rg == 2 || m > 8 ? 2 : 3;
+    const int stages = (blocks + c.split_k * c.waves - 1) / (c.split_k * c.waves);
+    c.depth = std::max(2, std::min(c.depth, stages));
+    while (c.depth > 2 && (size_t)c.waves * c.depth * (c.rg * 5 + xu2) * 1024 + 8192 > 159 * 1024) c.depth--;
+}
+
+// `split`: the caller can give a K split its workspace
+static Config pick_sparse(int m, int n, int k, int cu_count, bool split) {
     Config c;
     c.engine = ENGINE_LDS;
     c.nt = 1;
@@ -841,7 +882,10 @@ static Config pick_sparse(int m, int n, int k, int cu_count) {
     while (c.depth > 2 && ((c.depth - 1) * (c.rg * 5 + xu2) > 63 ||
                            (size_t)c.waves * c.depth * (c.rg * 5 + xu2) * 1024 + 8192 > 159 * 1024))
         c.depth--;
-    if (c.mt == 1 && m > 4 && tiles16 * 4 >= cu_count * 5) {
+    const bool timed = m <= 32 && n <= 32768 && k <= 28672;    // (beyond: the rules above, which were)
+    if (timed) pick_sparse_tile(c, m, tiles16, blocks, cu_count, split);
+    // (at most two tiles per CU one-wave workgroups are ahead up to 8 rows: 5 x 6170 x 8192 10.0 -> 7.7 us)
+    if (c.mt == 1 && m > 4 && tiles16 * 4 >= cu_count * 5 && !(timed && m <= 8 && tiles16 <= 2 * cu_count)) {
         // 5..16 activation rows and more than one tile per CU: the activation matrix stays resident in LDS and
         // four waves per CU each stream whole tiles (4-33 % faster on ten shapes than refetching 4-8 KB of
         // activations with every 5 KB weight stage; at four rows and below the two are level)
@@ -856,6 +900,7 @@ static Config pick_sparse(int m, int n, int k, int cu_count) {
             c.depth = depth;
             c.persist = 1;
             c.wavetile = 1;
+            c.split_k = 1;
             break;
         }
     }
@@ -869,6 +914,7 @@ static Config pick_sparse(int m, int n, int k, int cu_count) {
                 c.waves = w;
                 c.persist = 1;
                 c.wavetile = 2;
+                c.split_k = 1;
                 return c;
             }
     }
@@ -877,6 +923,19 @@ static Config pick_sparse(int m, int n, int k, int cu_count) {
     // 7.85 -> 7.83-8.0 us, where 32 x 14336 x 4096 on the same ring goes 12.3 -> 11.9 and 16 x 4096 x 14336 10.6 -> 10.1)
     if (m <= 4 && c.depth == 2 && c.waves == 1) c.ku = 1;
     return c;
+}
+
+// The library's own 2:4 launch.  A K split takes partials of its stream's workspace.  Under capture there is none: a recorded
+// launch could replay next to other work of that stream, as graphs of these launches always could.  Nor where no memory can
+// be had for it.
+static int launch_sparse_chosen(const StreamArgs& a, const uint8_t* meta, int cu_count, hipStream_t stream) {
+    Config c = pick_sparse(a.m, a.n, a.k, cu_count, true);
+    if (c.split_k > 1 && !stream_is_capturing(stream)) {
+        const int rc = launch_sparse_engine(c, a, meta, stream);
+        if (rc != SG_NO_DEVICE && rc != SG_WORKSPACE_TOO_SMALL) return rc;
+    }
+    if (c.split_k > 1) c = pick_sparse(a.m, a.n, a.k, cu_count, false);
+    return launch_sparse_engine(c, a, meta, stream);
 }
 
 // Split-K partial bytes and arrival counters the launch of `c` on an m x n x k problem takes from its workspace
@@ -1543,11 +1602,13 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
         } else if (tiles <= cu) {
             if (blocks < 28) return false;
             tile(4, 1, 4, 1);
+        } else if (tiles * 2 <= 3 * cu) {            // (one round of the record's 24-row tiles)
+            return false;
         } else if (tiles <= 2 * cu) {                // 32-row tiles; a long K on four waves, whose K offsets spread over the
-            if (blocks < (m > 8 || (m > 4 && tiles * 2 > 3 * cu) ? 16 : 28)) return false;   // memory channels (pitch 16448: 34.8 -> 24.7 us)
+            if (blocks < (m > 4 ? 16 : 28)) return false;    // memory channels (8 x 8192 x 16448 34.8 -> 24.7 us)
             if (blocks >= 60) tile(4, 2, 3, 1);
             else tile(2, 2, 4, 1);
-        } else if (blocks < 3) {
+        } else if (blocks < (tiles <= 4 * cu ? 4 : 3)) {
             return false;
         } else if (tiles <= 4 * cu) {
             if (resident(4, 4)) {}
@@ -2460,12 +2521,11 @@ int sg_sparse24_gemm(const uint8_t* A, const uint8_t* B_vals, const uint8_t* B_m
     if (reinterpret_cast<uintptr_t>(D) & 7u) return SG_BAD_ALIGNMENT;
     DeviceInfo* dev;
     if (int rc = get_device_info(&dev)) return rc;
-    const Config c = pick_sparse(m, n, k, dev->cu_count);
     StreamArgs a{};
     a.A = A; a.B = B_vals; a.D = D; a.scale = scale_tensor;
     a.m = m; a.n = n; a.k = k; a.b_stride = k / 2;
     a.out_f32 = 0;
-    return launch_sparse_engine(c, a, B_meta, static_cast<hipStream_t>(stream));
+    return launch_sparse_chosen(a, B_meta, dev->cu_count, static_cast<hipStream_t>(stream));
 }
 
 int sg_sparse24_compress(const uint8_t* B, uint8_t* B_vals, uint8_t* B_meta, int n, int k, int b_stride, void* stream) {
@@ -2490,23 +2550,22 @@ int sg_sparse24_gemm_tuned(const uint8_t* A, const uint8_t* B_vals, const uint8_
     if (reinterpret_cast<uintptr_t>(D) & 7u) return SG_BAD_ALIGNMENT;
     DeviceInfo* dev;
     if (int rc = get_device_info(&dev)) return rc;
-    Config c = pick_sparse(m, n, k, dev->cu_count);
-    if (t->engine != ENGINE_AUTO) {
-        c.rg = t->row_tiles;
-        c.waves = t->waves;
-        c.depth = t->depth;
-        c.split_k = t->split_k;
-        c.mt = t->m_blocks;
-        c.persist = t->persistent_wgs_per_cu;
-        c.wavetile = t->wave_tiles;
-        c.ku = t->k_chunks;   // 1: metadata by 64-byte pieces per stage also where whole lines are possible
-        if (c.mt != 1 && c.mt != 2) return SG_INVALID_CONFIG;
-        if (c.wavetile != 0 && c.wavetile != 1) return SG_INVALID_CONFIG;
-    }
     StreamArgs a{};
     a.A = A; a.B = B_vals; a.D = D; a.scale = scale_tensor;
     a.m = m; a.n = n; a.k = k; a.b_stride = k / 2;
     a.out_f32 = 0;
+    if (t->engine == ENGINE_AUTO) return launch_sparse_chosen(a, B_meta, dev->cu_count, static_cast<hipStream_t>(stream));
+    Config c = pick_sparse(m, n, k, dev->cu_count, false);
+    c.rg = t->row_tiles;
+    c.waves = t->waves;
+    c.depth = t->depth;
+    c.split_k = t->split_k;
+    c.mt = t->m_blocks;
+    c.persist = t->persistent_wgs_per_cu;
+    c.wavetile = t->wave_tiles;
+    c.ku = t->k_chunks;   // 1: metadata by 64-byte pieces per stage also where whole lines are possible
+    if (c.mt != 1 && c.mt != 2) return SG_INVALID_CONFIG;
+    if (c.wavetile != 0 && c.wavetile != 1) return SG_INVALID_CONFIG;
     return launch_sparse_engine(c, a, B_meta, static_cast<hipStream_t>(stream));
 }
 
