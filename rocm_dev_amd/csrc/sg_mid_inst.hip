@@ -52,14 +52,29 @@ static int launch_mid_tail(int rgw, int mh, int depth, int dx, int wn, const Str
     return SG_K_NOT_DIVISIBLE_BY_WARPTILE_K;
 }
 
-int launch_mid_reduce(int rgw, int mh, int wn, const StreamArgs& a, hipStream_t stream) {
-    const int frags_wg = 2 * wn * rgw * mh;                   // fragments of a tile; a workgroup of four waves takes 4 * kReduceFrags
-    if ((rgw * mh) % kReduceFrags != 0) return SG_INVALID_CONFIG;
-    const size_t grid = (size_t)a.n_tiles * a.m_tiles * ((frags_wg + 4 * kReduceFrags - 1) / (4 * kReduceFrags));
+template <int FRAGS, int BATCH>
+static int launch_reduce_one(int rgw, int mh, int wn, const StreamArgs& a, hipStream_t stream) {
+    const int frags_wg = 2 * wn * rgw * mh;                   // fragments of a tile; a workgroup of four waves takes 4 * FRAGS
+    const size_t grid = (size_t)a.n_tiles * a.m_tiles * ((frags_wg + 4 * FRAGS - 1) / (4 * FRAGS));
     if (grid == 0 || grid > 0x7fffffffu) return SG_BAD_ARGUMENT;
-    if (a.row_scale || a.col_scale) mid_reduce_kernel<true><<<dim3((unsigned)grid), dim3(256), 0, stream>>>(a, rgw, mh, wn);
-    else mid_reduce_kernel<false><<<dim3((unsigned)grid), dim3(256), 0, stream>>>(a, rgw, mh, wn);
+    if (a.row_scale || a.col_scale) mid_reduce_kernel<true, FRAGS, BATCH><<<dim3((unsigned)grid), dim3(256), 0, stream>>>(a, rgw, mh, wn);
+    else mid_reduce_kernel<false, FRAGS, BATCH><<<dim3((unsigned)grid), dim3(256), 0, stream>>>(a, rgw, mh, wn);
     return report_hip("mid_reduce_kernel launch", hipGetLastError()) == hipSuccess ? SG_SUCCESS : SG_LAUNCH_FAILED;
+}
+
+// Four fragments a wave fill the device from about 500 workgroups on; below that the launch is the chain of a wave's round trips,
+// two splits each, and one fragment a wave with four or eight splits in flight is shorter the fewer workgroups there are: GEMM
+// and sum of 103 x 174 x 12864, twelve splits on 6 workgroups, 13.5 -> 11.3 us, 640 x 222 x 9152 (40) 15.8 -> 13.8, 624 x 300 x 5120
+// (50, five splits) 10.8 -> 9.8, 371 x 816 x 7600 (84) 15.2 -> 14.5, 166 x 1750 x 26704 (84) 28.1 -> 27.6, launches of
+// 300 to 500 workgroups 1 % ahead, 2 to 4 with factors.  170 random launches timed both ways: 0.95 of the time
+// before in the geometric mean.  Three splits are level from 130 workgroups on and behind from 300 (192 x 8720 x 6464 27.9 against
+// 29.1); two are asked for at once either way (45 x 15894 x 12528 38.0 against 38.9).
+int launch_mid_reduce(int rgw, int mh, int wn, const StreamArgs& a, hipStream_t stream) {
+    if ((rgw * mh) % kReduceFrags != 0) return SG_INVALID_CONFIG;
+    const size_t wgs = (size_t)a.n_tiles * a.m_tiles * ((2 * wn * rgw * mh + 4 * kReduceFrags - 1) / (4 * kReduceFrags));
+    if (a.split_k > 4 && wgs < 512) return launch_reduce_one<1, 8>(rgw, mh, wn, a, stream);
+    if (a.split_k > 2 && wgs < (a.split_k == 4 ? 512 : 128)) return launch_reduce_one<1, 4>(rgw, mh, wn, a, stream);
+    return launch_reduce_one<kReduceFrags, 2>(rgw, mh, wn, a, stream);
 }
 
 int launch_mid(int rgw, int mh, int depth, int dx, int wn, const StreamArgs& a, unsigned grid, size_t lds, hipStream_t stream) {

@@ -14,20 +14,22 @@ namespace sg {
 // fragments per wave of the GEMM, wn x 2 waves per tile.
 // FACTORS: there are row or column factors (requested ahead of the partials, in 34 registers that the other build does not
 // hold: five waves a SIMD instead of eight).
+// FRAGS, BATCH: fragments of a wave and splits it asks for at once, up to eight 1 KB loads in flight.  Four and two; one and four or
+// eight where four would make so few waves that the launch is the chain of their round trips (launch_mid_reduce).
 constexpr int kReduceFrags = 4;
-template <bool FACTORS>
+template <bool FACTORS, int FRAGS, int BATCH>
 __global__ void __launch_bounds__(256) mid_reduce_kernel(const StreamArgs a, int rgw, int mh, int wn) {
-    const int fr = rgw * mh, frags_wg = 2 * wn * fr;   // fr is a multiple of kReduceFrags (launch_mid_reduce)
+    const int fr = rgw * mh, frags_wg = 2 * wn * fr;   // fr is a multiple of FRAGS (launch_mid_reduce)
     const int lane = lane_id();
-    // a workgroup takes 4 * kReduceFrags consecutive fragments of one tile; the workgroups of a weight tile sit on the
+    // a workgroup takes 4 * FRAGS consecutive fragments of one tile; the workgroups of a weight tile sit on the
     // XCD that computed it (the grid is n_tiles * m_tiles * chunks workgroups, chunks per tile)
-    const int chunks = (frags_wg + 4 * kReduceFrags - 1) / (4 * kReduceFrags);   // (the last one may have idle waves)
+    const int chunks = (frags_wg + 4 * FRAGS - 1) / (4 * FRAGS);   // (the last one may have idle waves)
     int pos;
     const int tile_n = xcd_weight_tile((int)blockIdx.x, (int)gridDim.x, a.m_tiles * chunks, a.n_tiles, pos);
     const int tile_m = pos / chunks, chunk = pos - tile_m * chunks;
     if (tile_n >= a.n_tiles || tile_m >= a.m_tiles) return;
     const unsigned tile_id = (unsigned)(tile_m * a.n_tiles + tile_n);
-    const unsigned rem = (unsigned)((chunk * 4 + wave_id()) * kReduceFrags);     // (wave of the tile, fragment of the wave)
+    const unsigned rem = (unsigned)((chunk * 4 + wave_id()) * FRAGS);     // (wave of the tile, fragment of the wave)
     if (rem >= (unsigned)frags_wg) return;
     const int wave = (int)rem / fr, f0 = (int)rem - wave * fr;
     const int wq = wave % wn, wm = wave / wn;
@@ -38,11 +40,11 @@ __global__ void __launch_bounds__(256) mid_reduce_kernel(const StreamArgs a, int
         m_idx = tile_m * (32 * mh) + (wm * mh + mb) * 16 + r;
         n_idx = tile_n * (16 * rgw * wn) + (wq * rgw + rg) * 16 + 4 * g;
     };
-    f32x4 col[kReduceFrags];
-    float row[kReduceFrags];
+    f32x4 col[FRAGS];
+    float row[FRAGS];
     if constexpr (FACTORS) {
 #pragma unroll
-        for (int j = 0; j < kReduceFrags; j++) {
+        for (int j = 0; j < FRAGS; j++) {
             int m_idx, n_idx;
             place(j, m_idx, n_idx);
             col[j] = col_scale_ahead(a, n_idx);
@@ -52,19 +54,30 @@ __global__ void __launch_bounds__(256) mid_reduce_kernel(const StreamArgs a, int
     const f32x4* p = reinterpret_cast<const f32x4*>(a.ws + ((size_t)tile_id * a.split_k) * ((size_t)frags_wg * 256) +
                                                     (size_t)wave * (fr * 256) + (size_t)f0 * 256) + lane;
     const size_t split_stride = (size_t)frags_wg * 64;
-    f32x4 v[kReduceFrags];
+    f32x4 v[FRAGS];
 #pragma unroll
-    for (int j = 0; j < kReduceFrags; j++) v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int sp = 0; sp < a.split_k; sp++) {
-        f32x4 t[kReduceFrags];
+    for (int j = 0; j < FRAGS; j++) v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (FRAGS > 1) {
+#pragma unroll BATCH
+        for (int sp = 0; sp < a.split_k; sp++) {
+            f32x4 t[FRAGS];
 #pragma unroll
-        for (int j = 0; j < kReduceFrags; j++) t[j] = p[(size_t)sp * split_stride + j * 64];
+            for (int j = 0; j < FRAGS; j++) t[j] = p[(size_t)sp * split_stride + j * 64];
 #pragma unroll
-        for (int j = 0; j < kReduceFrags; j++) v[j] += t[j];
+            for (int j = 0; j < FRAGS; j++) v[j] += t[j];
+        }
+    } else {
+        for (int sp = 0; sp < a.split_k; sp += BATCH) {   // (behind the last split it is read again and not added)
+            f32x4 t[BATCH];
+#pragma unroll
+            for (int i = 0; i < BATCH; i++) t[i] = p[(size_t)(sp + i < a.split_k ? sp + i : a.split_k - 1) * split_stride];
+#pragma unroll
+            for (int i = 0; i < BATCH; i++)
+                if (sp + i < a.split_k) v[0] += t[i];
+        }
     }
 #pragma unroll
-    for (int j = 0; j < kReduceFrags; j++) {
+    for (int j = 0; j < FRAGS; j++) {
         int m_idx, n_idx;
         place(j, m_idx, n_idx);
         if constexpr (FACTORS) {
