@@ -246,7 +246,11 @@ int sg_skinny_gemm_pick(int m, int n, int k, int out[8]);
  *   rows off their 128-byte lines (sg_debug_line_choice; 33 to 768 rows, k or b_stride no multiple of 128).  The record is
  *     the launch that it replaces - or, where it splits K and that launch does not, a mid-batch record of the same split on
  *     the tile nearest to its own, so that split_k says of either whether a workspace is needed (k = b_stride)
- *   wide tiles (sg_debug_wide_choice; above 128 rows).  The record is the mid-batch launch that it replaces. */
+ *   wide tiles (sg_debug_wide_choice; above 128 rows).  The record is the mid-batch launch that it replaces.
+ * Above 128 rows on few weight rows with a long k the record may split K in place of an unsplit one that needs no workspace.
+ * That one runs where the split cannot: on a caller's smaller workspace or none, without device memory for the library's own, and
+ * under capture without a caller's, so that graphs of such launches may replay side by side (the sums are added up in
+ * another order there than in an eager call). */
 int sg_skinny_gemm_choice(int m, int n, int k, SgTuning* out, int* from_table);
 
 /* Per-shape tuning table - the run-time form of what the reference's grid search produces: there the

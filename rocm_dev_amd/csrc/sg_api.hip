@@ -621,6 +621,29 @@ static double mid_model_us(int m, int n, int k, int bn, int bm, int sk, int cu_c
     return t * 1e6;
 }
 
+// (weight slots, activation slots; 0 = as many) of a mid-batch tile: the deepest ring that fits 160 KB.  A shallower
+// activation ring (activations come from L2, weights from HBM) is what lets the 256 x 256 tile keep
+// two weight stages in flight, and the 224 x 128 tile three (86 -> 80 us at 128 x 57344 x 8192).
+static void deepest_mid_ring(Config& c) {
+    const int bn = 8 * c.rg * c.waves, bm = 32 * c.mt;
+    const int per_wave_w = bn / (8 * c.waves), per_wave_x = bm / (8 * c.waves);   // DMA instructions per wave and stage
+    static const int rings[][2] = {{4, 0}, {4, 3}, {3, 0}, {3, 2}, {2, 0}};
+    c.depth = 2;
+    c.ku = 0;
+    for (const auto& r : rings) {
+        const int dw = r[0], dx = r[1] ? r[1] : r[0];
+        if (dw == 4 && dx == 3 && c.waves != 14) continue;   // compiled for the 224 x 128 tile, which it fills to 160 KB
+        const int in_flight_x = per_wave_w + (dx - 2) * (per_wave_w + per_wave_x);
+        const int in_flight_w = (dw - 2) * (per_wave_w + per_wave_x);
+        const size_t lds = ((size_t)dw * bn + (size_t)dx * bm) * 128;   // (a split's sum is a second launch: no arrival word)
+        if (lds > 160 * 1024) continue;
+        if ((in_flight_x < in_flight_w ? in_flight_x : in_flight_w) > 63) continue;
+        c.depth = dw;
+        c.ku = r[1];
+        break;
+    }
+}
+
 // Mid-batch heuristic, fitted to timings of the Llama-3-70B projection shapes at M = 64..256:
 // what matters first is that one round of workgroups covers the device (a second, partly
 // filled round costs more than any tile-shape effect), then that the round is as full as
@@ -731,30 +754,11 @@ static Config pick_mid(int m, int n, int k, int cu_count) {
     // sum on every split record of the Llama-3-70B shapes (128 x 128 tiles split three ways at 128 x 10240 x 8192
     // 32.1 -> 26.6 us, 128 x 64 split four ways at 64 x 8192 x 28672 46.8 -> 43.6, 64 x 64 split in two 19.1 -> 18.5)
     c.wavetile = c.split_k > 1 ? 1 : 0;
-    const int bn = 8 * c.rg * c.waves, bm = 32 * c.mt;
-    const int per_wave_w = bn / (8 * c.waves), per_wave_x = bm / (8 * c.waves);   // DMA instructions per wave and stage
-    // (weight slots, activation slots; 0 = as many): the deepest ring that fits 160 KB.  A shallower
-    // activation ring (activations come from L2, weights from HBM) is what lets the 256 x 256 tile keep
-    // two weight stages in flight, and the 224 x 128 tile three (86 -> 80 us at 128 x 57344 x 8192).
-    static const int rings[][2] = {{4, 0}, {4, 3}, {3, 0}, {3, 2}, {2, 0}};
-    c.depth = 2;
-    c.ku = 0;
     if (co_resident) {
         c.depth = 4;
         c.ku = 2;
     } else {
-        for (const auto& r : rings) {
-            const int dw = r[0], dx = r[1] ? r[1] : r[0];
-            if (dw == 4 && dx == 3 && c.waves != 14) continue;   // compiled for the 224 x 128 tile, which it fills to 160 KB
-            const int in_flight_x = per_wave_w + (dx - 2) * (per_wave_w + per_wave_x);
-            const int in_flight_w = (dw - 2) * (per_wave_w + per_wave_x);
-            const size_t lds = ((size_t)dw * bn + (size_t)dx * bm) * 128;   // (a split's sum is a second launch: no arrival word)
-            if (lds > 160 * 1024) continue;
-            if ((in_flight_x < in_flight_w ? in_flight_x : in_flight_w) > 63) continue;
-            c.depth = dw;
-            c.ku = r[1];
-            break;
-        }
+        deepest_mid_ring(c);
     }
     return c;
 }
@@ -1566,6 +1570,62 @@ static bool line_config(const Config& record, const Config* wide, double wide_us
     return true;
 }
 
+// More than 128 rows on so few weight rows that the record's tiles leave CUs idle: the mid-batch tile and K split that this
+// model puts first, 5 % ahead of the record.  (pick_mid's own splits go to four, with a third of a weight row's bytes of partials
+// at most and K blocks of 128 only: 1061 x 128 x 6128 ran on 34 workgroups.)  Microseconds with every CU busy, fitted to
+// timings of nine tiles with up to 32 splits on 190 random shapes (129..2048 rows, 128..12000 weight rows, K of 1600 to 32768), rows of
+// whole lines and others: 5 % off in the root mean square.  On 60 other shapes that the rule takes, padded rows and factors among
+// them, 0.65 of the time before in the geometric mean, none behind (with the sum of launch_mid_reduce for few workgroups): 1405 x 184
+// x 28048 109 -> 33 us, 1257 x 178 x 30144 100 -> 29, 1635 x 626 x 19056 108 -> 51, 1817 x 1146 x 18160 173 -> 82, 915 x 188 x 8640
+// 27.5 -> 12.8, 295 x 144 x 4224 12.7 -> 8.8, 822 x 5518 x 14880 141 -> 127.  Rows off their lines up to 768 rows are
+// line_config's.  Where the record stays ahead - one round of tiles that fills the CUs, K below about 3000 - the model says so.
+static double deep_split_us(int m, int n, int k, int bn, int bm, int sk, int cu_count) {
+    const bool lines = k % 128 == 0;
+    const long wgs = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm) * sk;
+    const double stages = (double)(((k + 127) / 128 + sk - 1) / sk);
+    const double per_stage = lines ? 0.232 * bn / 128 + 0.247 * bm / 128 + 0.12 * bn * bm / 16384
+                                   : 0.458 * bn / 128 + 0.384 * bm / 128 + 0.073 * bn * bm / 16384;
+    double us = rounds_of(wgs, cu_count, lines ? 0.87 : 0.84) * stages * per_stage;
+    us += lines ? 3.5 + (double)((wgs + cu_count - 1) / cu_count) : 4.2;
+    if (sk > 1) us += lines ? 3.1 + 1.36e-6 * (double)wgs * bn * bm : 2.7 + 1.57e-6 * (double)wgs * bn * bm;
+    return us;
+}
+
+constexpr double kDeepSplitWork = 1024.0 * 8192 * 8192;   // none of the shapes timed is larger
+static bool deep_split_config(const Config& record, int m, int n, int k, int cu_count, const Workspace* fixed_ws, Config* out) {
+    if (m <= 128 || m > 2048 || n > 12000 || k < 1024 || k > 32768 || (double)m * n * k > kDeepSplitWork || record.engine != ENGINE_MID || record.waves == 14) return false;
+    if (k % 128 != 0 && m <= kLineMaxM) return false;
+    struct Tile { int waves, rg, mt; };
+    static const Tile tiles[] = {{4, 2, 2}, {4, 2, 4}, {4, 4, 4}, {8, 2, 2}, {8, 2, 4}, {8, 2, 8}, {8, 4, 2}, {8, 4, 4}, {8, 4, 8}};
+    const int blocks = (k + 127) / 128;
+    // (ahead of a record that splits already by less than 12 %, it was behind as often: 554 x 346 x 16000 16.7 against 18.4)
+    double best = (record.split_k > 1 ? 0.88 : 0.95) * deep_split_us(m, n, k, 8 * record.rg * record.waves, 32 * record.mt, record.split_k, cu_count);
+    bool found = false;
+    Config c{};
+    for (const Tile& t : tiles) {
+        const int bn = 8 * t.waves * t.rg, bm = 32 * t.mt;
+        if (k % 128 != 0 && t.waves == 4 && t.rg == 4) continue;    // not built with part of a block at the end of K
+        const long of_m_n = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm);
+        for (int sk = 2; sk <= 16 && blocks / sk >= 4 && of_m_n * sk <= 2L * cu_count; sk++) {
+            // (kMaxPartialBytes holds any such split)
+            if (fixed_ws && ((size_t)(of_m_n * sk) * bn * bm * 4 > fixed_ws->partial_bytes || (size_t)of_m_n > fixed_ws->n_counters)) break;
+            const double us = deep_split_us(m, n, k, bn, bm, sk, cu_count);
+            if (us >= best) continue;
+            best = us;
+            found = true;
+            c.waves = t.waves; c.rg = t.rg; c.mt = t.mt; c.split_k = sk;
+        }
+    }
+    if (!found) return false;
+    c.engine = ENGINE_MID;
+    c.nt = 1;
+    c.persist = 0;
+    c.wavetile = 1;
+    deepest_mid_ring(c);
+    *out = c;
+    return true;
+}
+
 // Up to 32 activation rows and weight rows off their lines (a row stride that 128 does not divide): the skinny kernels of
 // sg_skinny_line_kernel.h in place of heuristic_config's record.  Which of them was read off timings of all their builds
 // (waves, ring slots, row tiles, K splits) against that record on 510 random shapes, n of 128..65536, K of 272..32768, 236 of
@@ -1658,16 +1718,19 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
     return true;
 }
 
-// What stands in for heuristic_config's record, if anything does: a wide tile or a kernel for rows off their lines.
+// What stands in for heuristic_config's record, if anything does: a wide tile, a kernel for rows off their lines or a mid-batch
+// launch with more K splits.
 static bool stand_in_config(const Config& record, int m, int n, int k, int b_stride, bool factors, int cu_count, const Workspace* fixed_ws,
                             Config* out) {
     if (m <= 32) return skinny_line_config(m, n, k, b_stride, cu_count, out);
     double wide_us = 0;
     const bool wide = wide_config(record, m, n, k, b_stride, factors, cu_count, fixed_ws, out, &wide_us);
     Config line;
-    if (!line_config(record, wide ? out : nullptr, wide_us, m, n, k, b_stride, cu_count, fixed_ws, &line)) return wide;
-    *out = line;
-    return true;
+    if (line_config(record, wide ? out : nullptr, wide_us, m, n, k, b_stride, cu_count, fixed_ws, &line)) {
+        *out = line;
+        return true;
+    }
+    return wide || deep_split_config(record, m, n, k, cu_count, fixed_ws, out);
 }
 
 // The record that sg_skinny_gemm_choice reports: heuristic_config's - or, where that has no K split and a kernel for rows
@@ -1677,6 +1740,7 @@ static bool stand_in_config(const Config& record, int m, int n, int k, int b_str
 static Config reported_config(int m, int n, int k, int cu_count) {
     const Config base = heuristic_config(m, n, k, cu_count);
     Config c;
+    if (m > 128 && stand_in_config(base, m, n, k, k, false, cu_count, nullptr, &c) && !c.line && !c.wide) return c;   // (a record's own launch)
     if (k % 128 == 0 || base.split_k > 1 || !stand_in_config(base, m, n, k, k, false, cu_count, nullptr, &c) || !c.line || c.split_k == 1) return base;
     if (m <= 32) {
         c.line = false;
@@ -1748,6 +1812,9 @@ static bool rejected_before_launch(int rc) {
 static bool launch_stand_in(const Config& record, const StreamArgs& a, int cu_count, hipStream_t stream, const Workspace* fixed_ws, int* rc) {
     Config c;
     if (!stand_in_config(record, a.m, a.n, a.k, a.b_stride, a.row_scale || a.col_scale, cu_count, fixed_ws, &c)) return false;
+    // A mid-batch split of deep_split_config's in place of an unsplit record takes partials of the stream's workspace, which under
+    // capture it leaves: a recorded launch may replay next to other work of that stream, as graphs of the record always could.
+    if (!c.line && !c.wide && a.m > 32 && c.split_k > 1 && record.split_k == 1 && !fixed_ws && stream_is_capturing(stream)) return false;
     c.fixed_ws = fixed_ws;
     *rc = launch_config(c, a, stream);
     return !rejected_before_launch(*rc) && !(c.split_k > 1 && *rc == SG_NO_DEVICE);

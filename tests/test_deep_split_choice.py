@@ -1,0 +1,82 @@
+"""K splits of the mid-batch kernel beyond its record's, on few weight rows (no GPU: the library's host code, its launches on a
+stand-in for the runtime)."""
+import ctypes as C
+import random
+
+import launch_recorder
+import pytest
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    return launch_recorder.build(tmp_path_factory.mktemp("fake"))
+
+
+# shapes whose heuristic record has no K split where the rule takes one: whole lines, a part of a block at the end of K
+UNSPLIT_RECORDS = [(1061, 128, 6128), (339, 432, 3840), (915, 188, 8640), (1257, 178, 30144), (1817, 1146, 18160)]
+
+
+def chosen_and_launched(rec, count):
+    """[shape, record, bytes asked for, launches] of random shapes that the mid-batch kernel takes with a K split above 128 rows"""
+    r, out = random.Random(5), []
+    record, four, three = (C.c_int * 10)(), (C.c_int * 4)(), (C.c_int * 3)()
+    need = C.c_size_t()
+    for i in range(count):
+        m, n, k = int(129 * 20 ** r.random()), 2 * int(1 + 4000 ** r.random()), 16 * int(64 * 40 ** r.random())
+        if r.random() < 0.5:
+            k = max(1024, k // 128 * 128)
+        pad = r.choice([0, 0, 16, 128])
+        if i < len(UNSPLIT_RECORDS):
+            (m, n, k), pad = UNSPLIT_RECORDS[i], 0
+        assert rec.call("sg_skinny_gemm_choice", m, n, k, record, None) == 0
+        assert rec.call("sg_debug_line_choice", m, n, k, k + pad, 0, four) == 0
+        assert rec.call("sg_debug_wide_choice", m, n, k, k + pad, 0, three) == 0
+        if record[0] != 4 or record[1] == 1 or four[0] or three[0]:
+            continue
+        assert rec.call("sg_workspace_query", m, n, k, C.byref(need)) == 0
+        rc, launches = rec.of("sg_skinny_gemm_auto", rec.A, rec.B, rec.D, rec.S, m, n, k, k + pad, None)
+        assert rc == 0
+        out.append([(m, n, k, pad), list(record), need.value, [x for x in launches if "fill_zero" not in x[0]]])
+    return out
+
+
+def test_the_reported_record_is_what_runs_and_fits_the_workspace_asked_for(fake):
+    seen = launch_recorder.scenario(fake, "test_deep_split_choice", "chosen_and_launched", 4000)
+    assert len(seen) > 500 and sum(s[0][2] % 128 != 0 for s in seen) > 100
+    assert [tuple(s[0][:3]) for s in seen[:len(UNSPLIT_RECORDS)]] == UNSPLIT_RECORDS
+    for shape, record, need, launches in seen:
+        m, n, k, _ = shape
+        _, split, waves, rg, mb = record[:5]
+        tiles = -(-n // (8 * waves * rg)) * -(-m // (32 * mb))
+        assert len(launches) == 2 and "mid_gemm_kernel" in launches[0][0] and "mid_reduce_kernel" in launches[1][0], (shape, record, launches)
+        assert launches[0][1:3] == [tiles * split, 64 * waves], (shape, record, launches)
+        assert need >= 65536 + tiles * split * 8 * waves * rg * 32 * mb * 4, (shape, record, need)
+
+
+def records_at_the_edges(rec):
+    """K splits of the choice on either side of the ranges that were timed"""
+    record, out = (C.c_int * 10)(), []
+    for m, n, k in [(2048, 128, 6144), (2049, 128, 6144), (915, 188, 32768), (915, 188, 32784), (1024, 8192, 8192 + 128)]:
+        assert rec.call("sg_skinny_gemm_choice", m, n, k, record, None) == 0
+        out.append(record[1])
+    return out
+
+
+def test_nothing_beyond_the_timed_ranges(fake):
+    at = launch_recorder.scenario(fake, "test_deep_split_choice", "records_at_the_edges")
+    assert at[0] > 1 and at[1] == 1 and at[2] > 4 and at[3] == 2 and at[4] == 1, at    # (2: the record's own)
+
+
+def without_room_for_partials(rec):
+    out = []
+    rec.fake.rec_largest_allocation(1 << 18)
+    for m, n, k in UNSPLIT_RECORDS:
+        out.append(rec.of("sg_skinny_gemm_auto", rec.A, rec.B, rec.D, rec.S, m, n, k, k, None))
+        out.append(rec.of("sg_skinny_gemm_auto_ws", rec.A, rec.B, rec.D, rec.S, m, n, k, k, None, C.c_size_t(0), None))
+    return out
+
+
+def test_the_record_runs_where_there_is_no_room_for_the_partials(fake):
+    """... and a caller who brings no workspace, as the record without a K split let it, is not refused"""
+    for rc, launches in launch_recorder.scenario(fake, "test_deep_split_choice", "without_room_for_partials"):
+        assert rc == 0 and len(launches) == 1 and "mid_gemm_kernel" in launches[0][0], (rc, launches)
