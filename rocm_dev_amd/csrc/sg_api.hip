@@ -1194,6 +1194,18 @@ static Config pick_config(int m, int n, int k, int cu_count) {
             c.waves = 1;
             c.depth = 8;
             c.split_k = few_tiles_split;
+            // With fewer workgroups than CUs the launch is a workgroup's chain of stages, and one wave has eight in flight: two
+            // waves of six slots keep twelve (1 x 2786 x 18816 13.2 -> 10.2 us, 7 x 2592 x 25472 17.7 -> 15.2, 2 x 766 x 6016 5.5 -> 4.8,
+            // 1 x 178 x 29440 8.1 -> 6.9).  From 200 workgroups on - 240 with thirty blocks of K each, 100 at 9..16 rows - HBM
+            // is busy either way and the sum over two waves costs up to 3 %; below fifteen blocks it costs 10 to 25 %, and with K off
+            // the 128-byte lines it pays from about 36 (5 x 1378 x 5840 5.9 against 6.1, 1 x 2676 x 16144 11.9 -> 9.9).  80 random
+            // shapes that it takes: 0.93 of the time before in the geometric mean, one behind by more than 3 %, which the limit of
+            // 200 off the lines has since left out (1 x 3646 x 11728 10.0 against 9.5).
+            const int wgs = tiles16 * c.split_k, of_each = blocks / c.split_k;
+            if (of_each >= (k % 128 == 0 ? 17 : 36) && wgs <= (m > 8 ? 100 : (k % 128 == 0 && of_each >= 30 ? 240 : 200))) {
+                c.waves = 2;
+                c.depth = 6;
+            }
             // between one and two 16-row tiles per CU half of the CUs stream twice what the others do (all
             // workgroups are resident at once); 24-row tiles that give every CU one workgroup level that.  Measured
             // on 6144 x 4096: level with 16-row tiles up to 8 activation rows (6.75 against 6.70 us - the launch is
