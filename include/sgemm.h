@@ -247,7 +247,7 @@ int sg_skinny_gemm_pick(int m, int n, int k, int out[8]);
  *     the launch that it replaces - or, where it splits K and that launch does not, a mid-batch record of the same split on
  *     the tile nearest to its own, so that split_k says of either whether a workspace is needed (k = b_stride)
  *   wide tiles (sg_debug_wide_choice; above 128 rows).  The record is the mid-batch launch that it replaces.
- * Above 128 rows on few weight rows with a long k the record may split K in place of an unsplit one that needs no workspace.
+ * Above 32 rows on few weight rows with a long k the record may split K in place of an unsplit one that needs no workspace.
  * That one runs where the split cannot: on a caller's smaller workspace or none, without device memory for the library's own, and
  * under capture without a caller's, so that graphs of such launches may replay side by side (the sums are added up in
  * another order there than in an eager call). */

@@ -1638,6 +1638,44 @@ static bool deep_split_config(const Config& record, int m, int n, int k, int cu_
     return true;
 }
 
+// 33..256 rows on the skinny ring (two_pass_config) with so few tiles that a workgroup's chain of stages is the launch: K splits
+// where the record has none (below K = 16384), on four waves of two slots over 16- or 32-row weight tiles, where this model puts them
+// 7 % ahead.
+// Microseconds fitted to 110 random shapes (33..256 rows, 128..5000 weight rows, K of 512..32768) timed with every split: 3.3 for
+// a launch, 0.17 or 0.25 a stage of 256 bytes of K, 1.23 times that with K off the 128-byte lines, 0.5 and 0.37 a split.  Of those
+// shapes it takes 38 and of others 100 were timed, padded rows and factors among them: 0.78 of the time before in the geometric
+// mean, two behind by more than 3 % (4): 40 x 192 x 13056 12.4 -> 7.2 us,
+// 130 x 160 x 11904 11.5 -> 7.6, 90 x 464 x 10144 12.9 -> 8.5, 49 x 570 x 6400 7.7 -> 6.6; below about 4000 of K an unsplit
+// launch stays ahead.
+static double ring_split_us(int k, int rg, int sk, double fill) {
+    const double stages = (double)((k + 255) / 256) / sk * (k % 128 ? 1.23 : 1.0);
+    return 3.34 + stages * (rg == 1 ? 0.17 : 0.25 + 0.019 * fill) + (sk > 1 ? 0.51 + 0.37 * sk : 0.0);
+}
+
+static bool ring_split_config(const Config& record, int m, int n, int k, int cu_count, const Workspace* fixed_ws, Config* out) {
+    if (m <= 32 || m > 256 || n < 128 || n > 5000 || record.engine != ENGINE_LDS || record.rg > 2 || record.split_k > 1) return false;
+    const int blocks = (k + 255) / 256, m_tiles = (m + 31) / 32;
+    double best = 0.93 * ring_split_us(k, record.rg, 1, (double)((n + 16 * record.rg - 1) / (16 * record.rg)) * m_tiles / cu_count);
+    Config c = record;
+    c.waves = 4;
+    c.depth = 2;
+    bool found = false;
+    for (int rg = 1; rg <= 2; rg++) {
+        const long tiles = (long)((n + 16 * rg - 1) / (16 * rg)) * m_tiles;
+        for (int sk = 2; sk <= 6 && blocks / sk >= 5 && tiles * sk <= cu_count; sk++) {
+            if (fixed_ws && ((size_t)(tiles * sk) * rg * 2048 > fixed_ws->partial_bytes || (size_t)tiles > fixed_ws->n_counters)) break;
+            const double us = ring_split_us(k, rg, sk, (double)(tiles * sk) / cu_count);
+            if (us >= best) continue;
+            best = us;
+            found = true;
+            c.rg = rg;
+            c.split_k = sk;
+        }
+    }
+    if (found) *out = c;
+    return found;
+}
+
 // Up to 32 activation rows and weight rows off their lines (a row stride that 128 does not divide): the skinny kernels of
 // sg_skinny_line_kernel.h in place of heuristic_config's record.  Which of them was read off timings of all their builds
 // (waves, ring slots, row tiles, K splits) against that record on 510 random shapes, n of 128..65536, K of 272..32768, 236 of
@@ -1730,8 +1768,8 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
     return true;
 }
 
-// What stands in for heuristic_config's record, if anything does: a wide tile, a kernel for rows off their lines or a mid-batch
-// launch with more K splits.
+// What stands in for heuristic_config's record, if anything does: a wide tile, a kernel for rows off their lines or a launch of the
+// record's kind with more K splits.
 static bool stand_in_config(const Config& record, int m, int n, int k, int b_stride, bool factors, int cu_count, const Workspace* fixed_ws,
                             Config* out) {
     if (m <= 32) return skinny_line_config(m, n, k, b_stride, cu_count, out);
@@ -1742,7 +1780,7 @@ static bool stand_in_config(const Config& record, int m, int n, int k, int b_str
         *out = line;
         return true;
     }
-    return wide || deep_split_config(record, m, n, k, cu_count, fixed_ws, out);
+    return wide || deep_split_config(record, m, n, k, cu_count, fixed_ws, out) || ring_split_config(record, m, n, k, cu_count, fixed_ws, out);
 }
 
 // The record that sg_skinny_gemm_choice reports: heuristic_config's - or, where that has no K split and a kernel for rows
@@ -1752,7 +1790,7 @@ static bool stand_in_config(const Config& record, int m, int n, int k, int b_str
 static Config reported_config(int m, int n, int k, int cu_count) {
     const Config base = heuristic_config(m, n, k, cu_count);
     Config c;
-    if (m > 128 && stand_in_config(base, m, n, k, k, false, cu_count, nullptr, &c) && !c.line && !c.wide) return c;   // (a record's own launch)
+    if (m > 32 && stand_in_config(base, m, n, k, k, false, cu_count, nullptr, &c) && !c.line && !c.wide) return c;   // (a record's own launch)
     if (k % 128 == 0 || base.split_k > 1 || !stand_in_config(base, m, n, k, k, false, cu_count, nullptr, &c) || !c.line || c.split_k == 1) return base;
     if (m <= 32) {
         c.line = false;
@@ -1824,7 +1862,7 @@ static bool rejected_before_launch(int rc) {
 static bool launch_stand_in(const Config& record, const StreamArgs& a, int cu_count, hipStream_t stream, const Workspace* fixed_ws, int* rc) {
     Config c;
     if (!stand_in_config(record, a.m, a.n, a.k, a.b_stride, a.row_scale || a.col_scale, cu_count, fixed_ws, &c)) return false;
-    // A mid-batch split of deep_split_config's in place of an unsplit record takes partials of the stream's workspace, which under
+    // A split of deep_split_config's or ring_split_config's in place of an unsplit record takes partials of the stream's workspace, which under
     // capture it leaves: a recorded launch may replay next to other work of that stream, as graphs of the record always could.
     if (!c.line && !c.wide && a.m > 32 && c.split_k > 1 && record.split_k == 1 && !fixed_ws && stream_is_capturing(stream)) return false;
     c.fixed_ws = fixed_ws;

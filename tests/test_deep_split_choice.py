@@ -1,5 +1,5 @@
-"""K splits of the mid-batch kernel beyond its record's, on few weight rows (no GPU: the library's host code, its launches on a
-stand-in for the runtime)."""
+"""K splits of the mid-batch kernel and of the skinny ring over several activation tiles beyond their records', on few weight rows
+(no GPU: the library's host code, its launches on a stand-in for the runtime)."""
 import ctypes as C
 import random
 
@@ -53,6 +53,40 @@ def test_the_reported_record_is_what_runs_and_fits_the_workspace_asked_for(fake)
         assert need >= 65536 + tiles * split * 8 * waves * rg * 32 * mb * 4, (shape, record, need)
 
 
+RINGS = [(130, 160, 11904), (56, 302, 12288), (90, 464, 10144), (256, 130, 5792), (33, 4998, 2048)]
+
+
+def rings_chosen_and_launched(rec, count):
+    """The same of 33..256 rows on the skinny ring: [shape, record, bytes asked for, launches]"""
+    r, out = random.Random(6), []
+    record, four, need = (C.c_int * 10)(), (C.c_int * 4)(), C.c_size_t()
+    for i in range(count):
+        m, n, k = int(33 * 7.8 ** r.random()), 2 * int(1 + 2500 ** r.random()), 16 * int(64 * 32 ** r.random())
+        if i < len(RINGS):
+            m, n, k = RINGS[i]
+        assert rec.call("sg_skinny_gemm_choice", m, n, k, record, None) == 0
+        assert rec.call("sg_debug_line_choice", m, n, k, k, 0, four) == 0
+        if record[0] != 2 or four[0]:
+            continue
+        assert rec.call("sg_workspace_query", m, n, k, C.byref(need)) == 0
+        rc, launches = rec.of("sg_skinny_gemm_auto", rec.A, rec.B, rec.D, rec.S, m, n, k, k, None)
+        assert rc == 0
+        out.append([(m, n, k), list(record), need.value, [x for x in launches if "fill_zero" not in x[0]]])
+    return out
+
+
+def test_the_rings_reported_record_is_what_runs_and_fits_the_workspace_asked_for(fake):
+    seen = launch_recorder.scenario(fake, "test_deep_split_choice", "rings_chosen_and_launched", 3000)
+    assert sum(s[1][1] > 1 and s[0][2] < 16384 for s in seen) > 100
+    for shape, record, need, launches in seen:
+        m, n, k = shape
+        _, split, waves, rg, mt = record[:5]
+        tiles = -(-n // (16 * rg)) * -(-m // (16 * mt))
+        assert len(launches) == 1 and "lds_gemm_kernel" in launches[0][0], (shape, record, launches)
+        assert launches[0][1:3] == [tiles * split, 64 * waves], (shape, record, launches)
+        assert need == (65536 + tiles * split * rg * mt * 1024 if split > 1 else 0), (shape, record, need)
+
+
 def records_at_the_edges(rec):
     """K splits of the choice on either side of the ranges that were timed"""
     record, out = (C.c_int * 10)(), []
@@ -69,8 +103,8 @@ def test_nothing_beyond_the_timed_ranges(fake):
 
 def without_room_for_partials(rec):
     out = []
-    rec.fake.rec_largest_allocation(1 << 18)
-    for m, n, k in UNSPLIT_RECORDS:
+    rec.fake.rec_largest_allocation(1 << 12)
+    for m, n, k in UNSPLIT_RECORDS + [(130, 160, 11904), (92, 316, 12416)]:
         out.append(rec.of("sg_skinny_gemm_auto", rec.A, rec.B, rec.D, rec.S, m, n, k, k, None))
         out.append(rec.of("sg_skinny_gemm_auto_ws", rec.A, rec.B, rec.D, rec.S, m, n, k, k, None, C.c_size_t(0), None))
     return out
@@ -79,4 +113,4 @@ def without_room_for_partials(rec):
 def test_the_record_runs_where_there_is_no_room_for_the_partials(fake):
     """... and a caller who brings no workspace, as the record without a K split let it, is not refused"""
     for rc, launches in launch_recorder.scenario(fake, "test_deep_split_choice", "without_room_for_partials"):
-        assert rc == 0 and len(launches) == 1 and "mid_gemm_kernel" in launches[0][0], (rc, launches)
+        assert rc == 0 and len(launches) == 1 and "_gemm_kernel" in launches[0][0] and "line" not in launches[0][0], (rc, launches)
