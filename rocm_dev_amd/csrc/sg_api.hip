@@ -1591,17 +1591,28 @@ static bool line_config(const Config& record, const Config* wide, double wide_us
 // x 28048 109 -> 33 us, 1257 x 178 x 30144 100 -> 29, 1635 x 626 x 19056 108 -> 51, 1817 x 1146 x 18160 173 -> 82, 915 x 188 x 8640
 // 27.5 -> 12.8, 295 x 144 x 4224 12.7 -> 8.8, 822 x 5518 x 14880 141 -> 127.  Rows off their lines up to 768 rows are
 // line_config's.  Where the record stays ahead - one round of tiles that fills the CUs, K below about 3000 - the model says so.
-static double deep_split_us(int m, int n, int k, int bn, int bm, int sk, int cu_count) {
-    const bool lines = k % 128 == 0;
-    const long wgs = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm) * sk;
-    const double stages = (double)(((k + 127) / 128 + sk - 1) / sk);
-    const double per_stage = lines ? 0.232 * bn / 128 + 0.247 * bm / 128 + 0.12 * bn * bm / 16384
-                                   : 0.458 * bn / 128 + 0.384 * bm / 128 + 0.073 * bn * bm / 16384;
-    double us = rounds_of(wgs, cu_count, lines ? 0.87 : 0.84) * stages * per_stage;
-    us += lines ? 3.5 + (double)((wgs + cu_count - 1) / cu_count) : 4.2;
-    if (sk > 1) us += lines ? 3.1 + 1.36e-6 * (double)wgs * bn * bm : 2.7 + 1.57e-6 * (double)wgs * bn * bm;
-    return us;
-}
+struct DeepSplitModel {     // (of one tile; a choice evaluates it some hundred times per call)
+    double stage_us, split_us, first_us, round_us, part, per_cu;
+    int blocks, cu_count;
+    DeepSplitModel(int k, int bn, int bm, int cus) : per_cu(1.0 / cus), blocks((k + 127) / 128), cu_count(cus) {
+        const bool lines = k % 128 == 0;
+        stage_us = lines ? (0.232 / 128) * bn + (0.247 / 128) * bm + (0.12 / 16384) * bn * bm
+                         : (0.458 / 128) * bn + (0.384 / 128) * bm + (0.073 / 16384) * bn * bm;
+        split_us = (lines ? 1.36e-6 : 1.57e-6) * bn * bm;
+        first_us = lines ? 3.1 : 2.7;
+        round_us = lines ? 1.0 : 0.0;
+        part = lines ? 0.87 : 0.84;
+    }
+    double us(long of_m_n, int sk) const {
+        const long wgs = of_m_n * sk;
+        const int full = wgs < cu_count ? 0 : (int)(wgs / cu_count);
+        const long rest = wgs - (long)full * cu_count;
+        const double stages = (double)((unsigned)(blocks + sk - 1) / (unsigned)sk);
+        const double us = ((double)full + (rest ? part + (1.0 - part) * (double)rest * per_cu : 0.0)) * stages * stage_us +
+                          (round_us > 0 ? 3.5 + (double)(full + (rest ? 1 : 0)) : 4.2);
+        return sk > 1 ? us + first_us + split_us * (double)wgs : us;
+    }
+};
 
 constexpr double kDeepSplitWork = 1024.0 * 8192 * 8192;   // none of the shapes timed is larger
 static bool deep_split_config(const Config& record, int m, int n, int k, int cu_count, const Workspace* fixed_ws, Config* out) {
@@ -1610,18 +1621,22 @@ static bool deep_split_config(const Config& record, int m, int n, int k, int cu_
     struct Tile { int waves, rg, mt; };
     static const Tile tiles[] = {{4, 2, 2}, {4, 2, 4}, {4, 4, 4}, {8, 2, 2}, {8, 2, 4}, {8, 2, 8}, {8, 4, 2}, {8, 4, 4}, {8, 4, 8}};
     const int blocks = (k + 127) / 128;
+    const int own_bn = 8 * record.rg * record.waves;
+    const DeepSplitModel own(k, own_bn, 32 * record.mt, cu_count);
     // (ahead of a record that splits already by less than 12 %, it was behind as often: 554 x 346 x 16000 16.7 against 18.4)
-    double best = (record.split_k > 1 ? 0.88 : 0.95) * deep_split_us(m, n, k, 8 * record.rg * record.waves, 32 * record.mt, record.split_k, cu_count);
+    double best = (record.split_k > 1 ? 0.88 : 0.95) * own.us((long)((n + own_bn - 1) / own_bn) * ((m + 32 * record.mt - 1) / (32 * record.mt)), record.split_k);
     bool found = false;
     Config c{};
     for (const Tile& t : tiles) {
         const int bn = 8 * t.waves * t.rg, bm = 32 * t.mt;
         if (k % 128 != 0 && t.waves == 4 && t.rg == 4) continue;    // not built with part of a block at the end of K
         const long of_m_n = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm);
-        for (int sk = 2; sk <= 16 && blocks / sk >= 4 && of_m_n * sk <= 2L * cu_count; sk++) {
+        const DeepSplitModel model(k, bn, bm, cu_count);
+        const int most = (int)std::min<long>(std::min(16, blocks / 4), 2L * cu_count / of_m_n);
+        for (int sk = 2; sk <= most; sk++) {
             // (kMaxPartialBytes holds any such split)
             if (fixed_ws && ((size_t)(of_m_n * sk) * bn * bm * 4 > fixed_ws->partial_bytes || (size_t)of_m_n > fixed_ws->n_counters)) break;
-            const double us = deep_split_us(m, n, k, bn, bm, sk, cu_count);
+            const double us = model.us(of_m_n, sk);
             if (us >= best) continue;
             best = us;
             found = true;
