@@ -1877,9 +1877,12 @@ static bool rejected_before_launch(int rc) {
 static bool launch_stand_in(const Config& record, const StreamArgs& a, int cu_count, hipStream_t stream, const Workspace* fixed_ws, int* rc) {
     Config c;
     if (!stand_in_config(record, a.m, a.n, a.k, a.b_stride, a.row_scale || a.col_scale, cu_count, fixed_ws, &c)) return false;
-    // A split of deep_split_config's or ring_split_config's in place of an unsplit record takes partials of the stream's workspace, which under
-    // capture it leaves: a recorded launch may replay next to other work of that stream, as graphs of the record always could.
-    if (!c.line && !c.wide && a.m > 32 && c.split_k > 1 && record.split_k == 1 && !fixed_ws && stream_is_capturing(stream)) return false;
+    // A split of skinny_line_config's, deep_split_config's or ring_split_config's in place of an unsplit record takes partials and
+    // counters of the stream's workspace, which under capture it leaves: a recorded launch may replay next to other work of that
+    // stream, as graphs of the record always could.  (The kernel for rows off their lines from 33 rows on splits under capture too,
+    // in the capture stream's workspace, as sgemm.h says of recorded launches with a K split.)
+    const bool keeps_split = c.line && a.m > 32;
+    if (c.split_k > 1 && record.split_k == 1 && !keeps_split && !fixed_ws && stream_is_capturing(stream)) return false;
     c.fixed_ws = fixed_ws;
     *rc = launch_config(c, a, stream);
     return !rejected_before_launch(*rc) && !(c.split_k > 1 && *rc == SG_NO_DEVICE);

@@ -19,7 +19,7 @@ std::mutex g_lock;
 std::map<const void*, std::string> g_names;   // host stub -> kernel
 std::vector<Launch> g_launches;
 size_t g_next = 1ul << 40, g_largest = ~(size_t)0;
-int g_pause_us = 0;
+int g_pause_us = 0, g_capturing = 0, g_allocations = 0;
 thread_local Call t_call;
 }  // namespace
 
@@ -30,6 +30,8 @@ int rec_count() { std::lock_guard<std::mutex> l(g_lock); return (int)g_launches.
 void rec_get(int i, Launch* out) { std::lock_guard<std::mutex> l(g_lock); *out = g_launches[(size_t)i]; }
 void rec_pause(int us) { g_pause_us = us; }              // every launch takes that long to return
 void rec_largest_allocation(size_t bytes) { g_largest = bytes; }
+void rec_capturing(int on) { g_capturing = on; }         // every stream is being captured
+int rec_allocations() { std::lock_guard<std::mutex> l(g_lock); return g_allocations; }
 
 // ---- what hipcc's host code calls
 void** __hipRegisterFatBinary(const void*) { static void* handle; return &handle; }
@@ -63,6 +65,7 @@ hipError_t hipLaunchKernel(const void* host, dim3 grid, dim3 block, void**, size
 hipError_t hipMalloc(void** p, size_t bytes) {
     std::lock_guard<std::mutex> l(g_lock);
     if (bytes > g_largest) return hipErrorOutOfMemory;
+    g_allocations++;
     *p = reinterpret_cast<void*>(g_next);
     g_next += (bytes + 4095) & ~(size_t)4095;
     return hipSuccess;
@@ -84,6 +87,9 @@ hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = reinterpret_cast<hipStream_t>(0x1000); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) { *s = hipStreamCaptureStatusNone; return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
+    *s = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
 }
