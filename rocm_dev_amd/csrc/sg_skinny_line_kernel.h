@@ -293,8 +293,10 @@ __global__ void __launch_bounds__(512) skinny_line_resident_kernel(const StreamA
             pair = 0;
             // The result of a matrix instruction may be read 12 wait states behind it.  The compiler did not see that across
             // the branches between the two (the store read the accumulators 3 states behind the last instruction, and took
-            // them without it).
-            asm volatile("s_nop 15" : "+v"(acc[0]));
+            // them without it).  Tied to every accumulator, so that none of their last instructions sinks behind it.
+            static_assert(MT <= 2);
+            if constexpr (MT == 2) asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[1]));
+            else asm volatile("s_nop 15" : "+v"(acc[0]));
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
                 store_fragment(a, acc[mt], scale, mt * 16 + r, tile * 16 + 4 * g);

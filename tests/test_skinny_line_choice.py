@@ -48,32 +48,91 @@ def test_shapes_timed_on_both_sides_of_the_rule():
             api.skinny_gemm_skinny_line_choice(*bad)
 
 
+# wait states (an instruction is one) from an eight-pass matrix instruction to a read of its result, and to a vector instruction
+# that overwrites it
+READ, OVERWRITE = 12, 11
+
+
+def _registers(text):
+    regs = set(int(x) for x in re.findall(r"\bv(\d+)\b", text))
+    for lo, hi in re.findall(r"\bv\[(\d+):(\d+)\]", text):
+        regs.update(range(int(lo), int(hi) + 1))
+    return regs
+
+
+def _functions(text):
+    """{kernel: (instructions, {label: index})}"""
+    out = {}
+    for m in re.finditer(r"^(_ZN2sg\w+):[^\n]*\n(.*?)^\s*\.section", text, re.S | re.M):
+        code, labels = [], {}
+        for line in m.group(2).splitlines():
+            line = line.split(";")[0].strip()
+            if line.endswith(":"):
+                labels[line[:-1]] = len(code)
+            elif line and not line.startswith("."):
+                code.append(line)
+        out[m.group(1)] = code, labels
+    return out
+
+
+def _early(code, labels):
+    """(matrix instructions, accesses to their results that come too early), along every branch, both ways"""
+    parsed = []
+    for instruction in code:
+        op, _, operands = instruction.replace("\t", " ").partition(" ")
+        first, _, rest = operands.partition(", ")
+        stores = "store" in op or op.startswith("ds_write") or " lds" in operands
+        valu = op.startswith("v_") and not op.startswith(("v_cmp", "v_readlane", "v_readfirstlane"))
+        reads = _registers(rest if valu or not stores and "load" in op or op.startswith("ds_read") else operands)
+        if op.startswith("v_mfma"):       # (a sum goes on in the registers it is in without waiting)
+            reads = _registers(", ".join(re.findall(r"v\[\d+:\d+\]", rest)[:2]))
+        parsed.append((op, operands, reads, _registers(first) if valu else set()))
+    early, matrix = [], 0
+    for start, (op, _, _, result) in enumerate(parsed):
+        if not op.startswith("v_mfma"):
+            continue
+        matrix += 1
+        paths, seen = [(start + 1, 0, frozenset(result))], {}
+        while paths:
+            at, states, live = paths.pop()
+            while at < len(code) and states < READ and live and seen.get((at, live), READ) > states:
+                seen[at, live] = states
+                op, operands, reads, writes = parsed[at]
+                if op.startswith(("s_endpgm", "s_setpc")):
+                    break
+                if reads & live or (states < OVERWRITE and writes & live and not op.startswith("v_mfma")):
+                    early.append((code[start], code[at], states))
+                    break
+                live -= writes
+                if op.startswith("s_cbranch"):
+                    paths.append((labels[operands], states + 1, live))
+                states += int(operands) + 1 if op == "s_nop" else 1
+                at = labels[operands] if op == "s_branch" else at + 1
+    return matrix, early
+
+
 def test_no_result_is_read_while_it_is_being_written():
-    """A vector instruction may read a matrix instruction's result 11 wait states behind it (one instruction is one; as the code
-    lies, not followed across taken branches).  The compiler missed some across branches in a tile's last step."""
+    """A vector or memory instruction may read a matrix instruction's result 12 wait states behind it, whichever way the branches
+    in between go.  The compiler missed some across branches in a tile's last step."""
     if not shutil.which("hipcc") and not os.path.exists("/opt/rocm/bin/hipcc"):
         pytest.skip("no hipcc")
     subprocess.run(["make", "-s", "-C", CSRC, "obj/sg_skinny_line_inst.s"], check=True, capture_output=True)
-    code = [line.split(";")[0].strip() for line in open(os.path.join(CSRC, "obj", "sg_skinny_line_inst.s"))]
-    busy, matrix = {}, 0
-    for instruction in code:
-        if not instruction or instruction.endswith(":") or instruction.startswith((".", "#")):
-            continue
-        operands = instruction.split(None, 1)[1] if " " in instruction or "\t" in instruction else ""
-        regs = set(int(x) for x in re.findall(r"\bv(\d+)\b", operands))
-        for lo, hi in re.findall(r"\bv\[(\d+):(\d+)\]", operands):
-            regs.update(range(int(lo), int(hi) + 1))
-        if instruction.startswith(("s_branch", "s_endpgm")):
-            busy = {}
-            continue
-        if instruction.startswith("v_mfma"):
-            matrix += 1
-            first = re.search(r"v\[(\d+):(\d+)\]", operands)
-            busy = {r: s + 1 for r, s in busy.items()}
-            busy.update({r: 0 for r in range(int(first.group(1)), int(first.group(2)) + 1)})
-            continue
-        early = [r for r in regs if busy.get(r, 99) < 11]
-        assert not early, "%s: v%d is read %d wait states behind its matrix instruction" % (instruction, early[0], busy[early[0]])
-        nop = re.match(r"s_nop (\d+)", instruction)
-        busy = {r: s + (int(nop.group(1)) + 1 if nop else 1) for r, s in busy.items() if s < 20}
-    assert matrix > 100
+    kernels = _functions(open(os.path.join(CSRC, "obj", "sg_skinny_line_inst.s")).read())
+    assert len(kernels) == 21       # the builds of launch_skinny_line
+    total = 0
+    for name, (code, labels) in kernels.items():
+        matrix, early = _early(code, labels)
+        assert not early, "%s: %s is %d wait states in front of %s" % (name, early[0][0], early[0][2], early[0][1])
+        total += matrix
+    assert total > 100
+
+
+def test_the_check_follows_branches_both_ways_and_counts_idle_states():
+    matrix = "v_mfma_f32_16x16x128_f8f6f4 v[0:3], v[10:17], v[20:27], v[0:3]"
+    for code, early in ((["s_nop 10", "v_mov_b32_e32 v9, v1"], 1), (["s_nop 11", "v_mov_b32_e32 v9, v1"], 0),
+                        (["s_nop 9", "v_mov_b32_e32 v1, 0"], 1), (["s_nop 10", "v_mov_b32_e32 v1, 0"], 0), ([matrix], 0),
+                        (["global_store_dwordx4 v[30:31], v[0:3], off"], 1), (["ds_read_b128 v[40:43], v3"], 1),
+                        (["s_cbranch_scc1 there", "s_nop 15", "there:", "ds_write_b128 v40, v[0:3]"], 1),
+                        (["s_branch there", "v_mov_b32_e32 v9, v1", "there:", "s_nop 15", "v_mov_b32_e32 v9, v1"], 0)):
+        code = "_ZN2sg1xEv: ; @\n\t" + "\n\t".join([matrix] + code + ["s_endpgm"]) + "\n\t.section\n"
+        assert len(_early(*_functions(code)["_ZN2sg1xEv"])[1]) == early, code
