@@ -1783,11 +1783,16 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
     return true;
 }
 
+// Records that skinny_line_config's kernels do not replace, wherever their rows lie: those of 17..32 rows with three K splits (in
+// the place of two or four: on 70 random shapes of 1030 to 1350 weight rows 0.94 of the time with two, 20 x 1156 x 28608 12.8 us against
+// 14.9; of fewer rows 0.99 of it with four on 13).
+static bool skinny_record_stays(const Config& record) { return record.split_k == 3; }
+
 // What stands in for heuristic_config's record, if anything does: a wide tile, a kernel for rows off their lines or a launch of the
 // record's kind with more K splits.
 static bool stand_in_config(const Config& record, int m, int n, int k, int b_stride, bool factors, int cu_count, const Workspace* fixed_ws,
                             Config* out) {
-    if (m <= 32) return skinny_line_config(m, n, k, b_stride, cu_count, out);
+    if (m <= 32) return !skinny_record_stays(record) && skinny_line_config(m, n, k, b_stride, cu_count, out);
     double wide_us = 0;
     const bool wide = wide_config(record, m, n, k, b_stride, factors, cu_count, fixed_ws, out, &wide_us);
     Config line;
@@ -2185,7 +2190,7 @@ int sg_debug_skinny_line_choice(int m, int n, int k, int b_stride, int out[5]) {
     int cu = 256;
     if (get_device_info(&dev) == SG_SUCCESS) cu = dev->cu_count;
     Config c;
-    if (skinny_line_config(m, n, k, b_stride, cu, &c)) {
+    if (m <= 32 && stand_in_config(heuristic_config(m, n, k, cu), m, n, k, b_stride, false, cu, nullptr, &c)) {
         out[0] = c.waves; out[1] = c.rg; out[2] = c.depth; out[3] = c.split_k; out[4] = c.wavetile;
     }
     return SG_SUCCESS;

@@ -48,6 +48,19 @@ def test_shapes_timed_on_both_sides_of_the_rule():
             api.skinny_gemm_skinny_line_choice(*bad)
 
 
+# where these kernels were timed behind the record, us: theirs / the record's
+RECORD_STAYS = [
+    # two K splits (four in the last) in the place of three: 14.9 / 12.8, 14.4 / 13.2, 13.4 / 12.1, 8.2 / 7.7, 7.7 / 7.3
+    (20, 1156, 28608, 0), (31, 1224, 22048, 0), (18, 1172, 24112, 0), (19, 1192, 8496, 16), (18, 998, 7376, 0),
+]
+
+
+@pytest.mark.parametrize("m,n,k,pad", RECORD_STAYS)
+def test_the_record_stays_where_it_was_timed_ahead(m, n, k, pad):
+    from rocm_dev_amd import api
+    assert api.skinny_gemm_skinny_line_choice(m, n, k, k + pad) is None
+
+
 # wait states (an instruction is one) from an eight-pass matrix instruction to a read of its result, and to a vector instruction
 # that overwrites it
 READ, OVERWRITE = 12, 11
