@@ -1785,8 +1785,12 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
 
 // Records that skinny_line_config's kernels do not replace, wherever their rows lie: those of 17..32 rows with three K splits (in
 // the place of two or four: on 70 random shapes of 1030 to 1350 weight rows 0.94 of the time with two, 20 x 1156 x 28608 12.8 us against
-// 14.9; of fewer rows 0.99 of it with four on 13).
-static bool skinny_record_stays(const Config& record) { return record.split_k == 3; }
+// 14.9; of fewer rows 0.99 of it with four on 13) and those with the activations in the waves' registers (of K from 3072 to 4096 on
+// rows 16 to 80 bytes further apart, 41 random shapes: 0.87 of the time, 23 x 10462 x 4096 on rows of 4112 0.86, 32 x 35948 x 3072 on
+// rows of 3136 0.68).
+static bool skinny_record_stays(const Config& record) {
+    return record.split_k == 3 || (record.engine == ENGINE_LDS && (record.wavetile & 3) == 3);
+}
 
 // What stands in for heuristic_config's record, if anything does: a wide tile, a kernel for rows off their lines or a launch of the
 // record's kind with more K splits.

@@ -52,6 +52,8 @@ def test_shapes_timed_on_both_sides_of_the_rule():
 RECORD_STAYS = [
     # two K splits (four in the last) in the place of three: 14.9 / 12.8, 14.4 / 13.2, 13.4 / 12.1, 8.2 / 7.7, 7.7 / 7.3
     (20, 1156, 28608, 0), (31, 1224, 22048, 0), (18, 1172, 24112, 0), (19, 1192, 8496, 16), (18, 998, 7376, 0),
+    # in the place of the activations in registers: 1.16, 1.48, 1.13 and 1.39 times
+    (23, 10462, 4096, 16), (32, 35948, 3072, 64), (32, 8354, 3584, 16), (28, 34268, 4096, 80),
 ]
 
 
