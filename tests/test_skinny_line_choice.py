@@ -54,6 +54,8 @@ RECORD_STAYS = [
     (20, 1156, 28608, 0), (31, 1224, 22048, 0), (18, 1172, 24112, 0), (19, 1192, 8496, 16), (18, 998, 7376, 0),
     # in the place of the activations in registers: 1.16, 1.48, 1.13 and 1.39 times
     (23, 10462, 4096, 16), (32, 35948, 3072, 64), (32, 8354, 3584, 16), (28, 34268, 4096, 80),
+    # four to five and a half 16-row tiles a CU on four waves: 13.3 / 10.9, 14.3 / 11.2, 12.5 / 10.6
+    (20, 16452, 2384, 0), (21, 16956, 2720, 0), (30, 19340, 1968, 16), (30, 21804, 2240, 0),
 ]
 
 
@@ -61,6 +63,12 @@ RECORD_STAYS = [
 def test_the_record_stays_where_it_was_timed_ahead(m, n, k, pad):
     from rocm_dev_amd import api
     assert api.skinny_gemm_skinny_line_choice(m, n, k, k + pad) is None
+
+
+@pytest.mark.parametrize("m,n,k,pad", [(21, 22968, 2272, 0), (20, 16384, 2384, 0), (20, 16452, 2832, 0), (20, 1400, 28608, 0)])
+def test_just_beyond_they_are_taken(m, n, k, pad):
+    from rocm_dev_amd import api
+    assert api.skinny_gemm_skinny_line_choice(m, n, k, k + pad)
 
 
 # wait states (an instruction is one) from an eight-pass matrix instruction to a read of its result, and to a vector instruction
