@@ -834,7 +834,7 @@ static int launch_sparse_engine(const Config& c, StreamArgs a, const uint8_t* me
 // activations (23 x 7542 x 10240 18.8 -> 15.2), or, up to four stages, on one wave (24 x 4464 x 1024 6.41 -> 3.83); beyond two
 // tiles per CU 16-row tiles where all workgroups are resident in as few rounds (17 x 10622 x 1792 7.74 -> 6.73).  No more slots
 // than a wave has stages.  `split` false: as many K splits as there can be without a workspace, none.
-static void pick_sparse_tile(Config& c, int m, int tiles16, int blocks, int cu, bool split) {
+static void pick_sparse_tile(Config& c, int m, int tiles16, int blocks, bool meta_lines, int cu, bool split) {
     const int xu2 = c.mt == 2 ? 16 : 2 * activation_instructions(1, m);
     int most = 1;
     c.rg = 1;
@@ -849,8 +849,9 @@ static void pick_sparse_tile(Config& c, int m, int tiles16, int blocks, int cu, 
     } else if (c.mt == 2 && tiles16 <= 2 * cu) {
         c.rg = c.waves = blocks <= 4 ? 1 : 2;
     } else if (c.mt == 2) {
-        // three workgroups of 16-row tiles on a CU, or two of 32-row tiles
-        c.rg = (tiles16 + 3 * cu - 1) / (3 * cu) <= (tiles16 + 4 * cu - 1) / (4 * cu) ? 1 : 2;
+        // three workgroups of 16-row tiles on a CU, or two of 32-row tiles - and two of either where the metadata comes by whole
+        // lines, whose ring takes 4 KB of LDS more (28 x 10414 x 1024 5.20 us on 32-row tiles, 6.76 on 16; 25 x 9984 x 10240 25.1, 28.2)
+        c.rg = !meta_lines && (tiles16 + 3 * cu - 1) / (3 * cu) <= (tiles16 + 4 * cu - 1) / (4 * cu) ? 1 : 2;
         c.waves = c.rg == 2 && blocks >= 16 ? 2 : 1;
     } else {
         if (m > 8 ? tiles16 > 4 * cu : tiles16 >= 4 * cu && (m > 4 || blocks > 2 || tiles16 > 6 * cu)) c.rg = 2;
@@ -887,7 +888,7 @@ static Config pick_sparse(int m, int n, int k, int cu_count, bool split) {
                            (size_t)c.waves * c.depth * (c.rg * 5 + xu2) * 1024 + 8192 > 159 * 1024))
         c.depth--;
     const bool timed = m <= 32 && n <= 32768 && k <= 28672;    // (beyond: the rules above, which were)
-    if (timed) pick_sparse_tile(c, m, tiles16, blocks, cu_count, split);
+    if (timed) pick_sparse_tile(c, m, tiles16, blocks, k % 1024 == 0, cu_count, split);
     // (at most two tiles per CU one-wave workgroups are ahead up to 8 rows: 5 x 6170 x 8192 10.0 -> 7.7 us)
     if (c.mt == 1 && m > 4 && tiles16 * 4 >= cu_count * 5 && !(timed && m <= 8 && tiles16 <= 2 * cu_count)) {
         // 5..16 activation rows and more than one tile per CU: the activation matrix stays resident in LDS and
