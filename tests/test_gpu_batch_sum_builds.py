@@ -6,27 +6,37 @@ import torch
 
 CU = 256
 # floats -> (pieces a lane, batches at once, threads) at 2 and at 9 batches
-BUILDS = {257: ((1, 8, 64),) * 2, 1152 * CU: ((1, 8, 64),) * 2, 1152 * CU + 1: ((2, 4, 256),) * 2, 2048 * CU: ((2, 4, 256),) * 2,
-          2048 * CU + 1: ((1, 1, 256),) * 2, 2944 * CU + 1: ((2, 1, 256),) * 2, 4096 * CU + 1: ((1, 1, 256),) * 2, 5120 * CU + 3: ((2, 1, 256),) * 2,
-          6144 * CU + 1: ((4, 1, 512),) * 2, 8192 * CU: ((4, 1, 512),) * 2, 8192 * CU + 1: ((2, 1, 256),) * 2, 9728 * CU + 2: ((4, 1, 256),) * 2,
+ONE = (1, 1, 256)
+BUILDS = {257: (ONE,) * 2, 1024: (ONE,) * 2, 1025: (ONE, (1, 8, 64)), 4096: (ONE, (1, 8, 64)), 4097: ((1, 8, 64),) * 2,
+          1152 * CU: ((1, 8, 64),) * 2, 1152 * CU + 1: ((2, 4, 256),) * 2, 2048 * CU: ((2, 4, 256),) * 2,
+          2048 * CU + 1: (ONE,) * 2, 2944 * CU + 1: (ONE, (2, 1, 256)), 4096 * CU: (ONE, (2, 1, 256)), 4096 * CU + 1: (ONE,) * 2,
+          5120 * CU + 3: ((2, 1, 256),) * 2, 6144 * CU + 1: ((4, 1, 512),) * 2, 8192 * CU: ((4, 1, 512),) * 2,
+          8192 * CU + 1: (ONE, (2, 1, 256)), 9728 * CU: (ONE, (2, 1, 256)), 9728 * CU + 2: ((4, 1, 256),) * 2,
           12288 * CU + 1: ((8, 1, 256),) * 2, 16384 * CU + 1: ((4, 1, 256),) * 2, 20480 * CU + 1: ((2, 1, 256), (8, 1, 256))}
+# other numbers of batches: (floats, batches) -> build
+OTHERS = {(256, 2): ONE, (256, 9): ONE, (2048, 3): ONE, (2049, 3): (1, 8, 64), (1025, 4): (1, 8, 64), (4096 * CU, 4): ONE,
+          (4096 * CU, 5): (2, 1, 256), (9728 * CU, 3): (2, 1, 256)}
+
+
+def build_of(mn, b):
+    """(pieces a lane, batches at once, threads)"""
+    if (mn, b) in OTHERS:
+        return OTHERS[mn, b]
+    return ONE if b == 1 and mn <= 4096 * CU else BUILDS[mn][b == 9]
 
 
 def choices(rec):
     out = []
-    for mn in list(BUILDS) + [256]:
-        for b in (2, 9, 1):
-            rc, launches = rec.of("sg_tiled_sum_reduce", rec.A, rec.B, rec.D, b, 1, mn, None)
-            assert rc == 0 and len(launches) == 1
-            out.append([mn, b, launches[0][0], launches[0][1], launches[0][2]])
+    for mn, b in [(mn, b) for mn in BUILDS for b in (2, 9, 1)] + list(OTHERS):
+        rc, launches = rec.of("sg_tiled_sum_reduce", rec.A, rec.B, rec.D, b, 1, mn, None)
+        assert rc == 0 and len(launches) == 1
+        out.append([mn, b, launches[0][0], launches[0][1], launches[0][2]])
     return out
 
 
 def test_build_of_every_size(tmp_path):
     for mn, b, kernel, grid, threads in launch_recorder.scenario(launch_recorder.build(tmp_path), "test_gpu_batch_sum_builds", "choices"):
-        pieces, batches, wide = BUILDS[mn][b == 9] if mn > 256 else (1, 1, 256)
-        if b == 1 and mn <= 2944 * CU:
-            pieces, batches, wide = 1, 1, 256
+        pieces, batches, wide = build_of(mn, b)
         assert "tiled_sum_reduce_kernel<%d, %d, %d," % (pieces, batches, wide) in kernel and threads == wide, (mn, b, kernel)
         # whole workgroups, then one-piece workgroups over what they leave
         whole = mn // (4 * wide * pieces)
