@@ -1743,8 +1743,8 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
             if (blocks < (m > 4 ? 16 : 28)) return false;    // memory channels (8 x 8192 x 16448 34.8 -> 24.7 us)
             if (blocks >= 60) tile(4, 2, 3, 1);
             else tile(2, 2, 4, 1);
-        } else if (blocks < (tiles <= 3 * cu ? 8 : (tiles <= 4 * cu ? 4 : 3))) {    // (up to three tiles a CU, 4 to 7 blocks: the record
-            return false;                            // 0.98 of the time on 204 random shapes, 1 x 8228 x 1696 4.9 us against 5.4)
+        } else if (blocks < (tiles <= 4 * cu ? 4 : 3)) {
+            return false;
         } else if (tiles <= 4 * cu) {
             if (resident(4, 4)) {}
             else if (m > 8 && tiles > 3 * cu) tile(2, 4, 3, 1);
