@@ -222,15 +222,13 @@ static const SumBuild kSums[] = {
     {16384 * kSumCus, launch_sum<8, 1, 256, 6>}, {20480 * kSumCus, launch_sum<4, 1, 256, 8>}, {0, launch_sum<2, 1, 256, 8>},
     {0, launch_sum<8, 1, 256, 6>}};
 
-// Sums that take a piece a lane out of their turn.  Where nothing is gained by asking for several batches at once - a float a lane,
-// one batch, two or three batches of up to 4096 or 2048 floats, anything up to 1024 -, the shorter code is ahead (2 x 12 x 79 1.8 us against
-// 2.3 with eight batches asked for, 3 x 16 x 113 2.3, 2.7, 5 x 10 x 78 2.5, 2.9; from nine batches on level).  And with few batches two of the
-// marks do not pay: up to four batches of 2944 to 4096 floats a CU (2 x 1217 x 664 4.7 us, 5.0 with two pieces; 1.035 times on 107
-// random sums), up to two of 8192 to 9728 (1.02).
+// Sums that take a piece a lane out of their turn: a float a lane or one batch, where nothing is gained by asking for several at
+// once, and up to four batches of 2944 to 4096 floats a CU (one behind the other 1.045 times as long with two pieces, on 109 random
+// sums; 2 x 1217 x 664 by itself 4.7 us, 5.0).  Timed by itself, a sum of two or three batches of up to 4096 or 2048 floats, or of up to
+// 1024 floats, is 0.1 to 0.5 us ahead that way too (2 x 12 x 79 1.8 us against 2.3 with eight batches asked for), but 0.75 to 0.95 times as
+// long with eight asked for where launches stand one behind the other.
 static bool one_piece_sum(size_t mn, int b) {
-    if (mn <= 1024 || (b == 2 && mn <= 4096) || (b == 3 && mn <= 2048)) return true;
-    if (b < 2 && mn <= kSums[kOnePiece].most) return true;
-    return (b <= 4 && mn > 2944 * kSumCus && mn <= 4096 * kSumCus) || (b <= 2 && mn > 8192 * kSumCus && mn <= 9728 * kSumCus);
+    return mn <= 256 || (b < 2 && mn <= kSums[kOnePiece].most) || (b <= 4 && mn > 2944 * kSumCus && mn <= 4096 * kSumCus);
 }
 
 int launch_tiled_sum_reduce(const float* A, const float* B, float* D, int b, int m, int n, hipStream_t stream) {

@@ -7,15 +7,13 @@ import torch
 CU = 256
 # floats -> (pieces a lane, batches at once, threads) at 2 and at 9 batches
 ONE = (1, 1, 256)
-BUILDS = {257: (ONE,) * 2, 1024: (ONE,) * 2, 1025: (ONE, (1, 8, 64)), 4096: (ONE, (1, 8, 64)), 4097: ((1, 8, 64),) * 2,
-          1152 * CU: ((1, 8, 64),) * 2, 1152 * CU + 1: ((2, 4, 256),) * 2, 2048 * CU: ((2, 4, 256),) * 2,
+BUILDS = {257: ((1, 8, 64),) * 2, 1152 * CU: ((1, 8, 64),) * 2, 1152 * CU + 1: ((2, 4, 256),) * 2, 2048 * CU: ((2, 4, 256),) * 2,
           2048 * CU + 1: (ONE,) * 2, 2944 * CU + 1: (ONE, (2, 1, 256)), 4096 * CU: (ONE, (2, 1, 256)), 4096 * CU + 1: (ONE,) * 2,
           5120 * CU + 3: ((2, 1, 256),) * 2, 6144 * CU + 1: ((4, 1, 512),) * 2, 8192 * CU: ((4, 1, 512),) * 2,
-          8192 * CU + 1: (ONE, (2, 1, 256)), 9728 * CU: (ONE, (2, 1, 256)), 9728 * CU + 2: ((4, 1, 256),) * 2,
+          8192 * CU + 1: ((2, 1, 256),) * 2, 9728 * CU + 2: ((4, 1, 256),) * 2,
           12288 * CU + 1: ((8, 1, 256),) * 2, 16384 * CU + 1: ((4, 1, 256),) * 2, 20480 * CU + 1: ((2, 1, 256), (8, 1, 256))}
 # other numbers of batches: (floats, batches) -> build
-OTHERS = {(256, 2): ONE, (256, 9): ONE, (2048, 3): ONE, (2049, 3): (1, 8, 64), (1025, 4): (1, 8, 64), (4096 * CU, 4): ONE,
-          (4096 * CU, 5): (2, 1, 256), (9728 * CU, 3): (2, 1, 256)}
+OTHERS = {(256, 2): ONE, (256, 9): ONE, (257, 1): ONE, (4096 * CU, 4): ONE, (4096 * CU, 5): (2, 1, 256)}
 
 
 def build_of(mn, b):
