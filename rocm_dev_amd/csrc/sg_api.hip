@@ -1723,13 +1723,19 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
     };
     // Pitches a little off a power of two put a tile's rows within 512 bytes to 1.5 KB of each other modulo the channels' period; with
     // many tiles, all at one place of K, the CUs then meet in a few channels, and the record, which starts its tiles at different
-    // places, is ahead.  Times its time on 16600, 18500, 22000, 27000 and 34000 weight rows, one launch behind the other: pitch 4128 1.25 to 1.02,
-    // 8224 1.41 to 1.14 (2 x 18500 x 8224 by itself 27.6 us against 41.6), 16448 1.24 to 1.15, and 8160, 8256 and 8288 1.18 to 1.01 but
-    // 0.97 on the last.  From 9 rows on only 4128 is behind (14 x 18500 x 8224 0.71), and at 5 to 8 rows 16448 no more.  (A map of
-    // pitches 16 to 416 bytes off the multiples of 1024 up to 24576: the others are 0.8 to 1.07.)
-    if (c.mt == 1 && tiles > 4 * cu &&
-        (b_stride == 4096 + 32 || (m <= 8 && b_stride == 8192 + 32) || (m <= 4 && b_stride == 16384 + 64) ||
-         (m <= 8 && tiles <= 7 * cu && (b_stride == 8192 - 32 || b_stride == 8192 + 64 || b_stride == 8192 + 96)))) return false;
+    // places, is ahead.  Times its time, one launch behind the other, on 9216 to 12288 weight rows and on 16600 to 34000: pitch 4128 1.00
+    // (K of 4096 1.10) and 1.25 to 1.02, 8224 1.08 to 1.01 (K of 8192 1.20) and 1.41 to 1.14 (2 x 18500 x 8224 by itself 27.6 us against
+    // 41.6), 16448 1.15 to 1.02 and 1.27 to 1.15, 8160, 8256 and 8288 1.07 to 1.00 and 1.18 to 1.01, but 0.97 on the last.  In between
+    // four waves a CU have a tile each, and the two are level.  From 9 rows on only 4128 is behind (14 x 18500 x 8224 0.71), and at 5 to 8
+    // rows 16448 no more.  8256 is behind on one to two tiles a CU as well, 1.05 to 1.15.  (Maps of pitches 16 to 416 bytes off the
+    // multiples of 1024 up to 24576, and of twelve pitches on 2048 to 57344 weight rows: the others are 0.6 to 1.07.)
+    if (c.mt == 1 && tiles > cu) {
+        const bool uneven = tiles > 2 * cu && (tiles <= 3 * cu || tiles > 4 * cu);
+        if (b_stride == 4096 + 32 && (tiles > 4 * cu || (tiles > 2 * cu && k % 256 == 0))) return false;
+        if (uneven && ((m <= 8 && b_stride == 8192 + 32) || (m <= 4 && b_stride == 16384 + 64))) return false;
+        if (uneven && m <= 8 && tiles <= 7 * cu && (b_stride == 8192 - 32 || b_stride == 8192 + 64 || b_stride == 8192 + 96)) return false;
+        if (tiles <= 2 * cu && b_stride == 8192 + 64) return false;
+    }
     if (c.mt == 1) {
         if (tiles * 2 <= cu) {                       // few tiles: only long K, on K splits
             if (!split_ok || blocks < (tiles * 5 <= cu ? 100 : 60) || (tiles * 5 > cu && tiles * 3 <= cu)) return false;
