@@ -1734,6 +1734,7 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
         if (b_stride == 4096 + 32 && (tiles > 4 * cu || (tiles > 2 * cu && k % 256 == 0))) return false;
         if (uneven && ((m <= 8 && b_stride == 8192 + 32) || (m <= 4 && b_stride == 16384 + 64))) return false;
         if (uneven && m <= 8 && tiles <= 7 * cu && (b_stride == 8192 - 32 || b_stride == 8192 + 64 || b_stride == 8192 + 96)) return false;
+        if (uneven && m <= 8 && k % 256 == 0 && b_stride == 8192 + 64) return false;    // (1 x 57344 x 8192 82 us against 94)
         if (tiles <= 2 * cu && b_stride == 8192 + 64) return false;
     }
     if (c.mt == 1) {
