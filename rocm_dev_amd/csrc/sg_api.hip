@@ -1761,10 +1761,17 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
             if ((blocks <= 10 && resident(8, 4)) || resident(8, 3)) {}
             else tile(1, 2, 3, 1);
         } else {
+            // A record of whole K blocks splits K among the waves of persistent workgroups.  It is ahead where four waves a CU begin
+            // another round of tiles that stays up to three quarters empty (33794 weight rows, K of 3072 to 9728 on rows 16 or 48 bytes
+            // further apart: 1.07 times its time at 8 rows; 50178 at 14 1.05 to 1.17), and from 5 rows on at K of 4096 to 4608 on most
+            // numbers of weight rows (8 x 38914 x 4096 on rows of 4112 28.8 us against 31.6; 40962 32.9, 31.8)
+            const bool whole = k % 256 == 0 && tiles > 8 * cu;
+            if (whole && m > 4 && blocks >= 16 && blocks <= 18) return false;
             if (blocks <= 6 && (resident(8, 4) || resident(8, 3))) {}
             else if (tiles > 12 * cu && resident(8, 3)) {}
-            else if (resident(4, 4)) {}
-            else if (m > 8) tile(1, 4, 3, 1);
+            else if (resident(4, 4)) {
+                if (whole && blocks >= 12 && (tiles - 1) % (4 * cu) < cu) return false;
+            } else if (m > 8) tile(1, 4, 3, 1);
             else {      // (a record of whole K blocks keeps the activations resident too: 0.92 of the time on 60 random shapes of 5..8 rows,
                 if (m > 4 && k % 256 == 0 && tiles <= 10 * cu) return false;     // 5 x 27638 x 15616 on rows of 15680 72 us against 89)
                 tile(1, 2, 4, 1);

@@ -61,6 +61,9 @@ RECORD_STAYS = [
     (2, 27000, 16448, 0),
     # two to three tiles a CU, whole K blocks and on one to two: 1.16, 1.08, 1.15, 1.11, 1.13, 1.12 and 1.14 times
     (8, 10240, 8192, 32), (8, 10240, 8192, 64), (1, 10240, 16448, 0), (4, 14336, 4096, 32), (8, 14336, 4096, 32), (4, 8192, 8192, 64), (1, 57344, 8192, 64),
+    # whole K blocks, where a round of tiles is begun: 1.09, 1.15, 1.11, 1.07 and 1.17 times; from 5 rows on with K of 4096 to 4608: 1.10, 1.10
+    (8, 33794, 3072, 48), (14, 35842, 4096, 16), (2, 34050, 4096, 16), (8, 33794, 3584, 16), (14, 50178, 4608, 16),
+    (8, 38914, 4096, 16), (14, 59394, 4096, 16),
     # 5..8 rows of whole K blocks, too many for the LDS: 1.24, 1.22 and 1.29 times
     (5, 27638, 15616, 64), (8, 31854, 13312, 16), (8, 28558, 16128, 64),
 ]
@@ -76,7 +79,8 @@ def test_the_record_stays_where_it_was_timed_ahead(m, n, k, pad):
                                        (2, 18500, 4112, 0), (2, 18500, 8240, 0), (2, 14336, 8224, 0), (14, 18500, 8224, 0), (8, 18500, 16448, 0),
                                        (4, 28690, 8160, 0), (4, 28690, 8256, 0), (8, 28690, 8288, 0),
                                        (8, 31854, 13328, 0), (4, 31854, 13312, 16), (8, 41300, 13312, 16),
-                                       (8, 8192, 8192, 32), (24, 8192, 8192, 64), (8, 14336, 4128, 0), (8, 10240, 16448, 0)])
+                                       (8, 8192, 8192, 32), (24, 8192, 8192, 64), (8, 14336, 4128, 0), (8, 10240, 16448, 0), (8, 33794, 2560, 16),
+                                       (8, 37890, 3072, 48), (8, 32768, 4096, 16), (2, 38914, 4096, 16), (8, 33794, 3600, 0)])
 def test_just_beyond_they_are_taken(m, n, k, pad):
     from rocm_dev_amd import api
     assert api.skinny_gemm_skinny_line_choice(m, n, k, k + pad)
