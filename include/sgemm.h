@@ -84,9 +84,9 @@ int    sg_release_workspaces(void);
  * else, nothing is allocated, and a launch that would need more than it is given returns SG_WORKSPACE_TOO_SMALL.
  *   sg_workspace_query  *bytes = what sg_skinny_gemm_auto_ws needs for the shape with the tuning table as it is now
  *                       (0 when the launch it would choose has no K split; then workspace may be NULL) to run what
- *                       sg_skinny_gemm_auto runs, bit for bit; where the kernel for rows off their 128-byte lines would
- *                       split K, less is accepted too, down to what the launch that it replaces needs (NULL, if
- *                       that has no K split), and runs what fits
+ *                       sg_skinny_gemm_auto runs, bit for bit; where that is a K split in the place of the heuristics'
+ *                       own launch (sg_skinny_gemm_choice), less is accepted too, down to what the launch that it
+ *                       replaces needs (NULL, if that has no K split), and runs what fits
  *   sg_workspace_init   zeroes the counter region (the first 64 KB) of a workspace with a kernel in stream order:
  *                       once per buffer, before its first use; every launch that completes leaves it zero again
  * workspace: device memory, 256-byte aligned, [16384 arrival counters][fp32 partials]; one buffer serves launches of
@@ -217,7 +217,7 @@ int sg_skinny_gemm_tuned_noalloc(const uint8_t* A, const uint8_t* B, void* D_bf1
  * stages are in flight.  That repeats the quantisation in every workgroup, so the library uses it only where it
  * measured faster than the two launches - m <= 8 and at least three 16-row tiles per CU (8 x 28672 x 4096: 22.5
  * against 22.8 us, 4 rows 21.0 against 23.8) - and otherwise runs the two launches itself, with the codes in a per-stream scratch buffer it
- * keeps.  sg_skinny_gemm_bf16act_choice says which (*fused) and with which record.  sg_skinny_gemm_bf16act_tuned
+ * keeps.  sg_skinny_gemm_bf16act_choice says which (*fused) and with which record, whatever the row stride.  sg_skinny_gemm_bf16act_tuned
  * always runs the fused kernel: with the given record (LDS ring, persistent_wgs_per_cu >= 1, wave_tiles 2 or 6,
  * row_tiles 1, depth 2; at most 8 streaming waves), or - engine 0 - the library's own for the shape;
  * SG_INVALID_CONFIG where the kernel does not apply. */
@@ -235,22 +235,26 @@ int sg_skinny_gemm_bf16act_choice(int m, int n, int k, SgTuning* out, int* fused
  * The eight cannot say everything a launch here depends on (persistent workgroups, resident activations,
  * the epilogue wave, the mid-batch tiles): passed back through sg_skinny_gemm they select a kernel of the
  * same ring geometry, not necessarily the one sg_skinny_gemm_auto runs.  sg_skinny_gemm_choice below
- * returns the complete record, and sg_skinny_gemm_tuned replays exactly that - but for the two kernels that no
+ * returns the complete record, and sg_skinny_gemm_tuned replays exactly that - but for the kernels that no
  * record describes, which engine = 0 replays. */
 int sg_skinny_gemm_pick(int m, int n, int k, int out[8]);
 
 /* The complete record sg_skinny_gemm_auto would launch for the shape: the tuning table's entry when
  * there is one (*from_table = 1), the built-in heuristics' otherwise (0).  from_table may be NULL.
- * Two kernels that no record describes may run in place of the heuristics' record; engine = 0 replays them, sgemm_debug.h
+ * Kernels that no record describes may run in place of the heuristics' record; engine = 0 replays them, sgemm_debug.h
  * says whether they do and on which tile, and the record, stored in the table, is what runs from then on:
+ *   up to 32 rows off their 128-byte lines (sg_debug_skinny_line_choice; b_stride no multiple of 128).  The record is the
+ *     launch that they replace - or, where they split K and that launch does not, an LDS-ring record of the same split, so that
+ *     split_k says whether a workspace is needed (k = b_stride)
  *   rows off their 128-byte lines (sg_debug_line_choice; 33 to 768 rows, k or b_stride no multiple of 128).  The record is
  *     the launch that it replaces - or, where it splits K and that launch does not, a mid-batch record of the same split on
  *     the tile nearest to its own, so that split_k says of either whether a workspace is needed (k = b_stride)
  *   wide tiles (sg_debug_wide_choice; above 128 rows).  The record is the mid-batch launch that it replaces.
  * Above 32 rows on few weight rows with a long k the record may split K in place of an unsplit one that needs no workspace.
- * That one runs where the split cannot: on a caller's smaller workspace or none, without device memory for the library's own, and
- * under capture without a caller's, so that graphs of such launches may replay side by side (the sums are added up in
- * another order there than in an eager call). */
+ * Wherever a K split stands in for a launch that needs no workspace, that launch runs where the split cannot: on a caller's smaller
+ * workspace or none, and without device memory for the library's own - and under capture without a caller's, so that graphs
+ * of such launches may replay side by side (the sums are added up in another order there than in an eager call).  Only
+ * the kernel for 33 to 768 rows off their lines keeps its split under capture, in the workspace of the capture stream. */
 int sg_skinny_gemm_choice(int m, int n, int k, SgTuning* out, int* from_table);
 
 /* Per-shape tuning table - the run-time form of what the reference's grid search produces: there the

@@ -828,7 +828,8 @@ static int launch_sparse_engine(const Config& c, StreamArgs a, const uint8_t* me
 // Row tiles, waves, ring slots and K splits of sparse24_gemm_kernel for up to 32 rows, as read off timings of 1, 2 and 4 of the
 // first two, 2..4 slots and up to eight splits on 139 random shapes (1..32 rows, n of 64..32768, k of 512..28672; every side
 // timed in turn, cold weights): 0.885 of the time of what ran before in the geometric mean, the best of them 0.878, none behind
-// by more than 3 %; on 169 further shapes whose launch it changes 0.83.  Few tiles and a long K: splits until the CUs have one each (14 x 198 x 24576 12.0 -> 7.2 us,
+// by more than 3 %, of which the rule takes up to six splits; on 250 other shapes 0.92 eagerly, where the short ones are the host's time, and
+// 0.95 recorded, without splits, at most 5 % behind.  Few tiles and a long K: splits until the CUs have one each (14 x 198 x 24576 12.0 -> 7.2 us,
 // 25 x 930 x 24576 17.7 -> 9.4, 19 x 1378 x 27776 20.5 -> 13.9); a K too short for one wave's ring on two of them (9 x 328 x 6144
 // 5.74 -> 4.67, 2 x 2308 x 7168 6.09 -> 4.84); 17..32 rows on one to two tiles per CU on 32-row tiles, which share the
 // activations (23 x 7542 x 10240 18.8 -> 15.2), or, up to four stages, on one wave (24 x 4464 x 1024 6.41 -> 3.83); beyond two
@@ -1587,8 +1588,8 @@ static bool line_config(const Config& record, const Config* wide, double wide_us
 // model puts first, 5 % ahead of the record.  (pick_mid's own splits go to four, with a third of a weight row's bytes of partials
 // at most and K blocks of 128 only: 1061 x 128 x 6128 ran on 34 workgroups.)  Microseconds with every CU busy, fitted to
 // timings of nine tiles with up to 32 splits on 190 random shapes (129..2048 rows, 128..12000 weight rows, K of 1600 to 32768), rows of
-// whole lines and others: 5 % off in the root mean square.  On 60 other shapes that the rule takes, padded rows and factors among
-// them, 0.65 of the time before in the geometric mean, none behind (with the sum of launch_mid_reduce for few workgroups): 1405 x 184
+// whole lines and others: 5 % off in the root mean square.  On 250 other shapes that the rule takes, padded rows and factors among
+// them, 0.68 of the time before in the geometric mean, three behind by more than 3 % (2022 x 1820 x 8128 by 11): 1405 x 184
 // x 28048 109 -> 33 us, 1257 x 178 x 30144 100 -> 29, 1635 x 626 x 19056 108 -> 51, 1817 x 1146 x 18160 173 -> 82, 915 x 188 x 8640
 // 27.5 -> 12.8, 295 x 144 x 4224 12.7 -> 8.8, 822 x 5518 x 14880 141 -> 127.  Rows off their lines up to 768 rows are
 // line_config's.  Where the record stays ahead - one round of tiles that fills the CUs, K below about 3000 - the model says so.
@@ -1660,7 +1661,7 @@ static bool deep_split_config(const Config& record, int m, int n, int k, int cu_
 // Microseconds fitted to 110 random shapes (33..256 rows, 128..5000 weight rows, K of 512..32768) timed with every split: 3.3 for
 // a launch, 0.17 or 0.25 a stage of 256 bytes of K, 1.23 times that with K off the 128-byte lines, 0.5 and 0.37 a split.  Of those
 // shapes it takes 38 and of others 100 were timed, padded rows and factors among them: 0.78 of the time before in the geometric
-// mean, two behind by more than 3 % (4): 40 x 192 x 13056 12.4 -> 7.2 us,
+// mean, two behind by more than 3 % (4), of 250 more 0.76, one (3.7): 40 x 192 x 13056 12.4 -> 7.2 us,
 // 130 x 160 x 11904 11.5 -> 7.6, 90 x 464 x 10144 12.9 -> 8.5, 49 x 570 x 6400 7.7 -> 6.6; below about 4000 of K an unsplit
 // launch stays ahead.
 static double ring_split_us(int k, int rg, int sk, double fill) {
@@ -1694,9 +1695,12 @@ static bool ring_split_config(const Config& record, int m, int n, int k, int cu_
 
 // Up to 32 activation rows and weight rows off their lines (a row stride that 128 does not divide): the skinny kernels of
 // sg_skinny_line_kernel.h in place of heuristic_config's record.  Which of them was read off timings of all their builds
-// (waves, ring slots, row tiles, K splits) against that record on 510 random shapes, n of 128..65536, K of 272..32768, 236 of
-// which the rule takes: 0.88 of the time before in the geometric mean (the best build of each shape: 0.87), and seven behind by
-// more than 2 %, at most 6 %.  32 x 32768 x 4112 35.7 -> 26.7 us, 1 x 16384 x 4112 15.5 -> 13.8, 13 x 20660 x 9664 57.5 -> 35.6,
+// (waves, ring slots, row tiles, K splits) against that record on 510 random shapes, n of 128..65536, K of 272..32768: 0.89 of the time
+// before in the geometric mean on the 231 that it took, at most 3.4 % behind.  Denser samples of single ranges, timed by themselves and one
+// behind the other, then found where the record is ahead (skinny_record_stays and the early returns below).  Of others that it takes
+// now, 300 run in 0.90 of the time before, four more than 3 % behind eagerly (at most 5.6) and seven recorded (at most 8); 300 of whole K
+// blocks on padded rows, whose records are the better ones, in 0.93, nineteen more than 3 % behind (at most 13).
+// 32 x 32768 x 4112 35.7 -> 26.7 us, 1 x 16384 x 4112 15.5 -> 13.8, 13 x 20660 x 9664 57.5 -> 35.6,
 // 5 x 39438 x 4016 35.6 -> 28.1, 28 x 13116 x 6960 25.0 -> 20.7, 5 x 2434 x 21584 18.0 -> 13.5, 1 x 8522 x 2832 7.3 -> 6.8.
 // What it leaves alone - weights of a megabyte or two, two K blocks, few tiles with a K below about 7000 at up to 16 rows - is
 // bound by the launch, or runs as fast there on its deeper rings.  Beyond those ranges it was not timed and is not taken.

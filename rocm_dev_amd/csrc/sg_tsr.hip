@@ -209,6 +209,8 @@ static int launch_sum(const float* A, const float* B, float* D, int b, size_t mn
 //     8192) 96.4 -> 83.8.  In between two such marks shorter workgroups are ahead: 12 x 78 x 14953 20.4, 22-24 with longer ones;
 //   * beyond 20480 floats a CU the length of a stream's visit decides, but not with up to four batches, whose few streams
 //     do better on more workgroups: 2 x 5061 x 4226 73.6 -> 68.3, 1 x 157034 x 89 32.7 -> 29.7; 5 x 6246 x 2092 level.
+// 250 other random sums, one launch behind the other: 0.74 of the time before in the geometric mean, nine more than 3 % behind (7 x 53 x
+// 14392 9.0 -> 9.9, 1 x 2519 x 869 6.2 -> 6.8, whose launch is the one before).
 struct SumBuild {
     size_t most;
     int (*launch)(const float*, const float*, float*, int, size_t, hipStream_t);
