@@ -1729,15 +1729,17 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
     // many tiles, all at one place of K, the CUs then meet in a few channels, and the record, which starts its tiles at different
     // places, is ahead.  Times its time, one launch behind the other, on 9216 to 12288 weight rows and on 16600 to 34000: pitch 4128 1.00
     // (K of 4096 1.10) and 1.25 to 1.02, 8224 1.08 to 1.01 (K of 8192 1.20) and 1.41 to 1.14 (2 x 18500 x 8224 by itself 27.6 us against
-    // 41.6), 16448 1.15 to 1.02 and 1.27 to 1.15, 8160, 8256 and 8288 1.07 to 1.00 and 1.18 to 1.01, but 0.97 on the last.  In between
+    // 41.6), 16448 1.15 to 1.02 and 1.27 to 1.15, 8160, 8256 and 8288 1.07 to 1.00 and 1.18 to 1.01, but 0.97 on the last, as 4128 is with
+    // a K below its pitch (2 x 47816 x 4000 46.6 us against 41.4).  In between
     // four waves a CU have a tile each, and the two are level.  From 9 rows on only 4128 is behind (14 x 18500 x 8224 0.71), and at 5 to 8
     // rows 16448 no more.  8256 is behind on one to two tiles a CU as well, 1.05 to 1.15.  (Maps of pitches 16 to 416 bytes off the
     // multiples of 1024 up to 24576, and of twelve pitches on 2048 to 57344 weight rows: the others are 0.6 to 1.07.)
     if (c.mt == 1 && tiles > cu) {
         const bool uneven = tiles > 2 * cu && (tiles <= 3 * cu || tiles > 4 * cu);
-        if (b_stride == 4096 + 32 && (tiles > 4 * cu || (tiles > 2 * cu && k % 256 == 0))) return false;
+        if (b_stride == 4096 + 32 && tiles <= 7 * cu && (tiles > 4 * cu || (tiles > 2 * cu && k % 256 == 0))) return false;
+        if (b_stride == 4096 + 32 && k > 4096 && tiles > 7 * cu && (m <= 8 || tiles <= 12 * cu)) return false;
         if (uneven && ((m <= 8 && b_stride == 8192 + 32) || (m <= 4 && b_stride == 16384 + 64))) return false;
-        if (uneven && m <= 8 && tiles <= 7 * cu && (b_stride == 8192 - 32 || b_stride == 8192 + 64 || b_stride == 8192 + 96)) return false;
+        if (uneven && m <= 8 && tiles <= 6 * cu && (b_stride == 8192 - 32 || b_stride == 8192 + 64 || b_stride == 8192 + 96)) return false;
         if (uneven && m <= 8 && k % 256 == 0 && b_stride == 8192 + 64) return false;    // (1 x 57344 x 8192 82 us against 94)
         if (tiles <= 2 * cu && b_stride == 8192 + 64) return false;
     }
@@ -1770,14 +1772,14 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
             // further apart: 1.07 times its time at 8 rows; 50178 at 14 1.05 to 1.17), and from 5 rows on at K of 4096 to 4608 on most
             // numbers of weight rows (8 x 38914 x 4096 on rows of 4112 28.8 us against 31.6; 40962 32.9, 31.8)
             const bool whole = k % 256 == 0 && tiles > 8 * cu;
-            if (whole && m > 4 && blocks >= 16 && blocks <= 18) return false;
+            if (whole && m > 4 && (blocks == 16 || blocks == 18)) return false;
             if (blocks <= 6 && (resident(8, 4) || resident(8, 3))) {}
             else if (tiles > 12 * cu && resident(8, 3)) {}
             else if (resident(4, 4)) {
                 if (whole && blocks >= 12 && (tiles - 1) % (4 * cu) < cu) return false;
             } else if (m > 8) tile(1, 4, 3, 1);
             else {      // (a record of whole K blocks keeps the activations resident too: 0.92 of the time on 60 random shapes of 5..8 rows,
-                if (m > 4 && k % 256 == 0 && tiles <= 10 * cu) return false;     // 5 x 27638 x 15616 on rows of 15680 72 us against 89)
+                if (m > 4 && k % 256 == 0 && tiles <= 9 * cu) return false;      // 5 x 27638 x 15616 on rows of 15680 72 us against 89)
                 tile(1, 2, 4, 1);
             }
         }
@@ -1806,7 +1808,8 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
         } else {
             // four waves a CU find four tiles at once: just beyond that the record is ahead, to five and a half
             // (42 random shapes 0.91 of the time: 20 x 16452 x 2384 10.9 us against 13.3, 21 x 16956 x 2720 11.2 against 14.3)
-            if (blocks > 7 && blocks <= 11 && tiles * 2 <= 11 * cu) return false;
+            // - but with eleven whole K blocks (30 x 22458 x 2816 21.4 us against 16.2)
+            if (blocks > 7 && blocks <= 11 && k != 11 * 256 && tiles * 2 <= 11 * cu) return false;
             if (blocks <= 7 && resident(8, 3)) {}
             else if (resident(4, 4)) {}
             else tile(1, 4, 3, 1);
@@ -1817,20 +1820,22 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
     return true;
 }
 
-// Records that skinny_line_config's kernels do not replace, wherever their rows lie: those of 17..32 rows with three K splits (in
-// the place of two or four: on 70 random shapes of 1030 to 1350 weight rows 0.94 of the time with two, 20 x 1156 x 28608 12.8 us against
+// Records of 17..32 rows that skinny_line_config's kernels do not replace, wherever their rows lie: those with three K splits (in the
+// place of two or four: on 70 random shapes of 1030 to 1350 weight rows 0.94 of the time with two, 20 x 1156 x 28608 12.8 us against
 // 14.9; of fewer rows 0.99 of it with four on 13) and those with the activations in the waves' registers (of K from 3072 to 4096 on
 // rows 16 to 80 bytes further apart, 41 random shapes: 0.87 of the time, 23 x 10462 x 4096 on rows of 4112 0.86, 32 x 35948 x 3072 on
-// rows of 3136 0.68).
-static bool skinny_record_stays(const Config& record) {
-    return record.split_k == 3 || (record.engine == ENGINE_LDS && (record.wavetile & 3) == 3);
+// rows of 3136 0.68) - but on seven to eight tiles a CU, where each of eight would have one (22 x 31862 x 4096 27.6 us against 25.1).
+static bool skinny_record_stays(const Config& record, int m, int n, int cu_count) {
+    if (m <= 16) return false;
+    const int tiles = (n + 15) / 16;
+    return record.split_k == 3 || (record.engine == ENGINE_LDS && (record.wavetile & 3) == 3 && (tiles <= 7 * cu_count || tiles > 8 * cu_count));
 }
 
 // What stands in for heuristic_config's record, if anything does: a wide tile, a kernel for rows off their lines or a launch of the
 // record's kind with more K splits.
 static bool stand_in_config(const Config& record, int m, int n, int k, int b_stride, bool factors, int cu_count, const Workspace* fixed_ws,
                             Config* out) {
-    if (m <= 32) return !skinny_record_stays(record) && skinny_line_config(m, n, k, b_stride, cu_count, out);
+    if (m <= 32) return !skinny_record_stays(record, m, n, cu_count) && skinny_line_config(m, n, k, b_stride, cu_count, out);
     double wide_us = 0;
     const bool wide = wide_config(record, m, n, k, b_stride, factors, cu_count, fixed_ws, out, &wide_us);
     Config line;

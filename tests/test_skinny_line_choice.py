@@ -80,7 +80,8 @@ def test_the_record_stays_where_it_was_timed_ahead(m, n, k, pad):
                                        (4, 28690, 8160, 0), (4, 28690, 8256, 0), (8, 28690, 8288, 0),
                                        (8, 31854, 13328, 0), (4, 31854, 13312, 16), (8, 41300, 13312, 16),
                                        (8, 8192, 8192, 32), (24, 8192, 8192, 64), (8, 14336, 4128, 0), (8, 10240, 16448, 0), (8, 33794, 2560, 16),
-                                       (8, 37890, 3072, 48), (8, 32768, 4096, 16), (2, 38914, 4096, 16), (8, 33794, 3600, 0)])
+                                       (8, 37890, 3072, 48), (8, 32768, 4096, 16), (2, 38914, 4096, 16), (8, 33794, 3600, 0), (30, 22458, 2816, 16),
+                                       (14, 14698, 8192, 16), (2, 47816, 4000, 128), (8, 54274, 4352, 16), (22, 31862, 4096, 16), (8, 39590, 15360, 80)])
 def test_just_beyond_they_are_taken(m, n, k, pad):
     from rocm_dev_amd import api
     assert api.skinny_gemm_skinny_line_choice(m, n, k, k + pad)
