@@ -1593,10 +1593,14 @@ static bool line_config(const Config& record, const Config* wide, double wide_us
 // x 28048 109 -> 33 us, 1257 x 178 x 30144 100 -> 29, 1635 x 626 x 19056 108 -> 51, 1817 x 1146 x 18160 173 -> 82, 915 x 188 x 8640
 // 27.5 -> 12.8, 295 x 144 x 4224 12.7 -> 8.8, 822 x 5518 x 14880 141 -> 127.  Rows off their lines up to 768 rows are
 // line_config's.  Where the record stays ahead - one round of tiles that fills the CUs, K below about 3000 - the model says so.
-struct DeepSplitModel {     // (of one tile; a choice evaluates it some hundred times per call)
+// The search is host time of every launch above 128 rows, also of those that it leaves alone: on 390 random shapes of whole blocks
+// above 256 rows that launch as many kernels without it 0.07 us a call in the mean, 0.16 in nine of ten; 0.14 and 0.54 with 64-bit
+// counts and every split of every tile looked at.
+struct DeepSplitModel {     // (of one tile)
     double stage_us, split_us, first_us, round_us, part, per_cu;
-    int blocks, cu_count;
-    DeepSplitModel(int k, int bn, int bm, int cus) : per_cu(1.0 / cus), blocks((k + 127) / 128), cu_count(cus) {
+    int blocks;
+    unsigned cu_count;
+    DeepSplitModel(int k, int bn, int bm, int cus) : per_cu(1.0 / cus), blocks((k + 127) / 128), cu_count((unsigned)cus) {
         const bool lines = k % 128 == 0;
         stage_us = lines ? (0.232 / 128) * bn + (0.247 / 128) * bm + (0.12 / 16384) * bn * bm
                          : (0.458 / 128) * bn + (0.384 / 128) * bm + (0.073 / 16384) * bn * bm;
@@ -1605,14 +1609,20 @@ struct DeepSplitModel {     // (of one tile; a choice evaluates it some hundred 
         round_us = lines ? 1.0 : 0.0;
         part = lines ? 0.87 : 0.84;
     }
-    double us(long of_m_n, int sk) const {
-        const long wgs = of_m_n * sk;
-        const int full = wgs < cu_count ? 0 : (int)(wgs / cu_count);
-        const long rest = wgs - (long)full * cu_count;
+    double us(unsigned of_m_n, int sk) const {     // (32-bit: at most 6016 tiles of up to 16 splits)
+        const unsigned wgs = of_m_n * (unsigned)sk;
+        const unsigned full = wgs < cu_count ? 0 : wgs / cu_count;
+        const unsigned rest = wgs - full * cu_count;
         const double stages = (double)((unsigned)(blocks + sk - 1) / (unsigned)sk);
         const double us = ((double)full + (rest ? part + (1.0 - part) * (double)rest * per_cu : 0.0)) * stages * stage_us +
                           (round_us > 0 ? 3.5 + (double)(full + (rest ? 1 : 0)) : 4.2);
         return sk > 1 ? us + first_us + split_us * (double)wgs : us;
+    }
+    // what none of 2..most splits is below: an even share of all stages, or one workgroup's, and the partials
+    double least_us(unsigned of_m_n, int most) const {
+        const double even = (double)of_m_n * per_cu, sum = split_us * (double)of_m_n, stages_us = blocks * stage_us;
+        const double sk = std::max(2.0, std::min((double)most, std::min(part / even, std::sqrt(part * stages_us / sum))));
+        return std::max(even, part / sk) * stages_us + sum * sk + (round_us > 0 ? 4.5 : 4.2) + first_us;
     }
 };
 
@@ -1626,15 +1636,17 @@ static bool deep_split_config(const Config& record, int m, int n, int k, int cu_
     const int own_bn = 8 * record.rg * record.waves;
     const DeepSplitModel own(k, own_bn, 32 * record.mt, cu_count);
     // (ahead of a record that splits already by less than 12 %, it was behind as often: 554 x 346 x 16000 16.7 against 18.4)
-    double best = (record.split_k > 1 ? 0.88 : 0.95) * own.us((long)((n + own_bn - 1) / own_bn) * ((m + 32 * record.mt - 1) / (32 * record.mt)), record.split_k);
+    double best = (record.split_k > 1 ? 0.88 : 0.95) * own.us((unsigned)((n + own_bn - 1) / own_bn) * (unsigned)((m + 32 * record.mt - 1) / (32 * record.mt)), record.split_k);
     bool found = false;
     Config c{};
     for (const Tile& t : tiles) {
         const int bn = 8 * t.waves * t.rg, bm = 32 * t.mt;
         if (k % 128 != 0 && t.waves == 4 && t.rg == 4) continue;    // not built with part of a block at the end of K
-        const long of_m_n = (long)((n + bn - 1) / bn) * ((m + bm - 1) / bm);
+        const unsigned of_m_n = (unsigned)((n + bn - 1) / bn) * (unsigned)((m + bm - 1) / bm);
+        if (of_m_n > (unsigned)cu_count) continue;
         const DeepSplitModel model(k, bn, bm, cu_count);
-        const int most = (int)std::min<long>(std::min(16, blocks / 4), 2L * cu_count / of_m_n);
+        const int most = std::min(std::min(16, blocks / 4), (int)(2u * (unsigned)cu_count / of_m_n));
+        if (model.least_us(of_m_n, most) > best * (1 + 1e-9)) continue;
         for (int sk = 2; sk <= most; sk++) {
             // (kMaxPartialBytes holds any such split)
             if (fixed_ws && ((size_t)(of_m_n * sk) * bn * bm * 4 > fixed_ws->partial_bytes || (size_t)of_m_n > fixed_ws->n_counters)) break;
