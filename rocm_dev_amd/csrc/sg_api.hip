@@ -852,11 +852,25 @@ static void pick_sparse_tile(Config& c, int m, int tiles16, int blocks, bool met
     } else if (c.mt == 2) {
         // three workgroups of 16-row tiles on a CU, or two of 32-row tiles - and two of either where the metadata comes by whole
         // lines, whose ring takes 4 KB of LDS more (28 x 10414 x 1024 5.20 us on 32-row tiles, 6.76 on 16; 25 x 9984 x 10240 25.1, 28.2)
-        c.rg = !meta_lines && (tiles16 + 3 * cu - 1) / (3 * cu) <= (tiles16 + 4 * cu - 1) / (4 * cu) ? 1 : 2;
+        // Beyond four tiles per CU only up to fifteen stages: with more, and just beyond four, 32-row tiles - on two waves from sixteen stages
+        // on - are ahead, as they read the activations half as often (32 x 20120 x 13440 56.5 us, 67.4 on 16 rows; 31 x 24148 x 22144
+        // 90, 112; 152 random shapes 0.88 of the time)
+        const bool long_k = tiles16 > 4 * cu && (blocks >= 16 || tiles16 * 2 <= 9 * cu);
+        c.rg = !meta_lines && !long_k && (tiles16 + 3 * cu - 1) / (3 * cu) <= (tiles16 + 4 * cu - 1) / (4 * cu) ? 1 : 2;
         c.waves = c.rg == 2 && blocks >= 16 ? 2 : 1;
     } else {
         if (m > 8 ? tiles16 > 4 * cu : tiles16 >= 4 * cu && (m > 4 || blocks > 2 || tiles16 > 6 * cu)) c.rg = 2;
         c.waves = 1;
+        // 9..16 rows whose activations do not stay in LDS (below): two waves on 32-row tiles are ahead where a round of one-wave workgroups
+        // is begun - beyond three tiles per CU, and beyond six, where those found a third round - and from 28 stages on, where the
+        // metadata comes by whole lines between three and a half and six tiles per CU (15 x 27430 x 23808 86 us, 117; 16 x 14064 x
+        // 21248 41, 48; 160 random shapes 0.89 of the time)
+        if (m > 8 && (meta_lines ? tiles16 <= 6 * cu && (tiles16 * 2 > 7 * cu || (tiles16 > 3 * cu && blocks >= 36))
+                                 : tiles16 > 3 * cu && (tiles16 <= 4 * cu || tiles16 > 6 * cu || blocks >= 28)))
+            c.rg = c.waves = 2;
+        // up to 8 rows beyond six tiles per CU as well, but level there at 5 to 8 where the metadata does not come by whole lines
+        // (6 x 28004 x 24576 78.7 us, 100; 2 x 27050 x 20480 58.5, 64.3)
+        if (m <= 8 && tiles16 > 6 * cu && blocks >= 16 && (m <= 4 || meta_lines)) c.rg = c.waves = 2;
     }
     c.split_k = split ? std::max(1, std::min(cu / tiles16, most)) : 1;
     c.depth = 4;
