@@ -1737,7 +1737,7 @@ constexpr int kSkinnyLineMaxN = 65536, kSkinnyLineMaxK = 32768;
 static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, Config* out) {
     if (m > 32 || k <= 256 || k > kSkinnyLineMaxK || n < 128 || n > kSkinnyLineMaxN || b_stride % 128 == 0) return false;
     const int tiles = (n + 15) / 16, blocks = (k + 255) / 256, cu = cu_count;
-    const bool split_ok = k % 128 != 0;
+    const bool split_ok = k % 128 != 0, whole_k = k % 256 == 0;
     Config c{};
     c.engine = ENGINE_LDS;
     c.line = true;
@@ -1797,17 +1797,20 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
             // another round of tiles that stays up to three quarters empty (33794 weight rows, K of 3072 to 9728 on rows 16 or 48 bytes
             // further apart: 1.07 times its time at 8 rows; 50178 at 14 1.05 to 1.17), and from 5 rows on at K of 4096 to 4608 on most
             // numbers of weight rows (8 x 38914 x 4096 on rows of 4112 28.8 us against 31.6; 40962 32.9, 31.8)
-            const bool whole = k % 256 == 0 && tiles > 8 * cu;
+            const bool whole = whole_k && tiles > 8 * cu;
             if (whole && m > 4 && (blocks == 16 || blocks == 18)) return false;
             if (blocks <= 6 && (resident(8, 4) || resident(8, 3))) {}
             else if (tiles > 12 * cu && resident(8, 3)) {}
             else if (resident(4, 4)) {
-                if (whole && blocks >= 12 && (tiles - 1) % (4 * cu) < cu) return false;
+                if (whole && (blocks >= 12 || (blocks == 11 && tiles <= 9 * cu)) && (tiles - 1) % (4 * cu) < cu) return false;
+            } else if (whole_k && tiles <= (m > 8 ? (b_stride % 128 == 64 || blocks <= 34 ? 12 : 11) : 9) * cu && tiles > (m > 8 ? 8 : 6) * cu) {
+                // the record keeps the activations resident, or in registers, and here a second round of workgroups is begun: 0.92 of the
+                // time on 60 random shapes of 5..8 rows (5 x 27638 x 15616 on rows of 15680 72 us against 89), 0.90 on 16 of up to 4
+                // (4 x 30596 x 28928 140, 164), 0.95 on 285 of 9..16 (14 x 36870 x 6400 on rows of 6448 39.5, 53;
+                // beyond eleven tiles a CU level with more than 34 blocks, but on pitches of half a line)
+                return false;
             } else if (m > 8) tile(1, 4, 3, 1);
-            else {      // (a record of whole K blocks keeps the activations resident too: 0.92 of the time on 60 random shapes of 5..8 rows,
-                if (m > 4 && k % 256 == 0 && tiles <= 9 * cu) return false;      // 5 x 27638 x 15616 on rows of 15680 72 us against 89)
-                tile(1, 2, 4, 1);
-            }
+            else tile(1, 2, 4, 1);
         }
     } else {                                         // the activations weigh as much: taller tiles share them
         if (tiles <= cu) {

@@ -66,6 +66,8 @@ RECORD_STAYS = [
     (8, 38914, 4096, 16), (14, 59394, 4096, 16),
     # 5..8 rows of whole K blocks, too many for the LDS: 1.24, 1.22 and 1.29 times
     (5, 27638, 15616, 64), (8, 31854, 13312, 16), (8, 28558, 16128, 64),
+    # whole K blocks too many for the LDS, a second round of workgroups: 1.35, 1.23, 1.18, 1.18 and 1.17 times; eleven of them: 1.09
+    (14, 36870, 6400, 48), (16, 35794, 7168, 112), (4, 30596, 28928, 64), (2, 28002, 24832, 16), (11, 46854, 6400, 64), (2, 33168, 2816, 16),
 ]
 
 
@@ -81,7 +83,8 @@ def test_the_record_stays_where_it_was_timed_ahead(m, n, k, pad):
                                        (8, 31854, 13328, 0), (4, 31854, 13312, 16), (8, 41300, 13312, 16),
                                        (8, 8192, 8192, 32), (24, 8192, 8192, 64), (8, 14336, 4128, 0), (8, 10240, 16448, 0), (8, 33794, 2560, 16),
                                        (8, 37890, 3072, 48), (8, 32768, 4096, 16), (2, 38914, 4096, 16), (8, 33794, 3600, 0), (30, 22458, 2816, 16),
-                                       (14, 14698, 8192, 16), (2, 47816, 4000, 128), (8, 54274, 4352, 16), (22, 31862, 4096, 16), (8, 39590, 15360, 80)])
+                                       (14, 14698, 8192, 16), (2, 47816, 4000, 128), (8, 54274, 4352, 16), (22, 31862, 4096, 16), (8, 39590, 15360, 80),
+                                       (14, 32768, 6400, 48), (14, 51202, 6400, 48), (14, 46000, 9216, 16), (4, 22000, 24832, 16), (4, 38000, 24832, 16), (2, 38000, 2816, 16)])
 def test_just_beyond_they_are_taken(m, n, k, pad):
     from rocm_dev_amd import api
     assert api.skinny_gemm_skinny_line_choice(m, n, k, k + pad)
