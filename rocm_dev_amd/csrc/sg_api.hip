@@ -1763,11 +1763,20 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
     if (c.mt == 1 && tiles > cu) {
         const bool uneven = tiles > 2 * cu && (tiles <= 3 * cu || tiles > 4 * cu);
         if (b_stride == 4096 + 32 && tiles <= 7 * cu && (tiles > 4 * cu || (tiles > 2 * cu && k % 256 == 0))) return false;
-        if (b_stride == 4096 + 32 && k > 4096 && tiles > 7 * cu && (m <= 8 || tiles <= 12 * cu)) return false;
+        if (b_stride == 4096 + 32 && k >= 4096 && tiles > 7 * cu && (m <= 8 || tiles <= 12 * cu)) return false;
         if (uneven && ((m <= 8 && b_stride == 8192 + 32) || (m <= 4 && b_stride == 16384 + 64))) return false;
         if (uneven && m <= 8 && tiles <= 6 * cu && (b_stride == 8192 - 32 || b_stride == 8192 + 64 || b_stride == 8192 + 96)) return false;
         if (uneven && m <= 8 && k % 256 == 0 && b_stride == 8192 + 64) return false;    // (1 x 57344 x 8192 82 us against 94)
         if (tiles <= 2 * cu && b_stride == 8192 + 64) return false;
+        // of whole K blocks more such pitches: 40 random shapes 0.91 of the time on the record (7 x 21762 x 3584 on rows of 3616 0.86,
+        // 16 x 21804 x 4608 on rows of 4640 19.3 us against 21.9)
+        if (whole_k && tiles > 2 * cu && (b_stride == 3584 + 32 || b_stride == 4608 + 32 || b_stride == 5376 + 80 || b_stride == 8192 + 32 ||
+                                          (m > 8 && (b_stride == 8192 + 64 || b_stride == 8192 + 96))))
+            return false;
+        // Pitches of half a line: every other row begins on its line, and the ring asks for a quarter more instead of half.  With the
+        // activations resident the two are level in the mean (276 random shapes of whole K blocks 0.997), but 62 of them were more
+        // than 3 % behind here, up to 19 (6 x 37880 x 5376 on rows of 5440), by their pitch.
+        if (whole_k && tiles > 2 * cu && b_stride % 128 == 64 && ((m <= 8 && tiles > 12 * cu) || resident(4, 4))) return false;
     }
     if (c.mt == 1) {
         if (tiles * 2 <= cu) {                       // few tiles: only long K, on K splits
@@ -1835,6 +1844,8 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
             else if (blocks < 20 && tiles <= 3 * cu) tile(1, 2, 4, 1);
             else tile(2, 4, 3, 1);
         } else {
+            // (pitches of half a line, see above: 31 random shapes 0.97 of the time on the record)
+            if (whole_k && b_stride % 128 == 64 && blocks >= 12 && tiles > 8 * cu && tiles <= 12 * cu) return false;
             // four waves a CU find four tiles at once: just beyond that the record is ahead, to five and a half
             // (42 random shapes 0.91 of the time: 20 x 16452 x 2384 10.9 us against 13.3, 21 x 16956 x 2720 11.2 against 14.3)
             // - but with eleven whole K blocks (30 x 22458 x 2816 21.4 us against 16.2)

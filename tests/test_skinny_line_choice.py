@@ -68,6 +68,9 @@ RECORD_STAYS = [
     (5, 27638, 15616, 64), (8, 31854, 13312, 16), (8, 28558, 16128, 64),
     # whole K blocks too many for the LDS, a second round of workgroups: 1.35, 1.23, 1.18, 1.18 and 1.17 times; eleven of them: 1.09
     (14, 36870, 6400, 48), (16, 35794, 7168, 112), (4, 30596, 28928, 64), (2, 28002, 24832, 16), (11, 46854, 6400, 64), (2, 33168, 2816, 16),
+    # whole K blocks on further pitches: 1.16, 1.13, 1.13, 1.45, 1.24, 1.14 and 1.29 times; of half a line: 1.19, 1.18, 1.07, 1.04
+    (7, 21762, 3584, 32), (16, 21804, 4608, 32), (13, 63444, 5376, 80), (15, 35680, 8192, 32), (15, 49302, 8192, 64), (9, 46058, 8192, 96),
+    (2, 38000, 4096, 32), (6, 37880, 5376, 64), (4, 53472, 16128, 64), (7, 56582, 19200, 64), (24, 40000, 6400, 64),
 ]
 
 
@@ -84,7 +87,8 @@ def test_the_record_stays_where_it_was_timed_ahead(m, n, k, pad):
                                        (8, 8192, 8192, 32), (24, 8192, 8192, 64), (8, 14336, 4128, 0), (8, 10240, 16448, 0), (8, 33794, 2560, 16),
                                        (8, 37890, 3072, 48), (8, 32768, 4096, 16), (2, 38914, 4096, 16), (8, 33794, 3600, 0), (30, 22458, 2816, 16),
                                        (14, 14698, 8192, 16), (2, 47816, 4000, 128), (8, 54274, 4352, 16), (22, 31862, 4096, 16), (8, 39590, 15360, 80),
-                                       (14, 32768, 6400, 48), (14, 51202, 6400, 48), (14, 46000, 9216, 16), (4, 22000, 24832, 16), (4, 38000, 24832, 16), (2, 38000, 2816, 16)])
+                                       (14, 32768, 6400, 48), (14, 51202, 6400, 48), (14, 46000, 9216, 16), (4, 22000, 24832, 16), (4, 38000, 24832, 16), (2, 38000, 2816, 16),
+                                       (7, 21762, 3584, 48), (16, 21804, 4608, 48), (15, 49302, 8192, 112), (6, 37880, 5392, 48), (12, 23374, 8960, 64), (24, 30000, 6400, 64)])
 def test_just_beyond_they_are_taken(m, n, k, pad):
     from rocm_dev_amd import api
     assert api.skinny_gemm_skinny_line_choice(m, n, k, k + pad)
