@@ -1794,6 +1794,8 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
         } else if (blocks < (tiles <= 4 * cu ? 4 : 3)) {
             return false;
         } else if (tiles <= 4 * cu) {
+            // (21 random shapes of whole K blocks, up to 4 rows: 0.98 of the time on the record, 2 x 12000 x 1024 0.95)
+            if (whole_k && m <= 4 && (blocks == 4 || (blocks == 5 && tiles <= 3 * cu))) return false;
             if (resident(4, 4)) {}
             else if (m > 8 && tiles > 3 * cu) tile(2, 4, 3, 1);
             else if (tiles <= 3 * cu) tile(1, 1, 4, 1);
@@ -1840,6 +1842,7 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
         } else if (blocks < 3) {
             return false;
         } else if (tiles <= 4 * cu) {
+            if (blocks == 4 || blocks == 5 || (whole_k && blocks == 6)) return false;       // (few K blocks, see below)
             if (resident(4, 4)) {}
             else if (blocks < 20 && tiles <= 3 * cu) tile(1, 2, 4, 1);
             else tile(2, 4, 3, 1);
@@ -1850,6 +1853,11 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
             // (42 random shapes 0.91 of the time: 20 x 16452 x 2384 10.9 us against 13.3, 21 x 16956 x 2720 11.2 against 14.3)
             // - but with eleven whole K blocks (30 x 22458 x 2816 21.4 us against 16.2)
             if (blocks > 7 && blocks <= 11 && k != 11 * 256 && tiles * 2 <= 11 * cu) return false;
+            // Few K blocks, a tile's extra pair of lines for a part of one among them: the record is 2 to 10 % ahead with three of them
+            // (29 x 29346 x 704 7.0 us against 7.6), with four or five, or six whole ones, on two to four tiles a CU (28 x 10736 x 944 4.9,
+            // 5.4), and with five to eight whole ones on four to six; 215 random shapes 0.97 of the time
+            if (blocks <= 3 && tiles <= (whole_k ? 12 : 8) * cu) return false;
+            if (whole_k && blocks >= 5 && blocks <= 8 && tiles <= 6 * cu) return false;
             if (blocks <= 7 && resident(8, 3)) {}
             else if (resident(4, 4)) {}
             else tile(1, 4, 3, 1);
