@@ -852,10 +852,10 @@ static void pick_sparse_tile(Config& c, int m, int tiles16, int blocks, bool met
     } else if (c.mt == 2) {
         // three workgroups of 16-row tiles on a CU, or two of 32-row tiles - and two of either where the metadata comes by whole
         // lines, whose ring takes 4 KB of LDS more (28 x 10414 x 1024 5.20 us on 32-row tiles, 6.76 on 16; 25 x 9984 x 10240 25.1, 28.2)
-        // Beyond four tiles per CU only up to fifteen stages: with more, and just beyond four, 32-row tiles - on two waves from sixteen stages
-        // on - are ahead, as they read the activations half as often (32 x 20120 x 13440 56.5 us, 67.4 on 16 rows; 31 x 24148 x 22144
+        // Beyond four tiles per CU only up to fifteen stages, just beyond up to seven: with more 32-row tiles - on two waves from sixteen
+        // stages on - are ahead, as they read the activations half as often (32 x 20120 x 13440 56.5 us, 67.4 on 16 rows; 31 x 24148 x 22144
         // 90, 112; 152 random shapes 0.88 of the time)
-        const bool long_k = tiles16 > 4 * cu && (blocks >= 16 || tiles16 * 2 <= 9 * cu);
+        const bool long_k = tiles16 > 4 * cu && (blocks >= 16 || (blocks >= 8 && tiles16 * 2 <= 9 * cu));
         c.rg = !meta_lines && !long_k && (tiles16 + 3 * cu - 1) / (3 * cu) <= (tiles16 + 4 * cu - 1) / (4 * cu) ? 1 : 2;
         c.waves = c.rg == 2 && blocks >= 16 ? 2 : 1;
     } else {
