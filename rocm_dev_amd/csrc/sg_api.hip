@@ -851,7 +851,7 @@ static void pick_sparse_tile(Config& c, int m, int tiles16, int blocks, bool met
         c.rg = c.waves = blocks <= 4 ? 1 : 2;
     } else if (c.mt == 2) {
         // three workgroups of 16-row tiles on a CU, or two of 32-row tiles - and two of either where the metadata comes by whole
-        // lines, whose ring takes 4 KB of LDS more (28 x 10414 x 1024 5.20 us on 32-row tiles, 6.76 on 16; 25 x 9984 x 10240 25.1, 28.2)
+        // lines, whose ring takes 4 KB of LDS more (28 x 10414 x 1024 5.20 us on 32-row tiles, 6.76 on 16; 25 x 9984 x 10240 25.1, 28.2).
         // Beyond four tiles per CU only up to fifteen stages, just beyond up to seven: with more 32-row tiles - on two waves from sixteen
         // stages on - are ahead, as they read the activations half as often (32 x 20120 x 13440 56.5 us, 67.4 on 16 rows; 31 x 24148 x 22144
         // 90, 112; 152 random shapes 0.88 of the time)
@@ -1738,6 +1738,9 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
     if (m > 32 || k <= 256 || k > kSkinnyLineMaxK || n < 128 || n > kSkinnyLineMaxN || b_stride % 128 == 0) return false;
     const int tiles = (n + 15) / 16, blocks = (k + 255) / 256, cu = cu_count;
     const bool split_ok = k % 128 != 0, whole_k = k % 256 == 0;
+    // 19 or 22 whole blocks divide among no number of the record's waves that fits: at 9..16 rows it fetches the activations with every
+    // stage, and is 13 to 24 % behind wherever it was timed
+    const bool uneven_shares = blocks == 19 || blocks == 22;
     Config c{};
     c.engine = ENGINE_LDS;
     c.line = true;
@@ -1768,15 +1771,17 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
         if (uneven && m <= 8 && tiles <= 6 * cu && (b_stride == 8192 - 32 || b_stride == 8192 + 64 || b_stride == 8192 + 96)) return false;
         if (uneven && m <= 8 && k % 256 == 0 && b_stride == 8192 + 64) return false;    // (1 x 57344 x 8192 82 us against 94)
         if (tiles <= 2 * cu && b_stride == 8192 + 64) return false;
-        // of whole K blocks more such pitches: 40 random shapes 0.91 of the time on the record (7 x 21762 x 3584 on rows of 3616 0.86,
-        // 16 x 21804 x 4608 on rows of 4640 19.3 us against 21.9)
-        if (whole_k && tiles > 2 * cu && (b_stride == 3584 + 32 || b_stride == 4608 + 32 || b_stride == 5376 + 80 || b_stride == 8192 + 32 ||
-                                          (m > 8 && (b_stride == 8192 + 64 || b_stride == 8192 + 96))))
-            return false;
-        // Pitches of half a line: every other row begins on its line, and the ring asks for a quarter more instead of half.  With the
-        // activations resident the two are level in the mean (276 random shapes of whole K blocks 0.997), but 62 of them were more
-        // than 3 % behind here, up to 19 (6 x 37880 x 5376 on rows of 5440), by their pitch.
-        if (whole_k && tiles > 2 * cu && b_stride % 128 == 64 && ((m <= 8 && tiles > 12 * cu) || resident(4, 4))) return false;
+        // of whole K blocks more such pitches: 72 random shapes 0.91 of the time on the record (7 x 21762 x 3584 on rows of 3616 0.86,
+        // 6 x 37880 x 5376 on rows of 5440 32.5 us against 38.7, 15 x 35680 x 8192 on rows of 8224 52.5 against 76.4)
+        static const int meet[] = {3616, 4640, 4672, 5440, 5456, 7232, 8224, 9280, 16192};
+        if (whole_k && tiles > 2 * cu) {
+            for (const int pitch : meet)
+                if (b_stride == pitch) return false;
+            if (m > 8 && (b_stride == 8192 + 64 || b_stride == 8192 + 96)) return false;
+            // On pitches of half a line every other row begins on its line, and the ring asks for a quarter more instead of half: with
+            // the activations resident the record is ahead at 9..16 rows (70 random shapes 0.96 of the time), up to 8 the two are level
+            if (m > 8 && !uneven_shares && b_stride % 128 == 64 && resident(4, 4)) return false;
+        }
     }
     if (c.mt == 1) {
         if (tiles * 2 <= cu) {                       // few tiles: only long K, on K splits
@@ -1794,7 +1799,7 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
         } else if (blocks < (tiles <= 4 * cu ? 4 : 3)) {
             return false;
         } else if (tiles <= 4 * cu) {
-            // (21 random shapes of whole K blocks, up to 4 rows: 0.98 of the time on the record, 2 x 12000 x 1024 0.95)
+            // (35 random shapes of whole K blocks, up to 4 rows: 0.97 of the time on the record)
             if (whole_k && m <= 4 && (blocks == 4 || (blocks == 5 && tiles <= 3 * cu))) return false;
             if (resident(4, 4)) {}
             else if (m > 8 && tiles > 3 * cu) tile(2, 4, 3, 1);
@@ -1813,7 +1818,7 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
             if (blocks <= 6 && (resident(8, 4) || resident(8, 3))) {}
             else if (tiles > 12 * cu && resident(8, 3)) {}
             else if (resident(4, 4)) {
-                if (whole && (blocks >= 12 || (blocks == 11 && tiles <= 9 * cu)) && (tiles - 1) % (4 * cu) < cu) return false;
+                if (whole && (blocks >= 12 || (blocks == 11 && tiles <= 9 * cu)) && !(m > 8 && uneven_shares) && (tiles - 1) % (4 * cu) < cu) return false;
             } else if (whole_k && tiles <= (m > 8 ? (b_stride % 128 == 64 || blocks <= 34 ? 12 : 11) : 9) * cu && tiles > (m > 8 ? 8 : 6) * cu) {
                 // the record keeps the activations resident, or in registers, and here a second round of workgroups is begun: 0.92 of the
                 // time on 60 random shapes of 5..8 rows (5 x 27638 x 15616 on rows of 15680 72 us against 89), 0.90 on 16 of up to 4
