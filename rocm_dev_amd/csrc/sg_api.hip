@@ -1773,11 +1773,11 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
         if (tiles <= 2 * cu && b_stride == 8192 + 64) return false;
         // of whole K blocks more such pitches: 72 random shapes 0.91 of the time on the record (7 x 21762 x 3584 on rows of 3616 0.86,
         // 6 x 37880 x 5376 on rows of 5440 32.5 us against 38.7, 15 x 35680 x 8192 on rows of 8224 52.5 against 76.4)
-        static const int meet[] = {3616, 4640, 4672, 5440, 5456, 7232, 8224, 9280, 16192};
+        static const int meet[] = {3616, 4640, 4672, 5440, 5456, 7232, 8224};
         if (whole_k && tiles > 2 * cu) {
             for (const int pitch : meet)
                 if (b_stride == pitch) return false;
-            if (m > 8 && (b_stride == 8192 + 64 || b_stride == 8192 + 96)) return false;
+            if (m > 8 ? b_stride == 8192 + 64 || b_stride == 8192 + 96 : b_stride == 9216 + 64 || b_stride == 16128 + 64) return false;
             // On pitches of half a line every other row begins on its line, and the ring asks for a quarter more instead of half: with
             // the activations resident the record is ahead at 9..16 rows (70 random shapes 0.96 of the time), up to 8 the two are level
             if (m > 8 && !uneven_shares && b_stride % 128 == 64 && resident(4, 4)) return false;
@@ -1852,6 +1852,7 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
             else if (blocks < 20 && tiles <= 3 * cu) tile(1, 2, 4, 1);
             else tile(2, 4, 3, 1);
         } else {
+            if (b_stride == 3584 + 32 && whole_k && tiles > 7 * cu && tiles <= 8 * cu) return false;     // (17 x 30630 x 3584 21.2 us against 24.6)
             // (pitches of half a line, see above: 31 random shapes 0.97 of the time on the record)
             if (whole_k && b_stride % 128 == 64 && blocks >= 12 && tiles > 8 * cu && tiles <= 12 * cu) return false;
             // four waves a CU find four tiles at once: just beyond that the record is ahead, to five and a half
