@@ -861,13 +861,16 @@ static void pick_sparse_tile(Config& c, int m, int tiles16, int blocks, bool met
     } else {
         if (m > 8 ? tiles16 > 4 * cu : tiles16 >= 4 * cu && (m > 4 || blocks > 2 || tiles16 > 6 * cu)) c.rg = 2;
         c.waves = 1;
-        // 9..16 rows whose activations do not stay in LDS (below): two waves on 32-row tiles are ahead where a round of one-wave workgroups
-        // is begun - beyond three tiles per CU, and beyond six, where those found a third round - and from 28 stages on, where the
-        // metadata comes by whole lines between three and a half and six tiles per CU (15 x 27430 x 23808 86 us, 117; 16 x 14064 x
-        // 21248 41, 48; 160 random shapes 0.89 of the time)
-        if (m > 8 && (meta_lines ? tiles16 <= 6 * cu && (tiles16 * 2 > 7 * cu || (tiles16 > 3 * cu && blocks >= 36))
-                                 : tiles16 > 3 * cu && (tiles16 <= 4 * cu || tiles16 > 6 * cu || blocks >= 28)))
-            c.rg = c.waves = 2;
+        // 9..16 rows whose activations do not stay in LDS (below): 32-row tiles, on two waves from sixteen stages on, are ahead where a round
+        // of one-wave workgroups is begun - beyond three tiles per CU, and beyond six, where those found a third round - and from 28
+        // stages on; where the metadata comes by whole lines from three to six tiles per CU, up to four not with 16 to 27 stages
+        // (15 x 27430 x 23808 86 us, 117; 16 x 14064 x 21248 41, 48; 15 x 15786 x 7168 13.7 on one wave, 16.8 on two; 867 random
+        // shapes of 9..16 rows 0.90 of the time)
+        if (m > 8 && (meta_lines ? tiles16 > 3 * cu && tiles16 <= 6 * cu && (tiles16 > 4 * cu || blocks < 16 || blocks >= 28)
+                                 : tiles16 > 3 * cu && (tiles16 <= 4 * cu || tiles16 > 6 * cu || blocks >= 28))) {
+            c.rg = 2;
+            c.waves = blocks >= 16 ? 2 : 1;
+        }
         // up to 8 rows beyond six tiles per CU as well, but level there at 5 to 8 where the metadata does not come by whole lines
         // (6 x 28004 x 24576 78.7 us, 100; 2 x 27050 x 20480 58.5, 64.3)
         if (m <= 8 && tiles16 > 6 * cu && blocks >= 16 && (m <= 4 || meta_lines)) c.rg = c.waves = 2;

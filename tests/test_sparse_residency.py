@@ -44,7 +44,7 @@ def test_sixteen_row_tiles_only_where_three_workgroups_fit_a_cu(fake):
 # other line, us: 56.5 / 67.4, 40.6 / 42.9, 77.9 / 90.2; 86 / 117, 82.5 / 96, 41 / 48; 66.9 / 72.6, 78.7 / 100
 WAVES = {(32, 20120, 13440): (2, 2), (23, 18202, 9600): (2, 2), (21, 18168, 25088): (2, 2), (32, 17646, 4352): (2, 1), (22, 21052, 7296): (1, 1), (21, 18294, 1280): (1, 1),
          (15, 27430, 23808): (2, 2), (11, 25888, 23808): (2, 2), (16, 14064, 21248): (2, 2), (12, 17654, 12928): (2, 1), (13, 11224, 25600): (1, 1),
-         (15, 20000, 12288): (2, 2), (11, 26000, 12288): (2, 1), (12, 13200, 12288): (1, 1), (12, 13200, 20480): (2, 2),
+         (15, 20000, 12288): (2, 2), (11, 26000, 12288): (2, 1), (12, 13200, 12288): (1, 1), (15, 15786, 7168): (2, 1), (15, 13732, 7168): (2, 1), (10, 14850, 11264): (1, 1), (12, 13200, 20480): (2, 2),
          (3, 25732, 24576): (2, 2), (6, 28004, 24576): (2, 2), (7, 28004, 24448): (2, 1), (6, 20480, 24576): (2, 1), (2, 26624, 7680): (2, 1)}
 
 
