@@ -1822,11 +1822,11 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
             else if (tiles > 12 * cu && resident(8, 3)) {}
             else if (resident(4, 4)) {
                 if (whole && (blocks >= 12 || (blocks == 11 && tiles <= 9 * cu)) && !(m > 8 && uneven_shares) && (tiles - 1) % (4 * cu) < cu) return false;
-            } else if (whole_k && tiles <= (m > 8 ? (b_stride % 128 == 64 || blocks <= 34 ? 12 : 11) : 9) * cu && tiles > (m > 8 ? 8 : 6) * cu) {
+            } else if (whole_k && tiles <= (m > 8 ? (b_stride % 128 == 64 || blocks <= 34 ? 12 : 10) : 9) * cu && tiles > (m > 8 ? 8 : 6) * cu) {
                 // the record keeps the activations resident, or in registers, and here a second round of workgroups is begun: 0.92 of the
                 // time on 60 random shapes of 5..8 rows (5 x 27638 x 15616 on rows of 15680 72 us against 89), 0.90 on 16 of up to 4
                 // (4 x 30596 x 28928 140, 164), 0.95 on 285 of 9..16 (14 x 36870 x 6400 on rows of 6448 39.5, 53;
-                // beyond eleven tiles a CU level with more than 34 blocks, but on pitches of half a line)
+                // beyond ten tiles a CU level with more than 34 blocks, but on pitches of half a line)
                 return false;
             } else if (m > 8) tile(1, 4, 3, 1);
             else tile(1, 2, 4, 1);

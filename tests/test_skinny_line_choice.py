@@ -89,7 +89,7 @@ def test_the_record_stays_where_it_was_timed_ahead(m, n, k, pad):
                                        (8, 8192, 8192, 32), (24, 8192, 8192, 64), (8, 14336, 4128, 0), (8, 10240, 16448, 0), (8, 33794, 2560, 16),
                                        (8, 37890, 3072, 48), (8, 32768, 4096, 16), (2, 38914, 4096, 16), (8, 33794, 3600, 0), (30, 22458, 2816, 16),
                                        (14, 14698, 8192, 16), (2, 47816, 4000, 128), (8, 54274, 4352, 16), (22, 31862, 4096, 16), (8, 39590, 15360, 80),
-                                       (14, 32768, 6400, 48), (14, 51202, 6400, 48), (14, 46000, 9216, 16), (4, 22000, 24832, 16), (4, 38000, 24832, 16), (2, 38000, 2816, 16),
+                                       (14, 32768, 6400, 48), (14, 51202, 6400, 48), (14, 46000, 9216, 16), (15, 41982, 12544, 32), (4, 22000, 24832, 16), (4, 38000, 24832, 16), (2, 38000, 2816, 16),
                                        (7, 21762, 3584, 48), (16, 21804, 4608, 48), (15, 49302, 8192, 112), (6, 37880, 5392, 48), (12, 23374, 8960, 64), (24, 30000, 6400, 64),
                                        (14, 24512, 16128, 64), (16, 22126, 9216, 64), (3, 20792, 12544, 64), (11, 36524, 4864, 16), (13, 36492, 5632, 80), (16, 27498, 5632, 64),
                                        (2, 17000, 1024, 16), (6, 12000, 1024, 48), (29, 33000, 704, 0), (26, 50000, 768, 32), (26, 9000, 688, 0), (26, 12000, 1520, 0), (24, 25000, 1280, 80)])
