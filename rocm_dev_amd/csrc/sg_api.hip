@@ -828,8 +828,8 @@ static int launch_sparse_engine(const Config& c, StreamArgs a, const uint8_t* me
 // Row tiles, waves, ring slots and K splits of sparse24_gemm_kernel for up to 32 rows, as read off timings of 1, 2 and 4 of the
 // first two, 2..4 slots and up to eight splits on 139 random shapes (1..32 rows, n of 64..32768, k of 512..28672; every side
 // timed in turn, cold weights): 0.885 of the time of what ran before in the geometric mean, the best of them 0.878, none behind
-// by more than 3 %, of which the rule takes up to six splits; on 250 other shapes 0.92 eagerly, where the short ones are the host's time, and
-// 0.95 recorded, without splits, at most 5 % behind.  Few tiles and a long K: splits until the CUs have one each (14 x 198 x 24576 12.0 -> 7.2 us,
+// by more than 3 %, of which the rule takes up to six splits; on 983 other shapes, recorded and so without splits, 0.88, one of them
+// more than 3 % behind (at most 4), on 1721 eagerly 0.80.  Few tiles and a long K: splits until the CUs have one each (14 x 198 x 24576 12.0 -> 7.2 us,
 // 25 x 930 x 24576 17.7 -> 9.4, 19 x 1378 x 27776 20.5 -> 13.9); a K too short for one wave's ring on two of them (9 x 328 x 6144
 // 5.74 -> 4.67, 2 x 2308 x 7168 6.09 -> 4.84); 17..32 rows on one to two tiles per CU on 32-row tiles, which share the
 // activations (23 x 7542 x 10240 18.8 -> 15.2), or, up to four stages, on one wave (24 x 4464 x 1024 6.41 -> 3.83); beyond two
@@ -1727,8 +1727,8 @@ static bool ring_split_config(const Config& record, int m, int n, int k, int cu_
 // (waves, ring slots, row tiles, K splits) against that record on 510 random shapes, n of 128..65536, K of 272..32768: 0.89 of the time
 // before in the geometric mean on the 231 that it took, at most 3.4 % behind.  Denser samples of single ranges, timed by themselves and one
 // behind the other, then found where the record is ahead (skinny_record_stays and the early returns below).  Of others that it takes
-// now, 300 run in 0.90 of the time before, four more than 3 % behind eagerly (at most 5.6) and seven recorded (at most 8); 300 of whole K
-// blocks on padded rows, whose records are the better ones, in 0.93, nineteen more than 3 % behind (at most 13).
+// now, 790 run in 0.90 of the time before, recorded, eleven of them more than 3 % behind (at most 7); 3246 of whole K blocks on padded
+// rows, whose records are the better ones, in 0.91, 121 more than 3 % behind and 28 more than 6 (at most 23, by their pitch).
 // 32 x 32768 x 4112 35.7 -> 26.7 us, 1 x 16384 x 4112 15.5 -> 13.8, 13 x 20660 x 9664 57.5 -> 35.6,
 // 5 x 39438 x 4016 35.6 -> 28.1, 28 x 13116 x 6960 25.0 -> 20.7, 5 x 2434 x 21584 18.0 -> 13.5, 1 x 8522 x 2832 7.3 -> 6.8.
 // What it leaves alone - weights of a megabyte or two, two K blocks, few tiles with a K below about 7000 at up to 16 rows - is
