@@ -1763,7 +1763,7 @@ static bool skinny_line_config(int m, int n, int k, int b_stride, int cu_count, 
     // (K of 4096 1.10) and 1.25 to 1.02, 8224 1.08 to 1.01 (K of 8192 1.20) and 1.41 to 1.14 (2 x 18500 x 8224 by itself 27.6 us against
     // 41.6), 16448 1.15 to 1.02 and 1.27 to 1.15, 8160, 8256 and 8288 1.07 to 1.00 and 1.18 to 1.01, but 0.97 on the last, as 4128 is with
     // a K below its pitch (2 x 47816 x 4000 46.6 us against 41.4).  In between
-    // four waves a CU have a tile each, and the two are level.  From 9 rows on only 4128 is behind (14 x 18500 x 8224 0.71), and at 5 to 8
+    // four waves a CU have a tile each, and the two are level.  From 9 rows on, with K as long as the pitch, only 4128 is behind (14 x 18500 x 8224 0.71), and at 5 to 8
     // rows 16448 no more.  8256 is behind on one to two tiles a CU as well, 1.05 to 1.15.  (Maps of pitches 16 to 416 bytes off the
     // multiples of 1024 up to 24576, and of twelve pitches on 2048 to 57344 weight rows: the others are 0.6 to 1.07.)
     if (c.mt == 1 && tiles > cu) {
